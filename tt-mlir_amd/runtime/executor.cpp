@@ -50,6 +50,7 @@ struct ProgramContext {
   // [B, H, S, D] view of.  The id is not in the pool; the attention kernel reads the source in place.
   std::unordered_map<std::uint32_t, Tensor> headViews;
   std::set<std::uint32_t> skip;
+  std::optional<Layout> layoutOnTheWay;   // of the result of a to_layout that the from_device behind it brings about
 
   Tensor &get(const fb::Table &ref, const char *what) {
     TTRT_ASSERT(static_cast<bool>(ref), std::string("missing tensor reference: ") + what);
@@ -204,14 +205,15 @@ OpRefs opRefs(const fb::Table &operation) {
 Tensor onDevice(ProgramContext &ctx, const Tensor &t) { return t.handle->storage == StorageType::Device ? t : toDevice(t, ctx.dev); }
 
 // a device tensor in (layout, dtype); never frees its argument
-Tensor as(ProgramContext &ctx, const Tensor &t, TensorLayout layout, DataType dtype) { return convertOnDevice(onDevice(ctx, t), layout, dtype); }
+Tensor as(ProgramContext &ctx, const Tensor &t, TensorLayout layout, DataType dtype) {
+  return t.handle->storage == StorageType::Host ? uploadAs(t, ctx.dev, layout, dtype) : convertOnDevice(t, layout, dtype);
+}
 
 Tensor convertTo(ProgramContext &ctx, const Tensor &t, const Layout &target) {
-  Tensor cur = t;
-  const bool change = cur.handle->layout != target.layout || cur.handle->dtype != target.dataType;
-  if (change || target.storageType == StorageType::Device) cur = as(ctx, cur, target.layout, target.dataType);
-  if (target.storageType == StorageType::Host && cur.handle->storage == StorageType::Device) cur = fromDevice(cur);
-  return cur;
+  const bool change = t.handle->layout != target.layout || t.handle->dtype != target.dataType;
+  if (target.storageType == StorageType::Device) return as(ctx, t, target.layout, target.dataType);
+  if (t.handle->storage == StorageType::Device) return fetchAs(t, target.layout, target.dataType);
+  return change ? fromDevice(as(ctx, t, target.layout, target.dataType)) : t;
 }
 
 std::vector<std::int64_t> rowMajorStrides(const std::vector<std::uint32_t> &shape) {
@@ -335,13 +337,32 @@ std::string matmulActivation(const fb::Table &op, int configTypeSlot, int config
   return std::string(op.string(activationSlot));
 }
 
+std::uint32_t refId(const fb::Table &ref);
+// The result `ref` of the operation at hand is read by the next operation of the program, of this type, and by nothing else.
+bool onlyFeedsNext(ProgramContext &ctx, const fb::Table &ref, OpType type, int operandSlot) {
+  const std::uint32_t next = ctx.opIndex + 1;
+  if (!ctx.fuseViews || next >= ctx.ops.size()) return false;
+  if (static_cast<OpType>(ctx.ops[next].scalar<std::uint8_t>(schema::Operation::f_type_type, 0)) != type) return false;
+  const auto use = ctx.uses.find(refId(ref));
+  return use != ctx.uses.end() && use->second == 1 && refId(ctx.ops[next].table(schema::Operation::f_type).table(operandSlot)) == refId(ref);
+}
+
 // ---- layout ops (runtime/lib/ttnn/operations/layout/*.cpp)
+// Host tensors change layout on their way over PCIe: a to_device whose result only feeds the next to_layout leaves the tensor
+// on the host for it, and a to_layout whose result only feeds the next from_device leaves its operand as it is and hands it the
+// layout (`layoutOnTheWay`); the tilize then reads the staged host memory, the untilize stores into the host tensor.
 void runToLayout(const fb::Table &op, ProgramContext &ctx) {
   Tensor in = ctx.get(op.table(schema::ToLayoutOp::f_in), "to_layout in");
   auto outRef = op.table(schema::ToLayoutOp::f_out);
   Layout want = layoutFromTensorRef(outRef);
   want.layout = static_cast<TensorLayout>(op.scalar<std::uint16_t>(schema::ToLayoutOp::f_layout, 0));
   if (op.has(schema::ToLayoutOp::f_dtype)) want.dataType = static_cast<DataType>(op.scalar<std::uint16_t>(schema::ToLayoutOp::f_dtype, 0));
+  if (in.handle->storage == StorageType::Device && want.storageType == StorageType::Device &&
+      onlyFeedsNext(ctx, outRef, OpType::FromDeviceOp, schema::FromDeviceOp::f_in)) {
+    ctx.layoutOnTheWay = want;
+    ctx.put(outRef, in);
+    return;
+  }
   ctx.put(outRef, convertTo(ctx, in, want));
 }
 void runTypecast(const fb::Table &op, ProgramContext &ctx) {
@@ -355,10 +376,17 @@ void runTypecast(const fb::Table &op, ProgramContext &ctx) {
 }
 void runToDevice(const fb::Table &op, ProgramContext &ctx) {
   Tensor in = ctx.get(op.table(schema::ToDeviceOp::f_in), "to_device in");
-  ctx.put(op.table(schema::ToDeviceOp::f_out), onDevice(ctx, in));
+  auto outRef = op.table(schema::ToDeviceOp::f_out);
+  ctx.put(outRef, onlyFeedsNext(ctx, outRef, OpType::ToLayoutOp, schema::ToLayoutOp::f_in) ? in : onDevice(ctx, in));
 }
 void runFromDevice(const fb::Table &op, ProgramContext &ctx) {
   Tensor in = ctx.get(op.table(schema::FromDeviceOp::f_in), "from_device in");
+  if (ctx.layoutOnTheWay.has_value()) {
+    const Layout l = *ctx.layoutOnTheWay;
+    ctx.layoutOnTheWay.reset();
+    ctx.put(op.table(schema::FromDeviceOp::f_out), fetchAs(in, l.layout, l.dataType));
+    return;
+  }
   ctx.put(op.table(schema::FromDeviceOp::f_out), in.handle->storage == StorageType::Device ? fromDevice(in) : in);
 }
 void runToMemoryConfig(const fb::Table &op, ProgramContext &ctx) {
@@ -2181,6 +2209,7 @@ void runExecuteTrace(const fb::Table &op, ProgramContext &ctx) {
 // dst <- src for tensors of one shape; src is brought to dst's layout and dtype first (on the device)
 void overwriteTensor(ProgramContext &ctx, Tensor &dst, const Tensor &src, const char *what) {
   TTRT_ASSERT(dst.handle->shape == src.handle->shape, std::string(what) + ": shape mismatch");
+  if (src.handle->storage == StorageType::Host && dst.handle->storage == StorageType::Device && uploadInto(src, dst)) return;
   Tensor conv = src;
   if (conv.handle->layout != dst.handle->layout || conv.handle->dtype != dst.handle->dtype)
     conv = as(ctx, conv, dst.handle->layout, dst.handle->dtype);
@@ -2543,7 +2572,7 @@ void updateTensorInPool(CallbackContext cc, std::uint32_t globalId, Tensor src) 
   Layout want = getTensorLayout(dst);
   Tensor conv = src;
   if (want.storageType == StorageType::Device || conv.handle->layout != want.layout || conv.handle->dtype != want.dataType)
-    conv = convertOnDevice(conv.handle->storage == StorageType::Device ? conv : toDevice(conv, ctx->dev), want.layout, want.dataType);
+    conv = as(*ctx, conv, want.layout, want.dataType);
   if (want.storageType == StorageType::Host && conv.handle->storage == StorageType::Device) conv = fromDevice(conv);
   memcpy(dst, conv);
   // new contents, new version (runtime/lib/ttnn/runtime.cpp:2588): a const-eval result or a trace slot computed from the

@@ -54,6 +54,11 @@ struct DeviceState {
   int deviceId = 0;
   void *stream = nullptr;  // hipStream_t: all work of this device is ordered on it
   bool open = false;
+  // Page-locked block through which host tensors go up (runtime.cpp, stage()): filled from `stagingHead` on, free again from
+  // the start after every wait for the stream.  `kernelsReachHost`: kernels may read and write page-locked memory.
+  void *staging = nullptr;
+  size_t stagingHead = 0;
+  bool kernelsReachHost = false;
   // Work on the stream of a device is issued by one thread at a time: submit, toLayout, toHost, wait and device copies
   // take this lock (recursive: a hook running inside submit may call toHost).  A capture in progress is thereby never
   // interleaved with the launches or the synchronisation of another thread.
@@ -131,6 +136,12 @@ Tensor convertOnDevice(const Tensor &src, TensorLayout layout, DataType dtype);
 std::vector<Tensor> invokeCpuOpOf(const Binary &binary, std::uint32_t programIndex, OpContext opContext, const std::vector<Tensor> &inputs);
 Tensor toDevice(const Tensor &hostTensor, const std::shared_ptr<DeviceState> &dev);
 Tensor fromDevice(const Tensor &deviceTensor);
+// the same together with a change of layout and data type: one pass over the host memory where one kernel can do it
+Tensor uploadAs(const Tensor &hostTensor, const std::shared_ptr<DeviceState> &dev, TensorLayout layout, DataType dtype);
+Tensor fetchAs(const Tensor &deviceTensor, TensorLayout layout, DataType dtype);
+// a host tensor's values into the memory of a device tensor of the same shape, in the latter's layout and data type; false
+// (and nothing done) when that takes more than one launch
+bool uploadInto(const Tensor &hostTensor, const Tensor &deviceTensor);
 
 Layout layoutFromTensorRef(const fb::Table &tensorRef);
 std::vector<std::uint32_t> shapeFromTensorRef(const fb::Table &tensorRef);
