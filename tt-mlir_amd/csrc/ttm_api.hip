@@ -2,6 +2,7 @@
 #include <stdarg.h>
 #include <string.h>
 
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <string>
@@ -23,19 +24,21 @@ int ttm_set_error(int code, const char *fmt, ...) {
 TTM_EXPORT const char *ttm_last_error(void) { return g_err; }
 
 // ---- options
-static std::mutex g_opt_mu;
-static std::map<std::string, int> &opts() {
-  static std::map<std::string, int> m = {
-      {"tilize_variant", 0}, {"untilize_variant", 0}, {"pack_variant", 0}, {"unpack_variant", 0},
-      {"rowwise_variant", 0}, {"sdpa_variant", 0}, {"linear_variant", 0}, {"linear_small_m_max", 64}, {"linear_ntw", 0}, {"linear_split_k", 0}, {"linear_two_part", 0}, {"linear_decode_split", 0}, {"linear_decode_wide", 0}, {"linear_glu_main", 0}, {"linear_decode_variant", 0}, {"linear_two_pass", 0}, {"linear_img_variant", 0},
-      {"check_extents", getenv("TTMLIR_AMD_CHECK_EXTENTS") && getenv("TTMLIR_AMD_CHECK_EXTENTS")[0] == '1' ? 1 : 0},
-  };
-  return m;
-}
-int ttm_option(const char *name) {
-  std::lock_guard<std::mutex> g(g_opt_mu);
-  auto it = opts().find(name);
-  return it == opts().end() ? 0 : it->second;
+namespace {
+struct Option {
+  const char *name;
+  std::atomic<int> value;
+};
+Option g_options[] = {
+    {"tilize_variant", {0}}, {"untilize_variant", {0}}, {"pack_variant", {0}}, {"unpack_variant", {0}},
+    {"rowwise_variant", {0}}, {"sdpa_variant", {0}}, {"linear_variant", {0}}, {"linear_small_m_max", {64}}, {"linear_ntw", {0}}, {"linear_split_k", {0}}, {"linear_two_part", {0}}, {"linear_decode_split", {0}}, {"linear_decode_wide", {0}}, {"linear_glu_main", {0}}, {"linear_decode_variant", {0}}, {"linear_two_pass", {0}}, {"linear_img_variant", {0}},
+    {"check_extents", {getenv("TTMLIR_AMD_CHECK_EXTENTS") && getenv("TTMLIR_AMD_CHECK_EXTENTS")[0] == '1' ? 1 : 0}},
+};
+}  // namespace
+std::atomic<int> *ttm_option_slot(const char *name) {
+  for (Option &o : g_options)
+    if (strcmp(o.name, name) == 0) return &o.value;
+  return nullptr;
 }
 // ---- operand extents
 bool ttm_check_extents_on() { return ttm_option("check_extents") != 0; }
@@ -59,18 +62,16 @@ int TtmExtentChecker::operator()(const char *what, const void *p, int64_t bytes,
 
 TTM_EXPORT int ttm_set_option(const char *name, int value) {
   TTM_REQUIRE(name != nullptr, "ttm_set_option: null name");
-  std::lock_guard<std::mutex> g(g_opt_mu);
-  auto it = opts().find(name);
-  if (it == opts().end()) return ttm_set_error(TTM_ERR_INVALID, "ttm_set_option: unknown option '%s'", name);
-  it->second = value;
+  std::atomic<int> *slot = ttm_option_slot(name);
+  if (!slot) return ttm_set_error(TTM_ERR_INVALID, "ttm_set_option: unknown option '%s'", name);
+  slot->store(value);
   return TTM_OK;
 }
 TTM_EXPORT int ttm_get_option(const char *name, int *value) {
   TTM_REQUIRE(name != nullptr && value != nullptr, "ttm_get_option: null argument");
-  std::lock_guard<std::mutex> g(g_opt_mu);
-  auto it = opts().find(name);
-  if (it == opts().end()) return ttm_set_error(TTM_ERR_INVALID, "ttm_get_option: unknown option '%s'", name);
-  *value = it->second;
+  std::atomic<int> *slot = ttm_option_slot(name);
+  if (!slot) return ttm_set_error(TTM_ERR_INVALID, "ttm_get_option: unknown option '%s'", name);
+  *value = slot->load();
   return TTM_OK;
 }
 

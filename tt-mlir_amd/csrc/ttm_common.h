@@ -4,6 +4,8 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <atomic>
+
 #include "ttmlir_amd_hip.h"
 #include "ttm_extents.h"
 
@@ -31,7 +33,14 @@ int ttm_set_error(int code, const char *fmt, ...) __attribute__((format(printf, 
 
 #define TTM_LAUNCH_CHECK() TTM_HIP(hipGetLastError())
 
-int ttm_option(const char *name);  // 0 when unset
+// Value of an option.  The name is looked up once per call site: an entry point reads up to a dozen of them per call, and as map
+// look-ups under a lock they were a third of the host time of a small launch.
+std::atomic<int> *ttm_option_slot(const char *name);
+#define ttm_option(name)                                                     \
+  ([&]() -> int {                                                            \
+    static std::atomic<int> *const slot_ = ttm_option_slot(name);            \
+    return slot_->load(std::memory_order_relaxed);                           \
+  }())
 
 // Opt-in host-side check of operand extents (option "check_extents", or TTMLIR_AMD_CHECK_EXTENTS=1 in the environment):
 // before anything is launched, the bytes the kernels touch behind every pointer argument (ttm_extents.h) must lie inside
