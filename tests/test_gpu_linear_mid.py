@@ -1,0 +1,72 @@
+"""The mid-size linear kernel under every plan it can take (row tiles and K shares per workgroup, slices of K), at the edges of its
+tiles: ragged rows, columns and K, fewer k-tiles than shares, one column tile, more rows than a workgroup holds; groups and the
+gated form against separate launches of the same plan.  Against the CPU oracle on the weights the device multiplies; outputs are
+O(1), so one bf16 step is at most 2^-6 and the accumulation order adds less than that (2^-5 as in the other linear tests)."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from ttmlir_amd import datagen
+from test_gpu_linear import check, metrics, pack_weight, run_linear, tilize_dev, untilize_dev  # noqa: F401 (metrics: fixture)
+
+pytestmark = pytest.mark.gpu
+PLANS = [8101, 8102, 8201, 8202, 4201, 4204, 8401, 8404]
+
+
+@pytest.fixture
+def plan(hip, request):
+    hip.set_option("linear_mid", request.param)
+    yield request.param
+    hip.set_option("linear_mid", 0)
+
+
+@pytest.mark.parametrize("plan", PLANS, indirect=True)
+@pytest.mark.parametrize("wfmt_name", ["bfp8", "bfp4", "bf16", "bf16_nk"])
+@pytest.mark.parametrize("M,K,N,act,bias", [(33, 37 * 32 + 11, 5 * 32 + 7, "silu", True), (161, 70, 32, None, False), (1, 1030, 100, "gelu", True)])
+def test_every_plan_against_the_oracle(hip, dev, orc, metrics, plan, wfmt_name, M, K, N, act, bias):  # noqa: F811
+    wfmt = {"bfp8": hip.BFP8B, "bfp4": hip.BFP4B}.get(wfmt_name, hip.BF16)
+    a = datagen.randn((M, K), seed=M, dtype=torch.bfloat16)
+    w = datagen.randn((K, N), seed=N, std=K ** -0.5)
+    b = datagen.randn((N,), seed=7, std=0.5, dtype=torch.bfloat16) if bias else None
+    nk = wfmt_name == "bf16_nk"
+    got, w_eff = run_linear(hip, dev, a, w.t().contiguous() if nk else w, b, act, wfmt, transpose_w=nk)
+    check(orc, metrics, got, a, w_eff, b, act, max_abs=2.0 ** -5)
+
+
+@pytest.mark.parametrize("plan", [8101, 8202, 4201, 8404], indirect=True)
+def test_batches_and_groups_equal_separate_launches(hip, dev, plan):
+    M, K, Ns = 70, 300, (200, 40, 96)
+    a = datagen.randn((M, K), seed=1, dtype=torch.bfloat16)
+    ws = [datagen.randn((K, N), seed=2 + i, std=0.05) for i, N in enumerate(Ns)]
+    want = [run_linear(hip, dev, a, w, None, None, hip.BFP8B)[0] for w in ws]
+    at, wt = tilize_dev(hip, a, dev), [pack_weight(hip, w, hip.BFP8B, dev) for w in ws]
+    outs = [torch.full((96 * ((N + 31) // 32 * 32),), float("nan"), dtype=torch.bfloat16, device=dev) for N in Ns]
+    arr = lambda t, v: (t * len(v))(*v)
+    hip.call("ttm_linear_group", hip.ptr(at), 3, arr(ctypes.c_void_p, [t.data_ptr() for t in wt]), hip.BFP8B,
+             arr(ctypes.c_void_p, [t.data_ptr() for t in outs]), arr(ctypes.c_int64, Ns), None, M, K, hip.current_stream())
+    for o, N, w in zip(outs, Ns, want):
+        assert torch.equal(untilize_dev(hip, o, (M, N), dev).cpu(), w)
+    three, _ = run_linear(hip, dev, a.expand(3, M, K), datagen.randn((3, K, 64), seed=9, std=0.05), None, None, hip.BFP4B)
+    for i in range(3):
+        one, _ = run_linear(hip, dev, a, datagen.randn((3, K, 64), seed=9, std=0.05)[i], None, None, hip.BFP4B)
+        assert torch.equal(three[i], one)
+
+
+@pytest.mark.parametrize("plan", [4201, 4401], indirect=True)
+@pytest.mark.parametrize("M,K,N", [(65, 64, 104), (65, 512, 5760)])
+def test_gated_form_against_the_oracle(hip, dev, orc, plan, M, K, N):
+    a = datagen.randn((M, K), seed=1, dtype=torch.bfloat16)
+    ws = [datagen.randn((K, N), seed=2 + i, std=K ** -0.5) for i in range(2)]
+    at, wt = tilize_dev(hip, a, dev), [pack_weight(hip, w, hip.BFP8B, dev) for w in ws]
+    out = torch.full(((M + 31) // 32 * 32 * ((N + 31) // 32 * 32),), float("nan"), dtype=torch.bfloat16, device=dev)
+    assert hip.lib().ttm_linear_glu_supported(hip.BFP8B, M, N, K) == 1
+    hip.call("ttm_linear_glu", hip.ptr(at), hip.ptr(wt[0]), hip.ptr(wt[1]), hip.BFP8B, hip.ptr(out), M, N, K, hip.ACT["silu"], 0, hip.current_stream())
+    got = untilize_dev(hip, out, (M, N), dev).float().cpu().numpy()
+    q = lambda w: orc.bfp_unpack(orc.bfp_pack(w.numpy(), 8), w.shape, 8)
+    r, an = orc.round_bf16, a.float().numpy()
+    ref = r(r(orc.linear(an, q(ws[0]), None, "silu")) * r(orc.linear(an, q(ws[1]))))
+    # two factors of up to 4, each within a bf16 step (2^-6 at magnitudes below 4) of the oracle's, and the product's own step
+    assert np.max(np.abs(got - ref)) <= 2.0 ** -3
+    assert np.mean(got == ref) >= 0.97

@@ -1,0 +1,208 @@
+// What the kernels of ttm_linear.hip and ttm_linear_mid.hip share: launch arguments, epilogue pieces, operand helpers.
+#pragma once
+#include <type_traits>
+
+#include "ttm_common.h"
+#include "ttm_math.h"
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+enum { WF_BFP8 = 0, WF_BFP4 = 1, WF_BF16_KN = 2, WF_BF16_NK = 3 };
+
+struct LinearArgs {
+  const uint8_t *A;     // bf16, tile order, [Mt*32, Kt*32]
+  const uint8_t *W;     // weights, format WF_*
+  const uint16_t *bias; // bf16 or null
+  uint8_t *C;           // bf16, tile order, [Mt*32, Nt*32]
+  int Mt, Nt, Kt;       // extents in tiles
+  int act, bias_tiled;
+  int64_t a_batch, w_batch, c_batch;  // byte strides between batch entries (w_batch 0 = shared weights)
+  int m_blocks, n_blocks;
+  int ntw;                            // block-float main kernel: column tiles per wavefront (block width / 2)
+  int nt_split, n_blocks1, ntw2;      // two-part grid: blocks [0, n_blocks1) cover column tiles [0, nt_split) at width ntw,
+                                      // the rest cover [nt_split, Nt) at width ntw2; nt_split = 0: one part
+  int k_slice;                        // k-tiles per grid.y slice (split-K); Kt when the reduction is not split
+  float *partial;                     // split-K: fp32 partial sums [slices][Mt * Nt * 1024] in output tile order
+  int img_zero_step;                  // two-pass launch: W points at the dequantised images, this step index holds zeros
+  // group launch (group_n >= 2): several weight matrices [K, N_i] applied to the same activations, each with its own
+  // output; W / C / Nt above describe the virtual concatenation (Nt = sum of the members' column tiles) and are not
+  // dereferenced.  Each member may have its own activation; no bias, tail or batch in a group.
+  int group_n;
+  const uint8_t *gW[4];
+  uint8_t *gC[4];
+  int gNt[4];
+  int gAct[4];                        // per-member activation
+  int glu;                            // gated pair (decode kernel only): C = gC[0] = act0(A gW[0]) x act1(A gW[1]), both [K, gNt[0] * 32]
+  int tail;                           // 0 none, 1 add, 2 multiply: element-wise tail with a tensor laid out like the output
+  int64_t tail_delta;                 // byte distance from an output element to its tail operand
+  int plan_batch;                     // host side only: batch entries the launch plan counts (a pair of matrices plans as one alone)
+  const struct QkvFinishArgs *qkv;    // host side only: the decode launch leaves partial sums and ttm_qkv_finish_k ends it
+  const struct NormFinishArgs *norm;  // host side only: ... and the RMSNorm kernel ends it (residual add, then the norm)
+};
+
+// x1 = residual + projection (stored to sum_out), then out = rms_norm(x1): the operands of the second launch
+struct NormFinishArgs {
+  const void *residual, *weight, *bias;
+  int weight_layout, bias_layout;
+  void *sum_out, *out;
+  int64_t rows, cols;
+  float eps;
+};
+
+// What follows the Q, K and V projections of a decode step (one token per user): head split, rotary embedding of q and k
+// at the cos / sin row `cos_row`, q to its own tensor, k and v into the cache row of position *index.
+struct QkvFinishArgs {
+  const float *partial;               // [slices][per] fp32 in tile order over the concatenation q | k | v (one row tile)
+  int slices;
+  int64_t per;
+  int users, heads, heads_pad, kv_heads, dim;
+  const uint16_t *cosc, *sinc;        // [.., dim] bf16 tiles
+  int64_t cos_row;
+  uint16_t *q_out;                    // [1, users, heads, dim] bf16 tiles
+  uint16_t *k_cache, *v_cache;        // [cache users, kv_heads, max_seq, dim] bf16 tiles
+  int64_t max_seq, seq_pad, batch_offset;
+  const int32_t *index;               // device memory: the position all users write
+};
+
+// The member of a group launch that owns column unit `u`, where a unit is `unit_tiles` column tiles and every member's
+// units are numbered one after another (a member's last unit may be partial).  Constant indices only: the arrays stay in
+// scalar registers.
+struct GroupMember {
+  const uint8_t *W;
+  uint8_t *C;
+  int Nt, local, tile_base, act;   // column tiles, unit index inside the member, first column tile in the concatenation
+};
+__device__ __forceinline__ GroupMember group_member(const LinearArgs &p, int u, int unit_tiles) {
+  GroupMember m = {p.gW[0], p.gC[0], p.gNt[0], u, 0, p.gAct[0]};
+  int start = 0, tiles = 0;
+  bool found = false;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (j < p.group_n) {
+      const int n = (p.gNt[j] + unit_tiles - 1) / unit_tiles;
+      if (!found && (u < start + n || j == p.group_n - 1)) {
+        found = true;
+        m.W = p.gW[j]; m.C = p.gC[j]; m.Nt = p.gNt[j]; m.local = u - start; m.tile_base = tiles; m.act = p.gAct[j];
+      }
+      start += n; tiles += p.gNt[j];
+    }
+  }
+  return m;
+}
+
+template <int ACT>
+__device__ __forceinline__ float apply_act(float x) {
+  if (ACT == TTM_ACT_GELU) return ttm_gelu_fast(x);
+  if (ACT == TTM_ACT_SILU) return ttm_silu(x);
+  if (ACT == TTM_ACT_SIGMOID) return ttm_sigmoid(x);
+  if (ACT == TTM_ACT_RELU) return ttm_max(x, 0.0f);   // keeps NaN, as arith.maximumf does
+  return x;
+}
+
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+// two floats -> packed bf16 pair, round to nearest even (v_cvt_pk_bf16_f32)
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+  f32x2_t v = {a, b};
+  bf16x2_t h = __builtin_convertvector(v, bf16x2_t);
+  return *(uint32_t *)&h;
+}
+
+// Four consecutive outputs -> bf16, optionally followed by the element-wise tail.  The result is rounded to bf16 before the
+// tail and again after it, exactly as a separate binary op on the stored result would do.
+__device__ __forceinline__ u32x2 finish_quad(const LinearArgs &p, const uint8_t *cptr, const float (&v)[4]) {
+  u32x2 o = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+  if (p.tail != 0) {   // uniform
+    const u32x2 r = *(const u32x2 *)(cptr + p.tail_delta);
+    const float y[4] = {__uint_as_float(o.x << 16), __uint_as_float(o.x & 0xFFFF0000u), __uint_as_float(o.y << 16),
+                        __uint_as_float(o.y & 0xFFFF0000u)};
+    const float t[4] = {__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xFFFF0000u), __uint_as_float(r.y << 16),
+                        __uint_as_float(r.y & 0xFFFF0000u)};
+    float z[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) z[i] = p.tail == 1 ? y[i] + t[i] : y[i] * t[i];
+    o = u32x2{pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3])};
+  }
+  return o;
+}
+
+// LDS image of an operand block: [row][8 chunks of 8 k], chunk slot XOR-swizzled by the row so that every
+// group of 8 consecutive lanes hits 8 distinct 16-byte slots in all three access patterns: fragment
+// reads (8 consecutive rows), activation copies (4 rows x 2 chunks) and dequantised weight writes
+// (rows 8 apart x 2 chunks).
+__device__ __forceinline__ int lds_swz(int row) { return (((row << 1) & 6) | ((row >> 2) & 1)) ^ (((row >> 3) & 3) << 1); }
+__device__ __forceinline__ int lds_chunk(int row, int kc) { return row * 8 + (kc ^ lds_swz(row)); }
+// The images of the two-pass route (written by the image pass, read by the second pass as 16 rows x four chunks per
+// ds_read_b128 for v_mfma_f32_16x16x32_bf16) swizzle the slot by the low three row bits instead: under that read the
+// swizzle above puts pairs of lanes on one bank group (51 against 32 cycles per instruction with eight wavefronts reading),
+// this one none.
+__device__ __forceinline__ int lds_swz16(int row) { return row & 7; }
+__device__ __forceinline__ int lds_chunk16(int row, int kc) { return row * 8 + (kc ^ lds_swz16(row)); }
+
+// high halves of two floats -> packed bf16 pair (lo = a, hi = b); exact for dequantised weights
+__device__ __forceinline__ uint32_t pack_hi(float a, float b) {
+  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+
+__device__ __forceinline__ float linear_act_rt(int act, float x) {
+  switch (act) {
+  case TTM_ACT_GELU: return apply_act<TTM_ACT_GELU>(x);
+  case TTM_ACT_SILU: return apply_act<TTM_ACT_SILU>(x);
+  case TTM_ACT_SIGMOID: return apply_act<TTM_ACT_SIGMOID>(x);
+  case TTM_ACT_RELU: return apply_act<TTM_ACT_RELU>(x);
+  default: return x;
+  }
+}
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+
+// 4 x 4 transpose of dwords within every quad of lanes: lane q ends up with dword q of the rows that lanes 0..3 hold
+__device__ __forceinline__ void quad_transpose(uint32_t *v, int lane) {
+  const bool odd = (lane & 1) != 0, hi = (lane & 2) != 0;
+#pragma unroll
+  for (int a = 0; a < 4; a += 2) {   // lanes 2 j and 2 j + 1 exchange (v[a + 1] of the even, v[a] of the odd)
+    const uint32_t ta = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[a], 0xB1, 0xF, 0xF, true);
+    const uint32_t tb = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[a + 1], 0xB1, 0xF, 0xF, true);
+    v[a + 1] = odd ? v[a + 1] : ta;
+    v[a] = odd ? tb : v[a];
+  }
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {      // lanes j and j + 2 exchange (v[a + 2] of the lower, v[a] of the upper)
+    const uint32_t ta = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[a], 0x4E, 0xF, 0xF, true);
+    const uint32_t tb = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[a + 2], 0x4E, 0xF, 0xF, true);
+    v[a + 2] = hi ? v[a + 2] : ta;
+    v[a] = hi ? tb : v[a];
+  }
+}
+
+
+static inline int device_cu_count() {
+  static int cus = 0;
+  if (cus == 0) {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
+    else cus = 256;
+  }
+  return cus;
+}
+
+// column units of `unit_tiles` tiles in a launch: a group numbers its members' units one after another
+static inline int column_units(const LinearArgs &p, int unit_tiles) {
+  if (p.group_n <= 1) return (p.Nt + unit_tiles - 1) / unit_tiles;
+  int n = 0;
+  for (int j = 0; j < p.group_n; ++j) n += (p.gNt[j] + unit_tiles - 1) / unit_tiles;
+  return n;
+}
+
+
+// Split-K partial sums -> output (ttm_linear.hip): grid ((per / 4 + 255) / 256, 1, batch) of 256 lanes, per = Mt * Nt * 1024
+void ttm_linear_launch_reduce(const LinearArgs &p, int slices, int64_t batch, hipStream_t s);
+
+// The mid-size kernel (ttm_linear_mid.hip).  Launch plan: row tiles per workgroup, shares of K in a workgroup (wavefronts), slices
+// of K over grid.y, modelled time.
+struct MidPlan {
+  int mt = 0, wk = 8, slices = 1;
+  double us = 0;
+};
+MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu);
+int ttm_linear_launch_mid(const LinearArgs &a, int wf, const MidPlan &plan, int64_t batch, bool glu, hipStream_t s);

@@ -21,149 +21,7 @@
 // Kernels, by use: ttm_linear_dma_k (block-float weights, M > 64), ttm_linear_reg_k (bf16 weights, M > 64),
 // ttm_linear_big_k (64-bit-addressed fallback), ttm_linear_decode_k / ttm_linear_small_k (M <= 64),
 // ttm_linear_reduce_k (second half of a split-K launch).
-#include <type_traits>
-
-#include "ttm_common.h"
-#include "ttm_math.h"
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-enum { WF_BFP8 = 0, WF_BFP4 = 1, WF_BF16_KN = 2, WF_BF16_NK = 3 };
-
-struct LinearArgs {
-  const uint8_t *A;     // bf16, tile order, [Mt*32, Kt*32]
-  const uint8_t *W;     // weights, format WF_*
-  const uint16_t *bias; // bf16 or null
-  uint8_t *C;           // bf16, tile order, [Mt*32, Nt*32]
-  int Mt, Nt, Kt;       // extents in tiles
-  int act, bias_tiled;
-  int64_t a_batch, w_batch, c_batch;  // byte strides between batch entries (w_batch 0 = shared weights)
-  int m_blocks, n_blocks;
-  int ntw;                            // block-float main kernel: column tiles per wavefront (block width / 2)
-  int nt_split, n_blocks1, ntw2;      // two-part grid: blocks [0, n_blocks1) cover column tiles [0, nt_split) at width ntw,
-                                      // the rest cover [nt_split, Nt) at width ntw2; nt_split = 0: one part
-  int k_slice;                        // k-tiles per grid.y slice (split-K); Kt when the reduction is not split
-  float *partial;                     // split-K: fp32 partial sums [slices][Mt * Nt * 1024] in output tile order
-  int img_zero_step;                  // two-pass launch: W points at the dequantised images, this step index holds zeros
-  // group launch (group_n >= 2): several weight matrices [K, N_i] applied to the same activations, each with its own
-  // output; W / C / Nt above describe the virtual concatenation (Nt = sum of the members' column tiles) and are not
-  // dereferenced.  Each member may have its own activation; no bias, tail or batch in a group.
-  int group_n;
-  const uint8_t *gW[4];
-  uint8_t *gC[4];
-  int gNt[4];
-  int gAct[4];                        // per-member activation
-  int glu;                            // gated pair (decode kernel only): C = gC[0] = act0(A gW[0]) x act1(A gW[1]), both [K, gNt[0] * 32]
-  int tail;                           // 0 none, 1 add, 2 multiply: element-wise tail with a tensor laid out like the output
-  int64_t tail_delta;                 // byte distance from an output element to its tail operand
-  const struct QkvFinishArgs *qkv;    // host side only: the decode launch leaves partial sums and ttm_qkv_finish_k ends it
-  const struct NormFinishArgs *norm;  // host side only: ... and the RMSNorm kernel ends it (residual add, then the norm)
-};
-
-// x1 = residual + projection (stored to sum_out), then out = rms_norm(x1): the operands of the second launch
-struct NormFinishArgs {
-  const void *residual, *weight, *bias;
-  int weight_layout, bias_layout;
-  void *sum_out, *out;
-  int64_t rows, cols;
-  float eps;
-};
-
-// What follows the Q, K and V projections of a decode step (one token per user): head split, rotary embedding of q and k
-// at the cos / sin row `cos_row`, q to its own tensor, k and v into the cache row of position *index.
-struct QkvFinishArgs {
-  const float *partial;               // [slices][per] fp32 in tile order over the concatenation q | k | v (one row tile)
-  int slices;
-  int64_t per;
-  int users, heads, heads_pad, kv_heads, dim;
-  const uint16_t *cosc, *sinc;        // [.., dim] bf16 tiles
-  int64_t cos_row;
-  uint16_t *q_out;                    // [1, users, heads, dim] bf16 tiles
-  uint16_t *k_cache, *v_cache;        // [cache users, kv_heads, max_seq, dim] bf16 tiles
-  int64_t max_seq, seq_pad, batch_offset;
-  const int32_t *index;               // device memory: the position all users write
-};
-
-// The member of a group launch that owns column unit `u`, where a unit is `unit_tiles` column tiles and every member's
-// units are numbered one after another (a member's last unit may be partial).  Constant indices only: the arrays stay in
-// scalar registers.
-struct GroupMember {
-  const uint8_t *W;
-  uint8_t *C;
-  int Nt, local, tile_base, act;   // column tiles, unit index inside the member, first column tile in the concatenation
-};
-__device__ __forceinline__ GroupMember group_member(const LinearArgs &p, int u, int unit_tiles) {
-  GroupMember m = {p.gW[0], p.gC[0], p.gNt[0], u, 0, p.gAct[0]};
-  int start = 0, tiles = 0;
-  bool found = false;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    if (j < p.group_n) {
-      const int n = (p.gNt[j] + unit_tiles - 1) / unit_tiles;
-      if (!found && (u < start + n || j == p.group_n - 1)) {
-        found = true;
-        m.W = p.gW[j]; m.C = p.gC[j]; m.Nt = p.gNt[j]; m.local = u - start; m.tile_base = tiles; m.act = p.gAct[j];
-      }
-      start += n; tiles += p.gNt[j];
-    }
-  }
-  return m;
-}
-
-template <int ACT>
-__device__ __forceinline__ float apply_act(float x) {
-  if (ACT == TTM_ACT_GELU) return ttm_gelu_fast(x);
-  if (ACT == TTM_ACT_SILU) return ttm_silu(x);
-  if (ACT == TTM_ACT_SIGMOID) return ttm_sigmoid(x);
-  if (ACT == TTM_ACT_RELU) return ttm_max(x, 0.0f);   // keeps NaN, as arith.maximumf does
-  return x;
-}
-
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-// two floats -> packed bf16 pair, round to nearest even (v_cvt_pk_bf16_f32)
-__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-  f32x2_t v = {a, b};
-  bf16x2_t h = __builtin_convertvector(v, bf16x2_t);
-  return *(uint32_t *)&h;
-}
-
-// Four consecutive outputs -> bf16, optionally followed by the element-wise tail.  The result is rounded to bf16 before the
-// tail and again after it, exactly as a separate binary op on the stored result would do.
-__device__ __forceinline__ u32x2 finish_quad(const LinearArgs &p, const uint8_t *cptr, const float (&v)[4]) {
-  u32x2 o = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
-  if (p.tail != 0) {   // uniform
-    const u32x2 r = *(const u32x2 *)(cptr + p.tail_delta);
-    const float y[4] = {__uint_as_float(o.x << 16), __uint_as_float(o.x & 0xFFFF0000u), __uint_as_float(o.y << 16),
-                        __uint_as_float(o.y & 0xFFFF0000u)};
-    const float t[4] = {__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xFFFF0000u), __uint_as_float(r.y << 16),
-                        __uint_as_float(r.y & 0xFFFF0000u)};
-    float z[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) z[i] = p.tail == 1 ? y[i] + t[i] : y[i] * t[i];
-    o = u32x2{pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3])};
-  }
-  return o;
-}
-
-// LDS image of an operand block: [row][8 chunks of 8 k], chunk slot XOR-swizzled by the row so that every
-// group of 8 consecutive lanes hits 8 distinct 16-byte slots in all three access patterns: fragment
-// reads (8 consecutive rows), activation copies (4 rows x 2 chunks) and dequantised weight writes
-// (rows 8 apart x 2 chunks).
-__device__ __forceinline__ int lds_swz(int row) { return (((row << 1) & 6) | ((row >> 2) & 1)) ^ (((row >> 3) & 3) << 1); }
-__device__ __forceinline__ int lds_chunk(int row, int kc) { return row * 8 + (kc ^ lds_swz(row)); }
-// The images of the two-pass route (written by the image pass, read by the second pass as 16 rows x four chunks per
-// ds_read_b128 for v_mfma_f32_16x16x32_bf16) swizzle the slot by the low three row bits instead: under that read the
-// swizzle above puts pairs of lanes on one bank group (51 against 32 cycles per instruction with eight wavefronts reading),
-// this one none.
-__device__ __forceinline__ int lds_swz16(int row) { return row & 7; }
-__device__ __forceinline__ int lds_chunk16(int row, int kc) { return row * 8 + (kc ^ lds_swz16(row)); }
-
-// high halves of two floats -> packed bf16 pair (lo = a, hi = b); exact for dequantised weights
-__device__ __forceinline__ uint32_t pack_hi(float a, float b) {
-  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
-}
+#include "ttm_linear.h"
 
 // ---- bfp8: 8 rows (k) x 8 bytes (n) + 8 exponents -> 8 chunks (one per n) of 8 k
 __device__ __forceinline__ void dequant_bfp8_block(const u32x2 (&rows)[8], u32x2 exps, u32x4 (&out)[8]) {
@@ -368,15 +226,6 @@ __device__ __forceinline__ void linear_store_partial(const LinearArgs &p, float 
 // gated launch: the wavefront's accumulator tiles alternate between the two matrices (tile 2 j: columns of the first, tile
 // 2 j + 1: the same columns of the second); out = round(round(act0(first)) x round(act1(second))) into column tile
 // ntw / 2 + j of the output, whose rows are NtR tiles long.  No bias.
-__device__ __forceinline__ float linear_act_rt(int act, float x) {
-  switch (act) {
-  case TTM_ACT_GELU: return apply_act<TTM_ACT_GELU>(x);
-  case TTM_ACT_SILU: return apply_act<TTM_ACT_SILU>(x);
-  case TTM_ACT_SIGMOID: return apply_act<TTM_ACT_SIGMOID>(x);
-  case TTM_ACT_RELU: return apply_act<TTM_ACT_RELU>(x);
-  default: return x;
-  }
-}
 template <int NA, int MB>
 __device__ __forceinline__ void linear_epilogue_glu(const LinearArgs &p, uint8_t *C, f32x16 (&acc)[NA][MB], int mtw, int ntw, int nt_end, int NtR, int lane) {
   static_assert(NA % 2 == 0, "pairs of column tiles");
@@ -429,7 +278,7 @@ __global__ __launch_bounds__(256) void ttm_linear_reduce_k(LinearArgs p, int sli
   }
   GroupMember m = {};
   int act = p.act;
-  if (p.group_n > 1) {   // one row tile (decode): tile nt of the concatenation belongs to one member
+  if (p.group_n > 1) {   // tile nt of the concatenation belongs to one member
     m = group_member(p, nt, 1);
     act = m.act;
   }
@@ -447,7 +296,7 @@ __global__ __launch_bounds__(256) void ttm_linear_reduce_k(LinearArgs p, int sli
     v[r] = x;
   }
   if (p.group_n > 1) {
-    uint8_t *Cm = m.C + ((int64_t)m.local * 1024 + in) * 2;
+    uint8_t *Cm = m.C + (((off >> 10) / p.Nt * m.Nt + m.local) * 1024 + in) * 2;
     *(u32x2 *)Cm = finish_quad(p, Cm, v);
     return;
   }
@@ -1684,8 +1533,6 @@ __global__ __launch_bounds__(256) void ttm_linear_small_k(LinearArgs p) {
 // MFMAs is four consecutive n again.  Loads run two k-tiles ahead (register ring): with eight wavefronts that is
 // 74 KiB in flight per CU; four ahead measured 5 % slower ([4096, 14336] at M = 32: 17.4 -> 16.5 us), one or five slower still.
 // =============================================================================================
-typedef float f32x4v __attribute__((ext_vector_type(4)));
-
 // BFP4 = true reads bfp4_b tiles (576 bytes, two elements per byte, low nibble first): a lane's 4 (n) of a k row are one
 // 16-bit word, whose nibbles are spread into the bytes of a word before the same sign-magnitude -> offset-binary step.
 //
@@ -1769,27 +1616,9 @@ __global__ __launch_bounds__(512) void ttm_linear_decode_k(LinearArgs p) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) af[s][h] = *(const u32x4 *)(Ak + offA + h * 1024);
   };
-  // 4 x 4 transpose of dwords within every quad of lanes: lane q ends up with dword q of the rows that lanes 0..3 hold
-  auto quad_transpose = [&](uint32_t *v) __attribute__((always_inline)) {
-    const bool odd = (lane & 1) != 0, hi = (lane & 2) != 0;
-#pragma unroll
-    for (int a = 0; a < 4; a += 2) {   // lanes 2 j and 2 j + 1 exchange (v[a + 1] of the even, v[a] of the odd)
-      const uint32_t ta = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[a], 0xB1, 0xF, 0xF, true);
-      const uint32_t tb = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[a + 1], 0xB1, 0xF, 0xF, true);
-      v[a + 1] = odd ? v[a + 1] : ta;
-      v[a] = odd ? tb : v[a];
-    }
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {      // lanes j and j + 2 exchange (v[a + 2] of the lower, v[a] of the upper)
-      const uint32_t ta = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[a], 0x4E, 0xF, 0xF, true);
-      const uint32_t tb = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[a + 2], 0x4E, 0xF, 0xF, true);
-      v[a + 2] = hi ? v[a + 2] : ta;
-      v[a] = hi ? tb : v[a];
-    }
-  };
   auto process_pair = [&](int s, int pr) __attribute__((always_inline)) {
     if constexpr (WL) {
-      if (!TWO_TERM || keeps[s] != 0u) { quad_transpose(&rows[s][pr][0]); quad_transpose(&rows[s][pr][4]); }
+      if (!TWO_TERM || keeps[s] != 0u) { quad_transpose(&rows[s][pr][0], lane); quad_transpose(&rows[s][pr][4], lane); }
     }
     if constexpr (TWO_TERM) {
       if (keeps[s] == 0u) return;   // wavefront-uniform: a k-tile past the end contributes nothing
@@ -2032,30 +1861,12 @@ __global__ __launch_bounds__(256) void ttm_qkv_finish_k(QkvFinishArgs p) {
   else *(u32x2 *)(p.k_cache + ((p.batch_offset + m) * p.kv_heads + h) * p.seq_pad * D + ttm_tiled_offset(pos, d, ct)) = packed;
 }
 
-static int device_cu_count() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
-    else cus = 256;
-  }
-  return cus;
-}
-
 // Grid of the block-float main kernel: block width (8, 6 or 4 column tiles) and number of k-slices, chosen by a
 // small cost model fitted to measurements on the config shapes.  A block costs (k-steps + 12) x 1.65 us at full width
 // (the 12 stand for prologue and epilogue), 0.92 / 0.78 of that at 6 / 4 tiles (a narrower block keeps the whole
 // activation traffic of a wide one); blocks run in rounds of one per CU; a split reduction adds its fp32 partial
 // traffic, (slices + 0.5) x M x N x 4 bytes, at 4 TB/s.  force_* != 0 pin a choice (tests, measurements).
-// column units of `unit_tiles` tiles in a launch: a group numbers its members' units one after another
-static int column_units(const LinearArgs &p, int unit_tiles) {
-  if (p.group_n <= 1) return (p.Nt + unit_tiles - 1) / unit_tiles;
-  int n = 0;
-  for (int j = 0; j < p.group_n; ++j) n += (p.gNt[j] + unit_tiles - 1) / unit_tiles;
-  return n;
-}
-
-static int plan_dma_grid(LinearArgs &p, int cus, int force_ntw, int force_slices, int two_part = 0) {
+static int plan_dma_grid(LinearArgs &p, int cus, int force_ntw, int force_slices, int two_part = 0, double *us = nullptr) {
   const int mbk = p.m_blocks, ksteps = (p.Kt + 1) / 2;
   static const double width_cost[5] = {0, 0, 0.78, 0.92, 1.0};
   double best = 1e30;
@@ -2071,6 +1882,7 @@ static int plan_dma_grid(LinearArgs &p, int cus, int force_ntw, int force_slices
       if (t < best * 0.97) { best = t; best_ntw = ntw; best_slices = slices; }   // ties go to the wider, unsplit choice
     }
   }
+  if (us) *us = best;
   if (force_slices) best_slices = force_slices;
   p.ntw = best_ntw;
   p.n_blocks = mbk * column_units(p, 2 * best_ntw);   // blocks per k-slice
@@ -2110,9 +1922,43 @@ static int set_lds_limit(K kernel, int bytes) {
   return 0;
 }
 
+void ttm_linear_launch_reduce(const LinearArgs &p, int slices, int64_t batch, hipStream_t s) {
+  const int64_t per = (int64_t)p.Mt * p.Nt * 1024;
+  hipLaunchKernelGGL(ttm_linear_reduce_k, dim3((unsigned)((per / 4 + 255) / 256), 1, (unsigned)batch), dim3(256), 0, s, p, slices);
+}
+
+// The mid-size kernel is the library's own choice: an option that pins another kernel or its plan rules it out.
+static bool mid_allowed() {
+  return ttm_option("linear_mid") != 1 && !ttm_option("linear_variant") && !ttm_option("linear_ntw") && !ttm_option("linear_split_k") &&
+         !ttm_option("linear_two_part") && !ttm_option("linear_two_pass") && !ttm_option("linear_img_variant") && !ttm_option("linear_decode_split") &&
+         !ttm_option("linear_decode_wide") && !ttm_option("linear_decode_variant") && ttm_option("linear_small_m_max") == 64;
+}
+// What the launch would take without it, in the models its plans are made with.  Up to 64 rows that is a launch of the decode
+// kernel per row tile (block-float weights; [4096, 14336] bfp8_b at 48 rows 27 us against 19, [4096, 6144] 23.6 / 13.5,
+// [1024, 1024] 10.8 / 5.9: never the better one) or ttm_linear_small_k (bf16 weights, one row tile: one workgroup per 32 columns,
+// four wavefronts over K).
+template <int WF>
+static double other_us(const LinearArgs &a) {
+  constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
+  const int cus = device_cu_count(), ksteps = (a.Kt + 1) / 2;
+  if (BFP && a.Mt * 32 <= 64) return 1e30;
+  if (!BFP && a.Mt == 1) return 3.5 + (a.Nt * a.plan_batch + cus - 1) / cus * ((a.Kt + 15) / 16) * 1.9;
+  LinearArgs p = a;
+  double us = 0;
+  const int slices = plan_dma_grid(p, cus, 0, a.group_n > 1 ? 1 : 0, 0, &us);
+  us *= a.plan_batch > 1 ? (double)a.plan_batch : 1.0;
+  const double first = 3.0 + (double)a.Kt * a.Nt * (a.w_batch ? a.plan_batch : 1) * ((WF == WF_BFP8 ? 1088.0 : WF == WF_BFP4 ? 576.0 : 2048.0) + 2048.0) / 5.5e6;
+  const double gain = WF == WF_BFP4 ? (slices == 1 ? 0.22 : 0.08) : (slices == 1 ? 0.28 : 0.18);
+  return BFP ? std::min(us, first + (1.0 - gain) * us) : first + (1.0 - gain) * us;
+}
+
 template <int WF>
 static int launch_linear(const LinearArgs &a, int64_t batch, hipStream_t s) {
   constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
+  if (!a.qkv && !a.norm && !a.glu && mid_allowed() && !(BFP && a.Mt == 1 && ttm_option("linear_mid") < 1000)) {
+    const MidPlan plan = ttm_linear_plan_mid(a, WF, false);
+    if (ttm_option("linear_mid") >= 1000 || plan.us < 0.93 * other_us<WF>(a)) return ttm_linear_launch_mid(a, WF, plan, batch, false, s);
+  }
   // up to linear_small_m_max rows (64) the small kernels run once per row tile; bf16 weights leave them after one row tile
   // (from two on the image route is faster: [14336, 4096] at M = 64 116 us against 75 us)
   if (a.Mt == 1 || (BFP && a.Mt * 32 <= ttm_option("linear_small_m_max"))) {
@@ -2388,6 +2234,7 @@ static int linear_entry(const void *a, int a_dtype, const void *w, int w_dtype, 
   for (int j = 0; j < 4; ++j) { p.gW[j] = nullptr; p.gC[j] = nullptr; p.gNt[j] = 0; p.gAct[j] = TTM_ACT_NONE; }
   p.tail = tail_op;
   p.tail_delta = tail ? (const uint8_t *)tail - (const uint8_t *)out : 0;
+  p.plan_batch = strides ? 1 : (int)batch;
   p.qkv = nullptr;
   p.norm = norm;
   if (strides) { p.a_batch = strides[0]; p.w_batch = strides[1]; p.c_batch = strides[2]; }
@@ -2467,7 +2314,14 @@ static bool glu_main_ok(int w_dtype, int64_t M, int64_t N, int64_t K) {
   const int64_t ksteps = (Kt + 1) / 2, blocks = ttm_cdiv(Mt, 8) * ttm_cdiv(2 * Nt, 8), rounds = (blocks + cus - 1) / cus;
   const double fused = rounds * (ksteps + 12) * 1.65, first = 3.0 + (double)Kt * 2 * Nt * (1088.0 + 2048.0) / 5.5e6;
   const double multiply = 3.0 + 3.0 * (double)Mt * Nt * 2048.0 / 5.5e6;
-  return !(0.28 * fused - first > multiply);
+  if (!(0.28 * fused - first > multiply)) return true;
+  // ... or where the gated form of the mid-size kernel beats that kernel on the group by more than the models' error
+  if (!mid_allowed()) return false;
+  LinearArgs p = {};
+  p.Mt = (int)Mt; p.Kt = (int)Kt; p.Nt = 2 * (int)Nt; p.m_blocks = (p.Mt + 7) / 8; p.plan_batch = 1;
+  p.group_n = 2; p.gNt[0] = p.gNt[1] = (int)Nt;
+  const double glu = ttm_linear_plan_mid(p, WF_BFP8, true).us;
+  return glu < 0.75 * (std::min(ttm_linear_plan_mid(p, WF_BFP8, false).us, other_us<WF_BFP8>(p)) + multiply);
 }
 
 TTM_EXPORT int ttm_linear_glu_supported(int w_dtype, int64_t M, int64_t N, int64_t K) {
@@ -2501,6 +2355,7 @@ TTM_EXPORT int ttm_linear_glu(const void *a, const void *w_gate, const void *w_u
   p.nt_split = p.n_blocks1 = p.ntw2 = 0;
   p.img_zero_step = 0;
   p.tail = TTM_TAIL_NONE; p.tail_delta = 0;
+  p.plan_batch = 1;
   p.qkv = nullptr; p.norm = nullptr;
   hipStream_t s = (hipStream_t)stream;
   if (M > 32) {   // the fused main kernel over the tile slots of both matrices: blocks of 256 rows x four column tiles of each
@@ -2508,6 +2363,18 @@ TTM_EXPORT int ttm_linear_glu(const void *a, const void *w_gate, const void *w_u
     p.Nt = 2 * p.gNt[0];
     p.m_blocks = (p.Mt + 7) / 8;
     p.n_blocks = p.m_blocks * ((p.Nt + 7) / 8);
+    if (mid_allowed()) {
+      // at few rows or small weights the mid-size kernel: [2048, 2 x 8192] at 237 tokens 28 against 59 us, [4096, 2 x 14336] at 128
+      // tokens 44 / 100, at 256 82 / 100; at 400 it would take 162, and stays here with 116
+      const MidPlan plan = ttm_linear_plan_mid(p, WF_BFP8, true);
+      const int cus = device_cu_count();
+      const double here = (double)((p.n_blocks + cus - 1) / cus) * ((p.Kt + 1) / 2 + 12) * 1.65;
+      if (ttm_option("linear_mid") >= 1000 || plan.us < 0.93 * here) {
+        if (int rc = ttm_linear_launch_mid(p, WF_BFP8, plan, 1, true, s)) return rc;
+        TTM_LAUNCH_CHECK();
+        return TTM_OK;
+      }
+    }
     static bool attr = false;
     if (!attr) {
       if (int rc = set_lds_limit(ttm_linear_dma_glu_k, 131072 + 32768)) return rc;
@@ -2558,6 +2425,7 @@ static int linear_group_entry(const void *a, int n, const void *const *w, int w_
   p.nt_split = p.n_blocks1 = p.ntw2 = 0;
   p.img_zero_step = 0;
   p.tail = TTM_TAIL_NONE; p.tail_delta = 0;
+  p.plan_batch = 1;
   p.qkv = qkv;
   p.norm = nullptr;
   hipStream_t s = (hipStream_t)stream;

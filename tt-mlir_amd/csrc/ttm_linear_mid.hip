@@ -1,0 +1,345 @@
+// Dense contraction at row counts between decode and prefill, and small products (see ttm_linear.hip for the operands).
+#include "ttm_linear.h"
+
+// =============================================================================================
+// Mid-size kernel: row counts between the decode kernel's and those that fill the device with 256-row blocks, and any product too
+// small for them.  A workgroup owns 32 MT rows x 128 columns; its 8 wavefronts are 2 column pairs (64 columns) x 4 shares of K
+// (every fourth k-tile), summed through LDS at the end.  No operand passes through LDS on the way in: weights go from global
+// memory to registers and become the MFMA operand there as in the decode kernel (byte j of eight row words feeds MFMA j, whose
+// row r stands for column 4 r + j), activation fragments are 16-byte loads of whole face-row halves, which the two column pairs of
+// a share find in L1.  That leaves no barrier in the loop and nothing to fill before it: a launch costs 3 us + its k-tiles, where
+// the LDS-direct kernels' blocks cost 12 k-steps (20 us) before and after theirs - what bounded every product below some
+// 10 GFLOP.  Bounds inside the loop, per 32 k of a wavefront: about 480 cycles of vector issue for the conversion (bf16
+// weights: 64), 128 MT of the matrix core, 32 + 32 MT of L1; MT = 2 balances them for short launches, MT = 4 halves the weight
+// traffic and conversions where the row count fills it.
+// =============================================================================================
+template <int WF, int MT, int WK, bool TT, bool GLU>
+__global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(LinearArgs p) {
+  constexpr int WN = GLU ? 2 : 1;    // column pairs of the workgroup
+  constexpr int THREADS = WN * WK * 64, D = 2;
+  __shared__ f32x4v part[WN * WK * 512];   // partial sums of one row tile: per wavefront 8 x 64 float4 = 8 KiB
+  constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
+  constexpr uint32_t TB = WF == WF_BFP8 ? 1088u : WF == WF_BFP4 ? 576u : 2048u;
+  constexpr uint32_t FACE = WF == WF_BFP8 ? 256u : WF == WF_BFP4 ? 128u : 512u, ROW = FACE / 16;
+  constexpr int RW = BFP ? 8 : 16;   // dwords of weights per lane, k-tile and column pair
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wn = GLU ? wave / WK : 0, wk = wave & (WK - 1);
+  // row blocks of one column unit are neighbours on one XCD: its L2 serves the weights to all but the first of them
+  const int mblocks = (p.Mt + MT - 1) / MT;
+  const int slot = (int)blockIdx.x >> 3, mt0 = slot % mblocks * MT;
+  int cg = slot / mblocks * 8 + ((int)blockIdx.x & 7);
+  if (cg >= p.n_blocks) return;
+  int Nt = p.Nt, tile_base = 0, act = p.act;
+  const uint8_t *A = p.A + (int64_t)blockIdx.z * p.a_batch;
+  const uint8_t *W = p.W + (int64_t)blockIdx.z * p.w_batch;
+  uint8_t *C = p.C + (int64_t)blockIdx.z * p.c_batch;
+  if constexpr (GLU) {
+    C = p.gC[0]; Nt = p.gNt[0];
+  } else if (p.group_n > 1) {   // workgroup-uniform
+    const GroupMember m = group_member(p, cg, 2);
+    W = m.W; C = m.C; Nt = m.Nt; cg = m.local; tile_base = m.tile_base; act = m.act;
+  }
+  const int q16 = lane & 15, kg = lane >> 4;   // weight operand row and 8-k group of this lane
+  const int fc = (q16 >> 2) & 1, quad = q16 & 3, fr = kg >> 1, half = kg & 1;
+  if (GLU) W = wn ? p.gW[1] : p.gW[0];
+  const uint32_t nt_l = (uint32_t)min(2 * cg + (q16 >> 3), Nt - 1);
+  // bfp8_b: two whole 16-byte rows of the quad's 128-byte line; bfp4_b: eight 2-byte words; bf16 [K, N]: eight 8-byte words;
+  // bf16 [N, K]: the 8 k of each of the four columns
+  const uint32_t offW = WF == WF_BF16_NK ? (uint32_t)(fc * 1024 + quad * 128 + fr * 512 + half * 16)
+                                         : (BFP ? 64u : 0u) + (fr * 2 + fc) * FACE + half * (FACE / 2) + quad * (WF == WF_BFP8 ? ROW : ROW / 4);
+  const uint32_t offE = (fr * 2 + fc) * 16 + half * 8;
+  const uint32_t offA = fr * 512 + q16 * 32 + half * 16;
+  int64_t rowA[MT];
+#pragma unroll
+  for (int r = 0; r < MT; ++r) rowA[r] = (int64_t)min(mt0 + r, p.Mt - 1) * p.Kt * 2048 + offA;
+
+  f32x4v acc[2 * MT][4], accs[TT ? 2 * MT : 1][4];   // accs: the sums over the S terms
+#pragma unroll
+  for (int h = 0; h < 2 * MT; ++h)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      acc[h][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
+      if (TT) accs[h][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    }
+  uint32_t rows[D][RW];
+  u32x2 ex[D];
+  bool live[D];
+  u32x4 af[D][2 * MT];
+  const int kbase = p.partial ? (int)blockIdx.y * p.k_slice : 0;
+  const int kend = p.partial ? min(kbase + p.k_slice, p.Kt) : p.Kt;
+  const int nchunks = (kend - kbase + WK - 1) / WK;
+  auto load_slot = [&](int s, int c) __attribute__((always_inline)) {
+    const int kt = kbase + wk + WK * c, ktc = min(kt, kend - 1);
+    live[s] = kt < kend;
+    uint32_t *rw = rows[s];
+    if constexpr (WF == WF_BF16_NK) {
+      const uint8_t *Wk = W + ((int64_t)nt_l * p.Kt + ktc) * TB + offW;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const u32x4 x = *(const u32x4 *)(Wk + j * 32);
+        rw[4 * j] = x.x; rw[4 * j + 1] = x.y; rw[4 * j + 2] = x.z; rw[4 * j + 3] = x.w;
+      }
+    } else {
+      const uint8_t *Wt = W + ((int64_t)ktc * Nt + nt_l) * TB, *Wk = Wt + offW;
+      if constexpr (WF == WF_BFP8) {
+        const u32x4 x = *(const u32x4 *)Wk, y = *(const u32x4 *)(Wk + 64);
+        rw[0] = x.x; rw[1] = x.y; rw[2] = x.z; rw[3] = x.w;
+        rw[4] = y.x; rw[5] = y.y; rw[6] = y.z; rw[7] = y.w;
+      } else if constexpr (WF == WF_BFP4) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) rw[i] = *(const uint16_t *)(Wk + i * ROW);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const u32x2 x = *(const u32x2 *)(Wk + i * ROW);
+          rw[2 * i] = x.x; rw[2 * i + 1] = x.y;
+        }
+      }
+      if constexpr (BFP) ex[s] = *(const u32x2 *)(Wt + offE);
+    }
+#pragma unroll
+    for (int h = 0; h < 2 * MT; ++h) af[s][h] = *(const u32x4 *)(A + rowA[h >> 1] + (int64_t)ktc * 2048 + (h & 1) * 1024);
+  };
+  auto process = [&](int s) __attribute__((always_inline)) {
+    if (!live[s]) return;   // wavefront-uniform: a k-tile past the end contributes nothing
+    uint32_t *rw = rows[s];
+    if constexpr (TT && BFP) {
+      if constexpr (WF == WF_BFP8) { quad_transpose(rw, lane); quad_transpose(rw + 4, lane); }
+      // (E + 1) << 7 for the rows 2 ip and 2 ip + 1, in the two halves of a word; E is capped so that the field stays 8 bits
+      uint32_t epk[4], pk[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int ip = 0; ip < 4; ++ip) {
+        uint32_t e2 = __builtin_amdgcn_perm(0u, ip < 2 ? ex[s].x : ex[s].y, (ip & 1) ? 0x0c030c02u : 0x0c010c00u);
+        typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+        const u16x2 capped = __builtin_elementwise_min(*(const u16x2 *)&e2, u16x2{0xFD, 0xFD});
+        e2 = *(const uint32_t *)&capped;
+        epk[ip] = (e2 + 0x00010001u) << 7;
+        if constexpr (WF == WF_BFP4) pk[ip] = rw[2 * ip] | (rw[2 * ip + 1] << 16);   // four nibbles per row
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        u32x4 wv, ws;
+#pragma unroll
+        for (int ip = 0; ip < 4; ++ip) {
+          if constexpr (WF == WF_BFP4) {
+            const uint32_t q = pk[ip] >> (4 * j);            // nibble j of either row in bits 0..3 and 16..19
+            ws[ip] = ((q & 0x00080008u) << 12) | epk[ip];
+            wv[ip] = ((q & 0x00070007u) << 4) | ws[ip];
+          } else {
+            const uint32_t q = __builtin_amdgcn_perm(rw[2 * ip + 1], rw[2 * ip], 0x0c040c00u + 0x00010001u * j);
+            ws[ip] = ((q & 0x00800080u) << 8) | epk[ip];
+            wv[ip] = (q & 0x007F007Fu) | ws[ip];
+          }
+        }
+#pragma unroll
+        for (int h = 0; h < 2 * MT; ++h) {
+          acc[h][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(bf16x8 *)&wv, *(bf16x8 *)&af[s][h], acc[h][j], 0, 0, 0);
+          accs[h][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(bf16x8 *)&ws, *(bf16x8 *)&af[s][h], accs[h][j], 0, 0, 0);
+        }
+      }
+      return;
+    }
+    float scale[8], nscale[8];
+    uint32_t t[8];
+    if constexpr (BFP) {
+      if constexpr (WF == WF_BFP8) { quad_transpose(rw, lane); quad_transpose(rw + 4, lane); }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        uint32_t E = ((i < 4 ? ex[s].x : ex[s].y) >> (8 * (i & 3))) & 0xFFu;
+        // value = magnitude x 2^(E - 127 - 6) (bfp8_b) or 2^(E - 127 - 2) (bfp4_b); smaller exponents flush to zero
+        constexpr uint32_t EB = WF == WF_BFP4 ? 2u : 6u, SIGN = WF == WF_BFP4 ? 0x08080808u : 0x80808080u, SH = WF == WF_BFP4 ? 3u : 7u;
+        E = max(E, EB);
+        scale[i] = __uint_as_float((E - EB) << 23);
+        nscale[i] = (WF == WF_BFP4 ? -8.0f : -128.0f) * scale[i];
+        uint32_t d = rw[i];
+        if (WF == WF_BFP4) {   // nibbles n3 n2 n1 n0 of the low half -> one per byte
+          d = (d | (d << 8)) & 0x00FF00FFu;
+          d = (d | (d << 4)) & 0x0F0F0F0Fu;
+        }
+        const uint32_t sg = d & SIGN, sb = sg >> SH;
+        t[i] = (d ^ SIGN ^ (sg - sb)) + sb;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      u32x4 w;
+      if constexpr (BFP) {
+        float f[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = fmaf((float)((t[i] >> (8 * j)) & 0xFFu), scale[i], nscale[i]);
+        w = u32x4{pack_hi(f[0], f[1]), pack_hi(f[2], f[3]), pack_hi(f[4], f[5]), pack_hi(f[6], f[7])};
+      } else if constexpr (WF == WF_BF16_KN) {
+        const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = __builtin_amdgcn_perm(rw[4 * i + 2 + (j >> 1)], rw[4 * i + (j >> 1)], sel);
+      } else {
+        w = u32x4{rw[4 * j], rw[4 * j + 1], rw[4 * j + 2], rw[4 * j + 3]};
+      }
+#pragma unroll
+      for (int h = 0; h < 2 * MT; ++h)
+        acc[h][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(bf16x8 *)&w, *(bf16x8 *)&af[s][h], acc[h][j], 0, 0, 0);
+      if constexpr (MT > 2) __builtin_amdgcn_sched_barrier(0);   // one column's operand at a time: more of them do not fit the registers
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < D; ++s) {
+    load_slot(s, s);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  for (int c0 = 0; c0 < nchunks; c0 += D) {
+#pragma unroll
+    for (int s = 0; s < D; ++s) {
+      process(s);
+      __builtin_amdgcn_sched_barrier(0);   // keep the loads in slot order, D - 1 slots ahead of their use
+      load_slot(s, c0 + s + D);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  if constexpr (TT && BFP) {
+#pragma unroll
+    for (int h = 0; h < 2 * MT; ++h)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[h][j] -= accs[h][j];
+  }
+  // one row tile at a time: the wavefronts' sums -> LDS as float4 (four consecutive n of one m), then the threads finish the 512
+  // slots, (h, i, lane) = (t >> 8, (t >> 6) & 3, t & 63)
+#pragma unroll
+  for (int r = 0; r < MT; ++r) {
+    if (mt0 + r >= p.Mt) break;      // workgroup-uniform
+    if (r > 0) __syncthreads();
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii)
+        part[(wave * 8 + hh * 4 + ii) * 64 + lane] = f32x4v{acc[2 * r + hh][0][ii], acc[2 * r + hh][1][ii], acc[2 * r + hh][2][ii], acc[2 * r + hh][3][ii]};
+    __syncthreads();
+#pragma unroll
+    for (int t0 = 0; t0 < 512; t0 += THREADS) {
+      const int t = t0 + tid, h = t >> 8, i = (t >> 6) & 3;
+      const int n_in = 16 * (kg & 1) + 4 * i, nt = 2 * cg + (kg >> 1);
+      if (nt >= Nt) continue;
+      const int in = (h * 2 + (n_in >> 4)) * 256 + q16 * 16 + (n_in & 15);
+      f32x4v sums[WN];
+#pragma unroll
+      for (int q = 0; q < WN; ++q) {
+        sums[q] = part[q * WK * 512 + t];
+#pragma unroll
+        for (int w = 1; w < WK; ++w) sums[q] += part[(q * WK + w) * 512 + t];
+      }
+      uint8_t *c = C + (((int64_t)(mt0 + r) * Nt + nt) * 1024 + in) * 2;
+      if constexpr (GLU) {
+        float v0[4], v1[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { v0[e] = linear_act_rt(p.gAct[0], sums[0][e]); v1[e] = linear_act_rt(p.gAct[1], sums[WN - 1][e]); }
+        const u32x2 g = {pack_bf16(v0[0], v0[1]), pack_bf16(v0[2], v0[3])}, u = {pack_bf16(v1[0], v1[1]), pack_bf16(v1[2], v1[3])};
+        const float z[4] = {__uint_as_float(g.x << 16) * __uint_as_float(u.x << 16), __uint_as_float(g.x & 0xFFFF0000u) * __uint_as_float(u.x & 0xFFFF0000u),
+                            __uint_as_float(g.y << 16) * __uint_as_float(u.y << 16), __uint_as_float(g.y & 0xFFFF0000u) * __uint_as_float(u.y & 0xFFFF0000u)};
+        *(u32x2 *)c = u32x2{pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3])};
+      } else if (p.partial) {   // bias, activation and rounding happen in ttm_linear_reduce_k
+        *(f32x4v *)(p.partial + (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * p.Mt + mt0 + r) * p.Nt * 1024 + (int64_t)(tile_base + nt) * 1024 + in) = sums[0];
+      } else {
+        float bv[4] = {0.f, 0.f, 0.f, 0.f};
+        if (p.bias) {
+          const uint16_t *bp = p.bias_tiled ? p.bias + (int64_t)nt * 1024 + (n_in >> 4) * 256 + (n_in & 15) : p.bias + nt * 32 + n_in;
+          const u32x2 raw = *(const u32x2 *)bp;
+          bv[0] = __uint_as_float(raw.x << 16); bv[1] = __uint_as_float(raw.x & 0xFFFF0000u);
+          bv[2] = __uint_as_float(raw.y << 16); bv[3] = __uint_as_float(raw.y & 0xFFFF0000u);
+        }
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = linear_act_rt(act, sums[0][e] + bv[e]);
+        *(u32x2 *)c = finish_quad(p, c, v);
+      }
+    }
+  }
+}
+
+// ---- the mid-size kernel's launch plan
+static int mid_units(const LinearArgs &p, bool glu) { return glu ? (p.gNt[0] + 1) / 2 : column_units(p, 2); }
+
+// The model was fitted to 36 shapes of 3 .. 1236 rows, 296 .. 7488 x 265 .. 14336 weights of all formats under every plan (11 % rms
+// over 380 timings; the plan it picks is 1 % slower than the best one on average): 3.3 us for launch, first loads and the last
+// wavefronts, the k-tiles that the wavefronts of a SIMD take, 0.2 + 0.95 us per row tile for the sums through LDS of each
+// round of workgroups, and for a split K the reduction's launch and its traffic at 2.5 TB/s.
+MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu) {
+  // option linear_mid: 0 by the model, 1 never, 1000 * shares + 100 * row tiles + slices pins a plan
+  const int force = ttm_option("linear_mid");
+  MidPlan best;
+  best.us = 1e30;
+  const int cus = device_cu_count(), units = mid_units(p, glu);
+  const int f = wf == WF_BFP8 || wf == WF_BFP4 ? 0 : 1;
+  // us per k-tile of a wavefront at 1 / 2 / 4 row tiles (wavefronts of a SIMD share it, so they add up)
+  static const double kChunk[2][5] = {{0, 0.25, 0.44, 0, 0.57}, {0, 0.32, 0.45, 0, 0.68}};
+  for (int mt = 1; mt <= 4; mt *= 2) {
+    const int blocks = units * ((p.Mt + mt - 1) / mt) * p.plan_batch;
+    for (int wk = 4; wk <= 8; wk += 4) {
+      if (glu ? wk != 4 || mt == 1 : (wk == 4 && mt != 2)) continue;
+      for (int slices = 1; slices <= (glu ? 1 : 16); slices *= 2) {
+        if (force >= 1000) {
+          if (force / 1000 != wk || force % 1000 / 100 != mt || force % 100 != slices) continue;
+        } else if ((mt > 1 && mt >= 2 * p.Mt) || (slices > 1 && p.Kt < 2 * wk * slices)) {
+          continue;
+        }
+        const int kt = (p.Kt + slices - 1) / slices, chunks = (kt + wk - 1) / wk, rounds = (blocks * slices + cus - 1) / cus;
+        if (force < 1000 && rounds > 8) continue;   // beyond what was measured; larger blocks amortise their ends better
+        const int waves = rounds * wk / 4 * (glu ? 2 : 1);            // per SIMD
+        double us = 3.3 + waves * chunks * kChunk[f][mt] + (wk == 8 || glu ? rounds : 1) * (0.2 + 0.95 * mt);
+        if (slices > 1) us += 2.7 + (slices + 0.5) * (double)p.Mt * p.Nt * p.plan_batch * 4096.0 / 2.5e6;
+        if (us < best.us) { best.us = us; best.mt = mt; best.wk = wk; best.slices = slices; }
+      }
+    }
+  }
+  return best;
+}
+
+template <int WF, int MT, int WK, bool TT>
+static void launch_mid_mt(const LinearArgs &p, dim3 grid, hipStream_t s) {
+  constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
+  hipLaunchKernelGGL((ttm_linear_mid_k<WF, MT, WK, TT && BFP, false>), grid, dim3(WK * 64), 0, s, p);
+}
+template <int WF>
+static int launch_mid(const LinearArgs &a, const MidPlan &plan, int64_t batch, bool glu, hipStream_t s) {
+  LinearArgs p = a;
+  int slices = plan.slices;
+  p.partial = nullptr;
+  p.k_slice = p.Kt;
+  const int64_t per = (int64_t)p.Mt * p.Nt * 1024;
+  if (slices > 1) {
+    p.k_slice = (p.Kt + slices - 1) / slices;
+    slices = (p.Kt + p.k_slice - 1) / p.k_slice;
+    void *ws = nullptr;
+    if (int rc = ttm_stream_workspace(s, (size_t)(per * slices * batch) * sizeof(float), &ws)) return rc;
+    p.partial = (float *)ws;
+  }
+  p.n_blocks = mid_units(a, glu);
+  const dim3 grid((unsigned)((p.n_blocks + 7) / 8 * 8 * ((p.Mt + plan.mt - 1) / plan.mt)), (unsigned)slices, (unsigned)batch);
+  if (glu) {
+    if constexpr (WF == WF_BFP8) {
+      if (plan.mt == 2) hipLaunchKernelGGL((ttm_linear_mid_k<WF_BFP8, 2, 4, false, true>), grid, dim3(512), 0, s, p);
+      else hipLaunchKernelGGL((ttm_linear_mid_k<WF_BFP8, 4, 4, false, true>), grid, dim3(512), 0, s, p);
+      return 0;
+    }
+    return ttm_set_error(TTM_ERR_INVALID, "ttm_linear_glu: the mid-size kernel's gated form takes bfp8_b weights");
+  }
+  switch (plan.wk * 10 + plan.mt) {
+  case 81: launch_mid_mt<WF, 1, 8, true>(p, grid, s); break;
+  case 82: launch_mid_mt<WF, 2, 8, false>(p, grid, s); break;
+  case 84: launch_mid_mt<WF, 4, 8, false>(p, grid, s); break;
+  case 42: launch_mid_mt<WF, 2, 4, false>(p, grid, s); break;
+  default: return ttm_set_error(TTM_ERR_INVALID, "ttm_linear: no such plan of the mid-size kernel (linear_mid = %d)", ttm_option("linear_mid"));
+  }
+  if (slices > 1)
+    ttm_linear_launch_reduce(p, slices, batch, s);
+  return 0;
+}
+
+
+int ttm_linear_launch_mid(const LinearArgs &a, int wf, const MidPlan &plan, int64_t batch, bool glu, hipStream_t s) {
+  switch (wf) {
+  case WF_BFP8: return launch_mid<WF_BFP8>(a, plan, batch, glu, s);
+  case WF_BFP4: return launch_mid<WF_BFP4>(a, plan, batch, glu, s);
+  case WF_BF16_KN: return launch_mid<WF_BF16_KN>(a, plan, batch, glu, s);
+  default: return launch_mid<WF_BF16_NK>(a, plan, batch, glu, s);
+  }
+}
