@@ -74,12 +74,16 @@ def _ck(status, what):
 
 
 def _call(name, *args):
-    _ck(getattr(lib(), name)(*args), name)
+    status = getattr(_lib or lib(), name)(*args)
+    if status:
+        _ck(status, name)
+
+
+_U32x8 = ctypes.c_uint32 * 8
 
 
 def _shape_arg(shape):
-    arr = (ctypes.c_uint32 * 8)(*[int(s) for s in shape])
-    return arr, len(shape)
+    return _U32x8(*map(int, shape)), len(shape)
 
 
 class Binary:
@@ -205,7 +209,7 @@ class Tensor:
         self._keepalive = keepalive  # borrowed host memory must outlive the tensor
 
     def desc(self):
-        shape, rank, lay, nbytes = (ctypes.c_uint32 * 8)(), ctypes.c_int(), Layout(), ctypes.c_uint64()
+        shape, rank, lay, nbytes = _U32x8(), ctypes.c_int(), Layout(), ctypes.c_uint64()
         _call("ttrt_tensor_desc", self.h, shape, ctypes.byref(rank), ctypes.byref(lay), ctypes.byref(nbytes))
         return tuple(shape[: rank.value]), lay, nbytes.value
 
@@ -321,17 +325,34 @@ def create_borrowed_host_tensor(array, dtype):
     return _host(array, dtype, True)
 
 
+_torch_types = None
+
+
+def _torch_maps():
+    """({torch dtype: (DataType, element size)}, {DataType: torch dtype}), built once."""
+    global _torch_types
+    if _torch_types is None:
+        import torch
+        to_rt = {torch.float32: DataType.Float32, torch.bfloat16: DataType.BFloat16, torch.float16: DataType.Float16,
+                 torch.int32: DataType.Int32, torch.int64: DataType.Int64, torch.uint8: DataType.UInt8, torch.float64: DataType.Float64,
+                 torch.int16: DataType.Int16, torch.int8: DataType.Int8, torch.bool: DataType.Bool}
+        back = {DataType.Float32: torch.float32, DataType.BFloat16: torch.bfloat16, DataType.Float16: torch.float16,
+                DataType.Int32: torch.int32, DataType.UInt8: torch.uint8}
+        _torch_types = {k: (v, torch.empty(0, dtype=k).element_size()) for k, v in to_rt.items()}, back
+    return _torch_types
+
+
 def from_torch(t, borrowed=False):
     """Host tensor from a CPU torch tensor (bf16 / f32 / f16 / ints)."""
-    import torch
-    m = {torch.float32: (DataType.Float32, None), torch.bfloat16: (DataType.BFloat16, torch.int16),
-         torch.float16: (DataType.Float16, None), torch.int32: (DataType.Int32, None), torch.int64: (DataType.Int64, None),
-         torch.uint8: (DataType.UInt8, None), torch.float64: (DataType.Float64, None), torch.int16: (DataType.Int16, None),
-         torch.int8: (DataType.Int8, None), torch.bool: (DataType.Bool, None)}
-    dt, view = m[t.dtype]
+    dt, itemsize = _torch_maps()[0][t.dtype]
     a = t.contiguous()
-    arr = a.view(view).numpy().view(np.uint16) if view is not None else a.numpy()
-    return _host(arr, dt, borrowed)
+    if a.device.type != "cpu" or a.requires_grad or a.numel() == 0:
+        import torch
+        return _host(a.view(torch.int16).numpy().view(np.uint16) if dt == DataType.BFloat16 else a.numpy(), dt, borrowed)
+    shape, rank = _shape_arg(a.shape or (1,))
+    h = ctypes.c_void_p()
+    _call("ttrt_tensor_create_host", ctypes.c_void_p(a.data_ptr()), shape, rank, None, itemsize, dt, int(borrowed), ctypes.byref(h))
+    return Tensor(h, keepalive=a if borrowed else None)
 
 
 def create_unsafe_borrowed_host_tensor(owned):
@@ -439,11 +460,16 @@ def to_numpy(tensor, target_dtype=None):
 
 def to_torch(tensor):
     import torch
-    a = to_numpy(tensor)
     lay = tensor.desc()[1]
-    if lay.dtype == DataType.BFloat16:
-        return torch.from_numpy(a.view(np.int16)).view(torch.bfloat16)
-    return torch.from_numpy(a)
+    host = to_host(tensor, untilize=True)[0] if lay.storage != StorageType.Host else tensor
+    shape, hlay, nbytes = host.desc()
+    dt = _torch_maps()[1].get(hlay.dtype)
+    if dt is None or hlay.layout == TensorLayout.Tile or nbytes == 0:
+        a = to_numpy(host)
+        return torch.from_numpy(a.view(np.int16)).view(torch.bfloat16) if lay.dtype == DataType.BFloat16 else torch.from_numpy(a)
+    out = torch.empty(shape, dtype=dt)
+    _call("ttrt_memcpy_out", ctypes.c_void_p(out.data_ptr()), host.h, -1)
+    return out
 
 
 def buffer_cast(src, from_dtype, to_dtype):
