@@ -393,8 +393,8 @@ int ttm_rotary_embedding_llama(const void *x, const void *cos_cache, const void 
  * call hipMalloc: code under HIP graph capture, tight serving loops, harnesses that forbid allocation.  Same arguments, same
  * kernels and bit-identical results; the per-slice partial results (max, sum, unnormalised output) go to a static device
  * array of 8 MiB that the library holds on every GPU it runs on until the process ends, instead of the stream's grow-only
- * workspace.  A call whose partial results need more (batch * kv_heads * slices * min(heads / kv_heads, 8) * (head_dim + 2)
- * floats; the config-5 decode shape of 32 users x 8 kv heads x 2048 positions takes 1 MiB) fails with TTM_ERR_INVALID and
+ * workspace.  A call whose partial results need more (kv_heads * (key shares + batch) * min(heads / kv_heads, 8) * (head_dim + 2)
+ * floats; the config-5 decode shape of 32 users x 8 kv heads x 2048 positions takes 1.6 MB) fails with TTM_ERR_INVALID and
  * launches nothing.  No hipMalloc, hipFree or allocating library call is made; the first call on a device looks the
  * array's address up (hipGetSymbolAddress), so make that call outside a capture.  All calls on one GPU share the array:
  * calls that overlap in time on one GPU (different streams) race; calls on one stream are ordered and safe. */

@@ -241,20 +241,26 @@ __global__ __launch_bounds__(256) void ttm_rotary_llama_k(const uint16_t *__rest
 
 // ------------------------------------------------------------------------------------------------ attention, one query token
 // q [1, B, H, D], k / v [B, Hkv, S, D] (or pages [blocks, Hkv, block, D] behind a page table), out [1, B, H, D], bf16 tiles.
-// grid (splits, B * Hkv), 256 threads.  A block owns the G = H / Hkv query heads of one kv head and one slice of the keys:
-//   1. scores = Q K^T with v_mfma_f32_16x16x32_bf16 (queries are the 16 rows, padded with zeros), written to LDS
-//      as (score + mask) * scale, -inf outside the valid keys;
-//   2. softmax numerators per query head, rounded to bf16 and stored as pairs of keys 16 apart, and their sum;
-//   3. P V on the vector ALU with v_dot2_f32_bf16: a wave reads the two halves of a V tile (2 x 1 KiB contiguous), every
-//      lane keeps 8 columns x G heads of partial sums, lanes are combined once per column tile;
-//   4. (max, sum, unnormalised output) go to the split's slot of the workspace; ttm_sdpa_decode_combine_k merges the slots
-//      (merging in the last workgroup to arrive was measured: the device-scope fences it needs double the kernel time).
+// HBM-bound: K and V up to the users' positions are read once.  A workgroup owns the G = H / Hkv query heads of one kv head and a
+// range of 32-key tiles; its wavefronts take the tiles in turn, each with a running maximum, sum and output of its own:
+//   scores = K Q^T with v_mfma_f32_16x16x32_bf16 (keys are the rows, heads the columns: a lane holds four consecutive keys of one
+//   head), softmax numerators against the running maximum, rounded to bf16 and exchanged through 16 G dwords of LDS, then P V on
+//   the vector ALU with v_dot2_f32_bf16: a lane owns two adjacent columns for all keys of the tile, so nothing is summed across lanes.
+// The next tile's K is requested when the scores are made, its V behind the products, so a wavefront has 16 KiB (D = 128) on the
+// way at any time and no wavefront waits for another before the end, where the partial results meet in LDS.
+//
+// Two forms.  Direct: grid (Hkv, B), eight wavefronts, the whole context of a user and the output in one launch.  Shares: the
+// visible tiles of all users of a kv head form one line (user after user), workgroup j of grid (shares, Hkv) streams its j-th equal
+// part whatever the users' context lengths are; (max, sum, unnormalised output) of a piece go to slot j + user of the kv head
+// (along the line either j or the user advances from one piece to the next, so the sum numbers the pieces) and
+// ttm_sdpa_decode_combine_k merges a user's slots (merging in the last workgroup to arrive was measured: the device-scope
+// fences it needs double the kernel time).
 struct DecodeArgs {
   const uint16_t *q, *k, *v, *mask;
   const int32_t *cur_pos, *page_table;
-  float *part;        // [B * Hkv][splits][G][D + 2]
+  float *part;        // [Hkv][shares + B][G][D + 2]
   uint16_t *out;
-  int B, H, Hkv, G, S, D, splits, keys_per_split, block, pages_per_user, mask_heads, is_causal;
+  int B, H, Hkv, G, S, D, shares, block, pages_per_user, mask_heads, is_causal;
   int blocks;         // number of blocks in a paged cache: page-table entries outside [0, blocks) are masked
   int concat_heads;   // out is [B, H * D] (row b holds user b's heads side by side) instead of [B, H, D]
   int Gt, g0;         // query heads per kv head in the tensors, and the first of them this launch serves (it serves G of them)
@@ -266,19 +272,57 @@ struct DecodeArgs {
 
 constexpr int kMaxG = 8;
 // K and V are read once per launch: streaming (nontemporal) loads keep them from displacing each other in the caches on
-// the way (measured at 32 users x 8 kv heads x 2048 positions: 59 -> 54 us).  STREAM = false when several launches share
-// one cache (more than kMaxG query heads per kv head), where the later launches profit from what the first one left.
+// the way.  STREAM = false when several launches share one cache (more than kMaxG query heads per kv head), where the later
+// launches profit from what the first one left.
 template <bool STREAM, typename T>
 __device__ __forceinline__ T kv_load(const T *p) {
   if constexpr (STREAM) return __builtin_nontemporal_load(p);
   else return *p;
 }
-#ifndef SPLIT_TARGET
-#define SPLIT_TARGET 512
-#endif
+constexpr int kDecodeBlocks = 512;   // workgroups of the shares form: two of four wavefronts per CU
 
-__device__ __forceinline__ const uint16_t *kv_tile_row(const uint16_t *base, const DecodeArgs &p, int b, int hk, int key_tile, bool &ok) {
-  // start of the row of tiles holding keys [32 key_tile, 32 key_tile + 32) of (b, hk).  A page-table entry outside the
+// the visible keys of user b: [lo, valid); tiles in front of lo's are not read at all
+__device__ __forceinline__ void visible_keys(const DecodeArgs &p, int b, int &lo, int &valid) {
+  valid = p.S;
+  int pos = p.S - 1;
+  if (p.cur_pos) {
+    pos = p.cur_pos[b];
+    if (p.is_causal) valid = min(max(pos + 1, 0), p.S);
+  }
+  lo = p.window >= 0 && pos + 1 > p.window ? pos + 1 - p.window : 0;
+}
+__device__ __forceinline__ int visible_tiles(const DecodeArgs &p, int b) {
+  int lo, valid;
+  visible_keys(p, b, lo, valid);
+  return max(((valid + 31) >> 5) - (lo >> 5), 0);
+}
+// inclusive sum over the lanes of a wavefront, DPP moves only
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);   // row_shr 1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);   // row_bcast 15 into rows 1 and 3, row_bcast 31 into rows 2 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+  return v;
+}
+// tiles of the users in front of user b0 + lane (exclusive sum) for the chunk of 64 users that holds user b, and all users' tiles
+__device__ __forceinline__ void line_of(const DecodeArgs &p, int b, int lane, int &before, int &mine, int &total) {
+  total = before = mine = 0;
+  for (int b0 = 0; b0 < p.B; b0 += 64) {
+    const int own = b0 + lane < p.B ? visible_tiles(p, b0 + lane) : 0, sum = wave_scan(own);
+    if (b >= b0 && b < b0 + 64) {
+      mine = __builtin_amdgcn_readlane(own, b - b0);
+      before = total + __builtin_amdgcn_readlane(sum, b - b0) - mine;
+    }
+    total += __builtin_amdgcn_readlane(sum, 63);
+  }
+}
+// first tile of share j (the host keeps tiles x shares below 2^31)
+__device__ __forceinline__ int share_begin(int total, int shares, int j) { return (int)((uint32_t)(total * j) / (uint32_t)shares); }
+
+__device__ __forceinline__ int64_t kv_tile_row(const DecodeArgs &p, int b, int hk, int key_tile, bool &ok) {
+  // first element of the row of tiles holding keys [32 key_tile, 32 key_tile + 32) of (b, hk).  A page-table entry outside the
   // cache's blocks (an unused slot, -1) gives ok = false and the address of block 0: the caller treats those keys as masked
   const int64_t row_elems = (int64_t)32 * p.D;
   ok = true;
@@ -287,296 +331,383 @@ __device__ __forceinline__ const uint16_t *kv_tile_row(const uint16_t *base, con
     int page = p.page_table[(int64_t)b * p.pages_per_user + key_tile / tiles_per_block];
     ok = page >= 0 && page < p.blocks;
     page = ok ? page : 0;
-    return base + (((int64_t)page * p.Hkv + hk) * tiles_per_block + key_tile % tiles_per_block) * row_elems;
+    return (((int64_t)page * p.Hkv + hk) * tiles_per_block + key_tile % tiles_per_block) * row_elems;
   }
-  return base + (((int64_t)b * p.Hkv + hk) * (p.S >> 5) + key_tile) * row_elems;
+  return (((int64_t)b * p.Hkv + hk) * (p.S >> 5) + key_tile) * row_elems;
 }
 
-template <bool STREAM>
-__global__ __launch_bounds__(256) void ttm_sdpa_decode_k(DecodeArgs p) {
-  extern __shared__ float lds[];
-  const int split = blockIdx.x, bh = blockIdx.y, b = bh / p.Hkv, hk = bh % p.Hkv;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int G = p.G, D = p.D, DT = D >> 5;
-  int valid = p.S, pos = p.S - 1;
-  if (p.cur_pos) {
-    pos = p.cur_pos[b];
-    if (p.is_causal) {
-      const int cp = pos + 1;
-      valid = cp < valid ? (cp < 0 ? 0 : cp) : valid;
+// the output of head h of user b, column c; padding columns do not exist (D is a multiple of 32)
+__device__ __forceinline__ void store_head(const DecodeArgs &p, int b, int h, int c, float v) {
+  const uint16_t val = ttm_f32_to_bf16(v);
+  if (p.concat_heads) p.out[ttm_tiled_offset(b, h * p.D + c, (p.H * p.D) >> 5)] = val;
+  else p.out[(int64_t)b * ttm_round_up32(p.H) * p.D + ttm_tiled_offset(h, c, p.D >> 5)] = val;
+}
+// zeros in the padding rows of the output, by the workgroup(s) of the last user / last kv head
+__device__ __forceinline__ void store_padding(const DecodeArgs &p, int b, int hk, int tid, int threads) {
+  const int G = p.G, D = p.D;
+  if (p.concat_heads) {   // padding rows below the last user, this kv head's columns
+    if (b == p.B - 1) {
+      const int pad = (int)ttm_round_up32(p.B) - p.B;
+      for (int i = tid; i < pad * G * D; i += threads)
+        p.out[ttm_tiled_offset(p.B + i / (G * D), (hk * p.Gt + p.g0) * D + i % (G * D), (p.H * D) >> 5)] = 0;
     }
+  } else if (hk == p.Hkv - 1 && p.g0 + G == p.Gt) {   // padding rows of the last head tile
+    const int pad = (int)ttm_round_up32(p.H) - p.H;
+    for (int i = tid; i < pad * D; i += threads)
+      p.out[(int64_t)b * ttm_round_up32(p.H) * D + ttm_tiled_offset(p.H + i / D, i % D, D >> 5)] = 0;
   }
-  // first visible key; the tiles in front of it are not read at all
-  const int lo = p.window >= 0 && pos + 1 > p.window ? pos + 1 - p.window : 0;
-  const int k0 = max(split * p.keys_per_split, lo & ~31);
-  int k1 = (split + 1) * p.keys_per_split;
-  k1 = k1 < valid ? k1 : valid;
-  const int nkeys = k1 > k0 ? k1 - k0 : 0;
-  const int ngroups = (nkeys + 15) >> 4;
-  float *sc = lds;                                        // [G][keys_per_split] scores
-  float *osum = lds + (size_t)G * p.keys_per_split;       // [G][D]
-  float *stat = osum + (size_t)G * D;                     // [G][2]: max, sum
-  uint32_t *pp = (uint32_t *)(stat + 2 * G);              // [G][keys_per_split / 2] bf16 pairs of softmax numerators
-  float *slot = p.part + ((size_t)bh * p.splits + split) * G * (D + 2);
+}
 
-  for (int i = tid; i < G * D; i += 256) osum[i] = 0.0f;
-  if (nkeys == 0) {
-    for (int i = tid; i < G * (D + 2); i += 256) {
-      const int c = i % (D + 2);
-      slot[i] = c == D ? -INFINITY : 0.0f;
-    }
+// GM: most query heads, DM: most column tiles (1, 2, 4, 8), NW: wavefronts
+template <bool STREAM, int GM, int DM, bool EXACT, int NW, bool DIRECT>
+__global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void ttm_sdpa_decode_k(DecodeArgs p) {
+  constexpr int KS = DM >= 4 ? 1 : 4 / DM;   // lanes of a column pair that share the tile's keys
+  constexpr int NP = DM > 4 ? 2 : 1;         // column pairs of a lane
+  constexpr int KEYS = 32 / KS;              // keys of a tile a lane multiplies
+  __shared__ uint32_t pbuf[NW][GM][16];      // softmax numerators of a tile: pairs of adjacent keys
+  __shared__ float om[NW][GM][2];            // max, sum
+  extern __shared__ float oo[];              // [NW][G][D] outputs
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int G = p.G, D = EXACT ? 32 * DM : p.D, DT = D >> 5;
+  const int hk = DIRECT ? blockIdx.x : blockIdx.y;
+  int t0 = 0, t1 = 0, b = 0, first = 0;   // the share's tiles on the line, the user it begins in and that user's first tile
+  if (DIRECT) {
+    b = blockIdx.y;
+    t1 = visible_tiles(p, b);
   } else {
-
-  // ---- 1. scores
-  {
-    // query fragments: lane supplies query row lane % 16, columns 32 c + 8 (lane / 16) .. + 7
-    const int g = lane & 15, dq = (lane >> 4) * 8;
-    bf16x8 qf[8];
-    const int h = hk * p.Gt + p.g0 + g;
-    const uint16_t *qb = p.q + (int64_t)b * ttm_round_up32(p.H) * D;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      u32x4 z = {0, 0, 0, 0};
-      if (c < DT && g < G) z = *(const u32x4 *)(qb + ttm_tiled_offset(h, 32 * c + dq, DT));
-      qf[c] = *(bf16x8 *)&z;
-    }
-    const int hrow = hk * p.Gt + p.g0;  // mask rows of this block's heads
-    constexpr int KU = 1;
-    for (int g0 = wave; g0 < ngroups; g0 += 4 * KU) {
-      // KU groups of 16 keys per wavefront and pass, all their loads issued before the first product (one group: 8 KiB per
-      // wavefront in flight; two measured 1.5 % slower, three and four slower still)
-      u32x4 kf[KU][8];
-      int grp[KU];
-      bool kok[KU];
-#pragma unroll
-      for (int u = 0; u < KU; ++u) {
-        grp[u] = g0 + 4 * u < ngroups ? g0 + 4 * u : g0;   // the tail repeats a valid group and skips its result
-        const int key = k0 + grp[u] * 16 + (lane & 15);     // this lane's key column of the B operand
-        const uint16_t *kt = kv_tile_row(p.k, p, b, hk, key >> 5, kok[u]);
-        // inside a tile: face (key half, column half), row key % 16, columns dq % 16 .. + 7
-        const int in_tile = (((key >> 4) & 1) * 2 + (dq >> 4)) * 256 + (key & 15) * 16 + (dq & 15);
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-          if (c < DT) kf[u][c] = kv_load<STREAM>((const u32x4 *)(kt + (int64_t)c * 1024 + in_tile));
+    int unused, total;
+    line_of(p, 0, lane, unused, unused, total);
+    t0 = share_begin(total, p.shares, blockIdx.x);
+    t1 = share_begin(total, p.shares, blockIdx.x + 1);
+    if (t0 >= t1) return;
+    for (int b0 = 0; b0 < p.B; b0 += 64) {
+      const int own = b0 + lane < p.B ? visible_tiles(p, b0 + lane) : 0;
+      const int n = wave_scan(own);
+      const uint64_t past = __ballot(first + n > t0);   // users that end behind t0
+      if (past) {
+        const int l = __ffsll((unsigned long long)past) - 1;
+        b = b0 + l;
+        first += __builtin_amdgcn_readlane(n - own, l);
+        break;
       }
+      first += __builtin_amdgcn_readlane(n, 63);
+    }
+    b = __builtin_amdgcn_readfirstlane(b);
+    first = __builtin_amdgcn_readfirstlane(first);
+  }
+  // lane roles: score phase (head hq, keys 4 kq .. + 3 of 16), product phase (column pairs cp + 64 i, keys KEYS ks .. of 32)
+  const int hq = lane & 15, kq = lane >> 4, dq = kq * 8;
+  const int cp = DM == 1 ? lane & 15 : DM == 2 ? lane & 31 : lane, ks = DM == 1 ? lane >> 4 : DM == 2 ? lane >> 5 : 0;
+  const int k_off = (dq >> 4) * 256 + hq * 16 + (dq & 15);   // inside a tile; + 512 for keys 16 .. 31 (A operand row = lane % 16)
+  int v_off[NP];
 #pragma unroll
-      for (int u = 0; u < KU; ++u) {
-        if (u == 1 && g0 + 4 >= ngroups) break;
-        f32x4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int n = 0; n < NP; ++n) {
+    const int c = 2 * min(cp + 64 * n, 16 * DT - 1);
+    v_off[n] = (c >> 5) * 1024 + ((c >> 4) & 1) * 256 + (c & 15) + ks * (KEYS == 8 ? 0 : 512);
+    if (KEYS == 8) v_off[n] += (ks >> 1) * 512 + (ks & 1) * 128;
+  }
+  // (the line's last user ends the loop: t1 is at most the total)
+  for (int next; first < t1 || DIRECT; ++b, first = next) {   // workgroup-uniform
+  next = DIRECT ? t1 : first + visible_tiles(p, b);
+  if (!DIRECT && next == first) continue;
+  int lo, valid;
+  visible_keys(p, b, lo, valid);
+  const int tb = (lo >> 5) - first;                 // tile on the line + tb = tile of the user's cache
+  const int ta = max(t0, first), tz = min(t1, next);
+  // query fragments: lane supplies head lane % 16, columns 32 c + 8 (lane / 16) .. + 7
+  bf16x8 qf[DM];
+  const uint16_t *qb = p.q + (int64_t)b * ttm_round_up32(p.H) * D;
 #pragma unroll
-        for (int c = 0; c < 8; ++c)
-          if (c < DT) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf[c], *(bf16x8 *)&kf[u][c], acc, 0, 0, 0);
-        // acc[i] = score of query 4 (lane / 16) + i against key lane % 16 of the group
-        const int kk = grp[u] * 16 + (lane & 15);
+  for (int c = 0; c < DM; ++c) {
+    u32x4 z = {0, 0, 0, 0};
+    if (c < DT && hq < G) z = *(const u32x4 *)(qb + ttm_tiled_offset(hk * p.Gt + p.g0 + hq, 32 * c + dq, DT));
+    qf[c] = *(bf16x8 *)&z;
+  }
+  float m = -INFINITY, l = 0.0f, o[GM][NP][2];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int gq = (lane >> 4) * 4 + i;
-          if (gq < G) {
-            float sv = acc[i];
-            if (p.mask) {
-              const int mh = p.mask_heads == 1 ? 0 : hrow + gq;
-              const int64_t mrows = ttm_round_up32(p.mask_heads);
-              sv += ttm_bf16_to_f32(p.mask[(int64_t)b * p.mask_b * mrows * p.S + ttm_tiled_offset(mh, k0 + kk, p.S >> 5)]);
-            }
-            sc[gq * p.keys_per_split + kk] = (k0 + kk < k1 && k0 + kk >= lo && kok[u]) ? sv * p.scale : -INFINITY;
+  for (int g = 0; g < GM; ++g)
+#pragma unroll
+    for (int n = 0; n < NP; ++n) o[g][n][0] = o[g][n][1] = 0.0f;
+  u32x4 kf[2][DM];
+  uint32_t vf[NP][KEYS];
+  bool kok = true, vok = true;
+  int64_t krow = 0, vrow = 0;
+  auto load_k = [&](int t) __attribute__((always_inline)) {
+    krow = kv_tile_row(p, b, hk, t + tb, kok);
+    const uint16_t *kt = p.k + krow + k_off;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int c = 0; c < DM; ++c)
+        if (c < DT) kf[u][c] = kv_load<STREAM>((const u32x4 *)(kt + c * 1024 + u * 512));
+  };
+  auto load_v = [&]() __attribute__((always_inline)) {   // of the tile whose K was requested last
+    vrow = krow;
+    vok = kok;
+    const uint16_t *vt = p.v + vrow;
+#pragma unroll
+    for (int n = 0; n < NP; ++n)
+#pragma unroll
+      for (int r = 0; r < KEYS; ++r)   // four rows share a line
+        vf[n][r] = *(const uint32_t *)(vt + v_off[n] + (r >> 4) * 512 + (r & 15) * 16);
+  };
+  int t = ta + wave;
+  if (t < tz) { load_k(t); load_v(); }
+  for (; t < tz; t += NW) {
+    const int kb = (t + tb) * 32;   // first key
+    f32x4 s[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      s[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int c = 0; c < DM; ++c)
+        if (c < DT) s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(bf16x8 *)&kf[u][c], qf[c], s[u], 0, 0, 0);
+    }
+    const bool ok = kok;
+    // pins the products in front of the loads that overwrite their operands (left to itself the compiler copies the 64 registers
+    // and multiplies behind the next tile's requests)
+    asm volatile("" : "+v"(s[0]), "+v"(s[1]));
+    if (t + NW < tz) load_k(t + NW);   // wavefront-uniform
+    const bool inner = ok && kb >= lo && kb + 32 <= valid;   // wavefront-uniform: every key of the tile is visible
+    float tm = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = kb + u * 16 + kq * 4 + i;
+        float x = s[u][i];
+        if (p.mask && hq < G) {
+          const int mh = p.mask_heads == 1 ? 0 : hk * p.Gt + p.g0 + hq;
+          x += ttm_bf16_to_f32(p.mask[(int64_t)b * p.mask_b * ttm_round_up32(p.mask_heads) * p.S + ttm_tiled_offset(mh, key, p.S >> 5)]);
+        }
+        x *= p.scale;
+        s[u][i] = inner || (ok && key >= lo && key < valid) ? x : -INFINITY;
+        tm = fmaxf(tm, s[u][i]);
+      }
+    tm = fmaxf(tm, __shfl_xor(tm, 16));
+    tm = fmaxf(tm, __shfl_xor(tm, 32));
+    const float mn = fmaxf(m, tm);
+    const float alpha = m == mn ? 1.0f : __expf(m - mn);      // (-inf, -inf) -> 1, (-inf, finite) -> 0
+    l *= alpha;
+    m = mn;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      uint32_t pair[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float x = s[u][2 * e], y = s[u][2 * e + 1];
+        pair[e] = ttm_pack_bf16x2(x == -INFINITY ? 0.0f : __expf(x - mn), y == -INFINITY ? 0.0f : __expf(y - mn));
+        l += __uint_as_float(pair[e] << 16) + __uint_as_float(pair[e] & 0xFFFF0000u);   // numerator and denominator see the same rounding
+      }
+      if (hq < GM) *(u32x2 *)&pbuf[wave][hq][u * 8 + kq * 2] = u32x2{pair[0], pair[1]};
+    }
+    if (__any(alpha != 1.0f && hq < GM)) {
+#pragma unroll
+      for (int g = 0; g < GM; ++g) {
+        const float ag = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(alpha), g));
+#pragma unroll
+        for (int n = 0; n < NP; ++n) { o[g][n][0] *= ag; o[g][n][1] *= ag; }
+      }
+    }
+    // LDS traffic of one wavefront is processed in order; the fence only pins the compiler's order
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (!inner) {   // rows outside the visible keys may hold anything, NaN included
+#pragma unroll
+      for (int r = 0; r < KEYS; ++r) {
+        const int key = kb + ks * KEYS + r;
+        const bool in = ok && key >= lo && key < valid;
+#pragma unroll
+        for (int n = 0; n < NP; ++n) vf[n][r] = in ? vf[n][r] : 0u;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < KEYS / 2; j += 4) {
+      uint32_t vp[NP][4][2];   // (key 2 j, key 2 j + 1) of either column
+#pragma unroll
+      for (int n = 0; n < NP; ++n)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          vp[n][e][0] = __builtin_amdgcn_perm(vf[n][2 * (j + e) + 1], vf[n][2 * (j + e)], 0x05040100u);
+          vp[n][e][1] = __builtin_amdgcn_perm(vf[n][2 * (j + e) + 1], vf[n][2 * (j + e)], 0x07060302u);
+        }
+#pragma unroll
+      for (int g = 0; g < GM; ++g) {
+        const u32x4 pg = *(const u32x4 *)&pbuf[wave][g][ks * (KEYS / 2) + j];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int n = 0; n < NP; ++n) {
+            const uint32_t pe = pg[e];
+            o[g][n][0] = __builtin_amdgcn_fdot2_f32_bf16(*(bf16x2 *)&vp[n][e][0], *(const bf16x2 *)&pe, o[g][n][0], false);
+            o[g][n][1] = __builtin_amdgcn_fdot2_f32_bf16(*(bf16x2 *)&vp[n][e][1], *(const bf16x2 *)&pe, o[g][n][1], false);
           }
+      }
+      __builtin_amdgcn_sched_barrier(0);   // eight keys at a time: all numerators and pairs at once do not fit the registers
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int g = 0; g < GM; ++g)
+#pragma unroll
+      for (int n = 0; n < NP; ++n) asm volatile("" : "+v"(o[g][n][0]), "+v"(o[g][n][1]));
+    if (t + NW < tz) load_v();
+  }
+  // the wavefronts' results meet in LDS
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  if (kq == 0 && hq < GM) { om[wave][hq][0] = m; om[wave][hq][1] = l; }
+#pragma unroll
+  for (int g = 0; g < GM; ++g) {
+    if (g < G) {
+#pragma unroll
+      for (int n = 0; n < NP; ++n) {
+        float x = o[g][n][0], y = o[g][n][1];
+        if (KS >= 2) { x += __shfl_xor(x, 32); y += __shfl_xor(y, 32); }
+        if (KS == 4) { x += __shfl_xor(x, 16); y += __shfl_xor(y, 16); }
+        if (ks == 0 && cp + 64 * n < 16 * DT) {
+          oo[(wave * G + g) * D + 2 * (cp + 64 * n)] = x;
+          oo[(wave * G + g) * D + 2 * (cp + 64 * n) + 1] = y;
         }
       }
     }
   }
   __syncthreads();
-
-  // ---- 2. softmax numerators: wave w serves heads w, w + 4, ...  The numerators are rounded to bf16 and stored in pairs
-  // (key r, key r + 16 of a 32-key tile) so that the next phase multiplies two keys per instruction; their sum is taken
-  // over the rounded values, which keeps numerator and denominator consistent.
-  const int padded = ngroups * 16, ntiles = (ngroups + 1) >> 1;
-  for (int g = wave; g < G; g += 4) {
-    const float *row = sc + g * p.keys_per_split;
-    uint32_t *prow = pp + g * (p.keys_per_split >> 1);
-    float m = -INFINITY;
-    for (int i = lane; i < padded; i += 64) m = fmaxf(m, row[i]);
+  float *slot = DIRECT ? nullptr : p.part + ((size_t)hk * (p.shares + p.B) + blockIdx.x + b) * G * (D + 2);
+  for (int i = tid; i < G * D; i += NW * 64) {
+    const int g = i / D, c = i - g * D, h = hk * p.Gt + p.g0 + g;
+    const float sinkv = DIRECT && p.sink ? ttm_bf16_to_f32(p.sink[ttm_tiled_offset(h, 0, 1)]) * p.scale : -INFINITY;
+    float M = sinkv;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-    float l = 0.0f;
-    for (int i = lane; i < ntiles * 16; i += 64) {
-      const int klo = (i >> 4) * 32 + (i & 15), khi = klo + 16;
-      const float elo = (m == -INFINITY || klo >= padded) ? 0.0f : __expf(row[klo] - m);
-      const float ehi = (m == -INFINITY || khi >= padded) ? 0.0f : __expf(row[khi] - m);
-      const uint32_t pair = ttm_pack_bf16x2(elo, ehi);
-      prow[i] = pair;
-      l += __uint_as_float(pair << 16) + __uint_as_float(pair & 0xFFFF0000u);
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, om[w][g][0]);
+    float num = 0.0f, den = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float e = om[w][g][0] == -INFINITY ? 0.0f : __expf(om[w][g][0] - M);
+      num += oo[(w * G + g) * D + c] * e;
+      den += om[w][g][1] * e;
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
-    if (lane == 0) { stat[2 * g] = m; stat[2 * g + 1] = l; }
-  }
-  __syncthreads();
-
-  // ---- 3. P V with v_dot2_f32_bf16: work items are (column tile, stride class of key tiles).  Per key tile a lane reads
-  // 8 columns of key r (faces 0 / 1) and of key r + 16 (faces 2 / 3), r = (lane % 32) / 2, columns
-  // 16 (lane / 32) + 8 (lane % 2) .. + 7; the two rows are interleaved to (v[r][d], v[r + 16][d]) pairs and multiplied with
-  // the stored (p[r], p[r + 16]) pair.
-  {
-    const int share = DT == 1 ? 4 : (DT == 2 ? 2 : 1);   // with one or two column tiles several waves split the keys of one
-    const int items = DT * share;
-    const int krow = (lane & 31) >> 1;
-    constexpr int UT = 4;                                  // key tiles in flight per pass (8 KiB per wave)
-    for (int item = wave; item < items; item += 4) {
-      const int dt = item % DT, tfirst = item / DT;
-      float o[kMaxG][8];
-#pragma unroll
-      for (int g = 0; g < kMaxG; ++g)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o[g][j] = 0.0f;
-      for (int t0 = tfirst; t0 < ntiles; t0 += UT * share) {
-        u32x4 ra[UT], rb[UT];
-        bool vok[UT];
-#pragma unroll
-        for (int u = 0; u < UT; ++u) {
-          const int t = t0 + u * share < ntiles ? t0 + u * share : t0;
-          const uint16_t *vt = kv_tile_row(p.v, p, b, hk, (k0 >> 5) + t, vok[u]) + (int64_t)dt * 1024;
-          ra[u] = kv_load<STREAM>((const u32x4 *)(vt + lane * 8));
-          rb[u] = kv_load<STREAM>((const u32x4 *)(vt + 512 + lane * 8));
-        }
-#pragma unroll
-        for (int u = 0; u < UT; ++u) {
-          const int t = t0 + u * share;
-          if (t >= ntiles) break;
-          uint32_t a[4] = {ra[u].x, ra[u].y, ra[u].z, ra[u].w}, c[4] = {rb[u].x, rb[u].y, rb[u].z, rb[u].w};
-          if (t * 32 + 32 > nkeys || k0 + t * 32 < lo || !vok[u]) {   // boundary tile: rows outside the visible keys may hold anything, NaN included
-            const bool la = vok[u] && t * 32 + krow < nkeys && k0 + t * 32 + krow >= lo;
-            const bool lb = vok[u] && t * 32 + 16 + krow < nkeys && k0 + t * 32 + 16 + krow >= lo;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) { a[j] = la ? a[j] : 0u; c[j] = lb ? c[j] : 0u; }
-          }
-          uint32_t vp[8];   // vp[2 j] = (a.col 2j, c.col 2j), vp[2 j + 1] = (a.col 2j+1, c.col 2j+1)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            vp[2 * j] = __builtin_amdgcn_perm(c[j], a[j], 0x05040100u);
-            vp[2 * j + 1] = __builtin_amdgcn_perm(c[j], a[j], 0x07060302u);
-          }
-#pragma unroll
-          for (int g = 0; g < kMaxG; ++g) {
-            if (g < G) {
-              const uint32_t pg = pp[g * (p.keys_per_split >> 1) + t * 16 + krow];
-#pragma unroll
-              for (int j = 0; j < 8; ++j)
-                o[g][j] = __builtin_amdgcn_fdot2_f32_bf16(*(bf16x2 *)&vp[j], *(const bf16x2 *)&pg, o[g][j], false);
-            }
-          }
-        }
-      }
-      // combine the 16 lanes that hold the same columns (they differ in bits 1..4 of the lane id)
-#pragma unroll
-      for (int g = 0; g < kMaxG; ++g) {
-        if (g < G) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            float v = o[g][j];
-            v += __shfl_xor(v, 2);
-            v += __shfl_xor(v, 4);
-            v += __shfl_xor(v, 8);
-            v += __shfl_xor(v, 16);
-            o[g][j] = v;
-          }
-        }
-      }
-      if (((lane >> 1) & 15) == 0) {
-        const int col = dt * 32 + (lane >> 5) * 16 + (lane & 1) * 8;
-#pragma unroll
-        for (int g = 0; g < kMaxG; ++g)
-          if (g < G)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              if (share == 1) osum[g * D + col + j] = o[g][j];
-              else atomicAdd(&osum[g * D + col + j], o[g][j]);
-            }
-      }
+    if (DIRECT) {
+      if (p.sink) den += __expf(sinkv - M);
+      store_head(p, b, h, c, den > 0.0f ? num / den : 0.0f);
+    } else {
+      slot[g * (D + 2) + c] = num;
+      if (c == 0) { slot[g * (D + 2) + D] = M; slot[g * (D + 2) + D + 1] = den; }
     }
   }
-  __syncthreads();
-
-  // ---- 4. the split's slot
-  for (int i = tid; i < G * (D + 2); i += 256) {
-    const int g = i / (D + 2), c = i % (D + 2);
-    slot[i] = c < D ? osum[g * D + c] : stat[2 * g + (c - D)];
+  if (DIRECT) {
+    store_padding(p, b, hk, tid, NW * 64);
+    return;
   }
-  }  // nkeys != 0
+  __syncthreads();   // the next user's piece reuses the arrays
+  }  // users of this share
 }
 
-// merges the slots of one query head: out = sum_s o_s exp(m_s - M) / sum_s l_s exp(m_s - M).  grid (B * Hkv, G), 256 lanes:
-// the weights exp(m_s - M) of the slices are formed once in LDS; 256 / D lanes share a column and take every (256 / D)-th
-// slice, so that a long cache cut into many slices for a few users (one user, 32768 positions: 64 slices) is merged by all
-// lanes of 32 workgroups instead of by eight workgroups looping over the slices.
+// merges a user's slots: out = sum_s o_s exp(m_s - M) / sum_s l_s exp(m_s - M).  grid (B * Hkv, G D / 256), 256 lanes.  Up to 16
+// slots a lane per output forms everything itself; more (few users with long caches) go through LDS: the weights exp(m_s - M)
+// are formed once per head, 256 / D lanes share a column and take every (256 / D)-th slot.
 constexpr int kMaxCombineSlices = 1024;
 __global__ __launch_bounds__(256) void ttm_sdpa_decode_combine_k(DecodeArgs p) {
   __shared__ float wgt[kMaxCombineSlices];
   __shared__ float red[256];
-  __shared__ float stats[2];
+  __shared__ float stats[4];
   const int bh = blockIdx.x, tid = threadIdx.x;
   const int b = bh / p.Hkv, hk = bh % p.Hkv;
-  const int G = p.G, D = p.D, S = p.splits;
-  for (int g = blockIdx.y; g < G; g += gridDim.y) {   // grid.y = G: one head per workgroup (workgroup-uniform)
-  const float *base = p.part + (size_t)bh * S * G * (D + 2) + (size_t)g * (D + 2);   // slice s: + s * G * (D + 2)
+  const int G = p.G, D = p.D;
+  // the user's tiles on the line and the shares that hold them
+  int before, total, mine;
+  line_of(p, b, tid & 63, before, mine, total);
+  // share of tile t: the last one that begins at or before it
+  auto share_of = [&](int t) { return (int)(((uint32_t)((t + 1) * p.shares) - 1u) / (uint32_t)total); };
+  const int j0 = mine ? share_of(before) : 0, S = mine ? share_of(before + mine - 1) - j0 + 1 : 0;
+  const bool gaps = total < p.shares;   // fewer tiles than shares: some of them are empty and left their slots as they were
+  auto empty = [&](int s) { return gaps && share_begin(total, p.shares, j0 + s) == share_begin(total, p.shares, j0 + s + 1); };
+  if (S <= 16) {   // a lane per output: independent loads, no barriers
+    for (int idx = blockIdx.y * 256 + tid; idx < G * D; idx += gridDim.y * 256) {
+      const int g = idx / D, c = idx - g * D, h = hk * p.Gt + p.g0 + g;
+      const float *base = p.part + (((size_t)hk * (p.shares + p.B) + j0 + b) * G + g) * (D + 2);
+      const size_t sstride = (size_t)G * (D + 2);
+      const float sinkv = p.sink ? ttm_bf16_to_f32(p.sink[ttm_tiled_offset(h, 0, 1)]) * p.scale : -INFINITY;
+      float M = sinkv, num = 0.0f, den = 0.0f;
+      if (gaps) {
+        for (int s = 0; s < S; ++s)
+          if (!empty(s)) M = fmaxf(M, base[s * sstride + D]);
+        for (int s = 0; s < S; ++s) {
+          if (empty(s) || base[s * sstride + D] == -INFINITY) continue;
+          const float w = __expf(base[s * sstride + D] - M);
+          num += base[s * sstride + c] * w;
+          den += base[s * sstride + D + 1] * w;
+        }
+      } else {
+#pragma unroll 8
+        for (int s = 0; s < S; ++s) M = fmaxf(M, base[s * sstride + D]);
+#pragma unroll 8
+        for (int s = 0; s < S; ++s) {
+          const float ms = base[s * sstride + D], w = ms == -INFINITY ? 0.0f : __expf(ms - M);
+          num += base[s * sstride + c] * w;
+          den += base[s * sstride + D + 1] * w;
+        }
+      }
+      if (p.sink) den += __expf(sinkv - M);
+      store_head(p, b, h, c, den > 0.0f ? num / den : 0.0f);
+    }
+    if (blockIdx.y == 0) store_padding(p, b, hk, tid, 256);
+    return;
+  }
+  for (int g = blockIdx.y; g < G; g += gridDim.y) {   // workgroup-uniform
+  const float *base = p.part + ((size_t)hk * (p.shares + p.B) + j0 + b) * G * (D + 2) + (size_t)g * (D + 2);   // piece s: + s * G * (D + 2)
   const size_t sstride = (size_t)G * (D + 2);
   const int h = hk * p.Gt + p.g0 + g;
   const float sinkv = p.sink ? ttm_bf16_to_f32(p.sink[ttm_tiled_offset(h, 0, 1)]) * p.scale : -INFINITY;
   // M = max over the slices (and the sink)
   float m = sinkv;
-  for (int s = tid; s < S; s += 256) m = fmaxf(m, base[s * sstride + D]);
+  for (int s = tid; s < S; s += 256)
+    if (!empty(s)) m = fmaxf(m, base[s * sstride + D]);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
   if ((tid & 63) == 0) red[tid >> 6] = m;
   __syncthreads();
   const float M = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   __syncthreads();
-  // weights and the denominator
-  float den = 0.0f;
-  for (int s = tid; s < S; s += 256) {
-    const float ms = base[s * sstride + D];
-    const float w = ms == -INFINITY ? 0.0f : __expf(ms - M);
-    wgt[s] = w;
-    den += base[s * sstride + D + 1] * w;
+  // weights, denominator and numerators, kMaxCombineSlices pieces at a time: lane (c, sub) sums the pieces sub, sub + nsub, ... of
+  // column c
+  const int nsub = 256 / D > 0 ? 256 / D : 1;
+  const int c = tid % D, sub = tid / D;
+  float den = 0.0f, num = 0.0f;
+  for (int s0 = 0; s0 < S; s0 += kMaxCombineSlices) {
+    const int n = min(S - s0, kMaxCombineSlices);
+    for (int s = tid; s < n; s += 256) {
+      const float ms = empty(s0 + s) ? -INFINITY : base[(s0 + s) * sstride + D];
+      const float w = ms == -INFINITY ? 0.0f : __expf(ms - M);
+      wgt[s] = w;
+      if (w != 0.0f) den += base[(s0 + s) * sstride + D + 1] * w;
+    }
+    __syncthreads();
+    if (sub < nsub) {
+      if (gaps) {
+        for (int s = sub; s < n; s += nsub)
+          if (wgt[s] != 0.0f) num += base[(s0 + s) * sstride + c] * wgt[s];
+      } else {
+#pragma unroll 8
+        for (int s = sub; s < n; s += nsub) num += base[(s0 + s) * sstride + c] * wgt[s];
+      }
+    }
+    __syncthreads();
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) den += __shfl_xor(den, o);
-  if ((tid & 63) == 0) red[tid >> 6] = den;
+  if ((tid & 63) == 0) stats[tid >> 6] = den;
+  red[tid] = num;
   __syncthreads();
-  if (tid == 0) stats[0] = (red[0] + red[1]) + (red[2] + red[3]) + (p.sink ? __expf(sinkv - M) : 0.0f);
-  __syncthreads();
-  den = stats[0];
-  // numerators: lane (c, sub) sums the slices sub, sub + nsub, ... of column c
-  const int nsub = 256 / D > 0 ? 256 / D : 1;
-  for (int c0 = 0; c0 < D; c0 += 256) {   // one round unless D > 256
-    const int c = c0 + (tid % (D < 256 ? D : 256)), sub = D < 256 ? tid / D : 0;
-    float num = 0.0f;
-    if (c < D && sub < nsub)
-      for (int s = sub; s < S; s += nsub) num += base[s * sstride + c] * wgt[s];
-    red[tid] = num;
-    __syncthreads();
-    if (c < D && sub == 0) {
-      for (int u = 1; u < nsub; ++u) num += red[tid + u * D];
-      const uint16_t val = ttm_f32_to_bf16(den > 0.0f ? num / den : 0.0f);
-      if (p.concat_heads) p.out[ttm_tiled_offset(b, h * D + c, (p.H * D) >> 5)] = val;
-      else p.out[(int64_t)b * ttm_round_up32(p.H) * D + ttm_tiled_offset(h, c, D >> 5)] = val;
-    }
-    __syncthreads();
+  den = (stats[0] + stats[1]) + (stats[2] + stats[3]) + (p.sink ? __expf(sinkv - M) : 0.0f);
+  if (sub == 0) {
+    for (int u = 1; u < nsub; ++u) num += red[tid + u * D];
+    store_head(p, b, h, c, den > 0.0f ? num / den : 0.0f);
   }
+  __syncthreads();
   }  // heads of this workgroup
-  if (blockIdx.y != 0) return;   // the padding belongs to the first head's workgroup
-  if (p.concat_heads) {   // padding rows below the last user, this kv head's columns
-    if (b == p.B - 1) {
-      const int pad = (int)ttm_round_up32(p.B) - p.B;
-      for (int i = tid; i < pad * G * D; i += 256)
-        p.out[ttm_tiled_offset(p.B + i / (G * D), (hk * p.Gt + p.g0) * D + i % (G * D), (p.H * D) >> 5)] = 0;
-    }
-    return;
-  }
-  if (hk == p.Hkv - 1 && p.g0 + G == p.Gt) {   // padding rows of the last head tile
-    const int pad = (int)ttm_round_up32(p.H) - p.H;
-    for (int i = tid; i < pad * D; i += 256)
-      p.out[(int64_t)b * ttm_round_up32(p.H) * D + ttm_tiled_offset(p.H + i / D, i % D, D >> 5)] = 0;
-  }
+  if (blockIdx.y == 0) store_padding(p, b, hk, tid, 256);   // the padding belongs to the first head's workgroup
 }
 
 }  // namespace
@@ -740,6 +871,26 @@ static int decode_scratch_ptr(void **ptr) {
   return TTM_OK;
 }
 
+template <bool STREAM, int GM, int DM, bool EXACT, int NW, bool DIRECT>
+static void launch_decode(const DecodeArgs &p, dim3 grid, hipStream_t s) {
+  const size_t lds = (size_t)NW * p.G * p.D * sizeof(float);   // at most 32 KiB
+  hipLaunchKernelGGL((ttm_sdpa_decode_k<STREAM, GM, DM, EXACT, NW, DIRECT>), grid, dim3(NW * 64), lds, s, p);
+}
+// The head dims 32, 64, 128 and 256 have kernels of their own; others, and heads in several launches, the next larger one's loops
+// with a bound.  Up to four heads (and 128 columns) the direct form holds its state in 128 registers and takes 16 wavefronts.
+template <bool DIRECT>
+static void launch_decode(const DecodeArgs &p, dim3 grid, hipStream_t s) {
+  constexpr int NW = DIRECT ? 8 : 4, NWS = DIRECT ? 16 : 4;
+  const bool few = p.G <= 4 && p.Gt <= kMaxG, once = p.Gt <= kMaxG;
+  switch (p.D) {
+  case 32: return few ? launch_decode<true, 4, 1, true, NWS, DIRECT>(p, grid, s) : once ? launch_decode<true, 8, 1, true, NW, DIRECT>(p, grid, s) : launch_decode<false, 8, 1, true, NW, DIRECT>(p, grid, s);
+  case 64: return few ? launch_decode<true, 4, 2, true, NWS, DIRECT>(p, grid, s) : once ? launch_decode<true, 8, 2, true, NW, DIRECT>(p, grid, s) : launch_decode<false, 8, 2, true, NW, DIRECT>(p, grid, s);
+  case 128: return few ? launch_decode<true, 4, 4, true, NWS, DIRECT>(p, grid, s) : once ? launch_decode<true, 8, 4, true, NW, DIRECT>(p, grid, s) : launch_decode<false, 8, 4, true, NW, DIRECT>(p, grid, s);
+  case 256: return few ? launch_decode<true, 4, 8, true, NW, DIRECT>(p, grid, s) : once ? launch_decode<true, 8, 8, true, NW, DIRECT>(p, grid, s) : launch_decode<false, 8, 8, true, NW, DIRECT>(p, grid, s);
+  default: return p.D < 128 ? launch_decode<false, 8, 4, false, NW, DIRECT>(p, grid, s) : launch_decode<false, 8, 8, false, NW, DIRECT>(p, grid, s);
+  }
+}
+
 static int sdpa_decode_entry(const void *q, const void *k, const void *v, const int32_t *cur_pos, const void *mask, int mask_heads,
                              const int32_t *page_table, int64_t pages_per_user, int64_t page_block, int64_t page_blocks, void *out, int dtype, int64_t batch,
                              int64_t heads, int64_t kv_heads, int64_t seq, int64_t head_dim, int is_causal, float scale, int concat_heads,
@@ -760,20 +911,24 @@ static int sdpa_decode_entry(const void *q, const void *k, const void *v, const 
                 (long long)page_blocks);
   }
   hipStream_t s = (hipStream_t)stream;
-  // enough blocks to fill the device, slices small enough for the score rows to fit in LDS
-  int64_t splits = ttm_cdiv(SPLIT_TARGET, batch * kv_heads);
-  const int64_t max_keys = (48 * 1024 / 6) / G / 32 * 32;   // 4 bytes of score + 2 of numerator per key and head
-  if (splits > seq / 256) splits = seq / 256 > 0 ? seq / 256 : 1;
-  if (ttm_cdiv(seq, splits) > max_keys) splits = ttm_cdiv(seq, max_keys);
-  const int64_t keys = ttm_round_up32(ttm_cdiv(seq, splits));
-  splits = ttm_cdiv(seq, keys);
-  TTM_REQUIRE(splits <= kMaxCombineSlices, "ttm_sdpa_decode: a cache of %lld positions takes %lld key slices, the merge handles %d", (long long)seq,
-              (long long)splits, kMaxCombineSlices);
+  // Direct form where the users alone fill the device or their caches are short; shares for few users with long caches.  Measured
+  // (D = 128, 8 kv heads; direct / shares, us, contexts of a quarter of the cache to all of it | all of it): 1 user x 512
+  // positions 8.5 / 11.0 | 7.9 / 10.6, 1 x 1024 12.7 / 12.0 | 11.7 / 11.7, 1 x 2048 14.9 / 15.8 | 22.3 / 15.4, 8 x 1024 15.5 / 20.8 |
+  // 15.7 / 17.0, 8 x 2048 21.5 / 23.3 | 25.8 / 21.8, 16 x 2048 26.1 / 26.7 | 27.0 / 30.4, 16 x 4096 47.9 / 39.2 | 56.2 / 51.9,
+  // 32 x 2048 33.5 / 36.5 | 46.0 / 50.9, 32 x 4096 65.3 / 64.8 | 85.1 / 91.5.
+  const int form = ttm_option("sdpa_decode_form");   // 0 by this rule, 1 direct, 2 shares
+  // (the results of the wavefronts fit in 32 KiB of LDS)
+  const bool direct = G * head_dim <= 1024 && (form ? form == 1 : seq * head_dim <= 2048 * std::max<int64_t>(64, batch * kv_heads));
+  const int64_t all = batch * (seq / 32);          // tiles of a kv head when every cache is full
+  int64_t shares = ttm_cdiv(kDecodeBlocks, kv_heads);
+  if (shares > all / 4) shares = all / 4 > 0 ? all / 4 : 1;   // a tile for every wavefront
+  if (shares > INT32_MAX / (all + 1)) shares = INT32_MAX / (all + 1);
+  TTM_REQUIRE(all < INT32_MAX, "ttm_sdpa_decode: caches of %lld x %lld positions are too long", (long long)batch, (long long)seq);
   DecodeArgs p;
   p.q = (const uint16_t *)q; p.k = (const uint16_t *)k; p.v = (const uint16_t *)v; p.mask = (const uint16_t *)mask;
   p.cur_pos = cur_pos; p.page_table = page_table; p.out = (uint16_t *)out;
   p.B = (int)batch; p.H = (int)heads; p.Hkv = (int)kv_heads; p.G = (int)G; p.S = (int)seq; p.D = (int)head_dim;
-  p.splits = (int)splits; p.keys_per_split = (int)keys; p.block = (int)page_block; p.pages_per_user = (int)pages_per_user;
+  p.shares = (int)shares; p.block = (int)page_block; p.pages_per_user = (int)pages_per_user;
   p.blocks = (int)page_blocks;
   p.mask_heads = mask_heads; p.is_causal = is_causal; p.concat_heads = concat_heads;
   p.scale = scale > 0.0f ? scale : 1.0f / sqrtf((float)head_dim);
@@ -783,11 +938,11 @@ static int sdpa_decode_entry(const void *q, const void *k, const void *v, const 
   TTM_REQUIRE(!mask || mask_batch == 1 || mask_batch == batch, "ttm_sdpa_decode: mask batch must be 1 or %lld", (long long)batch);
   p.mask_b = mask_batch == 1 ? 0 : 1;
   void *ws = nullptr;
-  const size_t part_bytes = (size_t)(batch * kv_heads * splits * G * (head_dim + 2)) * sizeof(float);
+  const size_t part_bytes = (size_t)(kv_heads * (shares + batch) * G * (head_dim + 2)) * sizeof(float);
   if (static_scratch) {
     TTM_REQUIRE(part_bytes <= kDecodeScratchBytes,
                 "ttm_sdpa_decode_static: the per-slice partial results of this call take %zu bytes, the static scratch holds %zu "
-                "(batch * kv_heads * slices * heads-per-kv-head * (head_dim + 2) floats): use ttm_sdpa_decode_windowed",
+                "(kv_heads * (shares + batch) * heads-per-kv-head * (head_dim + 2) floats): use ttm_sdpa_decode_windowed",
                 part_bytes, (size_t)kDecodeScratchBytes);
     if (int rc = decode_scratch_ptr(&ws)) return rc;
   } else {
@@ -797,11 +952,14 @@ static int sdpa_decode_entry(const void *q, const void *k, const void *v, const 
   for (int64_t g0 = 0; g0 < Gt; g0 += kMaxG) {   // the launches of one call follow each other on the stream and share the workspace
     p.g0 = (int)g0;
     p.G = (int)(Gt - g0 < kMaxG ? Gt - g0 : kMaxG);
-    const size_t lds = (size_t)(p.G * keys + p.G * head_dim + 2 * p.G + p.G * keys / 2) * sizeof(float);
-    if (Gt <= kMaxG) hipLaunchKernelGGL(ttm_sdpa_decode_k<true>, dim3((unsigned)splits, (unsigned)(batch * kv_heads)), dim3(256), lds, s, p);
-    else hipLaunchKernelGGL(ttm_sdpa_decode_k<false>, dim3((unsigned)splits, (unsigned)(batch * kv_heads)), dim3(256), lds, s, p);
+    if (direct) {
+      launch_decode<true>(p, dim3((unsigned)kv_heads, (unsigned)batch), s);
+      TTM_LAUNCH_CHECK();
+      continue;
+    }
+    launch_decode<false>(p, dim3((unsigned)shares, (unsigned)kv_heads), s);
     TTM_LAUNCH_CHECK();
-    hipLaunchKernelGGL(ttm_sdpa_decode_combine_k, dim3((unsigned)(batch * kv_heads), (unsigned)p.G), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(ttm_sdpa_decode_combine_k, dim3((unsigned)(batch * kv_heads), (unsigned)ttm_cdiv(p.G * head_dim, 256)), dim3(256), 0, s, p);
     TTM_LAUNCH_CHECK();
   }
   return TTM_OK;
