@@ -521,6 +521,12 @@ const void *stage(DeviceState &dev, const void *src, size_t bytes) {
   return p;
 }
 
+// Over PCIe every access costs: a layout kernel goes to host memory itself only where the row-major rows are whole 16-byte chunks
+// (odd rows go by elements or shifted chunks, [2009, 463] bf16 by 190 us where the copy of its bytes takes 35).
+bool wholeChunkRows(const std::vector<std::uint32_t> &shape, DataType dtype) {
+  return utils::isBlockFormatDataType(dtype) || dims3(shape).cols * utils::dataTypeElementSize(dtype) % 16 == 0;
+}
+
 // src (a tensor of this shape in layout / dtype sl / sd) into dst in dl / dd with one launch; false when there is no such
 // kernel.  Either side may be page-locked host memory.
 bool convertInOneLaunch(const void *src, TensorLayout sl, DataType sd, void *dst, TensorLayout dl, DataType dd,
@@ -846,6 +852,7 @@ bool uploadInto(const Tensor &h, const Tensor &d) {
   DeviceState &dev = *d.handle->device;
   std::lock_guard<std::recursive_mutex> g(dev.mu);
   requireNotCapturing(d.handle->device, "a host to device transfer");
+  if (s.layout != d.handle->layout && !wholeChunkRows(s.shape, s.dtype)) return false;
   const void *p = stage(dev, s.data.get(), s.bytes);
   return p && convertInOneLaunch(p, s.layout, s.dtype, d.handle->data.get(), d.handle->layout, d.handle->dtype, s.shape, dev.stream);
 }
@@ -884,9 +891,11 @@ Tensor fetchAs(const Tensor &d, TensorLayout layout, DataType dtype) {
   t->version = nextTensorVersion();
   if (same && bytes > kKernelCopyMax) {
     TTM_CALL(ttm_memcpy_d2h(p, s.data.get(), bytes, dev.stream));
-  } else if (!convertInOneLaunch(s.data.get(), s.layout, s.dtype, p, layout, dtype, s.shape, dev.stream)) {
+  } else if ((s.layout != layout && !wholeChunkRows(s.shape, dtype)) ||
+             !convertInOneLaunch(s.data.get(), s.layout, s.dtype, p, layout, dtype, s.shape, dev.stream)) {
     const Tensor c = convertOnDevice(d, layout, dtype);
-    TTM_CALL(ttm_memcpy_d2h(p, c.handle->data.get(), bytes, dev.stream));
+    if (bytes <= kKernelCopyMax) TTM_CALL(ttm_copy_kernel(c.handle->data.get(), p, (bytes + 15) / 16 * 16, dev.stream));
+    else TTM_CALL(ttm_memcpy_d2h(p, c.handle->data.get(), bytes, dev.stream));
     syncStream(dev);
     return Tensor{t};
   }
