@@ -21,6 +21,10 @@ pytestmark = pytest.mark.gpu
     (2, 3, 1, 160, 96, [159, 3], -1, True),                    # no kernel of its own
     (2, 2, 2, 1024, 256, [1000, 64], -1, False),
     (2, 4, 4, 64, 128, [-1, 40], -1, False),                   # a user that sees nothing
+    (2, 4, 1, 4096, 128, [4095, 2000], -1, True),              # more pieces of a user than are requested ahead of their weights
+    (2, 8, 1, 8192, 256, [8191, 8000], -1, False),             # ... with a lane per column
+    (2, 4, 1, 4096, 64, [100, 40], -1, False),                 # most shares empty
+    (1, 2, 1, 65536, 32, [65535], -1, False),                  # as many pieces as there are shares
 ])
 def test_both_forms_against_the_oracle(hip, dev, orc, form, B, H, Hkv, S, D, cur, window, sink):
     q, k, v = (datagen.randn(s, seed=i, dtype=torch.bfloat16) for i, s in enumerate(((1, B, H, D), (B, Hkv, S, D), (B, Hkv, S, D))))

@@ -604,17 +604,19 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void ttm_sdpa_decode_k(D
   }  // users of this share
 }
 
-// merges a user's slots: out = sum_s o_s exp(m_s - M) / sum_s l_s exp(m_s - M).  grid (B * Hkv, G D / 256), 256 lanes.  Up to 16
-// slots a lane per output forms everything itself; more (few users with long caches) go through LDS: the weights exp(m_s - M)
-// are formed once per head, 256 / D lanes share a column and take every (256 / D)-th slot.
-constexpr int kMaxCombineSlices = 1024;
+// merges a user's slots: out = sum_s o_s exp(m_s - M) / sum_s l_s exp(m_s - M).  grid (B * Hkv, G), 256 lanes: a workgroup per head,
+// 256 / D lanes of it share a column and take every (256 / D)-th slot.  Bound by the memory round trips that follow each other (a few
+// hundred KiB in all), so there are two: the users' positions, then a lane's maxima and sums together with its first eight
+// numerators, which do not wait for the weights.  5 users x 4 heads of 4 kv heads, 1300 keys on average (about 20 slots each):
+// both launches 27.4 us with a workgroup per 256 outputs, one head after the other and numerators behind the weights -> 13.9 us.
 __global__ __launch_bounds__(256) void ttm_sdpa_decode_combine_k(DecodeArgs p) {
-  __shared__ float wgt[kMaxCombineSlices];
+  __shared__ float wgt[kDecodeBlocks];   // a user's slots lie in at most that many shares
   __shared__ float red[256];
-  __shared__ float stats[4];
-  const int bh = blockIdx.x, tid = threadIdx.x;
+  __shared__ float tops[4], sums[4];
+  constexpr int kAhead = 8;
+  const int bh = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
   const int b = bh / p.Hkv, hk = bh % p.Hkv;
-  const int G = p.G, D = p.D;
+  const int G = p.G, D = p.D, h = hk * p.Gt + p.g0 + g;
   // the user's tiles on the line and the shares that hold them
   int before, total, mine;
   line_of(p, b, tid & 63, before, mine, total);
@@ -622,92 +624,62 @@ __global__ __launch_bounds__(256) void ttm_sdpa_decode_combine_k(DecodeArgs p) {
   auto share_of = [&](int t) { return (int)(((uint32_t)((t + 1) * p.shares) - 1u) / (uint32_t)total); };
   const int j0 = mine ? share_of(before) : 0, S = mine ? share_of(before + mine - 1) - j0 + 1 : 0;
   const bool gaps = total < p.shares;   // fewer tiles than shares: some of them are empty and left their slots as they were
-  auto empty = [&](int s) { return gaps && share_begin(total, p.shares, j0 + s) == share_begin(total, p.shares, j0 + s + 1); };
-  if (S <= 16) {   // a lane per output: independent loads, no barriers
-    for (int idx = blockIdx.y * 256 + tid; idx < G * D; idx += gridDim.y * 256) {
-      const int g = idx / D, c = idx - g * D, h = hk * p.Gt + p.g0 + g;
-      const float *base = p.part + (((size_t)hk * (p.shares + p.B) + j0 + b) * G + g) * (D + 2);
-      const size_t sstride = (size_t)G * (D + 2);
-      const float sinkv = p.sink ? ttm_bf16_to_f32(p.sink[ttm_tiled_offset(h, 0, 1)]) * p.scale : -INFINITY;
-      float M = sinkv, num = 0.0f, den = 0.0f;
-      if (gaps) {
-        for (int s = 0; s < S; ++s)
-          if (!empty(s)) M = fmaxf(M, base[s * sstride + D]);
-        for (int s = 0; s < S; ++s) {
-          if (empty(s) || base[s * sstride + D] == -INFINITY) continue;
-          const float w = __expf(base[s * sstride + D] - M);
-          num += base[s * sstride + c] * w;
-          den += base[s * sstride + D + 1] * w;
-        }
-      } else {
-#pragma unroll 8
-        for (int s = 0; s < S; ++s) M = fmaxf(M, base[s * sstride + D]);
-#pragma unroll 8
-        for (int s = 0; s < S; ++s) {
-          const float ms = base[s * sstride + D], w = ms == -INFINITY ? 0.0f : __expf(ms - M);
-          num += base[s * sstride + c] * w;
-          den += base[s * sstride + D + 1] * w;
-        }
-      }
-      if (p.sink) den += __expf(sinkv - M);
-      store_head(p, b, h, c, den > 0.0f ? num / den : 0.0f);
-    }
-    if (blockIdx.y == 0) store_padding(p, b, hk, tid, 256);
-    return;
-  }
-  for (int g = blockIdx.y; g < G; g += gridDim.y) {   // workgroup-uniform
-  const float *base = p.part + ((size_t)hk * (p.shares + p.B) + j0 + b) * G * (D + 2) + (size_t)g * (D + 2);   // piece s: + s * G * (D + 2)
+  auto filled = [&](int s) { return s < S && !(gaps && share_begin(total, p.shares, j0 + s) == share_begin(total, p.shares, j0 + s + 1)); };
+  const float *base = p.part + (((size_t)hk * (p.shares + p.B) + j0 + b) * G + g) * (D + 2);   // piece s: + s * sstride
   const size_t sstride = (size_t)G * (D + 2);
-  const int h = hk * p.Gt + p.g0 + g;
+  const int nsub = 256 / D, c = tid % D, sub = tid / D;
   const float sinkv = p.sink ? ttm_bf16_to_f32(p.sink[ttm_tiled_offset(h, 0, 1)]) * p.scale : -INFINITY;
-  // M = max over the slices (and the sink)
-  float m = sinkv;
-  for (int s = tid; s < S; s += 256)
-    if (!empty(s)) m = fmaxf(m, base[s * sstride + D]);
+  float ms[kDecodeBlocks / 256], ls[kDecodeBlocks / 256], ahead[kAhead];
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-  if ((tid & 63) == 0) red[tid >> 6] = m;
+  for (int i = 0; i < kDecodeBlocks / 256; ++i) {
+    const bool in = filled(tid + 256 * i);
+    ms[i] = in ? base[(tid + 256 * i) * sstride + D] : -INFINITY;
+    ls[i] = in ? base[(tid + 256 * i) * sstride + D + 1] : 0.0f;
+  }
+#pragma unroll
+  for (int k = 0; k < kAhead; ++k) {
+    const int s = sub + nsub * k;
+    ahead[k] = sub < nsub && filled(s) ? base[s * sstride + c] : 0.0f;
+  }
+  float M = sinkv;
+#pragma unroll
+  for (int i = 0; i < kDecodeBlocks / 256; ++i) M = fmaxf(M, ms[i]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
+  if ((tid & 63) == 0) tops[tid >> 6] = M;
   __syncthreads();
-  const float M = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  __syncthreads();
-  // weights, denominator and numerators, kMaxCombineSlices pieces at a time: lane (c, sub) sums the pieces sub, sub + nsub, ... of
-  // column c
-  const int nsub = 256 / D > 0 ? 256 / D : 1;
-  const int c = tid % D, sub = tid / D;
+  M = fmaxf(fmaxf(tops[0], tops[1]), fmaxf(tops[2], tops[3]));
   float den = 0.0f, num = 0.0f;
-  for (int s0 = 0; s0 < S; s0 += kMaxCombineSlices) {
-    const int n = min(S - s0, kMaxCombineSlices);
-    for (int s = tid; s < n; s += 256) {
-      const float ms = empty(s0 + s) ? -INFINITY : base[(s0 + s) * sstride + D];
-      const float w = ms == -INFINITY ? 0.0f : __expf(ms - M);
-      wgt[s] = w;
-      if (w != 0.0f) den += base[(s0 + s) * sstride + D + 1] * w;
-    }
-    __syncthreads();
-    if (sub < nsub) {
-      if (gaps) {
-        for (int s = sub; s < n; s += nsub)
-          if (wgt[s] != 0.0f) num += base[(s0 + s) * sstride + c] * wgt[s];
-      } else {
-#pragma unroll 8
-        for (int s = sub; s < n; s += nsub) num += base[(s0 + s) * sstride + c] * wgt[s];
-      }
-    }
-    __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kDecodeBlocks / 256; ++i) {
+    const float w = ms[i] == -INFINITY ? 0.0f : __expf(ms[i] - M);
+    wgt[tid + 256 * i] = w;
+    den += ls[i] * w;
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) den += __shfl_xor(den, o);
-  if ((tid & 63) == 0) stats[tid >> 6] = den;
+  if ((tid & 63) == 0) sums[tid >> 6] = den;
+  __syncthreads();
+  if (sub < nsub) {
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k)
+      if (sub + nsub * k < S) num += ahead[k] * wgt[sub + nsub * k];
+    if (gaps) {
+      for (int s = sub + nsub * kAhead; s < S; s += nsub)
+        if (wgt[s] != 0.0f) num += base[s * sstride + c] * wgt[s];
+    } else {
+#pragma unroll 8
+      for (int s = sub + nsub * kAhead; s < S; s += nsub) num += base[s * sstride + c] * wgt[s];
+    }
+  }
   red[tid] = num;
   __syncthreads();
-  den = (stats[0] + stats[1]) + (stats[2] + stats[3]) + (p.sink ? __expf(sinkv - M) : 0.0f);
+  den = (sums[0] + sums[1]) + (sums[2] + sums[3]) + (p.sink ? __expf(sinkv - M) : 0.0f);
   if (sub == 0) {
     for (int u = 1; u < nsub; ++u) num += red[tid + u * D];
     store_head(p, b, h, c, den > 0.0f ? num / den : 0.0f);
   }
-  __syncthreads();
-  }  // heads of this workgroup
-  if (blockIdx.y == 0) store_padding(p, b, hk, tid, 256);   // the padding belongs to the first head's workgroup
+  if (g == 0) store_padding(p, b, hk, tid, 256);   // the padding belongs to the first head's workgroup
 }
 
 }  // namespace
@@ -912,10 +884,10 @@ static int sdpa_decode_entry(const void *q, const void *k, const void *v, const 
   }
   hipStream_t s = (hipStream_t)stream;
   // Direct form where the users alone fill the device or their caches are short; shares for few users with long caches.  Measured
-  // (D = 128, 8 kv heads; direct / shares, us, contexts of a quarter of the cache to all of it | all of it): 1 user x 512
-  // positions 8.5 / 11.0 | 7.9 / 10.6, 1 x 1024 12.7 / 12.0 | 11.7 / 11.7, 1 x 2048 14.9 / 15.8 | 22.3 / 15.4, 8 x 1024 15.5 / 20.8 |
-  // 15.7 / 17.0, 8 x 2048 21.5 / 23.3 | 25.8 / 21.8, 16 x 2048 26.1 / 26.7 | 27.0 / 30.4, 16 x 4096 47.9 / 39.2 | 56.2 / 51.9,
-  // 32 x 2048 33.5 / 36.5 | 46.0 / 50.9, 32 x 4096 65.3 / 64.8 | 85.1 / 91.5.
+  // (D = 128, 8 kv heads of 4 query heads, contexts of a quarter of the cache to all of it; direct / shares, us): 1 user x 512 positions
+  // 7.4 / 9.9, 1 x 1024 10.7 / 10.2, 1 x 2048 12.1 / 10.4, 1 x 4096 30.2 / 11.5, 8 x 1024 14.8 / 15.2, 8 x 2048 24.3 / 18.8, 16 x 2048
+  // 26.4 / 26.0, 16 x 4096 43.8 / 35.9, 32 x 1024 19.7 / 26.2, 32 x 2048 32.9 / 37.2; D = 64: 5 x 2048 12.2 / 13.6, 5 x 4096 21.6 / 15.6,
+  // 16 x 2048 15.4 / 18.1, 16 x 4096 26.5 / 25.5.
   const int form = ttm_option("sdpa_decode_form");   // 0 by this rule, 1 direct, 2 shares
   // (the results of the wavefronts fit in 32 KiB of LDS)
   const bool direct = G * head_dim <= 1024 && (form ? form == 1 : seq * head_dim <= 2048 * std::max<int64_t>(64, batch * kv_heads));
@@ -959,7 +931,7 @@ static int sdpa_decode_entry(const void *q, const void *k, const void *v, const 
     }
     launch_decode<false>(p, dim3((unsigned)shares, (unsigned)kv_heads), s);
     TTM_LAUNCH_CHECK();
-    hipLaunchKernelGGL(ttm_sdpa_decode_combine_k, dim3((unsigned)(batch * kv_heads), (unsigned)ttm_cdiv(p.G * head_dim, 256)), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(ttm_sdpa_decode_combine_k, dim3((unsigned)(batch * kv_heads), (unsigned)p.G), dim3(256), 0, s, p);
     TTM_LAUNCH_CHECK();
   }
   return TTM_OK;
