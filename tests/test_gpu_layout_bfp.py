@@ -219,3 +219,46 @@ def test_full_size_properties(hip, dev, orc, fmt):
     assert torch.equal(back, xd)
     assert int(t.view(torch.int32).to(torch.int64).sum()) == int(xd.view(torch.int32).to(torch.int64).sum())
     assert np.array_equal(t.reshape(-1).cpu().numpy(), orc.tilize(x.numpy()))
+
+
+@pytest.mark.parametrize("fmt", [8, 4])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape,shift", [((1, 1, 1), 0), ((2, 33, 129), 1), ((1, 64, 255), 3), ((3, 31, 257), 0), ((1, 95, 1023), 5), ((2, 40, 300), 2),
+                                         ((1, 32, 512), 1), ((1, 500, 384), 0), ((2, 1100, 2081), 7)])
+def test_bfp_ragged_strips(hip, dev, orc, fmt, dtype, shape, shift):
+    """Strips whose rows start and end anywhere, on buffers that start at any element: packed bytes and read-back against the oracle
+    and the generic kernel (random bit patterns: infinities, NaN and subnormal numbers among them), nothing written around them."""
+    hfmt, code = (hip.BFP8B if fmt == 8 else hip.BFP4B), (hip.F32 if dtype == torch.float32 else hip.BF16)
+    b, r, c = shape
+    n, pad, s = b * r * c, 64, hip.current_stream()
+    packed = b * ((r + 31) // 32) * ((c + 31) // 32) * hip.lib().ttm_bfp_tile_bytes(hfmt)
+    ints = torch.int32 if dtype == torch.float32 else torch.int16
+    limit = 2 ** (8 * ints.itemsize - 1)
+    rng = np.random.default_rng(n)
+    bits = torch.from_numpy(rng.integers(-limit, limit, n)).to(ints)
+    plain = torch.randn(n, generator=torch.Generator().manual_seed(n)).to(dtype)
+    for x, oracle in ((plain, True), (bits.view(dtype), False)):
+        src = torch.zeros(n + 2 * pad, dtype=dtype, device=dev)
+        src[pad + shift:pad + shift + n] = x.to(dev)
+        got = {}
+        for variant in (2, 1):
+            hip.set_option("pack_variant", variant)
+            hip.set_option("unpack_variant", variant)
+            try:
+                p = torch.full((packed + 32,), 9, dtype=torch.uint8, device=dev)
+                hip.call("ttm_bfp_pack", hip.ptr(src[pad + shift:]), code, hip.ROW_MAJOR, hip.ptr(p), hfmt, b, r, c, s)
+                back = torch.full((n + 2 * pad,), 5, dtype=ints, device=dev)
+                hip.call("ttm_bfp_unpack", hip.ptr(p), hfmt, hip.ptr(back[pad + shift:]), code, hip.ROW_MAJOR, b, r, c, s)
+                torch.cuda.synchronize()
+            finally:
+                hip.set_option("pack_variant", 0)
+                hip.set_option("unpack_variant", 0)
+            got[variant] = p.cpu(), back.cpu()
+        (p, back), (gp, gback) = got[2], got[1]
+        assert torch.equal(p, gp) and torch.equal(back, gback)
+        assert (p[packed:] == 9).all() and (back[:pad + shift] == 5).all() and (back[pad + shift + n:] == 5).all()
+        if oracle:
+            want = orc.bfp_pack(x.float().numpy().reshape(shape), fmt)
+            assert np.array_equal(p[:packed].numpy(), want)
+            vals = orc.bfp_unpack(want, shape, fmt).reshape(-1)
+            assert np.array_equal(back[pad + shift:pad + shift + n].view(dtype).float().numpy(), vals)

@@ -14,9 +14,11 @@
 // on a row-major plain side that is a strip of 32 rows x 512 bytes which is read / written in
 // fully contiguous 512-byte row segments and permuted through a padded LDS image, exactly like
 // the tilize kernel; the packed side of a strip is one contiguous run of tiles.
-// Shapes whose rows are not a multiple of 512 bytes, or that need zero padding, take a generic
-// kernel with one face row quad per lane group and bounds-checked scalar accesses.
+// Row-major shapes whose rows are not a multiple of 512 bytes, or that need zero padding, take strips whose
+// row-major side moves in shifted chunks; small or narrow ones, and tile-ordered tensors that are no whole number of
+// strips, a generic kernel with one face row quad per lane group and bounds-checked scalar accesses.
 #include "ttm_common.h"
+#include "ttm_ragged.h"
 
 // ------------------------------------------------------------------------------------ element math
 // W = magnitude bits (7 or 3).  Returns the magnitude only; signs are merged per chunk.
@@ -253,6 +255,78 @@ __global__ __launch_bounds__(256) TTM_MAX_WAVES((PACK && ROWMAJOR && W == 7 && E
   }
 }
 
+// ------------------------------------------------------------------------------------ ragged shapes
+// The row-major side in strips of 32 rows x 512 bytes that start and end anywhere, moved in shifted chunks (ttm_ragged.h), the
+// packed side as in the strip kernel.  HBM-bound; the generic kernel reads and writes single elements there and gives a tile its
+// own workgroup.  [3, 1966, 1888] fp32 pack / unpack bfp4_b 21.6 / 26.3 -> 12.2 / 16.9 us, [4096, 8190] bf16 bfp8_b 54.1 / 53.7 ->
+// 24.2 / 24.6 us (4.2 TB/s).
+template <int W, int ELEM, bool PACK>
+__global__ __launch_bounds__(256) void ttm_bfp_ragged_k(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int rows, int cols, int strips) {
+  constexpr int EPT = 16 / ELEM, CPT = 64 * ELEM, TPS = 16 / ELEM;   // elements per chunk, chunks per tile, tiles per strip
+  constexpr int TILE_BYTES = 64 + (W == 7 ? 1024 : 512), CHUNK_OUT = EPT * (W + 1) / 8;
+  constexpr bool VIA_LDS = PACK && W == 3;   // bfp4_b leaves as whole 16-byte chunks, as in the strip kernel
+  __shared__ u32x4 image[kRaggedImage];
+  __shared__ __attribute__((aligned(16))) uint8_t pk[VIA_LDS ? TPS * TILE_BYTES : 16];
+  const int tid = threadIdx.x;
+  const RaggedStrip st = ragged_strip<ELEM>(rows, cols, strips);
+  const int64_t b = blockIdx.y;
+  const int64_t tile_off = ((b * st.yt + st.ty) * st.ct + st.sx * TPS) * (int64_t)TILE_BYTES;
+  const uintptr_t rm = (uintptr_t)(PACK ? src : dst) + (b * rows + st.ty * 32) * st.stride + st.sx * 512;
+  if (PACK) {
+    ragged_load<ELEM>(image, st, rm, (uintptr_t)src, (uintptr_t)src + (int64_t)gridDim.y * rows * st.stride);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int oc = i * 256 + tid, tl = oc / CPT, w = oc % CPT;
+      if (tl >= st.tiles) continue;   // wavefront-uniform: a tile is a whole number of wavefronts
+      const int face = w / (16 * ELEM), dy = (w / ELEM) % 16, q = w % ELEM;
+      uint32_t bits[EPT], out[2];
+      chunk_to_bits<ELEM == 2, EPT>(ragged_read(image, st, rm, (face >> 1) * 16 + dy, (tl * 2 * ELEM + (face & 1) * ELEM + q) * 16), bits);
+      const uint32_t E = encode_chunk<W, EPT>(bits, out);
+      uint8_t *tile = (VIA_LDS ? pk : dst + tile_off) + tl * TILE_BYTES, *m = tile + 64 + w * CHUNK_OUT;
+      if (q == 0) tile[face * 16 + dy] = (uint8_t)E;
+      if (CHUNK_OUT == 8) __builtin_nontemporal_store(u32x2{out[0], out[1]}, (u32x2 *)m);
+      else if (CHUNK_OUT == 2) *(uint16_t *)m = (uint16_t)out[0];
+      else if (VIA_LDS) *(uint32_t *)m = out[0];
+      else __builtin_nontemporal_store(out[0], (uint32_t *)m);
+    }
+    if constexpr (VIA_LDS) {
+      __syncthreads();
+      for (int c = tid; c < st.tiles * (TILE_BYTES / 16); c += 256) __builtin_nontemporal_store(((const u32x4 *)pk)[c], (u32x4 *)(dst + tile_off) + c);
+    }
+  } else {
+    const bool more = ragged_left(st) > 512;
+    u32x4 v[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      // i = 4: row tid of the next tile's column 0
+      const int tl = i < 4 ? (i * 256 + tid) / CPT : TPS, w = i < 4 ? (i * 256 + tid) % CPT : (tid >> 4) * (32 * ELEM) + (tid & 15) * ELEM;
+      if (!(i < 4 ? tl < st.tiles : tid < 32 && more)) continue;
+      const uint8_t *tile = src + tile_off + tl * TILE_BYTES, *m = tile + 64 + w * CHUNK_OUT;
+      const int E = tile[w / ELEM];   // face rows in order
+      uint32_t in[2] = {0, 0};
+      if (CHUNK_OUT == 8) {
+        const u32x2 t = __builtin_nontemporal_load((const u32x2 *)m);
+        in[0] = t.x; in[1] = t.y;
+      } else if (CHUNK_OUT == 4) {
+        in[0] = __builtin_nontemporal_load((const uint32_t *)m);
+      } else {
+        in[0] = __builtin_nontemporal_load((const uint16_t *)m);
+      }
+      v[i] = decode_chunk<W, ELEM == 2, EPT>(in, E);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int oc = i * 256 + tid, tl = oc / CPT, w = oc % CPT;
+      const int face = w / (16 * ELEM), dy = (w / ELEM) % 16, q = w % ELEM;
+      if (tl < st.tiles) image[((face >> 1) * 16 + dy) * kRaggedPitch + tl * 2 * ELEM + (face & 1) * ELEM + q] = v[i];
+    }
+    if (tid < 32 && more) image[tid * kRaggedPitch + 32] = v[4];
+    __syncthreads();
+    ragged_store<ELEM>(image, st, rm);
+  }
+}
+
 // ------------------------------------------------------------------------------------ generic kernels
 // One lane per 4 elements of a face row; grid = (tile columns, tile rows, batch).
 template <int W, bool BF16, bool PACK>
@@ -320,7 +394,8 @@ static int run_bfp(const void *src, void *dst, int fmt, int dtype, int layout, i
   const bool padded = rm && (rows != pr || cols != pc);
   hipStream_t s = (hipStream_t)stream;
   const int tiles_per_wg = 16 / elem;
-  bool strip = aligned && !padded && ttm_option(PACK ? "pack_variant" : "unpack_variant") == 0;
+  const int variant = ttm_option(PACK ? "pack_variant" : "unpack_variant");   // 0 by the rules below, 1 generic, 2 strips of any size
+  bool strip = aligned && !padded && variant != 1;
   int64_t strips_per_row = 0, blocks = 0;
   if (strip) {
     if (rm) {
@@ -346,6 +421,20 @@ static int run_bfp(const void *src, void *dst, int fmt, int dtype, int layout, i
     else { if (bf16) STRIP_RM(3, 2); else STRIP_RM(3, 4); }
 #undef STRIP_RM
 #undef STRIP
+  } else if (const int64_t strips = ttm_cdiv(pc * elem, 512);
+             rm && variant != 1 && ((uintptr_t)(PACK ? dst : src) & 15) == 0 && (uintptr_t)(PACK ? src : dst) % elem == 0 &&
+             pr * pc < ((int64_t)1 << 31) && yt <= 65535 && batch <= 65535 &&
+             (variant == 2 || (ntiles >= (PACK ? 2304 : 1536) && rows >= 24 && cols * elem * 4 >= strips * 512 * 3))) {
+    // Strips where the tensor is large and its strips are mostly real columns.  Generic / strips, bfp8_b, us (pack | unpack):
+    // [1024, 1056] fp32 4.1 / 4.3 | 4.6 / 4.3, bf16 3.4 / 4.2 | 3.8 / 4.4; [1500, 1000] fp32 4.0 / 4.5 | 5.2 / 4.6, bf16 3.9 / 4.4 |
+    // 4.6 / 4.5; [1024, 2080] fp32 6.0 / 5.0 | 7.2 / 5.4, bf16 4.8 / 5.2 | 5.5 / 5.0; [3, 700, 1500] fp32 6.3 / 5.7 | 9.7 / 6.4, bf16
+    // 6.2 / 5.5 | 8.1 / 6.1; [2000, 3001] fp32 10.9 / 7.6 | 16.0 / 8.8, bf16 12.1 / 6.7 | 13.1 / 7.6; bfp4_b within 0.7 of these.
+    const dim3 grid((unsigned)(strips * yt), (unsigned)batch);
+#define RAGGED(Wv, EL) \
+  hipLaunchKernelGGL((ttm_bfp_ragged_k<Wv, EL, PACK>), grid, dim3(256), 0, s, (const uint8_t *)src, (uint8_t *)dst, (int)rows, (int)cols, (int)strips)
+    if (fmt == TTM_BFP8B) { if (bf16) RAGGED(7, 2); else RAGGED(7, 4); }
+    else { if (bf16) RAGGED(3, 2); else RAGGED(3, 4); }
+#undef RAGGED
   } else {
     TTM_REQUIRE(yt <= 65535 && batch <= 65535, "%s: more than 65535 tile rows or batches on the generic path", who);
     TTM_REQUIRE(((uintptr_t)(PACK ? dst : src) & 3) == 0, "%s: packed buffer must be 4-byte aligned", who);

@@ -8,9 +8,8 @@
 //   1  direct: one lane per 16-byte chunk of the tiled side, the row-major side is touched in
 //      face-row segments (16 elements).  No LDS; used when a strip does not divide the row.
 // Shapes that are not multiples of 32, and rows that start anywhere, have kernels of their own below (zero padding).
-#include <type_traits>
-
 #include "ttm_common.h"
+#include "ttm_ragged.h"
 
 typedef u32x4 chunk_t;  // 16 bytes
 
@@ -233,114 +232,48 @@ __global__ __launch_bounds__(256) void ttm_untilize_rows_k(const T *__restrict__
 
 // ------------------------------------------------------------------------------------ ragged shapes
 // Rows or columns that are not multiples of 32, or a row-major side that starts anywhere.  The strip kernel's plan (32 rows x 512
-// bytes per workgroup, the permutation through a row-major LDS image with a 33-chunk pitch) with the row-major side moved in
-// aligned 16-byte chunks whatever its rows start at: a row of the strip covers up to 33 of them.  Tilize keeps the chunks as they
-// are and shifts when it reads the image (five dwords and a funnel shift per output chunk); untilize shifts when it makes the
-// aligned chunks it stores.  Element accesses remain where a chunk crosses the end of the buffer (tilize) or of a row (untilize).  HBM-bound as the strip kernel is; before, a chunk whose address was not a multiple of 16 went by element accesses,
-// seven of eight for an odd bf16 width: [3, 1000, 3001] bf16 tilize / untilize 14.8 / 23.3 -> 7.8 / 10.0 us,
-// [4000, 7001] fp32 51 / 78 -> 41 / 38 us (5.5 / 5.9 TB/s).
+// bytes per workgroup) with the row-major side moved in shifted chunks (ttm_ragged.h).  HBM-bound as the strip kernel is; before,
+// a chunk whose address was not a multiple of 16 went by element accesses, seven of eight for an odd bf16 width: [3, 1000, 3001]
+// bf16 tilize / untilize 14.8 / 23.3 -> 7.8 / 10.0 us, [4000, 7001] fp32 51 / 78 -> 41 / 38 us (5.5 / 5.9 TB/s).
 // Tilize writes zeros into the padding; untilize skips it.  grid (strips x tile rows, matrices).
-__device__ __forceinline__ u32x4 lds_unaligned16(const uint8_t *image, int off) {
-  const uint32_t *w = (const uint32_t *)image + (off >> 2);
-  const int sh = (off & 3) * 8;
-  const uint32_t d0 = w[0], d1 = w[1], d2 = w[2], d3 = w[3], d4 = w[4];
-  return u32x4{__builtin_amdgcn_alignbit(d1, d0, sh), __builtin_amdgcn_alignbit(d2, d1, sh), __builtin_amdgcn_alignbit(d3, d2, sh),
-               __builtin_amdgcn_alignbit(d4, d3, sh)};
-}
 template <int ELEM, bool TILIZE>
 __global__ __launch_bounds__(256) void ttm_tile_ragged_k(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int rows, int cols,
                                                          int strips, int64_t matrices) {
-  constexpr int CPT = 64 * ELEM, PITCH = 33, BPR = PITCH * 16;   // chunks per tile; chunks and bytes per image row
-  typedef typename std::conditional<ELEM == 4, uint32_t, typename std::conditional<ELEM == 2, uint16_t, uint8_t>::type>::type T;
-  __shared__ u32x4 image[32 * PITCH + 1];   // one more: the shift reads a dword ahead
-  uint8_t *bytes = (uint8_t *)image;
+  constexpr int CPT = 64 * ELEM;   // chunks per tile
+  __shared__ u32x4 image[kRaggedImage];
   const int tid = threadIdx.x;
-  // neighbouring strips share the lines at their common edge: consecutive ones go to one XCD (workgroups are dealt to the eight
-  // XCDs in turn), whose L2 then puts the two parts of a line together
-  const int n8 = gridDim.x >> 3, id = (int)blockIdx.x < n8 * 8 ? ((int)blockIdx.x & 7) * n8 + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
-  const int sx = id % strips, ty = id / strips, ct = (cols + 31) >> 5, yt = (rows + 31) >> 5;
-  const int nrows = min(32, rows - ty * 32), nbytes = min(512, (cols - sx * (512 / ELEM)) * ELEM);   // of the strip's row segments
-  const int tiles = min(16 / ELEM, ct - sx * (16 / ELEM));
-  const int64_t stride = (int64_t)cols * ELEM;
+  const RaggedStrip st = ragged_strip<ELEM>(rows, cols, strips);
   for (int64_t b = blockIdx.y; b < matrices; b += gridDim.y) {
-    const int64_t rm_off = (b * rows + ty * 32) * stride + sx * 512;
-    const int64_t tile_off = ((b * yt + ty) * ct + sx * (16 / ELEM)) * (int64_t)(CPT * 16);
-    const uintptr_t rm = (uintptr_t)(TILIZE ? src : dst) + rm_off;
-    // chunk slot idx: row and number of the aligned chunk in the row; slots 1024 .. 1055 are the rows' 33rd chunks
-    auto row_of = [&](int idx) { return idx < 1024 ? idx >> 5 : idx - 1024; };
-    auto chunk_of = [&](int idx) { return idx < 1024 ? idx & 31 : 32; };
+    const int64_t tile_off = ((b * st.yt + st.ty) * st.ct + st.sx * (16 / ELEM)) * (int64_t)(CPT * 16);
+    const uintptr_t rm = (uintptr_t)(TILIZE ? src : dst) + (b * rows + st.ty * 32) * st.stride + st.sx * 512;
     if (TILIZE) {
-      const uintptr_t lo = (uintptr_t)src, hi = lo + matrices * rows * stride;
-      u32x4 v[5];
-#pragma unroll
-      for (int i = 0; i < 5; ++i) {
-        const int idx = i * 256 + tid, r = row_of(idx);
-        if (idx >= 1056 || r >= nrows) continue;
-        const uintptr_t a = rm + r * stride, c = (a & ~(uintptr_t)15) + chunk_of(idx) * 16;
-        if (c >= a + nbytes) continue;
-        if (c >= lo && c + 16 <= hi) {
-          v[i] = __builtin_nontemporal_load((const u32x4 *)c);
-        } else {
-          T e[16 / ELEM];
-#pragma unroll
-          for (int k = 0; k < 16 / ELEM; ++k) e[k] = c + k * ELEM >= lo && c + k * ELEM < hi ? *(const T *)(c + k * ELEM) : T(0);
-          v[i] = *(const u32x4 *)e;
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 5; ++i) {
-        const int idx = i * 256 + tid;
-        if (idx < 1056) image[row_of(idx) * PITCH + chunk_of(idx)] = v[i];
-      }
+      ragged_load<ELEM>(image, st, rm, (uintptr_t)src, (uintptr_t)src + matrices * rows * st.stride);
       __syncthreads();
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int oc = i * 256 + tid, tl = oc / CPT, w = oc % CPT;
-        if (tl >= tiles) continue;
+        if (tl >= st.tiles) continue;
         const int face = w / (16 * ELEM), dy = (w / ELEM) % 16, q = w % ELEM;
-        const int r = (face >> 1) * 16 + dy, at = (tl * 2 * ELEM + (face & 1) * ELEM + q) * 16;   // byte column of the strip
-        u32x4 o = lds_unaligned16(bytes, r * BPR + (int)((rm + r * stride) & 15) + at);
-        const int n = r < nrows ? nbytes - at : 0;   // valid bytes of the chunk
-        if (n < 16) {
-#pragma unroll
-          for (int k = 0; k < 4; ++k) o[k] = n >= 4 * k + 4 ? o[k] : n <= 4 * k ? 0u : o[k] & ((1u << (8 * (n - 4 * k))) - 1u);
-        }
+        const u32x4 o = ragged_read(image, st, rm, (face >> 1) * 16 + dy, (tl * 2 * ELEM + (face & 1) * ELEM + q) * 16);
         __builtin_nontemporal_store(o, (u32x4 *)(dst + tile_off) + oc);
       }
     } else {
-      // a strip stores the aligned chunks that begin in it: the last one of a row reaches into the next strip, whose first 16 bytes
-      // of every row (a face row or half of one) are the image's 33rd chunk
-      const int left = (int)min(stride - (int64_t)sx * 512, (int64_t)1024);   // bytes of a row from the strip on
-      const bool more = left > 512;
+      const bool more = ragged_left(st) > 512;
       u32x4 v[5];
 #pragma unroll
       for (int i = 0; i < 5; ++i) {
         const int oc = i < 4 ? i * 256 + tid : 16 / ELEM * CPT + (tid >> 4) * (32 * ELEM) + (tid & 15) * ELEM;   // i = 4: row tid of the next tile's column 0
-        if (i < 4 ? oc / CPT < tiles : tid < 32 && more) v[i] = __builtin_nontemporal_load((const u32x4 *)(src + tile_off) + oc);
+        if (i < 4 ? oc / CPT < st.tiles : tid < 32 && more) v[i] = __builtin_nontemporal_load((const u32x4 *)(src + tile_off) + oc);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int oc = i * 256 + tid, tl = oc / CPT, w = oc % CPT;
         const int face = w / (16 * ELEM), dy = (w / ELEM) % 16, q = w % ELEM;
-        if (tl < tiles) image[((face >> 1) * 16 + dy) * PITCH + tl * 2 * ELEM + (face & 1) * ELEM + q] = v[i];
+        if (tl < st.tiles) image[((face >> 1) * 16 + dy) * kRaggedPitch + tl * 2 * ELEM + (face & 1) * ELEM + q] = v[i];
       }
-      if (tid < 32 && more) image[tid * PITCH + 32] = v[4];
+      if (tid < 32 && more) image[tid * kRaggedPitch + 32] = v[4];
       __syncthreads();
-#pragma unroll
-      for (int i = 0; i < 5; ++i) {
-        const int idx = i * 256 + tid, r = row_of(idx);
-        if (idx >= 1056 || r >= nrows || (i == 4 && sx > 0)) continue;   // i = 4: the piece in front of the first whole chunk of a row
-        const uintptr_t a = rm + r * stride;
-        const int head = (int)(-a & 15), at = i == 4 ? head - 16 : head + chunk_of(idx) * 16;   // byte column of the chunk in the strip
-        if (at >= nbytes) continue;
-        if (at >= 0 && at + 16 <= left) {
-          *(u32x4 *)(a + at) = lds_unaligned16(bytes, r * BPR + at);
-        } else {   // the ends of a row
-#pragma unroll
-          for (int k = 0; k < 16 / ELEM; ++k)
-            if (at + k * ELEM >= 0 && at + k * ELEM < left) *(T *)(a + at + k * ELEM) = *(const T *)(bytes + r * BPR + at + k * ELEM);
-        }
-      }
+      ragged_store<ELEM>(image, st, rm);
     }
     if (matrices > gridDim.y) __syncthreads();
   }
@@ -362,7 +295,7 @@ static int run_layout(const void *src, void *dst, int64_t batch, int64_t rows, i
   const int64_t strips = ttm_cdiv(pc * elem, 512);
   const int variant = ttm_option(TILIZE ? "tilize_variant" : "untilize_variant");
   if ((!aligned || (cols * elem % 512 != 0 && variant == 0)) && pr * pc < ((int64_t)1 << 31) && ((uintptr_t)(TILIZE ? dst : src) & 15) == 0 &&   // the tile-order side moves in whole 16-byte chunks
-      batch * strips * (pr / 32) >= 256 && rows >= 24 && cols * elem * 4 >= strips * 512 * 3) {
+      (uintptr_t)(TILIZE ? src : dst) % elem == 0 && batch * strips * (pr / 32) >= 256 && rows >= 24 && cols * elem * 4 >= strips * 512 * 3) {
     const dim3 grid((unsigned)(strips * (pr / 32)), (unsigned)(batch > 65535 ? 65535 : batch));
 #define RAGGED(E) \
   hipLaunchKernelGGL((ttm_tile_ragged_k<E, TILIZE>), grid, dim3(256), 0, s, (const uint8_t *)src, (uint8_t *)dst, (int)rows, (int)cols, (int)strips, batch)
