@@ -11,6 +11,8 @@
 // A lane therefore owns one query column of every accumulator: the running max / sum and the
 // rescale factor are per-lane scalars, shared only with lane ^ 32.
 // Workgroup = 4 wavefronts x 32 queries; K and V^T blocks of 32 keys are staged in LDS.
+#include <algorithm>
+
 #include "ttm_common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -78,6 +80,23 @@ __device__ __forceinline__ void sdpa_xcd_order(const SdpaArgs &p, int &x, int &h
   b = group / p.Hkv;
   h = (group % p.Hkv) * gq + member % gq;
   x = member / gq;
+}
+
+// The same for a causal launch of one query block per workgroup, which should begin with its longest blocks: x is slowest, so the
+// workgroups of an XCD take the last blocks of all its heads first.
+__device__ __forceinline__ void sdpa_longest_first(const SdpaArgs &p, int &x, int &h, int &b) {
+  const int flat = x + (int)gridDim.x * (h + p.Hq * b), gq = p.Hq / p.Hkv, groups = p.B * p.Hkv;
+  if (groups % 8 == 0) {
+    const int xcd = flat % 8, idx = flat / 8, heads = groups / 8 * gq, member = idx % heads, group = member / gq * 8 + xcd;
+    x = idx / heads;
+    b = group / p.Hkv;
+    h = (group % p.Hkv) * gq + member % gq;
+  } else {
+    const int heads = p.Hq * p.B, member = flat % heads;
+    x = flat / heads;
+    b = member / p.Hq;
+    h = member % p.Hq;
+  }
 }
 
 template <int DT>  // head_dim / 32
@@ -1140,7 +1159,8 @@ __global__ __launch_bounds__(256 * KH) __attribute__((amdgpu_waves_per_eu(2, 2))
   uint8_t *lds = (uint8_t *)sdpa_ring;
   const int nqb = (p.sqt + 3) / 4;
   int x = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  sdpa_xcd_order(p, x, h, b);
+  if (KH == 2 && !paired && p.hi_off == 0) sdpa_longest_first(p, x, h, b);
+  else sdpa_xcd_order(p, x, h, b);
   if constexpr (KH == 1) {
     // One query block per workgroup, two workgroups per CU.  Under a causal mask a block's work grows with its number:
     // the first half of a matrix's workgroups (the first to be placed, one per CU) take the upper blocks from the last
@@ -1226,26 +1246,43 @@ static int sdpa_entry(const void *q, const void *k, const void *v, const void *m
   const int variant = ttm_option("sdpa_variant");   // 1 = 32 keys per pass, 2 = 64 keys without pairing query blocks
   const bool wide = variant != 1;
   const int nqb = (int)ttm_cdiv(p.sqt, 4);
-  const int paired = is_causal && nqb >= 2 && variant != 2;
+  int cus = 0, devid = 0;
+  if (hipGetDevice(&devid) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, devid) != hipSuccess || cus <= 0) cus = 256;
+  const int64_t blocks = (int64_t)nqb * Hq * B;
+  // Pairs (last and first query block of a matrix, second last and second, ...) give workgroups of equal work, but only whole rounds
+  // of them use the device: where the blocks have a CU each they are single, and where pairs would leave part of their last round
+  // idle, single blocks that begin with the longest ones end sooner.  Single / paired, causal, us: [1, 16 / 4, 440, 64] 9.3 / 14.5,
+  // [1, 32 / 8, 512, 128] 13.1 / 19.1, [1, 32 / 8, 1024, 128] 20.1 / 25.8, [1, 8 / 8, 4096, 128] 57.4 / 62.0, [1, 32 / 8, 1100, 128] (288
+  // blocks) 22.6 / 27.3, [1, 32 / 8, 1700, 128] (448) 38.1 / 39.1, [1, 32 / 8, 2400, 128] (608) 67.8 / 90.1, [1, 32 / 8, 3000, 64] (768)
+  // 67.8 / 80.4; whole rounds of pairs: [1, 32 / 8, 2048, 128] (512) 48.6 / 47.6, [1, 32 / 8, 4096, 64] (1024) 111.6 / 108.9; short ones:
+  // [4, 32 / 8, 300, 64] (384) 14.9 / 13.3.  Under a short window all blocks are as long: 2400 tokens, window 300 39.2 / 44.9, 1500, 187
+  // 19.6 / 18.1.  sdpa_variant 9 pairs always, 10 never.
+  bool single = blocks <= cus;
+  if (!single && (D == 64 || D == 128)) {
+    const int64_t rounds = ttm_cdiv((int64_t)((nqb + 1) / 2) * Hq * B, cus);   // of pairs
+    if (p.lo_off < Sq / 2) single = ttm_cdiv(blocks, cus) < 2 * rounds;
+    else single = nqb >= 6 && std::max(2 * nqb * (int64_t)cus, blocks * (nqb + 1)) * 33 < 2 * cus * rounds * (nqb + 1) * 32;
+  }
+  if (variant == 9) single = false;
+  if (variant == 10) single = true;
+  const int paired = is_causal && nqb >= 2 && variant != 2 && !single;
   const dim3 grid64(paired ? (unsigned)((nqb + 1) / 2) : (unsigned)nqb, (unsigned)Hq, (unsigned)B);
   // eight wavefronts per workgroup (two key halves per query tile) when the launch would otherwise leave every SIMD with a
   // single wavefront: no more workgroups than CUs (only one eight-wavefront workgroup fits a CU, so a larger launch would
   // take a second round where the four-wavefront kernel runs two workgroups side by side).  sdpa_variant 3 forces it, 4
   // forbids it, 6 keeps the chained form of it.
-  int cus = 0, devid = 0;
-  if (hipGetDevice(&devid) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, devid) != hipSuccess || cus <= 0) cus = 256;
   const int64_t wgs = (int64_t)grid64.x * grid64.y * grid64.z;
   // (with 64 or 128 columns the eight-wavefront form is the pipelined kernel, which is the faster one at every launch size:
   // [2, 32 / 8, 4096, 128] causal 293 against 350 us, [1, 32 / 8, 8192, 128] 539 against 665 us)
-  const bool split = wide && D <= 128 && (variant == 3 || ((variant == 0 || variant == 6) && wgs <= (int64_t)cus) ||
-                                          ((variant == 0 || variant == 7 || variant == 8) && (D == 64 || D == 128)));
+  const bool split = wide && D <= 128 && (variant == 3 || ((variant == 0 || variant == 6 || variant >= 9) && wgs <= (int64_t)cus) ||
+                                          ((variant == 0 || variant >= 7) && (D == 64 || D == 128)));
   p.ksplits = 1; p.part_o = nullptr; p.part_ml = nullptr;
   if (split) {
     const dim3 block8(512);
-    // few workgroups against many keys (not the paired causal launch, whose query blocks carry equal work already): the
+    // few workgroups against many keys (not under a causal mask: [1, 16 / 4, 1024, 128] 27.6 us shared out, 19.2 not): the
     // keys of a query block are shared out until the device is full, at least four 64-key passes per share
     int64_t ks = 1;
-    if (!paired && wgs * 2 <= (int64_t)cus && ttm_option("sdpa_variant") != 5) {
+    if ((!is_causal || nqb < 2) && wgs * 2 <= (int64_t)cus && variant != 5) {
       ks = (int64_t)cus / wgs;
       if (ks > p.skt / 8) ks = p.skt / 8;
       if (ks > 16) ks = 16;
@@ -1270,7 +1307,6 @@ static int sdpa_entry(const void *q, const void *k, const void *v, const void *m
       // 128 columns: [2..8, 32 / 8, 2048, 128] causal 5..13 % faster, [1, 32 / 8, 3000, 128] 12 %); a single sequence of 2048
       // tokens has only two blocks per CU, of very different length, and is 8 % slower that way, 4096 tokens 4 % slower,
       // 8192 the same.  sdpa_variant 7 forces it, 8 keeps the eight-wavefront form.
-      const int64_t blocks = (int64_t)nqb * Hq * B;
       const bool four = variant == 7 || (variant == 0 && D == 128 && blocks >= 3 * (int64_t)cus && nqb <= 24);
       const int ring = (int)D / 32 * (four ? 20480 : 40960);   // five stages of 32 or 64 keys of K and V
       const void *fn = four ? (D == 128 ? (const void *)ttm_sdpa_pipe_k<4, 1> : (const void *)ttm_sdpa_pipe_k<2, 1>)
