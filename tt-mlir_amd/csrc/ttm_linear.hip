@@ -1937,8 +1937,10 @@ static bool mid_allowed() {
 // kernel per row tile (block-float weights; [4096, 14336] bfp8_b at 48 rows 27 us against 19, [4096, 6144] 23.6 / 13.5,
 // [1024, 1024] 10.8 / 5.9: never the better one) or ttm_linear_small_k (bf16 weights, one row tile: one workgroup per 32 columns,
 // four wavefronts over K).
+// `measured`: what it takes rather than what the models say, which judge plans of one kernel against each other and are 3 (fused),
+// 18 (images of block-float weights) and 23 % (of bf16 weights) too high on average.
 template <int WF>
-static double other_us(const LinearArgs &a) {
+static double other_us(const LinearArgs &a, bool measured = false) {
   constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
   const int cus = device_cu_count(), ksteps = (a.Kt + 1) / 2;
   if (BFP && a.Mt * 32 <= 64) return 1e30;
@@ -1949,7 +1951,20 @@ static double other_us(const LinearArgs &a) {
   us *= a.plan_batch > 1 ? (double)a.plan_batch : 1.0;
   const double first = 3.0 + (double)a.Kt * a.Nt * (a.w_batch ? a.plan_batch : 1) * ((WF == WF_BFP8 ? 1088.0 : WF == WF_BFP4 ? 576.0 : 2048.0) + 2048.0) / 5.5e6;
   const double gain = WF == WF_BFP4 ? (slices == 1 ? 0.22 : 0.08) : (slices == 1 ? 0.28 : 0.18);
-  return BFP ? std::min(us, first + (1.0 - gain) * us) : first + (1.0 - gain) * us;
+  const double two = first + (1.0 - gain) * us;
+  if (measured) return !BFP ? 0.77 * two : us <= two ? 0.97 * us : 0.82 * two;
+  return BFP ? std::min(us, two) : two;
+}
+// Whether the mid-size kernel's plan beats it.  Its own model is 3 % low for block-float and 5 % high for bf16 weights (10 % at
+// these sizes, less where K is long: 14336 x 4096 bf16 at 700 rows 140 / 148).  Over 177 shapes
+// of 400 .. 1600 rows around the line the choice costs 0.7 % against always knowing the faster one (7 % without the kernel); at
+// 4096 x 6144 bf16, image route / mid-size kernel: 520 rows 60.5 / 48.3 us, 661 rows 61.7 / 71.3; 5120 x 2880 bfp8_b, 400 rows 38.6 /
+// 28.1, 661 rows 52.3 / 49.6, 930 rows 56.0 / 54.1, 1600 rows 71.5 / 85.8.
+template <int WF>
+static bool mid_beats_other(const LinearArgs &a, const MidPlan &plan) {
+  constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
+  if (!BFP && a.Mt == 1) return plan.us < 0.93 * other_us<WF>(a);
+  return (BFP ? 1.03 : 0.95) * plan.us < other_us<WF>(a, true);
 }
 
 template <int WF>
@@ -1957,7 +1972,7 @@ static int launch_linear(const LinearArgs &a, int64_t batch, hipStream_t s) {
   constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
   if (!a.qkv && !a.norm && !a.glu && mid_allowed() && !(BFP && a.Mt == 1 && ttm_option("linear_mid") < 1000)) {
     const MidPlan plan = ttm_linear_plan_mid(a, WF, false);
-    if (ttm_option("linear_mid") >= 1000 || plan.us < 0.93 * other_us<WF>(a)) return ttm_linear_launch_mid(a, WF, plan, batch, false, s);
+    if (ttm_option("linear_mid") >= 1000 || mid_beats_other<WF>(a, plan)) return ttm_linear_launch_mid(a, WF, plan, batch, false, s);
   }
   // up to linear_small_m_max rows (64) the small kernels run once per row tile; bf16 weights leave them after one row tile
   // (from two on the image route is faster: [14336, 4096] at M = 64 116 us against 75 us)

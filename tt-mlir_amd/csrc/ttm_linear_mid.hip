@@ -3,11 +3,10 @@
 
 // =============================================================================================
 // Mid-size kernel: row counts between the decode kernel's and those that fill the device with 256-row blocks, and any product too
-// small for them.  A workgroup owns 32 MT rows x 128 columns; its 8 wavefronts are 2 column pairs (64 columns) x 4 shares of K
-// (every fourth k-tile), summed through LDS at the end.  No operand passes through LDS on the way in: weights go from global
+// small for them.  A workgroup owns 32 MT rows x 64 columns; its 4 or 8 wavefronts are shares of K (every fourth or eighth k-tile; the
+// gated form: 2 matrices x 4 shares), summed through LDS at the end.  No operand passes through LDS on the way in: weights go from global
 // memory to registers and become the MFMA operand there as in the decode kernel (byte j of eight row words feeds MFMA j, whose
-// row r stands for column 4 r + j), activation fragments are 16-byte loads of whole face-row halves, which the two column pairs of
-// a share find in L1.  That leaves no barrier in the loop and nothing to fill before it: a launch costs 3 us + its k-tiles, where
+// row r stands for column 4 r + j), activation fragments are 16-byte loads of whole face-row halves.  That leaves no barrier in the loop and nothing to fill before it: a launch costs 3 us + its k-tiles, where
 // the LDS-direct kernels' blocks cost 12 k-steps (20 us) before and after theirs - what bounded every product below some
 // 10 GFLOP.  Bounds inside the loop, per 32 k of a wavefront: about 480 cycles of vector issue for the conversion (bf16
 // weights: 64), 128 MT of the matrix core, 32 + 32 MT of L1; MT = 2 balances them for short launches, MT = 4 halves the weight
@@ -272,7 +271,7 @@ MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu) {
   // us per k-tile of a wavefront at 1 / 2 / 4 row tiles (wavefronts of a SIMD share it, so they add up)
   static const double kChunk[2][5] = {{0, 0.25, 0.44, 0, 0.57}, {0, 0.32, 0.45, 0, 0.68}};
   for (int mt = 1; mt <= 4; mt *= 2) {
-    const int blocks = units * ((p.Mt + mt - 1) / mt) * p.plan_batch;
+    const int blocks = (units + 7) / 8 * 8 * ((p.Mt + mt - 1) / mt) * p.plan_batch;   // a column unit's row blocks run on one XCD
     for (int wk = 4; wk <= 8; wk += 4) {
       if (glu ? wk != 4 || mt == 1 : (wk == 4 && mt != 2)) continue;
       for (int slices = 1; slices <= (glu ? 1 : 16); slices *= 2) {
