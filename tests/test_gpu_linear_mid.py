@@ -70,3 +70,19 @@ def test_gated_form_against_the_oracle(hip, dev, orc, plan, M, K, N):
     # two factors of up to 4, each within a bf16 step (2^-6 at magnitudes below 4) of the oracle's, and the product's own step
     assert np.max(np.abs(got - ref)) <= 2.0 ** -3
     assert np.mean(got == ref) >= 0.97
+
+
+@pytest.mark.parametrize("plan", [8101, 8201, 8401, 4201], indirect=True)
+@pytest.mark.parametrize("wfmt_name", ["bfp8", "bfp4", "bf16"])
+def test_infinite_activations(hip, dev, plan, wfmt_name):
+    """An infinite activation gives the infinities and NaN (0 x inf) of its products with the weights the device holds."""
+    M, K, N = 97, 160, 96
+    a = datagen.randn((M, K), seed=3, dtype=torch.bfloat16)
+    a[5, 40] = float("inf")
+    a[70, 159] = float("-inf")
+    w = datagen.randn((K, N), seed=4, std=0.1)
+    got, w_eff = run_linear(hip, dev, a, w, None, None, {"bfp8": hip.BFP8B, "bfp4": hip.BFP4B}.get(wfmt_name, hip.BF16))
+    want = a.float() @ torch.as_tensor(w_eff).float()
+    got = got.float()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.isinf(got), torch.isinf(want)) and torch.equal(got[torch.isinf(got)], want[torch.isinf(want)])

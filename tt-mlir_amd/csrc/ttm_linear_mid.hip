@@ -322,7 +322,12 @@ static int launch_mid(const LinearArgs &a, const MidPlan &plan, int64_t batch, b
     return ttm_set_error(TTM_ERR_INVALID, "ttm_linear_glu: the mid-size kernel's gated form takes bfp8_b weights");
   }
   switch (plan.wk * 10 + plan.mt) {
-  case 81: launch_mid_mt<WF, 1, 8, true>(p, grid, s); break;
+  case 81:
+    // The two-term operand (1.m and 1.0 products, subtracted at the end) saves conversion work, but an infinite activation leaves
+    // inf - inf: only up to 64 rows, where the decode kernel multiplies the same way.
+    if (a.Mt <= 2) launch_mid_mt<WF, 1, 8, true>(p, grid, s);
+    else launch_mid_mt<WF, 1, 8, false>(p, grid, s);
+    break;
   case 82: launch_mid_mt<WF, 2, 8, false>(p, grid, s); break;
   case 84: launch_mid_mt<WF, 4, 8, false>(p, grid, s); break;
   case 42: launch_mid_mt<WF, 2, 4, false>(p, grid, s); break;
