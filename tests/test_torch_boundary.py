@@ -26,3 +26,15 @@ def test_other_kinds_of_tensors_keep_their_values():
     for t in (x.as_subclass(Named), torch.nn.Parameter(x, requires_grad=False), torch.tensor([1 - 2j, 3 + 4j]).imag, x.t(), x.expand(4, 2, 3),
               torch._neg_view(x).resolve_neg(), torch.empty(0, 3)):
         assert torch.equal(rt.to_torch(rt.from_torch(t)), torch.Tensor(t))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.int32, torch.uint8])
+def test_results_come_back_to_host_memory_whatever_the_default_device(dtype):
+    x = torch.arange(2000).reshape(50, 40).to(dtype)
+    host = rt.from_torch(x)
+    with torch.device("meta"):
+        back = rt.to_torch(host)
+    assert back.device.type == "cpu" and torch.equal(back, x)
+    with FakeTensorMode():
+        fake = rt.to_torch(host)
+    assert fake.shape == x.shape and fake.dtype == dtype

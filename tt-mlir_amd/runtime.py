@@ -329,15 +329,15 @@ _torch_types = None
 
 
 def _torch_maps():
-    """({torch dtype: (DataType, element size)}, {DataType: torch dtype}), built once."""
+    """({torch dtype: (DataType, element size)}, {DataType: (torch dtype, numpy dtype that holds its bits)}), built once."""
     global _torch_types
     if _torch_types is None:
         import torch
         to_rt = {torch.float32: DataType.Float32, torch.bfloat16: DataType.BFloat16, torch.float16: DataType.Float16,
                  torch.int32: DataType.Int32, torch.int64: DataType.Int64, torch.uint8: DataType.UInt8, torch.float64: DataType.Float64,
                  torch.int16: DataType.Int16, torch.int8: DataType.Int8, torch.bool: DataType.Bool}
-        back = {DataType.Float32: torch.float32, DataType.BFloat16: torch.bfloat16, DataType.Float16: torch.float16,
-                DataType.Int32: torch.int32, DataType.UInt8: torch.uint8}
+        back = {DataType.Float32: (torch.float32, np.float32), DataType.BFloat16: (torch.bfloat16, np.int16),
+                DataType.Float16: (torch.float16, np.float16), DataType.Int32: (torch.int32, np.int32), DataType.UInt8: (torch.uint8, np.uint8)}
         _torch_types = {k: (v, torch.empty(0, dtype=k).element_size()) for k, v in to_rt.items()}, back
     return _torch_types
 
@@ -465,13 +465,15 @@ def to_torch(tensor):
     lay = tensor.desc()[1]
     host = to_host(tensor, untilize=True)[0] if lay.storage != StorageType.Host else tensor
     shape, hlay, nbytes = host.desc()
-    dt = _torch_maps()[1].get(hlay.dtype)
+    dt, np_dtype = _torch_maps()[1].get(hlay.dtype, (None, None))
     if dt is None or hlay.layout == TensorLayout.Tile or nbytes == 0:
         a = to_numpy(host)
         return torch.from_numpy(a.view(np.int16)).view(torch.bfloat16) if lay.dtype == DataType.BFloat16 else torch.from_numpy(a)
-    out = torch.empty(shape, dtype=dt)
-    _call("ttrt_memcpy_out", ctypes.c_void_p(out.data_ptr()), host.h, -1)
-    return out
+    # the result in numpy's memory, not torch.empty's: a default device or an active FakeTensorMode would put that elsewhere
+    out = np.empty(shape, dtype=np_dtype)
+    memcpy(out, host)
+    out = torch.from_numpy(out)
+    return out if out.dtype == dt else out.view(dt)
 
 
 def buffer_cast(src, from_dtype, to_dtype):
