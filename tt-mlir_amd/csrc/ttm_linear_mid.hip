@@ -330,8 +330,7 @@ static int launch_mid(const LinearArgs &a, const MidPlan &plan, int64_t batch, b
     break;
   case 82: launch_mid_mt<WF, 2, 8, false>(p, grid, s); break;
   case 84: launch_mid_mt<WF, 4, 8, false>(p, grid, s); break;
-  case 42: launch_mid_mt<WF, 2, 4, false>(p, grid, s); break;
-  default: return ttm_set_error(TTM_ERR_INVALID, "ttm_linear: no such plan of the mid-size kernel (linear_mid = %d)", ttm_option("linear_mid"));
+  default: launch_mid_mt<WF, 2, 4, false>(p, grid, s);   // 42: ttm_linear_plan_mid has no others
   }
   if (slices > 1)
     ttm_linear_launch_reduce(p, slices, batch, s);
@@ -340,6 +339,8 @@ static int launch_mid(const LinearArgs &a, const MidPlan &plan, int64_t batch, b
 
 
 int ttm_linear_launch_mid(const LinearArgs &a, int wf, const MidPlan &plan, int64_t batch, bool glu, hipStream_t s) {
+  if (plan.mt == 0)
+    return ttm_set_error(TTM_ERR_INVALID, "ttm_linear: no such plan of the mid-size kernel%s (linear_mid = %d)", glu ? "'s gated form" : "", ttm_option("linear_mid"));
   switch (wf) {
   case WF_BFP8: return launch_mid<WF_BFP8>(a, plan, batch, glu, s);
   case WF_BFP4: return launch_mid<WF_BFP4>(a, plan, batch, glu, s);
