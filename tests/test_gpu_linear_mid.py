@@ -86,3 +86,11 @@ def test_infinite_activations(hip, dev, plan, wfmt_name):
     got = got.float()
     assert torch.equal(torch.isnan(got), torch.isnan(want))
     assert torch.equal(torch.isinf(got), torch.isinf(want)) and torch.equal(got[torch.isinf(got)], want[torch.isinf(want)])
+
+
+@pytest.mark.parametrize("plan", [8102, 8216, 8404], indirect=True)
+@pytest.mark.parametrize("K", [20, 70])
+def test_more_slices_than_k_tiles(hip, dev, orc, metrics, plan, K):  # noqa: F811
+    a, w = datagen.randn((70, K), seed=1, dtype=torch.bfloat16), datagen.randn((K, 96), seed=2, std=K ** -0.5)
+    got, w_eff = run_linear(hip, dev, a, w, None, None, hip.BFP8B)
+    check(orc, metrics, got, a, w_eff, None, None, max_abs=2.0 ** -5)

@@ -304,9 +304,11 @@ static int launch_mid(const LinearArgs &a, const MidPlan &plan, int64_t batch, b
   p.partial = nullptr;
   p.k_slice = p.Kt;
   const int64_t per = (int64_t)p.Mt * p.Nt * 1024;
-  if (slices > 1) {
+  if (slices > 1) {   // a pinned split of a short K may come down to fewer slices, or to one
     p.k_slice = (p.Kt + slices - 1) / slices;
     slices = (p.Kt + p.k_slice - 1) / p.k_slice;
+  }
+  if (slices > 1) {
     void *ws = nullptr;
     if (int rc = ttm_stream_workspace(s, (size_t)(per * slices * batch) * sizeof(float), &ws)) return rc;
     p.partial = (float *)ws;
