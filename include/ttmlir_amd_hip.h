@@ -390,12 +390,13 @@ int ttm_rotary_embedding_llama(const void *x, const void *cos_cache, const void 
                                int dtype, int64_t batch, int64_t rows, int64_t cols, int64_t cs_batch, int64_t cs_rows, void *stream);
 
 /* ttm_sdpa_decode_windowed that allocates nothing.  It has no counterpart in the reference; it is for callers that cannot
- * call hipMalloc: code under HIP graph capture, tight serving loops, harnesses that forbid allocation.  Same arguments, same
- * kernels and bit-identical results; the per-slice partial results (max, sum, unnormalised output) go to a static device
- * array of 8 MiB that the library holds on every GPU it runs on until the process ends, instead of the stream's grow-only
- * workspace.  A call whose partial results need more (kv_heads * (key shares + batch) * min(heads / kv_heads, 8) * (head_dim + 2)
- * floats; the config-5 decode shape of 32 users x 8 kv heads x 2048 positions takes 1.6 MB) fails with TTM_ERR_INVALID and
- * launches nothing.  No hipMalloc, hipFree or allocating library call is made; the first call on a device looks the
+ * call hipMalloc: code under HIP graph capture, tight serving loops, harnesses that forbid allocation.  Same arguments and
+ * the same kernels; partial results (max, sum, unnormalised output, one per user or share of the keys and head) go to a static
+ * device array of 8 MiB that the library holds on every GPU it runs on until the process ends, instead of the stream's grow-only
+ * workspace.  A call whose users alone would fill it (batch * kv_heads * min(heads / kv_heads, 8) * (head_dim + 2) floats: 1.1 MB
+ * for 32 users x 8 kv heads of 4 heads x 128) fails with TTM_ERR_INVALID and launches nothing.  Results are bit-identical, but
+ * for calls of some 500 and more users x kv heads with long caches, whose keys are not shared out here.
+ * No hipMalloc, hipFree or allocating library call is made; the first call on a device looks the
  * array's address up (hipGetSymbolAddress), so make that call outside a capture.  All calls on one GPU share the array:
  * calls that overlap in time on one GPU (different streams) race; calls on one stream are ordered and safe. */
 int ttm_sdpa_decode_static(const void *q, const void *k, const void *v, const int32_t *cur_pos, const void *mask,

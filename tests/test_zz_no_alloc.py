@@ -56,3 +56,24 @@ def test_static_scratch_refuses_what_does_not_fit(hip, dev):
                      hip.BF16, 64, 256, 32, 8192, 128, 1, 0.0, 0, -1, None, hip.current_stream())
     finally:
         hip.set_option("check_extents", 1)
+
+
+@pytest.mark.parametrize("B,H,Hkv,S,D", [
+    (220, 32, 8, 256, 256),     # the direct form: no partial results, though users and shares together would not fit
+    (400, 16, 2, 64, 256),      # users fit, users and shares do not, eight heads x 256 columns: two direct launches of four heads
+    (400, 24, 2, 64, 256),      # ... of twelve heads: three
+    (500, 16, 2, 64, 192),      # ... head dim without a kernel of its own: five heads and three
+    (500, 32, 4, 64, 128),      # ... in one
+])
+def test_static_scratch_takes_many_users(hip, dev, orc, B, H, Hkv, S, D):
+    """Calls whose users fit the array are served whatever the number of key shares; against the oracle within a bf16 step of outputs
+    below 1 (2^-7) and the rounding of the numerators (2^-8 of |v| < 5), 2^-6 together."""
+    q, k, v, qt, kt, vt = _operands(hip, dev, B, H, Hkv, S, D, 90)
+    cur = [(37 * u) % S for u in range(B)]
+    out = _run(hip, "ttm_sdpa_decode_static", qt, kt, vt, torch.tensor(cur, dtype=torch.int32, device=dev), B, H, Hkv, S, D)
+    have = untilize_dev(hip, out, q.shape, dev).float().cpu().numpy()
+    some = [0, 1, B // 2, B - 2, B - 1]
+    want = orc.sdpa_decode(q.float().numpy()[:, some], k[some].float().numpy(), v[some].float().numpy(), cur_pos=[cur[u] for u in some], is_causal=True)
+    assert np.max(np.abs(have[:, some] - want)) <= 2.0 ** -6
+    ref = _run(hip, "ttm_sdpa_decode_windowed", qt, kt, vt, torch.tensor(cur, dtype=torch.int32, device=dev), B, H, Hkv, S, D)
+    assert np.max(np.abs(have - untilize_dev(hip, ref, q.shape, dev).float().cpu().numpy())) <= 2.0 ** -6

@@ -858,7 +858,9 @@ static void launch_decode(const DecodeArgs &p, dim3 grid, hipStream_t s) {
   case 32: return few ? launch_decode<true, 4, 1, true, NWS, DIRECT>(p, grid, s) : once ? launch_decode<true, 8, 1, true, NW, DIRECT>(p, grid, s) : launch_decode<false, 8, 1, true, NW, DIRECT>(p, grid, s);
   case 64: return few ? launch_decode<true, 4, 2, true, NWS, DIRECT>(p, grid, s) : once ? launch_decode<true, 8, 2, true, NW, DIRECT>(p, grid, s) : launch_decode<false, 8, 2, true, NW, DIRECT>(p, grid, s);
   case 128: return few ? launch_decode<true, 4, 4, true, NWS, DIRECT>(p, grid, s) : once ? launch_decode<true, 8, 4, true, NW, DIRECT>(p, grid, s) : launch_decode<false, 8, 4, true, NW, DIRECT>(p, grid, s);
-  case 256: return few ? launch_decode<true, 4, 8, true, NW, DIRECT>(p, grid, s) : once ? launch_decode<true, 8, 8, true, NW, DIRECT>(p, grid, s) : launch_decode<false, 8, 8, true, NW, DIRECT>(p, grid, s);
+  case 256:
+    if constexpr (DIRECT) return once ? launch_decode<true, 4, 8, true, NW, DIRECT>(p, grid, s) : launch_decode<false, 4, 8, true, NW, DIRECT>(p, grid, s);   // at most 1024 outputs
+    else return few ? launch_decode<true, 4, 8, true, NW, DIRECT>(p, grid, s) : once ? launch_decode<true, 8, 8, true, NW, DIRECT>(p, grid, s) : launch_decode<false, 8, 8, true, NW, DIRECT>(p, grid, s);
   default: return p.D < 128 ? launch_decode<false, 8, 4, false, NW, DIRECT>(p, grid, s) : launch_decode<false, 8, 8, false, NW, DIRECT>(p, grid, s);
   }
 }
@@ -890,7 +892,7 @@ static int sdpa_decode_entry(const void *q, const void *k, const void *v, const 
   // 16 x 2048 15.4 / 18.1, 16 x 4096 26.5 / 25.5.
   const int form = ttm_option("sdpa_decode_form");   // 0 by this rule, 1 direct, 2 shares
   // (the results of the wavefronts fit in 32 KiB of LDS)
-  const bool direct = G * head_dim <= 1024 && (form ? form == 1 : seq * head_dim <= 2048 * std::max<int64_t>(64, batch * kv_heads));
+  bool direct = G * head_dim <= 1024 && (form ? form == 1 : seq * head_dim <= 2048 * std::max<int64_t>(64, batch * kv_heads));
   const int64_t all = batch * (seq / 32);          // tiles of a kv head when every cache is full
   int64_t shares = ttm_cdiv(kDecodeBlocks, kv_heads);
   if (shares > all / 4) shares = all / 4 > 0 ? all / 4 : 1;   // a tile for every wavefront
@@ -909,21 +911,30 @@ static int sdpa_decode_entry(const void *q, const void *k, const void *v, const 
   p.sink = (const uint16_t *)sink;
   TTM_REQUIRE(!mask || mask_batch == 1 || mask_batch == batch, "ttm_sdpa_decode: mask batch must be 1 or %lld", (long long)batch);
   p.mask_b = mask_batch == 1 ? 0 : 1;
+  const size_t slot_bytes = (size_t)(kv_heads * G * (head_dim + 2)) * sizeof(float);   // of one share or user, all kv heads
+  size_t part_bytes = direct ? 0 : slot_bytes * (size_t)(shares + batch);
+  int64_t per_launch = kMaxG;
   void *ws = nullptr;
-  const size_t part_bytes = (size_t)(kv_heads * (shares + batch) * G * (head_dim + 2)) * sizeof(float);
   if (static_scratch) {
-    TTM_REQUIRE(part_bytes <= kDecodeScratchBytes,
-                "ttm_sdpa_decode_static: the per-slice partial results of this call take %zu bytes, the static scratch holds %zu "
-                "(kv_heads * (shares + batch) * heads-per-kv-head * (head_dim + 2) floats): use ttm_sdpa_decode_windowed",
-                part_bytes, (size_t)kDecodeScratchBytes);
+    TTM_REQUIRE(slot_bytes * (size_t)batch <= kDecodeScratchBytes,
+                "ttm_sdpa_decode_static: one partial result per user and head of this call takes %zu bytes, the static scratch holds %zu "
+                "(batch * kv_heads * heads-per-kv-head * (head_dim + 2) floats): use ttm_sdpa_decode_windowed",
+                slot_bytes * (size_t)batch, (size_t)kDecodeScratchBytes);
+    if (part_bytes > kDecodeScratchBytes) {
+      // More than some 500 users x kv heads (a share and a user take a slot each): the direct form needs no slots, and that many
+      // workgroups fill the device; above 1024 outputs per kv head in several launches of fewer heads
+      direct = true;
+      part_bytes = 0;
+      per_launch = std::min<int64_t>(kMaxG, 1024 / head_dim);
+    }
     if (int rc = decode_scratch_ptr(&ws)) return rc;
-  } else {
+  } else if (part_bytes) {
     if (int rc = ttm_stream_workspace(s, part_bytes, &ws)) return rc;
   }
   p.part = (float *)ws;
-  for (int64_t g0 = 0; g0 < Gt; g0 += kMaxG) {   // the launches of one call follow each other on the stream and share the workspace
+  for (int64_t g0 = 0; g0 < Gt; g0 += per_launch) {   // the launches of one call follow each other on the stream and share the workspace
     p.g0 = (int)g0;
-    p.G = (int)(Gt - g0 < kMaxG ? Gt - g0 : kMaxG);
+    p.G = (int)(Gt - g0 < per_launch ? Gt - g0 : per_launch);
     if (direct) {
       launch_decode<true>(p, dim3((unsigned)kv_heads, (unsigned)batch), s);
       TTM_LAUNCH_CHECK();
