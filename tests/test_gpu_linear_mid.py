@@ -94,3 +94,33 @@ def test_more_slices_than_k_tiles(hip, dev, orc, metrics, plan, K):  # noqa: F81
     a, w = datagen.randn((70, K), seed=1, dtype=torch.bfloat16), datagen.randn((K, 96), seed=2, std=K ** -0.5)
     got, w_eff = run_linear(hip, dev, a, w, None, None, hip.BFP8B)
     check(orc, metrics, got, a, w_eff, None, None, max_abs=2.0 ** -5)
+
+
+@pytest.mark.parametrize("wfmt_name,M,K,N", [("bf16", 20, 4096, 512), ("bf16", 1, 2048, 128), ("bfp8", 100, 4096, 256)])
+def test_a_split_product_is_recorded_on_a_stream_without_workspace(hip, dev, orc, metrics, wfmt_name, M, K, N):  # noqa: F811
+    """Recorded as the first call of its stream and replayed on changing activations, with eager calls in between."""
+    wfmt = {"bfp8": hip.BFP8B, "bf16": hip.BF16}[wfmt_name]
+    w = datagen.randn((K, N), seed=N, std=K ** -0.5)
+    xs = [datagen.randn((M, K), seed=i, dtype=torch.bfloat16) for i in range(3)]
+    eager, w_eff = zip(*[run_linear(hip, dev, x, w, None, None, wfmt) for x in xs])
+    wt = tilize_dev(hip, w.to(torch.bfloat16), dev) if wfmt == hip.BF16 else pack_weight(hip, w, wfmt, dev)
+    a, out = tilize_dev(hip, xs[0], dev), torch.full(((M + 31) // 32 * 32 * N,), float("nan"), dtype=torch.bfloat16, device=dev)
+    torch.cuda.synchronize()
+    stream, graph, nodes = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_size_t()
+    hip.call("ttm_stream_create", ctypes.byref(stream))
+    hip.call("ttm_graph_begin_capture", stream)
+    try:
+        hip.call("ttm_linear", hip.ptr(a), hip.BF16, hip.ptr(wt), wfmt, 0, None, hip.BF16, hip.TILE, hip.ptr(out), hip.BF16, 1, 1, M, N, K, 0, stream)
+    finally:
+        hip.call("ttm_graph_end_capture", stream, ctypes.byref(graph), ctypes.byref(nodes))
+    assert nodes.value == 1
+    for x, e in zip(xs, eager):
+        a.copy_(tilize_dev(hip, x, dev))
+        torch.cuda.synchronize()
+        hip.call("ttm_graph_launch", graph, stream)
+        hip.call("ttm_stream_sync", stream)
+        got = untilize_dev(hip, out, (M, N), dev).cpu()
+        check(orc, metrics, got, x, w_eff[0], None, None, max_abs=2.0 ** -5)
+        assert torch.allclose(got.float(), e.float(), atol=2.0 ** -5)
+    hip.call("ttm_graph_destroy", graph)
+    hip.call("ttm_stream_destroy", stream)

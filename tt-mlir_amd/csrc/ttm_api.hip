@@ -213,6 +213,15 @@ int ttm_stream_workspace(hipStream_t stream, size_t bytes, void **ptr) {
   return TTM_OK;
 }
 
+bool ttm_stream_workspace_ready(hipStream_t stream, size_t bytes) {
+  int dev = 0;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &st) != hipSuccess || st == hipStreamCaptureStatusNone || hipGetDevice(&dev) != hipSuccess) return true;
+  std::lock_guard<std::mutex> g(g_ws_mu);
+  const auto it = g_ws.find({dev, stream});
+  return it != g_ws.end() && it->second.bytes >= bytes;
+}
+
 TTM_EXPORT int ttm_stream_destroy(void *stream) {
   if (!stream) return TTM_OK;
   TTM_HIP(hipStreamSynchronize((hipStream_t)stream));

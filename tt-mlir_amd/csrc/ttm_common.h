@@ -84,6 +84,8 @@ struct TtmExtentChecker {
 // Growing allocates with hipMalloc and is refused while the stream is capturing; an allocation that a captured graph may
 // have recorded is never freed before the stream is destroyed.
 int ttm_stream_workspace(hipStream_t stream, size_t bytes, void **ptr);
+// False when that call would be refused: the stream is capturing and its workspace is smaller.
+bool ttm_stream_workspace_ready(hipStream_t stream, size_t bytes);
 
 // RMSNorm that starts from the fp32 partial sums of a split-K projection of one row tile plus a residual (ttm_rowwise.hip)
 bool ttm_rowwise_partials_supported(int64_t rows, int64_t cols);

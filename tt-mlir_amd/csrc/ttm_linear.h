@@ -204,5 +204,5 @@ struct MidPlan {
   int mt = 0, wk = 8, slices = 1;
   double us = 0;
 };
-MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu);
+MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu, int max_slices = 16);
 int ttm_linear_launch_mid(const LinearArgs &a, int wf, const MidPlan &plan, int64_t batch, bool glu, hipStream_t s);

@@ -261,7 +261,7 @@ static int mid_units(const LinearArgs &p, bool glu) { return glu ? (p.gNt[0] + 1
 // over 380 timings; the plan it picks is 1 % slower than the best one on average): 3.3 us for launch, first loads and the last
 // wavefronts, the k-tiles that the wavefronts of a SIMD take, 0.2 + 0.95 us per row tile for the sums through LDS of each
 // round of workgroups, and for a split K the reduction's launch and its traffic at 2.5 TB/s.
-MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu) {
+MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu, int max_slices) {
   // option linear_mid: 0 by the model, 1 never, 1000 * shares + 100 * row tiles + slices pins a plan
   const int force = ttm_option("linear_mid");
   MidPlan best;
@@ -274,7 +274,7 @@ MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu) {
     const int blocks = (units + 7) / 8 * 8 * ((p.Mt + mt - 1) / mt) * p.plan_batch;   // a column unit's row blocks run on one XCD
     for (int wk = 4; wk <= 8; wk += 4) {
       if (glu ? wk != 4 || mt == 1 : (wk == 4 && mt != 2)) continue;
-      for (int slices = 1; slices <= (glu ? 1 : 16); slices *= 2) {
+      for (int slices = 1; slices <= (glu ? 1 : max_slices); slices *= 2) {
         if (force >= 1000) {
           if (force / 1000 != wk || force % 1000 / 100 != mt || force % 100 != slices) continue;
         } else if ((mt > 1 && mt >= 2 * p.Mt) || (slices > 1 && p.Kt < 2 * wk * slices)) {
@@ -340,7 +340,13 @@ static int launch_mid(const LinearArgs &a, const MidPlan &plan, int64_t batch, b
 }
 
 
-int ttm_linear_launch_mid(const LinearArgs &a, int wf, const MidPlan &plan, int64_t batch, bool glu, hipStream_t s) {
+int ttm_linear_launch_mid(const LinearArgs &a, int wf, const MidPlan &best, int64_t batch, bool glu, hipStream_t s) {
+  MidPlan plan = best;
+  // A recording stream cannot allocate the slices' partial sums: unless an earlier call left room for them, the best plan without
+  // (the kernels this one took over from ran such products unsplit, so they could always be recorded)
+  if (plan.slices > 1 && ttm_option("linear_mid") < 1000 &&
+      !ttm_stream_workspace_ready(s, (size_t)((int64_t)a.Mt * a.Nt * 1024 * plan.slices * batch) * sizeof(float)))
+    plan = ttm_linear_plan_mid(a, wf, glu, 1);
   if (plan.mt == 0)
     return ttm_set_error(TTM_ERR_INVALID, "ttm_linear: no such plan of the mid-size kernel%s (linear_mid = %d)", glu ? "'s gated form" : "", ttm_option("linear_mid"));
   switch (wf) {
