@@ -555,7 +555,7 @@ bool convertInOneLaunch(const void *src, TensorLayout sl, DataType sd, void *dst
 
 DeviceState::~DeviceState() {
   if (open && stream) ttm_stream_destroy(stream);
-  if (staging) hostPool().free(staging, kStagingBytes);
+  if (staging) hostPool().free(staging);
 }
 
 size_t getNumAvailableDevices() {
@@ -580,7 +580,7 @@ Device openMeshDevice(const MeshDeviceOptions &options) {
     std::memset(probe, 0, 16);
     st->kernelsReachHost = ttm_copy_kernel(probe, there, 16, st->stream) == 0 && ttm_stream_sync(st->stream) == 0;
     pool().free(there, 16);
-    hostPool().free(probe, kStagingBytes);
+    hostPool().free(probe);
   }
   {
     std::lock_guard<std::mutex> g(deviceRegistry().mu);
@@ -667,7 +667,7 @@ void closeMeshDevice(Device d) {
     }
   }
   pool().release();
-  if (d.handle->staging) hostPool().free(d.handle->staging, kStagingBytes);
+  if (d.handle->staging) hostPool().free(d.handle->staging);
   d.handle->staging = nullptr;
   hostPool().release();
   TTM_CALL(ttm_stream_destroy(d.handle->stream));
@@ -887,7 +887,7 @@ Tensor fetchAs(const Tensor &d, TensorLayout layout, DataType dtype) {
   auto t = std::make_shared<TensorImpl>();
   t->shape = s.shape; t->dtype = dtype; t->layout = layout; t->storage = StorageType::Host;
   t->bytes = bytes;
-  t->data = std::shared_ptr<void>(p, [bytes](void *q) { hostPool().free(q, bytes); });
+  t->data = std::shared_ptr<void>(p, [](void *q) { hostPool().free(q); });
   t->version = nextTensorVersion();
   if (same && bytes > kKernelCopyMax) {
     TTM_CALL(ttm_memcpy_d2h(p, s.data.get(), bytes, dev.stream));
