@@ -268,8 +268,25 @@ EXPORT int ttm_free(void *dptr) {
   free(dptr);
   return TTM_OK;
 }
-EXPORT int ttm_host_alloc(void **hptr, size_t bytes) { if (!hptr) return fail("null"); *hptr = malloc(bytes ? bytes : 1); return *hptr ? TTM_OK : fail("out of memory"); }
-EXPORT int ttm_host_free(void *hptr) { free(hptr); return TTM_OK; }
+// page-locked host memory is within the kernels' reach, as on the GPU; TTMLIR_AMD_NULL_DEVICE_PAGEABLE=1: it is not, and the runtime
+// takes its memcpy routes
+const bool g_host_reach = !(getenv("TTMLIR_AMD_NULL_DEVICE_PAGEABLE") && std::string(getenv("TTMLIR_AMD_NULL_DEVICE_PAGEABLE")) == "1");
+EXPORT int ttm_host_alloc(void **hptr, size_t bytes) {
+  if (!hptr) return fail("null");
+  *hptr = malloc(bytes ? bytes : 1);
+  if (!*hptr) return fail("out of memory");
+  std::lock_guard<std::mutex> g(g_mu);
+  if (g_host_reach) g_allocs[(uintptr_t)*hptr] = bytes;
+  return TTM_OK;
+}
+EXPORT int ttm_host_free(void *hptr) {
+  {
+    std::lock_guard<std::mutex> g(g_mu);
+    g_allocs.erase((uintptr_t)hptr);
+  }
+  free(hptr);
+  return TTM_OK;
+}
 EXPORT int ttm_memcpy_h2d(void *dst, const void *src, size_t bytes, void *) {
   if (!bytes) return TTM_OK;
   if (!src) return fail("ttm_memcpy_h2d: null source");

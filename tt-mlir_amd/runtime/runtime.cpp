@@ -514,7 +514,10 @@ const void *stage(DeviceState &dev, const void *src, size_t bytes) {
     if (!dev.staging) return nullptr;
   }
   const size_t room = (bytes + 511) / 512 * 512;   // device blocks are rounded the same way: copies move whole 16-byte chunks
-  if (dev.stagingHead + room > kStagingBytes) syncStream(dev);
+  if (dev.stagingHead + room > kStagingBytes) {
+    syncStream(dev);
+    debug::Stats::get().incrementStat("StagingBlockReused");
+  }
   auto *p = static_cast<std::uint8_t *>(dev.staging) + dev.stagingHead;
   dev.stagingHead += room;
   std::memcpy(p, src, bytes);
@@ -527,29 +530,32 @@ bool wholeChunkRows(const std::vector<std::uint32_t> &shape, DataType dtype) {
   return utils::isBlockFormatDataType(dtype) || dims3(shape).cols * utils::dataTypeElementSize(dtype) % 16 == 0;
 }
 
-// src (a tensor of this shape in layout / dtype sl / sd) into dst in dl / dd with one launch; false when there is no such
-// kernel.  Either side may be page-locked host memory.
-bool convertInOneLaunch(const void *src, TensorLayout sl, DataType sd, void *dst, TensorLayout dl, DataType dd,
-                        const std::vector<std::uint32_t> &shape, void *stream) {
-  const Dims3 d = dims3(shape);
+// Whether one kernel takes layout / dtype sl / sd to dl / dd.
+bool oneLaunch(TensorLayout sl, DataType sd, TensorLayout dl, DataType dd) {
   const auto plain = [](DataType t) { return t == DataType::Float32 || t == DataType::BFloat16; };
   const auto block = [](DataType t) { return t == DataType::BFP_BFloat8 || t == DataType::BFP_BFloat4; };
+  return (sl == dl && sd == dd) || (plain(sd) && block(dd) && dl == TensorLayout::Tile) || (block(sd) && sl == TensorLayout::Tile && plain(dd)) ||
+         (sd == dd && !utils::isBlockFormatDataType(sd));
+}
+
+// src (a tensor of this shape in layout / dtype sl / sd) into dst in dl / dd with that launch.  Either side may be page-locked host
+// memory.
+void convertInOneLaunch(const void *src, TensorLayout sl, DataType sd, void *dst, TensorLayout dl, DataType dd,
+                        const std::vector<std::uint32_t> &shape, void *stream) {
+  const Dims3 d = dims3(shape);
   const int lsl = static_cast<int>(sl), ldl = static_cast<int>(dl), lsd = static_cast<int>(sd), ldd = static_cast<int>(dd);
   if (sl == dl && sd == dd) {
     const size_t bytes = tensorBytes(shape, sd, sl);
     TTM_CALL(ttm_copy_kernel(src, dst, (bytes + 15) / 16 * 16, stream));
-  } else if (plain(sd) && block(dd) && dl == TensorLayout::Tile) {
+  } else if (utils::isBlockFormatDataType(dd)) {
     TTM_CALL(ttm_bfp_pack(src, lsd, lsl, dst, ldd, d.batch, d.rows, d.cols, stream));
-  } else if (block(sd) && sl == TensorLayout::Tile && plain(dd)) {
+  } else if (utils::isBlockFormatDataType(sd)) {
     TTM_CALL(ttm_bfp_unpack(src, lsd, dst, ldd, ldl, d.batch, d.rows, d.cols, stream));
-  } else if (sd == dd && !utils::isBlockFormatDataType(sd)) {
+  } else {
     const int es = static_cast<int>(utils::dataTypeElementSize(sd));
     if (dl == TensorLayout::Tile) TTM_CALL(ttm_tilize(src, dst, d.batch, d.rows, d.cols, es, stream));
     else TTM_CALL(ttm_untilize(src, dst, d.batch, d.rows, d.cols, es, stream));
-  } else {
-    return false;
   }
-  return true;
 }
 }  // namespace
 
@@ -852,9 +858,12 @@ bool uploadInto(const Tensor &h, const Tensor &d) {
   DeviceState &dev = *d.handle->device;
   std::lock_guard<std::recursive_mutex> g(dev.mu);
   requireNotCapturing(d.handle->device, "a host to device transfer");
+  if (!oneLaunch(s.layout, s.dtype, d.handle->layout, d.handle->dtype)) return false;   // before anything is staged
   if (s.layout != d.handle->layout && !wholeChunkRows(s.shape, s.dtype)) return false;
   const void *p = stage(dev, s.data.get(), s.bytes);
-  return p && convertInOneLaunch(p, s.layout, s.dtype, d.handle->data.get(), d.handle->layout, d.handle->dtype, s.shape, dev.stream);
+  if (!p) return false;
+  convertInOneLaunch(p, s.layout, s.dtype, d.handle->data.get(), d.handle->layout, d.handle->dtype, s.shape, dev.stream);
+  return true;
 }
 
 Tensor uploadAs(const Tensor &h, const std::shared_ptr<DeviceState> &dev, TensorLayout layout, DataType dtype) {
@@ -891,8 +900,9 @@ Tensor fetchAs(const Tensor &d, TensorLayout layout, DataType dtype) {
   t->version = nextTensorVersion();
   if (same && bytes > kKernelCopyMax) {
     TTM_CALL(ttm_memcpy_d2h(p, s.data.get(), bytes, dev.stream));
-  } else if ((s.layout != layout && !wholeChunkRows(s.shape, dtype)) ||
-             !convertInOneLaunch(s.data.get(), s.layout, s.dtype, p, layout, dtype, s.shape, dev.stream)) {
+  } else if (oneLaunch(s.layout, s.dtype, layout, dtype) && (s.layout == layout || wholeChunkRows(s.shape, dtype))) {
+    convertInOneLaunch(s.data.get(), s.layout, s.dtype, p, layout, dtype, s.shape, dev.stream);
+  } else {
     const Tensor c = convertOnDevice(d, layout, dtype);
     if (bytes <= kKernelCopyMax) TTM_CALL(ttm_copy_kernel(c.handle->data.get(), p, (bytes + 15) / 16 * 16, dev.stream));
     else TTM_CALL(ttm_memcpy_d2h(p, c.handle->data.get(), bytes, dev.stream));
