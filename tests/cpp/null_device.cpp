@@ -314,7 +314,9 @@ EXPORT int ttm_fill_u32(void *dst, uint32_t value, size_t count, void *) {
 }
 EXPORT int ttm_stream_create(void **stream) { if (!stream) return fail("null"); *stream = malloc(8); return TTM_OK; }
 EXPORT int ttm_stream_destroy(void *stream) { free(stream); return TTM_OK; }
-EXPORT int ttm_stream_sync(void *) { return TTM_OK; }
+std::atomic<long> g_syncs{0};
+EXPORT int ttm_stream_sync(void *) { ++g_syncs; return TTM_OK; }
+EXPORT long null_device_syncs(void) { return g_syncs; }   // for tests: how often a stream was waited for
 EXPORT int ttm_device_sync(void) { return TTM_OK; }
 EXPORT int ttm_event_create(void **event) { if (!event) return fail("null"); *event = malloc(8); return TTM_OK; }
 EXPORT int ttm_event_destroy(void *event) { free(event); return TTM_OK; }

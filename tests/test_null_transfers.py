@@ -37,3 +37,27 @@ assert rt.get_stat("StagingBlockReused") == 1, rt.get_stat("StagingBlockReused")
 for x, d in zip(xs, ds):
     assert torch.equal(rt.to_torch(d), x.to(torch.bfloat16))
 """)
+
+
+def test_uploads_are_waited_for_beside_another_open_handle(null_env):  # noqa: F811
+    """Every handle has a stream of its own and the device pool is common: a tensor that is still on its way on one stream could be
+    read, or its memory reused, on the other."""
+    run(null_env, """
+import ctypes
+null = ctypes.CDLL(os.environ["TTMLIR_AMD_HIP_LIB"])
+null.null_device_syncs.restype = ctypes.c_long
+def waits(f):
+    before = null.null_device_syncs()
+    f()
+    return null.null_device_syncs() - before
+plain, tiled = rt.Layout(ST.Device, TL.RowMajor, DT.Float32), rt.Layout(ST.Device, TL.Tile, DT.Float32)
+x = torch.randn(64, 96)
+up = lambda d, lay: rt.to_layout(rt.from_torch(x), d, lay)
+assert waits(lambda: up(device, plain)) == waits(lambda: up(device, tiled)) == 0
+others = []
+assert waits(lambda: others.append(rt.open_mesh_device())) >= 2      # its own probe, and what the first handle has under way
+for d in (device, others[0]):
+    assert waits(lambda: up(d, plain)) == waits(lambda: up(d, tiled)) == 1
+rt.close_mesh_device(others[0])
+assert waits(lambda: up(device, plain)) == waits(lambda: up(device, tiled)) == 0
+""")

@@ -245,6 +245,7 @@ namespace {
 struct DeviceRegistry {
   std::mutex mu;
   std::vector<std::weak_ptr<DeviceState>> devices;
+  std::atomic<int> open{0};   // open handles
 };
 DeviceRegistry &deviceRegistry() {
   static DeviceRegistry *r = new DeviceRegistry;
@@ -504,6 +505,13 @@ void syncStream(DeviceState &dev) {
   dev.stagingHead = 0;
 }
 
+// An upload is left pending only while this is the process's one open handle: its stream orders everything that may read the
+// tensor or reuse its memory.  Other handles have streams of their own and the pool is common to all, so beside them a tensor is
+// there when the call returns.
+void finishUpload(DeviceState &dev) {
+  if (deviceRegistry().open > 1) syncStream(dev);
+}
+
 // The bytes of a host tensor in the staging block, or null when they have to go another way.  Launches that read them must
 // be on the stream before the next wait.
 const void *stage(DeviceState &dev, const void *src, size_t bytes) {
@@ -560,6 +568,7 @@ void convertInOneLaunch(const void *src, TensorLayout sl, DataType sd, void *dst
 }  // namespace
 
 DeviceState::~DeviceState() {
+  if (counted) --deviceRegistry().open;
   if (open && stream) ttm_stream_destroy(stream);
   if (staging) hostPool().free(staging);
 }
@@ -588,9 +597,18 @@ Device openMeshDevice(const MeshDeviceOptions &options) {
     pool().free(there, 16);
     hostPool().free(probe);
   }
+  std::vector<std::shared_ptr<DeviceState>> others;
   {
     std::lock_guard<std::mutex> g(deviceRegistry().mu);
+    for (auto &w : deviceRegistry().devices)
+      if (auto o = w.lock()) others.push_back(o);
     deviceRegistry().devices.push_back(st);
+    ++deviceRegistry().open;
+    st->counted = true;
+  }
+  for (auto &o : others) {   // what they uploaded while they were alone
+    std::lock_guard<std::recursive_mutex> g(o->mu);
+    if (o->open && !o->capturing) syncStream(*o);
   }
   return Device{st};
 }
@@ -679,6 +697,8 @@ void closeMeshDevice(Device d) {
   TTM_CALL(ttm_stream_destroy(d.handle->stream));
   d.handle->stream = nullptr;
   d.handle->open = false;
+  d.handle->counted = false;
+  --deviceRegistry().open;
 }
 
 std::string getDeviceName(Device) {
@@ -846,6 +866,7 @@ Tensor toDevice(const Tensor &h, const std::shared_ptr<DeviceState> &dev) {
   if (const void *p = stage(*dev, s.data.get(), s.bytes)) {
     if (s.bytes <= kKernelCopyMax) TTM_CALL(ttm_copy_kernel(p, d.handle->data.get(), (s.bytes + 15) / 16 * 16, dev->stream));
     else TTM_CALL(ttm_memcpy_h2d(d.handle->data.get(), p, s.bytes, dev->stream));
+    finishUpload(*dev);
     return d;
   }
   TTM_CALL(ttm_memcpy_h2d(d.handle->data.get(), s.data.get(), s.bytes, dev->stream));
@@ -863,6 +884,7 @@ bool uploadInto(const Tensor &h, const Tensor &d) {
   const void *p = stage(dev, s.data.get(), s.bytes);
   if (!p) return false;
   convertInOneLaunch(p, s.layout, s.dtype, d.handle->data.get(), d.handle->layout, d.handle->dtype, s.shape, dev.stream);
+  finishUpload(dev);
   return true;
 }
 

@@ -54,6 +54,7 @@ struct DeviceState {
   int deviceId = 0;
   void *stream = nullptr;  // hipStream_t: all work of this device is ordered on it
   bool open = false;
+  bool counted = false;    // among the open handles of the registry
   // Page-locked block through which host tensors go up (runtime.cpp, stage()): filled from `stagingHead` on, free again from
   // the start after every wait for the stream.  `kernelsReachHost`: kernels may read and write page-locked memory.
   void *staging = nullptr;
