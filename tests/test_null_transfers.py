@@ -61,3 +61,30 @@ for d in (device, others[0]):
 rt.close_mesh_device(others[0])
 assert waits(lambda: up(device, plain)) == waits(lambda: up(device, tiled)) == 0
 """)
+
+
+def test_reading_a_tensor_of_a_busy_handle_does_not_wait_for_its_program(null_env):  # noqa: F811
+    """A thread that holds one handle's lock (to_layout on it) and reads a tensor of another, whose program waits for that thread."""
+    run(null_env, """
+import threading
+other = rt.open_mesh_device()
+x = torch.randn(64, 96)
+mine = rt.to_layout(rt.from_torch(x), device, rt.Layout(ST.Device, TL.Tile, DT.Float32), retain=True)
+got = []
+def reader():
+    got.append(rt.to_torch(rt.to_layout(mine, other, rt.Layout(ST.Host, TL.RowMajor, DT.Float32))))
+def hook(idx, name, dbg, h):
+    if not got and not threads:
+        threads.append(threading.Thread(target=reader, daemon=True))
+        threads[0].start()
+        threads[0].join(30)
+        finished.append(not threads[0].is_alive())
+        if not finished[0]:
+            os._exit(3)
+threads, finished = [], []
+rt.set_post_op_callback(hook)
+b = rt.Binary.load_from_memory(programs.c1_matmul())
+ins = [rt.to_layout(rt.from_torch(t), device, rt.get_layout(b, 0, i)) for i, t in enumerate(datagen.c1_matmul())]
+rt.submit(device, b, 0, ins)
+assert finished == [True] and torch.equal(got[0], x)
+""")

@@ -2209,7 +2209,9 @@ void runExecuteTrace(const fb::Table &op, ProgramContext &ctx) {
 // dst <- src for tensors of one shape; src is brought to dst's layout and dtype first (on the device)
 void overwriteTensor(ProgramContext &ctx, Tensor &dst, const Tensor &src, const char *what) {
   TTRT_ASSERT(dst.handle->shape == src.handle->shape, std::string(what) + ": shape mismatch");
-  if (src.handle->storage == StorageType::Host && dst.handle->storage == StorageType::Device && uploadInto(src, dst)) return;
+  // (a tensor of another handle is written on this program's stream, below, and without that handle's lock)
+  if (src.handle->storage == StorageType::Host && dst.handle->storage == StorageType::Device && dst.handle->device == ctx.dev &&
+      uploadInto(src, dst)) return;
   Tensor conv = src;
   if (conv.handle->layout != dst.handle->layout || conv.handle->dtype != dst.handle->dtype)
     conv = as(ctx, conv, dst.handle->layout, dst.handle->dtype);

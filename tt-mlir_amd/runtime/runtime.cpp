@@ -901,7 +901,13 @@ Tensor fetchAs(const Tensor &d, TensorLayout layout, DataType dtype) {
   TTRT_ASSERT(d.handle->device && d.handle->device->open, "the tensor belongs to a device that has been closed");
   requireNotCapturing(d.handle->device, "a device to host transfer");
   DeviceState &dev = *d.handle->device;
-  std::lock_guard<std::recursive_mutex> g(dev.mu);
+  // Callers that hold the lock of another handle read this one's tensors too, and two of them that waited for each other's lock would
+  // wait for ever.  Without it the staging block is not started over after the wait; nothing else here needs it.
+  const std::unique_lock<std::recursive_mutex> g(dev.mu, std::try_to_lock);
+  const auto finish = [&] {
+    if (g.owns_lock()) syncStream(dev);
+    else TTM_CALL(ttm_stream_sync(dev.stream));
+  };
   const TensorImpl &s = *d.handle;
   const size_t bytes = tensorBytes(s.shape, dtype, layout);
   const bool same = s.layout == layout && s.dtype == dtype;
@@ -912,7 +918,7 @@ Tensor fetchAs(const Tensor &d, TensorLayout layout, DataType dtype) {
     const Tensor c = same ? d : convertOnDevice(d, layout, dtype);
     Tensor h = makeHostTensor(s.shape, dtype, layout);
     TTM_CALL(ttm_memcpy_d2h(h.handle->data.get(), c.handle->data.get(), bytes, dev.stream));
-    syncStream(dev);
+    finish();
     return h;
   }
   auto t = std::make_shared<TensorImpl>();
@@ -928,10 +934,10 @@ Tensor fetchAs(const Tensor &d, TensorLayout layout, DataType dtype) {
     const Tensor c = convertOnDevice(d, layout, dtype);
     if (bytes <= kKernelCopyMax) TTM_CALL(ttm_copy_kernel(c.handle->data.get(), p, (bytes + 15) / 16 * 16, dev.stream));
     else TTM_CALL(ttm_memcpy_d2h(p, c.handle->data.get(), bytes, dev.stream));
-    syncStream(dev);
+    finish();
     return Tensor{t};
   }
-  syncStream(dev);
+  finish();
   return Tensor{t};
 }
 
