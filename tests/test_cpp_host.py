@@ -32,6 +32,12 @@ def test_host_pool_bookkeeping(tmp_path):
     assert r.returncode == 0, r.stdout
 
 
+def test_host_copy(tmp_path):
+    exe = compile_cpp(tmp_path, "test_host_copy")
+    r = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout
+
+
 def test_runtime_arm_sketch_compiles_and_runs(tmp_path):
     """The fourth arm of the reference's runtime dispatch: include/ttmlir_amd_runtime_arm.hpp over the C ABI, in its own namespace,
     linked against the exported ttrt_* symbols only."""

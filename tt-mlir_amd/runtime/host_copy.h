@@ -9,6 +9,7 @@
 #include <cstring>
 #include <memory>
 #include <mutex>
+#include <system_error>
 #include <thread>
 
 namespace tt::runtime {
@@ -48,7 +49,10 @@ private:
   HostCopy() {
     const unsigned cores = std::thread::hardware_concurrency();
     const int n = cores < 2 ? 0 : static_cast<int>(cores / 2 < kHelpers ? cores / 2 : kHelpers);
-    for (int i = 0; i < n; ++i) std::thread([this] { serve(); }).detach();
+    try {
+      for (int i = 0; i < n; ++i) std::thread([this] { serve(); }).detach();
+    } catch (const std::system_error &) {   // no more threads to be had: the caller copies with those there are, or alone
+    }
   }
   void serve() {
     std::uint64_t seen = 0;
