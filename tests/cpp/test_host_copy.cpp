@@ -1,4 +1,5 @@
-// Shared host copies: values at the edges of the chunks, several callers at once, a process that may start no thread.
+// Shared host copies: values at the edges of the chunks, several callers at once, a process that may start no thread, and a forked
+// child, which has none of its parent's helpers.
 // Build: g++ -std=c++17 -pthread -I tt-mlir_amd/runtime tests/cpp/test_host_copy.cpp -o <exe>; exit status 0 = all checks passed.
 #include <sys/resource.h>
 #include <sys/wait.h>
@@ -76,5 +77,11 @@ static int withoutThreads() {   // no room for another stack
 int main() {
   if (inChild(withoutThreads)) return 1;   // before this process has helpers
   if (sizes() || manyCallers()) return 1;
-  return 0;
+  for (int k = 0; k < 20; ++k)
+    if (inChild(sizes)) return 1;
+  std::thread busy([] { for (int k = 0; k < 200; ++k) (void)copies(size_t(4) << 20, k); });
+  int bad = 0;
+  for (int k = 0; k < 20 && !bad; ++k) bad = inChild(sizes);   // forked while another thread shares its copies out
+  busy.join();
+  return bad;
 }

@@ -2,6 +2,8 @@
 // into fresh pages at 30 GB/s, which is less than PCIe delivers ([2048, 4096] bf16, 16 MiB: 0.55 ms of the 1.4 ms a read-back
 // took), mostly in page faults and cache misses that further cores take beside it.
 #pragma once
+#include <unistd.h>
+
 #include <atomic>
 #include <condition_variable>
 #include <cstddef>
@@ -21,14 +23,16 @@ public:
   static constexpr int kHelpers = 5;
 
   // Returns when all bytes are there.  The caller takes chunks as the helpers do, so it never waits for a thread that has not
-  // been scheduled (or, after a fork, does not exist): only for chunks that were begun.
+  // been scheduled: only for chunks that were begun.  A forked child has neither the helpers nor a lock and a condition variable it
+  // could rely on, and copies alone.
   static void run(void *dst, const void *src, size_t bytes) {
     if (bytes < kShareFrom) {
       std::memcpy(dst, src, bytes);
       return;
     }
     static HostCopy *crew = new HostCopy;   // never destroyed: its threads wait until the process ends
-    crew->share(dst, src, bytes);
+    if (crew->owner != getpid()) std::memcpy(dst, src, bytes);
+    else crew->share(dst, src, bytes);
   }
 
 private:
@@ -85,6 +89,7 @@ private:
     if (job == j) job.reset();
   }
 
+  const pid_t owner = getpid();
   std::mutex mu;
   std::condition_variable cv;
   std::shared_ptr<Job> job;
