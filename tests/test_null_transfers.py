@@ -88,3 +88,33 @@ ins = [rt.to_layout(rt.from_torch(t), device, rt.get_layout(b, 0, i)) for i, t i
 rt.submit(device, b, 0, ins)
 assert finished == [True] and torch.equal(got[0], x)
 """)
+
+
+def test_a_callback_after_the_program_sees_every_result_as_declared(null_env):  # noqa: F811
+    """Layout changes that are made on the way over PCIe leave their operand in the result's place: not where a callback may read the
+    result (wrong layout and type) or write it (into the caller's input)."""
+    run(null_env, """
+pb = rt.ProgramBuilder()
+pb.begin_program("p")
+a = pb.input((64, 96), DT.Float32, TL.RowMajor, ST.Host)
+up = pb.to_device(a)
+t = pb.to_layout(up, TL.Tile)
+s = pb.unary(programs.UNARY["neg"], t)
+down = pb.to_layout(s, TL.RowMajor, DT.BFloat16)
+out = pb.from_device(down)
+pb.output(out)
+pb.end_program()
+b = rt.Binary.load_from_memory(pb.finish())
+x = torch.randn(64, 96)
+host = rt.from_torch(x)
+seen = {}
+def post(idx, hook):
+    seen["down"] = hook.retrieve(down, untilize=False).desc()[1]
+    seen["up"] = rt.to_torch(hook.retrieve(up))
+    hook.update(up, rt.from_torch(torch.zeros(64, 96)))
+rt.set_program_callbacks(post=post)
+(y,) = rt.submit(device, b, 0, [host])
+assert (seen["down"].layout, seen["down"].dtype) == (TL.RowMajor, DT.BFloat16)
+assert torch.equal(seen["up"], x) and torch.equal(rt.to_torch(host), x)
+assert torch.equal(rt.to_torch(y), -x.to(torch.bfloat16))
+""")

@@ -338,10 +338,11 @@ std::string matmulActivation(const fb::Table &op, int configTypeSlot, int config
 }
 
 std::uint32_t refId(const fb::Table &ref);
-// The result `ref` of the operation at hand is read by the next operation of the program, of this type, and by nothing else.
+// The result `ref` of the operation at hand is read by the next operation of the program, of this type, and by nothing else: no
+// callback after the program either, which may look at, or write, any tensor that is still in the pool.
 bool onlyFeedsNext(ProgramContext &ctx, const fb::Table &ref, OpType type, int operandSlot) {
   const std::uint32_t next = ctx.opIndex + 1;
-  if (!ctx.fuseViews || next >= ctx.ops.size()) return false;
+  if (!ctx.fuseViews || next >= ctx.ops.size() || debug::Hooks::get().postProgramCallback) return false;
   if (static_cast<OpType>(ctx.ops[next].scalar<std::uint8_t>(schema::Operation::f_type_type, 0)) != type) return false;
   const auto use = ctx.uses.find(refId(ref));
   return use != ctx.uses.end() && use->second == 1 && refId(ctx.ops[next].table(schema::Operation::f_type).table(operandSlot)) == refId(ref);
