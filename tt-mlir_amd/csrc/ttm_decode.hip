@@ -889,10 +889,12 @@ static int sdpa_decode_entry(const void *q, const void *k, const void *v, const 
   // (D = 128, 8 kv heads of 4 query heads, contexts of a quarter of the cache to all of it; direct / shares, us): 1 user x 512 positions
   // 7.4 / 9.9, 1 x 1024 10.7 / 10.2, 1 x 2048 12.1 / 10.4, 1 x 4096 30.2 / 11.5, 8 x 1024 14.8 / 15.2, 8 x 2048 24.3 / 18.8, 16 x 2048
   // 26.4 / 26.0, 16 x 4096 43.8 / 35.9, 32 x 1024 19.7 / 26.2, 32 x 2048 32.9 / 37.2; D = 64: 5 x 2048 12.2 / 13.6, 5 x 4096 21.6 / 15.6,
-  // 16 x 2048 15.4 / 18.1, 16 x 4096 26.5 / 25.5.
+  // 16 x 2048 15.4 / 18.1, 16 x 4096 26.5 / 25.5.  A tile of 32 columns takes about as long as one of 64, so narrower heads count as 64:
+  // D = 32, 16 kv heads of 5 query heads: 1 x 4096 15.3 / 11.0, 2 x 2048 12.0 / 13.7, 2 x 4096 18.0 / 14.1, 8 x 4096 25.4 / 24.1 (under a
+  // window they see few tiles: 4 x 2080, 8 kv heads of 12, window 100 9.6 / 20.9).
   const int form = ttm_option("sdpa_decode_form");   // 0 by this rule, 1 direct, 2 shares
   // (the results of the wavefronts fit in 32 KiB of LDS)
-  bool direct = G * head_dim <= 1024 && (form ? form == 1 : seq * head_dim <= 2048 * std::max<int64_t>(64, batch * kv_heads));
+  bool direct = G * head_dim <= 1024 && (form ? form == 1 : seq * (window < 0 ? std::max<int64_t>(64, head_dim) : head_dim) <= 2048 * std::max<int64_t>(64, batch * kv_heads));
   const int64_t all = batch * (seq / 32);          // tiles of a kv head when every cache is full
   int64_t shares = ttm_cdiv(kDecodeBlocks, kv_heads);
   if (shares > all / 4) shares = all / 4 > 0 ? all / 4 : 1;   // a tile for every wavefront
