@@ -1956,10 +1956,13 @@ static double other_us(const LinearArgs &a, bool measured = false) {
   return BFP ? std::min(us, two) : two;
 }
 // Whether the mid-size kernel's plan beats it.  Its own model is 3 % low for block-float and 5 % high for bf16 weights (10 % at
-// these sizes, less where K is long: 14336 x 4096 bf16 at 700 rows 140 / 148).  Over 177 shapes
-// of 400 .. 1600 rows around the line the choice costs 0.7 % against always knowing the faster one (7 % without the kernel); at
-// 4096 x 6144 bf16, image route / mid-size kernel: 520 rows 60.5 / 48.3 us, 661 rows 61.7 / 71.3; 5120 x 2880 bfp8_b, 400 rows 38.6 /
-// 28.1, 661 rows 52.3 / 49.6, 930 rows 56.0 / 54.1, 1600 rows 71.5 / 85.8.
+// these sizes, less where K is long: 14336 x 4096 bf16 at 700 rows 140 / 148).  4096 x 6144 bf16, image route / mid-size kernel: 520
+// rows 60.5 / 48.3 us, 661 rows 61.7 / 71.3; 5120 x 2880 bfp8_b, 400 rows 38.6 / 28.1, 661 rows 52.3 / 49.6, 930 rows 56.0 / 54.1, 1600
+// rows 71.5 / 85.8.  Of 2900 random shapes (33 .. 2048 rows, weights of 512 .. 8192 x 512 .. 14336, all formats) it is taken at 2116, on
+// average in 0.62 of the other's time, and is the slower one at 46 of them: by 5 % at the median, at worst 28.5 / 23.1 us at 897
+// rows x 518 x 8653 bf16 and 79.9 / 68.0 at 1514 rows x 3072 x 5024 bfp4_b, two in five of them with K below 850.  The models scatter by
+// 4 .. 10 %: lines that leave out more of the 46 (refitted models, an extra charge for short K) take away as much elsewhere, up
+// to 30 % a shape.
 template <int WF>
 static bool mid_beats_other(const LinearArgs &a, const MidPlan &plan) {
   constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
