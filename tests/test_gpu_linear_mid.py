@@ -124,3 +124,25 @@ def test_a_split_product_is_recorded_on_a_stream_without_workspace(hip, dev, orc
         assert torch.allclose(got.float(), e.float(), atol=2.0 ** -5)
     hip.call("ttm_graph_destroy", graph)
     hip.call("ttm_stream_destroy", stream)
+
+
+@pytest.mark.parametrize("wfmt_name", ["bfp8", "bfp4"])
+@pytest.mark.parametrize("M", [33, 64])
+def test_infinite_activations_up_to_64_rows(hip, dev, wfmt_name, M):
+    """The two-term operand leaves inf - inf in every column of such a row, here as in the decode kernel (which these sizes went to
+    before); other rows are those of a call without it."""
+    a = datagen.randn((M, 512), seed=3, dtype=torch.bfloat16)
+    w, wfmt = datagen.randn((512, 96), seed=4, std=0.1), {"bfp8": hip.BFP8B, "bfp4": hip.BFP4B}[wfmt_name]
+    clean, _ = run_linear(hip, dev, a, w, None, None, wfmt)
+    a[5, 40], a[M - 1, 511] = float("inf"), float("-inf")
+    hit = torch.zeros(M, dtype=torch.bool)
+    hit[[5, M - 1]] = True
+    for option in (0, 8101, 1):
+        hip.set_option("linear_mid", option)
+        try:
+            got, _ = run_linear(hip, dev, a, w, None, None, wfmt)
+        finally:
+            hip.set_option("linear_mid", 0)
+        assert torch.isnan(got[hit]).all() and torch.isfinite(got[~hit]).all()
+        if option == 0:
+            assert torch.equal(got[~hit], clean[~hit])

@@ -47,3 +47,16 @@ def test_host_tensors_of_earlier_read_backs_keep_their_values(device):
     for x, h in zip([xs[0], xs[2], xs[3], xs[4]], held):
         assert torch.equal(rt.to_torch(h), x)
     assert np.array_equal(rt.to_numpy(held[0]), xs[0].view(torch.int16).numpy().view(np.uint16))
+
+
+def test_the_routes_through_page_locked_memory_are_the_ones_that_run(device):
+    """What the tests above compare would be the same bytes if the device were found not to reach page-locked memory."""
+    x = datagen.randn((512, 1024), seed=1)
+    lay = rt.Layout(ST.Device, TL.Tile, DT.Float32)
+    rt.to_host(rt.to_layout(rt.from_torch(x), device, lay), untilize=True)    # a read-back waits: the staging block is empty
+    rt.clear_stats()
+    ds = [rt.to_layout(rt.from_torch(x), device, lay) for _ in range(5)]      # 5 x 2 MiB through 8 MiB
+    assert rt.get_stat("StagingBlockReused") == 1
+    for d in ds:
+        assert torch.equal(rt.to_torch(d), x)
+    assert rt.get_stat("HostPoolReadBack") == 5

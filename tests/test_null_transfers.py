@@ -118,3 +118,12 @@ assert (seen["down"].layout, seen["down"].dtype) == (TL.RowMajor, DT.BFloat16)
 assert torch.equal(seen["up"], x) and torch.equal(rt.to_torch(host), x)
 assert torch.equal(rt.to_torch(y), -x.to(torch.bfloat16))
 """)
+
+
+@pytest.mark.parametrize("pageable", ["0", "1"])
+def test_transfers_on_both_routes(null_env, pageable):  # noqa: F811
+    """The GPU's transfer tests, with page-locked memory within the kernels' reach and without (the memcpy routes)."""
+    skip = "not through_page_locked" if pageable == "1" else ""
+    r = subprocess.run([sys.executable, "-m", "pytest", os.path.join(ROOT, "tests", "test_gpu_transfers.py"), "-q", "-m", "gpu", "-p", "no:cacheprovider",
+                        "-k", skip], env=dict(null_env, TTMLIR_AMD_NULL_DEVICE_PAGEABLE=pageable), capture_output=True, text=True, timeout=600, cwd=ROOT)
+    assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-1000:]

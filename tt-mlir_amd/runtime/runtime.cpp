@@ -921,6 +921,7 @@ Tensor fetchAs(const Tensor &d, TensorLayout layout, DataType dtype) {
     finish();
     return h;
   }
+  debug::Stats::get().incrementStat("HostPoolReadBack");
   auto t = std::make_shared<TensorImpl>();
   t->shape = s.shape; t->dtype = dtype; t->layout = layout; t->storage = StorageType::Host;
   t->bytes = bytes;
