@@ -28,15 +28,6 @@ def test_other_kinds_of_tensors_keep_their_values():
         assert torch.equal(rt.to_torch(rt.from_torch(t)), torch.Tensor(t))
 
 
-def test_a_functionalized_tensor_keeps_its_values():
-    """Its own memory is not where they are."""
-    x = torch.arange(6.0).reshape(2, 3)
-    assert torch.equal(rt.to_torch(rt.from_torch(torch._to_functional_tensor(x))), x)
-    seen = []
-    torch.func.functionalize(lambda t: (seen.append(rt.to_torch(rt.from_torch(t))), t + 1)[1])(x)
-    assert torch.equal(seen[0], x)
-
-
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.int32, torch.uint8])
 def test_results_come_back_to_host_memory_whatever_the_default_device(dtype):
     x = torch.arange(2000).reshape(50, 40).to(dtype)

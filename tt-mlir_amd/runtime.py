@@ -348,9 +348,8 @@ def from_torch(t, borrowed=False):
     dt, itemsize = _torch_maps()[0][t.dtype]
     a = t.contiguous()
     # data_ptr() points at the values only of plain tensors in host memory: subclasses (a FakeTensor has no memory), negative views
-    # (the sign lives in a bit of the tensor), ZeroTensors and functionalized tensors (the values are another tensor's) go through
-    # numpy(), which converts them or refuses them
-    if type(a) not in (torch.Tensor, torch.nn.Parameter) or a.device.type != "cpu" or a.requires_grad or a.is_neg() or a._is_zerotensor() or torch._is_functional_tensor(a) or a.numel() == 0:
+    # (the sign lives in a bit of the tensor) and ZeroTensors go through numpy(), which converts them or refuses them
+    if type(a) not in (torch.Tensor, torch.nn.Parameter) or a.device.type != "cpu" or a.requires_grad or a.is_neg() or a._is_zerotensor() or a.numel() == 0:
         return _host(a.view(torch.int16).numpy().view(np.uint16) if dt == DataType.BFloat16 else a.numpy(), dt, borrowed)
     shape, rank = _shape_arg(a.shape or (1,))
     h = ctypes.c_void_p()
