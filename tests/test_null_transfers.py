@@ -120,6 +120,23 @@ assert torch.equal(rt.to_torch(y), -x.to(torch.bfloat16))
 """)
 
 
+def test_a_round_trip_through_the_device_is_a_copy(null_env):  # noqa: F811
+    """to_device, then a to_layout back to the host that changes nothing: the result is not the caller's tensor."""
+    run(null_env, """
+pb = rt.ProgramBuilder()
+pb.begin_program("p")
+a = pb.input((64, 96), DT.Float32, TL.RowMajor, ST.Host)
+pb.output(pb.to_layout(pb.to_device(a), TL.RowMajor, DT.Float32, ST.Host))
+pb.end_program()
+x = torch.randn(64, 96)
+host = rt.from_torch(x)
+(y,) = rt.submit(device, rt.Binary.load_from_memory(pb.finish()), 0, [host])
+assert rt.host_data_ptr(y) != rt.host_data_ptr(host)
+rt.memcpy_tensor(host, rt.from_torch(torch.zeros(64, 96)))
+assert torch.equal(rt.to_torch(y), x)
+""")
+
+
 @pytest.mark.parametrize("pageable", ["0", "1"])
 def test_transfers_on_both_routes(null_env, pageable):  # noqa: F811
     """The GPU's transfer tests, with page-locked memory within the kernels' reach and without (the memcpy routes)."""

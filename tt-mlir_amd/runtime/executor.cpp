@@ -378,7 +378,10 @@ void runTypecast(const fb::Table &op, ProgramContext &ctx) {
 void runToDevice(const fb::Table &op, ProgramContext &ctx) {
   Tensor in = ctx.get(op.table(schema::ToDeviceOp::f_in), "to_device in");
   auto outRef = op.table(schema::ToDeviceOp::f_out);
-  ctx.put(outRef, onlyFeedsNext(ctx, outRef, OpType::ToLayoutOp, schema::ToLayoutOp::f_in) ? in : onDevice(ctx, in));
+  // (a to_layout that ends on the host may have nothing to change: its result would be the operand itself, not a copy)
+  const bool leave = onlyFeedsNext(ctx, outRef, OpType::ToLayoutOp, schema::ToLayoutOp::f_in) &&
+                     layoutFromTensorRef(ctx.ops[ctx.opIndex + 1].table(schema::Operation::f_type).table(schema::ToLayoutOp::f_out)).storageType == StorageType::Device;
+  ctx.put(outRef, leave ? in : onDevice(ctx, in));
 }
 void runFromDevice(const fb::Table &op, ProgramContext &ctx) {
   Tensor in = ctx.get(op.table(schema::FromDeviceOp::f_in), "from_device in");
