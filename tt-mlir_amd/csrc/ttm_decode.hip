@@ -249,12 +249,12 @@ __global__ __launch_bounds__(256) void ttm_rotary_llama_k(const uint16_t *__rest
 // The next tile's K is requested when the scores are made, its V behind the products, so a wavefront has 16 KiB (D = 128) on the
 // way at any time and no wavefront waits for another before the end, where the partial results meet in LDS.
 //
-// Two forms.  Direct: grid (Hkv, B), eight wavefronts, the whole context of a user and the output in one launch.  Shares: the
-// visible tiles of all users of a kv head form one line (user after user), workgroup j of grid (shares, Hkv) streams its j-th equal
-// part whatever the users' context lengths are; (max, sum, unnormalised output) of a piece go to slot j + user of the kv head
-// (along the line either j or the user advances from one piece to the next, so the sum numbers the pieces) and
-// ttm_sdpa_decode_combine_k merges a user's slots (merging in the last workgroup to arrive was measured: the device-scope
-// fences it needs double the kernel time).
+// Two forms.  Direct: grid (Hkv, B), 16 wavefronts for up to four heads of 32, 64 or 128 columns, else eight; the whole context of a
+// user and the output in one launch.  Shares, four wavefronts: the visible tiles of all users of a kv head form one line (user after
+// user), workgroup j of grid (shares, Hkv) streams its j-th equal part whatever the users' context lengths are; (max, sum,
+// unnormalised output) of a piece go to slot j + user of the kv head (along the line either j or the user advances from one piece
+// to the next, so the sum numbers the pieces) and ttm_sdpa_decode_combine_k merges a user's slots (merging in the last workgroup to
+// arrive was measured: the device-scope fences it needs double the kernel time).
 struct DecodeArgs {
   const uint16_t *q, *k, *v, *mask;
   const int32_t *cur_pos, *page_table;
@@ -271,9 +271,9 @@ struct DecodeArgs {
 };
 
 constexpr int kMaxG = 8;
-// K and V are read once per launch: streaming (nontemporal) loads keep them from displacing each other in the caches on
-// the way.  STREAM = false when several launches share one cache (more than kMaxG query heads per kv head), where the later
-// launches profit from what the first one left.
+// K is read by streaming (nontemporal) loads: each line once per launch, by one instruction.  STREAM = false when several launches
+// share one cache (more than kMaxG query heads per kv head), where the later launches profit from what the first one left.  V's
+// loads are plain ones: a lane takes a dword of every row, so a line is fetched by four instructions and has to stay until the last.
 template <bool STREAM, typename T>
 __device__ __forceinline__ T kv_load(const T *p) {
   if constexpr (STREAM) return __builtin_nontemporal_load(p);

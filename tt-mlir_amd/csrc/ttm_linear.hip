@@ -18,9 +18,11 @@
 // and pairs along k are packed to bf16 by taking the high halves (exact: 7 significant bits).
 // Rows whose shared exponent is below 7 (|w| < 2^-120) are flushed to zero.
 //
-// Kernels, by use: ttm_linear_dma_k (block-float weights, M > 64), ttm_linear_reg_k (bf16 weights, M > 64),
-// ttm_linear_big_k (64-bit-addressed fallback), ttm_linear_decode_k / ttm_linear_small_k (M <= 64),
-// ttm_linear_reduce_k (second half of a split-K launch).
+// Kernels, by use: ttm_linear_decode_k (block-float weights, one row tile), ttm_linear_small_k (bf16 weights, one row tile, where the
+// weights are large), ttm_linear_mid_k (ttm_linear_mid.hip: from 33 rows to what fills the device, and small products),
+// ttm_linear_image_k + ttm_linear_img_k (beyond: weights as bf16 images first), ttm_linear_dma_k (beyond, block-float weights without
+// images), ttm_linear_dma_glu_k (the gated pair), ttm_linear_reg_k (bf16 weights whose images would not fit), ttm_linear_big_k
+// (64-bit-addressed fallback), ttm_linear_reduce_k (second half of a split-K launch).
 #include "ttm_linear.h"
 
 // ---- bfp8: 8 rows (k) x 8 bytes (n) + 8 exponents -> 8 chunks (one per n) of 8 k
