@@ -329,7 +329,8 @@ _torch_types = None
 
 
 def _torch_maps():
-    """({torch dtype: (DataType, element size)}, {DataType: (torch dtype, numpy dtype that holds its bits)}), built once."""
+    """({torch dtype: (DataType, element size)}, {DataType: (torch dtype, numpy dtype that holds its bits)}, the classes of plain
+    tensors), built once."""
     global _torch_types
     if _torch_types is None:
         import torch
@@ -338,18 +339,19 @@ def _torch_maps():
                  torch.int16: DataType.Int16, torch.int8: DataType.Int8, torch.bool: DataType.Bool}
         back = {DataType.Float32: (torch.float32, np.float32), DataType.BFloat16: (torch.bfloat16, np.int16),
                 DataType.Float16: (torch.float16, np.float16), DataType.Int32: (torch.int32, np.int32), DataType.UInt8: (torch.uint8, np.uint8)}
-        _torch_types = {k: (v, torch.empty(0, dtype=k).element_size()) for k, v in to_rt.items()}, back
+        _torch_types = {k: (v, torch.empty(0, dtype=k).element_size()) for k, v in to_rt.items()}, back, (torch.Tensor, torch.nn.Parameter)
     return _torch_types
 
 
 def from_torch(t, borrowed=False):
     """Host tensor from a CPU torch tensor (bf16 / f32 / f16 / ints)."""
-    import torch
-    dt, itemsize = _torch_maps()[0][t.dtype]
+    types, _, plain = _torch_maps()
+    dt, itemsize = types[t.dtype]
     a = t.contiguous()
     # data_ptr() points at the values only of plain tensors in host memory: subclasses (a FakeTensor has no memory), negative views
     # (the sign lives in a bit of the tensor) and ZeroTensors go through numpy(), which converts them or refuses them
-    if type(a) not in (torch.Tensor, torch.nn.Parameter) or a.device.type != "cpu" or a.requires_grad or a.is_neg() or a._is_zerotensor() or a.numel() == 0:
+    if type(a) not in plain or not a.is_cpu or a.requires_grad or a.is_neg() or a._is_zerotensor() or a.numel() == 0:
+        import torch
         return _host(a.view(torch.int16).numpy().view(np.uint16) if dt == DataType.BFloat16 else a.numpy(), dt, borrowed)
     shape, rank = _shape_arg(a.shape or (1,))
     h = ctypes.c_void_p()
@@ -470,8 +472,9 @@ def to_torch(tensor):
         a = to_numpy(host)
         return torch.from_numpy(a.view(np.int16)).view(torch.bfloat16) if lay.dtype == DataType.BFloat16 else torch.from_numpy(a)
     # the result in numpy's memory, not torch.empty's: a default device or an active FakeTensorMode would put that elsewhere
+    # (its address by way of the buffer protocol: .ctypes builds an object for 1 us)
     out = np.empty(shape, dtype=np_dtype)
-    memcpy(out, host)
+    _call("ttrt_memcpy_out", ctypes.byref(ctypes.c_char.from_buffer(out)), host.h, -1)
     out = torch.from_numpy(out)
     return out if out.dtype == dt else out.view(dt)
 
