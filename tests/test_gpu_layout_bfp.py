@@ -72,6 +72,46 @@ def test_tilize_ragged_zero_padded(hip, dev, orc, shape, dtype):
     assert np.all(got[n:] == np.asarray(7, dtype=back.cpu().numpy().dtype).view(dtype))
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.uint16, np.uint8])
+@pytest.mark.parametrize("shape,offset", [((70, 1002), 1), ((3, 33, 129), 3), ((5, 3, 8), 1), ((40, 4, 17), 5), ((1, 1), 1), ((2, 65, 515), 7)])
+def test_tilize_untilize_at_any_element(hip, dev, orc, shape, dtype, offset):
+    """The row-major side starts at any element of its buffer and nothing in front of it or behind it is written; rows narrower
+    than a wavefront's access, matrices shorter than a workgroup's."""
+    rng = np.random.default_rng(2)
+    x = rng.standard_normal(shape).astype(np.float32) if dtype == np.float32 else rng.integers(1, 250, shape).astype(dtype)
+    n = x.size
+    b, r, c = orc._split3(shape)
+    buf = torch.full((n + 64,), 7, dtype=NP2T[np.dtype(dtype)], device=dev)
+    rm = buf[offset:offset + n]
+    rm.copy_(to_dev(x, dev).reshape(-1))
+    t = torch.full((b * (-(-r // 32) * 32) * (-(-c // 32) * 32),), 0x55, dtype=buf.dtype, device=dev)
+    hip.call("ttm_tilize", hip.ptr(rm), hip.ptr(t), b, r, c, x.dtype.itemsize, hip.current_stream())
+    assert np.array_equal(t.cpu().numpy().view(dtype), orc.tilize(x).view(dtype).reshape(-1))
+    rm.fill_(9)
+    hip.call("ttm_untilize", hip.ptr(t), hip.ptr(rm), b, r, c, x.dtype.itemsize, hip.current_stream())
+    got = buf.cpu().numpy().view(dtype)
+    seven = np.full(1, 7, dtype=buf.cpu().numpy().dtype).view(dtype)[0]
+    assert np.array_equal(got[offset:offset + n].reshape(shape), x)
+    assert np.all(got[:offset] == seven) and np.all(got[offset + n:] == seven)
+
+
+@pytest.mark.parametrize("rows,cols", [(41000, 2051), (41024, 2048)])
+def test_large_tensors_take_strips(hip, dev, rows, cols):
+    """Above the size up to which every shape goes chunk by chunk: whole strips and rows that start anywhere, against torch."""
+    g = torch.Generator(device=dev).manual_seed(3)
+    x = torch.randint(-2**15, 2**15 - 1, (rows, cols), dtype=torch.int16, device=dev, generator=g)
+    pr, pc = -(-rows // 32) * 32, -(-cols // 32) * 32
+    assert pr * pc * 2 > 160 << 20
+    padded = torch.nn.functional.pad(x, (0, pc - cols, 0, pr - rows))
+    want = padded.reshape(pr // 32, 2, 16, pc // 32, 2, 16).permute(0, 3, 1, 4, 2, 5).contiguous().reshape(-1)
+    t = torch.full((pr * pc,), 0x55, dtype=torch.int16, device=dev)
+    hip.call("ttm_tilize", hip.ptr(x), hip.ptr(t), 1, rows, cols, 2, hip.current_stream())
+    assert torch.equal(t, want)
+    back = torch.full((rows * cols + 64,), 7, dtype=torch.int16, device=dev)
+    hip.call("ttm_untilize", hip.ptr(want), hip.ptr(back), 1, rows, cols, 2, hip.current_stream())
+    assert torch.equal(back[:rows * cols].reshape(rows, cols), x) and bool((back[rows * cols:] == 7).all())
+
+
 def test_c1_operands_layout(hip, dev, orc):
     a, b = datagen.c1_matmul()
     for m in (a, b):

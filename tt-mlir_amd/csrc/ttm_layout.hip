@@ -1,13 +1,13 @@
 // Tilize / untilize for Tenstorrent's 32x32 tile layout with 16x16 faces, plus the plain copy
 // kernel used as the measured HBM ceiling.  All kernels move 16 bytes per lane per access.
 //
-// Two formulations of each direction, selected with ttm_set_option("tilize_variant"/"untilize_variant"):
-//   0  LDS-staged: a workgroup owns a strip of 32 rows x 512 bytes (16/elem tiles).  Global reads
-//      and writes are both fully contiguous (512 B per row segment on the row-major side, 16 KiB
-//      on the tiled side); the face permutation happens between a padded LDS image and registers.
-//   1  direct: one lane per 16-byte chunk of the tiled side, the row-major side is touched in
-//      face-row segments (16 elements).  No LDS; used when a strip does not divide the row.
-// Shapes that are not multiples of 32, and rows that start anywhere, have kernels of their own below (zero padding).
+// Formulations of each direction (the rule with its measurements stands at run_layout):
+//   direct: one lane per 16-byte chunk of the tiled side, whose row-major half may start at any element (the part takes 16-byte
+//           accesses at any address).  No LDS, no barrier; every shape.
+//   strips: a workgroup owns a strip of 32 rows x 512 bytes (16/elem tiles).  Global reads and writes are both contiguous (512 B
+//           per row segment on the row-major side, 16 KiB on the tiled side); the face permutation happens between a padded LDS
+//           image and registers.  Tensors that pass through the last-level cache.
+// ttm_set_option("tilize_variant" / "untilize_variant"): 0 by the rule, 1 direct.
 #include "ttm_common.h"
 #include "ttm_ragged.h"
 
@@ -47,38 +47,76 @@ TTM_EXPORT int ttm_copy_kernel(const void *src, void *dst, size_t bytes, void *s
 }
 
 // ------------------------------------------------------------------------------------ direct
-// ELEM = element bytes.  A face row (16 elements) is ELEM chunks; a tile is 64*ELEM chunks.
-template <int ELEM, bool TILIZE>
-__global__ __launch_bounds__(256) void ttm_tile_direct_k(const chunk_t *__restrict__ src,
-                                                         chunk_t *__restrict__ dst, int64_t yt, int64_t xt,
-                                                         int64_t total_chunks) {
-  constexpr int CPT = 64 * ELEM;  // chunks per tile
-  const int64_t row_chunks = xt * 2 * ELEM;  // chunks per row-major row
-  int64_t base = (int64_t)blockIdx.x * (256 * 4) + threadIdx.x;
-  chunk_t v[4];
-  int64_t rm[4];
+// A wavefront's access covers 8 / ELEM rows x 8 ELEM chunks (more rows of narrower tensors): 8 / ELEM face rows of 16 ELEM bytes are one 128-byte line of the tiled
+// side, and a row's W chunks are 128 ELEM contiguous bytes of the row-major side, which starts and ends at any element: 16-byte
+// accesses at their own alignment (a lane whose chunk crosses the end of a row takes elements), so nothing outside the tensor is read
+// and nothing is shifted or exchanged.  U accesses per lane.  What bounds it is bytes in flight against the number of
+// workgroups: two loads per lane are best for tilize up to some 16 MiB, one beyond and for untilize (a store needs no more).
+// Tilize streams its stores past the caches, untilize does not (partial lines at the ends of rows meet in L2).  Against strips of 32
+// rows x 512 bytes through LDS with funnel shifts for odd rows: [3, 1000, 3001] bf16 tilize / untilize 9.0 / 10.6 -> 7.0 / 6.9 us,
+// [4000, 7001] fp32 42.0 / 37.2 -> 39.4 / 35.6, [2, 1266, 771] bf16 4.2 / 5.5 -> 3.1 / 3.2, [7, 33, 9000] fp32 7.7 / 6.2 -> 4.4 / 4.4,
+// [65536, 64] bf16 5.3 / 6.2 -> 3.1 / 3.6, [70000, 3, 100] bf16 590 / 528 -> 89 / 20.
+typedef chunk_t chunk_any __attribute__((aligned(1)));   // at any address
+template <int ELEM>
+using layout_elem = typename std::conditional<ELEM == 4, uint32_t, typename std::conditional<ELEM == 2, uint16_t, uint8_t>::type>::type;
+
+template <int ELEM, int U, bool TILIZE>
+__global__ __launch_bounds__(256) void ttm_tile_direct_k(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int rows, int cols, int lw, int wc,
+                                                         uint32_t xu, uint32_t matrices) {
+  typedef layout_elem<ELEM> T;
+  constexpr int V = 16 / ELEM;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ct = (cols + 31) >> 5, yt = (rows + 31) >> 5;
+  // a wavefront's accesses are 1 << lw chunks wide, a workgroup 1 << wc wavefronts; its other wavefronts lie below
+  const uint32_t by = blockIdx.x / xu;
+  const int chunk = (int)((((blockIdx.x - by * xu) << wc) + (wave & ((1 << wc) - 1))) << lw) + (lane & ((1 << lw) - 1));
+  const uint32_t row0 = ((by << (2 - wc)) + (wave >> wc)) * (64 >> lw) * U + (lane >> lw);   // of the rows of all matrices, padded ones for tilize
+  const uint32_t per = TILIZE ? yt * 32 : rows;
+  const int n = cols - chunk * V;                          // elements of the row from this chunk on
+  if (TILIZE ? chunk >= ct * 2 * ELEM : n <= 0) return;
+  const int tc = chunk / (2 * ELEM), in = (chunk / ELEM & 1) * (16 * ELEM) + chunk % ELEM;   // tile column, face column and chunk of a face row
+  chunk_t v[U];
+  int64_t tiled[U], rm[U];   // chunk of the tiled side, element of the other; rm < 0: padding
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    int64_t o = base + u * 256;  // chunk index on the tiled side
-    if (o < total_chunks) {
-      int64_t tile = o / CPT;
-      int w = (int)(o % CPT);
-      int face = w / (16 * ELEM), dy = (w / ELEM) % 16, q = w % ELEM;
-      int64_t tx = tile % xt, tyb = tile / xt;  // tyb = batch * yt + ty (rows are multiples of 32)
-      int64_t r = tyb * 32 + (face >> 1) * 16 + dy;
-      rm[u] = r * row_chunks + tx * 2 * ELEM + (face & 1) * ELEM + q;
-      v[u] = TILIZE ? __builtin_nontemporal_load(&src[rm[u]]) : __builtin_nontemporal_load(&src[o]);
+  for (int u = 0; u < U; ++u) {
+    const uint32_t g = row0 + u * (64 >> lw), b = matrices > 1 ? g / per : 0, r = g - b * per;
+    tiled[u] = g < per * (uint64_t)matrices ? (((int64_t)b * yt + (r >> 5)) * ct + tc) * (64 * ELEM) + (r >> 4 & 1) * (32 * ELEM) + (r & 15) * ELEM + in : -1;
+    rm[u] = (int)r < rows ? ((int64_t)b * rows + r) * cols + chunk * V : -1;
+    if (TILIZE) {
+      v[u] = chunk_t{0, 0, 0, 0};
+      if (tiled[u] >= 0 && rm[u] >= 0 && n >= V) v[u] = *(const chunk_any *)((const T *)src + rm[u]);
+    } else if (tiled[u] >= 0) {
+      v[u] = ((const chunk_t *)src)[tiled[u]];
+    }
+  }
+  if (TILIZE && n > 0 && n < V) {   // the end of a row
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (tiled[u] < 0 || rm[u] < 0) continue;
+      T e[V];
+#pragma unroll
+      for (int j = 0; j < V; ++j) e[j] = j < n ? ((const T *)src)[rm[u] + j] : T(0);
+      v[u] = *(const chunk_t *)e;
     }
   }
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    int64_t o = base + u * 256;
-    if (o < total_chunks) {
-      if (TILIZE) __builtin_nontemporal_store(v[u], &dst[o]);
-      else __builtin_nontemporal_store(v[u], &dst[rm[u]]);
+  for (int u = 0; u < U; ++u) {
+    if (tiled[u] < 0) continue;
+    if (TILIZE) {
+      __builtin_nontemporal_store(v[u], (chunk_t *)dst + tiled[u]);
+    } else {
+      T *p = (T *)dst + rm[u];
+      if (n >= V) {
+        *(chunk_any *)p = v[u];
+      } else {
+        T e[V];
+        *(chunk_t *)e = v[u];
+#pragma unroll
+        for (int j = 0; j < V; ++j)
+          if (j < n) p[j] = e[j];
+      }
     }
   }
-  (void)yt;
 }
 
 // ------------------------------------------------------------------------------------ LDS staged
@@ -142,7 +180,7 @@ __global__ __launch_bounds__(256) TTM_MAX_WAVES(TILIZE ? 3 : 4) void ttm_tile_st
   }
 }
 
-// ------------------------------------------------------------------------------------ scalar (padding)
+// ------------------------------------------------------------------------------------ scalar: tile-order sides at any address
 template <typename T, bool TILIZE>
 __global__ __launch_bounds__(256) void ttm_tile_scalar_k(const T *__restrict__ src, T *__restrict__ dst,
                                                          int64_t batch, int64_t rows, int64_t cols,
@@ -162,123 +200,47 @@ __global__ __launch_bounds__(256) void ttm_tile_scalar_k(const T *__restrict__ s
   }
 }
 
-// ------------------------------------------------------------------------------------ ragged shapes, small
-// Rows or columns that are not multiples of 32.  Lanes walk the tile-order side in 16-byte chunks (V elements of one face
-// row: one row, V consecutive columns), so that side is read or written in whole lines; the row-major side of a chunk is
-// one 16-byte access when it lies inside the row and its address allows it, else up to V element accesses.  grid.y numbers
-// the matrices.  Tilize writes zeros into the padding; untilize skips it.
-template <typename T, bool TILIZE>
-__global__ __launch_bounds__(256) void ttm_tile_chunks_k(const T *__restrict__ src, T *__restrict__ dst, uint32_t rows, uint32_t cols,
-                                                         uint32_t pr, uint32_t pc) {
-  constexpr uint32_t V = 16 / sizeof(T);
-  const uint32_t chunks = pr / V * pc, ct = pc / 32;
-  const int64_t b = blockIdx.y;
-  const T *rm_src = src + b * rows * (int64_t)cols;
-  T *rm_dst = dst + b * rows * (int64_t)cols;
-  const chunk_t *t_src = (const chunk_t *)(src + b * pr * (int64_t)pc);
-  chunk_t *t_dst = (chunk_t *)(dst + b * pr * (int64_t)pc);
-  for (uint32_t ch = blockIdx.x * 256 + threadIdx.x; ch < chunks; ch += gridDim.x * 256) {
-    const uint32_t e0 = ch * V, tile = e0 >> 10, e = e0 & 1023, face = e >> 8;
-    const uint32_t tr = tile / ct, tc = tile - tr * ct;
-    const uint32_t r = tr * 32 + (face >> 1) * 16 + ((e >> 4) & 15), c0 = tc * 32 + (face & 1) * 16 + (e & 15);
-    const bool row_in = r < rows;
-    const int64_t off = (int64_t)r * cols + c0;
-    if (TILIZE) {
-      chunk_t v = {0, 0, 0, 0};
-      if (row_in && c0 < cols) {
-        const T *p = rm_src + off;
-        if (c0 + V <= cols && ((uintptr_t)p & 15) == 0) {
-          v = __builtin_nontemporal_load((const chunk_t *)p);
-        } else {
-          T t[V];
-#pragma unroll
-          for (uint32_t j = 0; j < V; ++j) t[j] = c0 + j < cols ? p[j] : T(0);
-          v = *(const chunk_t *)t;
-        }
-      }
-      __builtin_nontemporal_store(v, t_dst + ch);
-    } else if (row_in && c0 < cols) {
-      const chunk_t v = __builtin_nontemporal_load(t_src + ch);
-      T *p = rm_dst + off;
-      if (c0 + V <= cols && ((uintptr_t)p & 15) == 0) {
-        __builtin_nontemporal_store(v, (chunk_t *)p);
-      } else {
-        T t[V];
-        *(chunk_t *)t = v;
-#pragma unroll
-        for (uint32_t j = 0; j < V; ++j)
-          if (c0 + j < cols) p[j] = t[j];
-      }
-    }
-  }
-}
-
-// Untilize of a ragged shape whose rows are whole 16-byte chunks (cols a multiple of V, destination 16-byte aligned): lanes
-// walk the row-major destination, so the stores are whole lines, and fetch each chunk from its face row on the tile side.
-template <typename T>
-__global__ __launch_bounds__(256) void ttm_untilize_rows_k(const T *__restrict__ src, T *__restrict__ dst, uint32_t rows, uint32_t cols,
-                                                           uint32_t pr, uint32_t pc) {
-  constexpr uint32_t V = 16 / sizeof(T);
-  const uint32_t cpr = cols / V, chunks = rows * cpr, ct = pc / 32;
-  const int64_t b = blockIdx.y;
-  const chunk_t *t_src = (const chunk_t *)(src + b * pr * (int64_t)pc);
-  chunk_t *o = (chunk_t *)(dst + b * rows * (int64_t)cols);
-  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < chunks; i += gridDim.x * 256) {
-    const uint32_t r = i / cpr, c0 = (i - r * cpr) * V;
-    const uint32_t e = ((r >> 5) * ct + (c0 >> 5)) * 1024 + (((r >> 4) & 1) * 2 + ((c0 >> 4) & 1)) * 256 + (r & 15) * 16 + (c0 & 15);
-    __builtin_nontemporal_store(__builtin_nontemporal_load(t_src + e / V), o + i);
-  }
-}
-
-// ------------------------------------------------------------------------------------ ragged shapes
+// ------------------------------------------------------------------------------------ untilize of ragged shapes, large
 // Rows or columns that are not multiples of 32, or a row-major side that starts anywhere.  The strip kernel's plan (32 rows x 512
-// bytes per workgroup) with the row-major side moved in shifted chunks (ttm_ragged.h).  HBM-bound as the strip kernel is; before,
-// a chunk whose address was not a multiple of 16 went by element accesses, seven of eight for an odd bf16 width: [3, 1000, 3001]
-// bf16 tilize / untilize 14.8 / 23.3 -> 7.8 / 10.0 us, [4000, 7001] fp32 51 / 78 -> 41 / 38 us (5.5 / 5.9 TB/s).
-// Tilize writes zeros into the padding; untilize skips it.  grid (strips x tile rows, matrices).
-template <int ELEM, bool TILIZE>
-__global__ __launch_bounds__(256) void ttm_tile_ragged_k(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int rows, int cols,
-                                                         int strips, int64_t matrices) {
+// bytes per workgroup) with the row-major side stored in shifted chunks (ttm_ragged.h).  HBM-bound as the strip kernel is.  The
+// padding is skipped.  grid (strips x tile rows, matrices).
+template <int ELEM>
+__global__ __launch_bounds__(256) void ttm_untilize_ragged_k(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int rows, int cols,
+                                                             int strips, int64_t matrices) {
   constexpr int CPT = 64 * ELEM;   // chunks per tile
   __shared__ u32x4 image[kRaggedImage];
   const int tid = threadIdx.x;
   const RaggedStrip st = ragged_strip<ELEM>(rows, cols, strips);
   for (int64_t b = blockIdx.y; b < matrices; b += gridDim.y) {
     const int64_t tile_off = ((b * st.yt + st.ty) * st.ct + st.sx * (16 / ELEM)) * (int64_t)(CPT * 16);
-    const uintptr_t rm = (uintptr_t)(TILIZE ? src : dst) + (b * rows + st.ty * 32) * st.stride + st.sx * 512;
-    if (TILIZE) {
-      ragged_load<ELEM>(image, st, rm, (uintptr_t)src, (uintptr_t)src + matrices * rows * st.stride);
-      __syncthreads();
+    const uintptr_t rm = (uintptr_t)dst + (b * rows + st.ty * 32) * st.stride + st.sx * 512;
+    const bool more = ragged_left(st) > 512;
+    u32x4 v[5];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int oc = i * 256 + tid, tl = oc / CPT, w = oc % CPT;
-        if (tl >= st.tiles) continue;
-        const int face = w / (16 * ELEM), dy = (w / ELEM) % 16, q = w % ELEM;
-        const u32x4 o = ragged_read(image, st, rm, (face >> 1) * 16 + dy, (tl * 2 * ELEM + (face & 1) * ELEM + q) * 16);
-        __builtin_nontemporal_store(o, (u32x4 *)(dst + tile_off) + oc);
-      }
-    } else {
-      const bool more = ragged_left(st) > 512;
-      u32x4 v[5];
-#pragma unroll
-      for (int i = 0; i < 5; ++i) {
-        const int oc = i < 4 ? i * 256 + tid : 16 / ELEM * CPT + (tid >> 4) * (32 * ELEM) + (tid & 15) * ELEM;   // i = 4: row tid of the next tile's column 0
-        if (i < 4 ? oc / CPT < st.tiles : tid < 32 && more) v[i] = __builtin_nontemporal_load((const u32x4 *)(src + tile_off) + oc);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int oc = i * 256 + tid, tl = oc / CPT, w = oc % CPT;
-        const int face = w / (16 * ELEM), dy = (w / ELEM) % 16, q = w % ELEM;
-        if (tl < st.tiles) image[((face >> 1) * 16 + dy) * kRaggedPitch + tl * 2 * ELEM + (face & 1) * ELEM + q] = v[i];
-      }
-      if (tid < 32 && more) image[tid * kRaggedPitch + 32] = v[4];
-      __syncthreads();
-      ragged_store<ELEM>(image, st, rm);
+    for (int i = 0; i < 5; ++i) {
+      const int oc = i < 4 ? i * 256 + tid : 16 / ELEM * CPT + (tid >> 4) * (32 * ELEM) + (tid & 15) * ELEM;   // i = 4: row tid of the next tile's column 0
+      if (i < 4 ? oc / CPT < st.tiles : tid < 32 && more) v[i] = __builtin_nontemporal_load((const u32x4 *)(src + tile_off) + oc);
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int oc = i * 256 + tid, tl = oc / CPT, w = oc % CPT;
+      const int face = w / (16 * ELEM), dy = (w / ELEM) % 16, q = w % ELEM;
+      if (tl < st.tiles) image[((face >> 1) * 16 + dy) * kRaggedPitch + tl * 2 * ELEM + (face & 1) * ELEM + q] = v[i];
+    }
+    if (tid < 32 && more) image[tid * kRaggedPitch + 32] = v[4];
+    __syncthreads();
+    ragged_store<ELEM>(image, st, rm);
     if (matrices > gridDim.y) __syncthreads();
   }
 }
 
+// The kernel of a shape.  `bytes` is one side; both together stay in the 256 MB last-level cache up to some 128 MiB each.
+//   aligned whole strips: direct up to there, strips beyond ([2048, 4096] bf16 tilize / untilize 6.6 / 6.5 strips, 6.0 / 6.1 us direct,
+//     [4096, 4096] fp32 21.6 / 22.2, 19.9 / 19.9, [8192, 8192] bf16 41.3 / 42.0, 38.8 / 41.2, fp32 80.6 / 82.2, 87 / 87)
+//   other shapes: tilize direct ([8192, 8191] fp32 93 strips, 88 direct, [3, 4000, 8001] fp32 136, 127); untilize direct up to there
+//     ([4000, 7001] fp32 36.8 strips, 35.1 direct), strips where a strip is mostly real rows and columns beyond ([3, 4096, 8190] bf16
+//     64 strips, 73 direct, [8192, 8191] fp32 78, 96)
+// To page-locked host memory the direct form, whose stores go through L2, is the faster one too ([2048, 8192] bf16 669 -> 631 us).
 template <bool TILIZE>
 static int run_layout(const void *src, void *dst, int64_t batch, int64_t rows, int64_t cols, int elem,
                       void *stream, const char *who) {
@@ -288,90 +250,73 @@ static int run_layout(const void *src, void *dst, int64_t batch, int64_t rows, i
   TTM_REQUIRE(src && dst, "%s: null pointer", who);
   TTM_REQUIRE(src != dst, "%s: in-place conversion is not supported", who);
   hipStream_t s = (hipStream_t)stream;
-  const int64_t pr = ttm_round_up32(rows), pc = ttm_round_up32(cols);
+  const int64_t pr = ttm_round_up32(rows), pc = ttm_round_up32(cols), bytes = batch * pr * pc * elem;
   const bool aligned = rows == pr && cols == pc && ((uintptr_t)src & 15) == 0 && ((uintptr_t)dst & 15) == 0;
-  // The strip kernel where its workgroups fill the device and their strips are mostly real rows and columns; small, short or
-  // narrow tensors are faster a chunk per lane ([53, 1023] bf16 2.6 / 2.9 us against 3.7 / 5.5, [2000, 5, 40] 3.8 / 3.3 against 7.3 / 6.9).
+  // whole 16-byte chunks on the tile-order side, whole elements on the other
+  const bool plain = pr < INT32_MAX && pc < INT32_MAX && ((uintptr_t)(TILIZE ? dst : src) & 15) == 0 && (uintptr_t)(TILIZE ? src : dst) % elem == 0;
+  const bool large = bytes > ((int64_t)(TILIZE ? 96 : 160) << 20) && ttm_option(TILIZE ? "tilize_variant" : "untilize_variant") == 0;
   const int64_t strips = ttm_cdiv(pc * elem, 512);
-  const int variant = ttm_option(TILIZE ? "tilize_variant" : "untilize_variant");
-  if ((!aligned || (cols * elem % 512 != 0 && variant == 0)) && pr * pc < ((int64_t)1 << 31) && ((uintptr_t)(TILIZE ? dst : src) & 15) == 0 &&   // the tile-order side moves in whole 16-byte chunks
-      (uintptr_t)(TILIZE ? src : dst) % elem == 0 && batch * strips * (pr / 32) >= 256 && rows >= 24 && cols * elem * 4 >= strips * 512 * 3) {
-    const dim3 grid((unsigned)(strips * (pr / 32)), (unsigned)(batch > 65535 ? 65535 : batch));
-#define RAGGED(E) \
-  hipLaunchKernelGGL((ttm_tile_ragged_k<E, TILIZE>), grid, dim3(256), 0, s, (const uint8_t *)src, (uint8_t *)dst, (int)rows, (int)cols, (int)strips, batch)
-    if (elem == 4) RAGGED(4);
-    else if (elem == 2) RAGGED(2);
-    else RAGGED(1);
-#undef RAGGED
-    TTM_LAUNCH_CHECK();
-    return TTM_OK;
-  }
-  if (!aligned && batch <= 65535 && pr * pc < ((int64_t)1 << 31) && rows * cols < ((int64_t)1 << 31) &&
-      ((uintptr_t)(TILIZE ? dst : src) & 15) == 0 &&   // the tile-order side moves in whole 16-byte chunks
-      (TILIZE || elem > 1 || cols % 16 == 0)) {       // bytes into rows that are not whole chunks: the element-wise kernel is faster
-    if (!TILIZE && cols % (16 / elem) == 0 && ((uintptr_t)dst & 15) == 0) {
-      const int64_t rchunks = rows * cols * elem / 16;
-      const dim3 rgrid((unsigned)(ttm_cdiv(rchunks, 256) > 262144 ? 262144 : ttm_cdiv(rchunks, 256)), (unsigned)batch);
-#define ROWS(T) \
-  hipLaunchKernelGGL((ttm_untilize_rows_k<T>), rgrid, dim3(256), 0, s, (const T *)src, (T *)dst, (uint32_t)rows, (uint32_t)cols, (uint32_t)pr, \
-                     (uint32_t)pc)
-      if (elem == 4) ROWS(uint32_t);
-      else if (elem == 2) ROWS(uint16_t);
-      else ROWS(uint8_t);
-#undef ROWS
-      TTM_LAUNCH_CHECK();
-      return TTM_OK;
-    }
-    const int64_t chunks = pr * pc * elem / 16;
-    const dim3 grid((unsigned)(ttm_cdiv(chunks, 256) > 262144 ? 262144 : ttm_cdiv(chunks, 256)), (unsigned)batch);
-#define RAGGED(T) \
-  hipLaunchKernelGGL((ttm_tile_chunks_k<T, TILIZE>), grid, dim3(256), 0, s, (const T *)src, (T *)dst, (uint32_t)rows, (uint32_t)cols, \
-                     (uint32_t)pr, (uint32_t)pc)
-    if (elem == 4) RAGGED(uint32_t);
-    else if (elem == 2) RAGGED(uint16_t);
-    else RAGGED(uint8_t);
-#undef RAGGED
-    TTM_LAUNCH_CHECK();
-    return TTM_OK;
-  }
-  if (!aligned) {
-    int64_t n = batch * pr * pc;
-    unsigned blocks = (unsigned)(ttm_cdiv(n, 256) > 1048576 ? 1048576 : ttm_cdiv(n, 256));
-#define SCALAR(T) \
-  hipLaunchKernelGGL((ttm_tile_scalar_k<T, TILIZE>), dim3(blocks), dim3(256), 0, s, (const T *)src, (T *)dst, \
-                     batch, rows, cols, pr, pc)
-    if (elem == 4) SCALAR(uint32_t);
-    else if (elem == 2) SCALAR(uint16_t);
-    else SCALAR(uint8_t);
-#undef SCALAR
-    TTM_LAUNCH_CHECK();
-    return TTM_OK;
-  }
-  const int64_t yt = batch * (pr / 32), xt = pc / 32;
-  const int64_t total_chunks = yt * xt * 64 * elem;
-  const int64_t row_bytes = cols * elem;
-  if (variant == 0 && row_bytes % 512 == 0) {
-    int64_t strips_per_row = row_bytes / 512;
-    int64_t blocks = yt * strips_per_row;
+  if (large && aligned && cols * elem % 512 == 0) {
+    const int64_t blocks = batch * (pr / 32) * strips;
     TTM_REQUIRE(blocks < (1ll << 31), "%s: tensor too large", who);
 #define STRIP(E) \
   hipLaunchKernelGGL((ttm_tile_strip_k<E, TILIZE>), dim3((unsigned)blocks), dim3(256), 0, s, \
-                     (const chunk_t *)src, (chunk_t *)dst, xt, strips_per_row)
+                     (const chunk_t *)src, (chunk_t *)dst, pc / 32, strips)
     if (elem == 4) STRIP(4);
     else if (elem == 2) STRIP(2);
     else STRIP(1);
 #undef STRIP
-  } else {
-    int64_t blocks = ttm_cdiv(total_chunks, 1024);
-    TTM_REQUIRE(blocks < (1ll << 31), "%s: tensor too large", who);
-#define DIRECT(E) \
-  hipLaunchKernelGGL((ttm_tile_direct_k<E, TILIZE>), dim3((unsigned)blocks), dim3(256), 0, s, \
-                     (const chunk_t *)src, (chunk_t *)dst, yt, xt, total_chunks)
-    if (elem == 4) DIRECT(4);
-    else if (elem == 2) DIRECT(2);
-    else DIRECT(1);
-#undef DIRECT
+    TTM_LAUNCH_CHECK();
+    return TTM_OK;
   }
+  if constexpr (!TILIZE) {
+    if (large && plain && pr * pc < ((int64_t)1 << 31) && rows >= 24 && cols * elem * 4 >= strips * 512 * 3) {
+      const dim3 grid((unsigned)(strips * (pr / 32)), (unsigned)(batch > 65535 ? 65535 : batch));
+#define RAGGED(E) \
+  hipLaunchKernelGGL((ttm_untilize_ragged_k<E>), grid, dim3(256), 0, s, (const uint8_t *)src, (uint8_t *)dst, (int)rows, (int)cols, (int)strips, batch)
+      if (elem == 4) RAGGED(4);
+      else if (elem == 2) RAGGED(2);
+      else RAGGED(1);
+#undef RAGGED
+      TTM_LAUNCH_CHECK();
+      return TTM_OK;
+    }
+  }
+  const int u = TILIZE && bytes <= ((int64_t)32 << 20) ? 2 : 1;   // accesses per lane
+  const int64_t across = ttm_cdiv((TILIZE ? pc : cols) * elem, 16);   // chunks of a row
+  int lw = 0, wc = 0;
+  while ((1 << lw) < 8 * elem && (1 << lw) < across) ++lw;
+  while (wc < 2 && ((int64_t)1 << (lw + wc)) < across) ++wc;
+  const int64_t xu = ttm_cdiv(across, 1 << (lw + wc)), rows_all = batch * (TILIZE ? pr : rows), groups = ttm_cdiv(rows_all, ((64 >> lw) * u) << (2 - wc));
+  if (plain && rows_all < INT32_MAX && groups * xu < INT32_MAX) {
+    const dim3 grid((unsigned)(groups * xu));
+#define DIRECT(E, U) \
+  hipLaunchKernelGGL((ttm_tile_direct_k<E, U, TILIZE>), grid, dim3(256), 0, s, (const uint8_t *)src, (uint8_t *)dst, (int)rows, (int)cols, lw, wc, \
+                     (uint32_t)xu, (uint32_t)batch)
+#define DIRECT_U(E)                                       \
+  do {                                                    \
+    if constexpr (TILIZE) {                               \
+      if (u == 2) DIRECT(E, 2);                           \
+      else DIRECT(E, 1);                                  \
+    } else DIRECT(E, 1);                                  \
+  } while (0)
+    if (elem == 4) DIRECT_U(4);
+    else if (elem == 2) DIRECT_U(2);
+    else DIRECT_U(1);
+#undef DIRECT_U
+#undef DIRECT
+    TTM_LAUNCH_CHECK();
+    return TTM_OK;
+  }
+  int64_t n = batch * pr * pc;
+  unsigned blocks = (unsigned)(ttm_cdiv(n, 256) > 1048576 ? 1048576 : ttm_cdiv(n, 256));
+#define SCALAR(T) \
+  hipLaunchKernelGGL((ttm_tile_scalar_k<T, TILIZE>), dim3(blocks), dim3(256), 0, s, (const T *)src, (T *)dst, \
+                     batch, rows, cols, pr, pc)
+  if (elem == 4) SCALAR(uint32_t);
+  else if (elem == 2) SCALAR(uint16_t);
+  else SCALAR(uint8_t);
+#undef SCALAR
   TTM_LAUNCH_CHECK();
   return TTM_OK;
 }
