@@ -95,6 +95,27 @@ def test_tilize_untilize_at_any_element(hip, dev, orc, shape, dtype, offset):
     assert np.all(got[:offset] == seven) and np.all(got[offset + n:] == seven)
 
 
+@pytest.mark.parametrize("fmt", [8, 4])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_bfp_large_tensors_take_strips(hip, dev, fmt, dtype):
+    """Above the size up to which odd shapes go chunk by chunk, packed and unpacked by strips: the same bytes and values."""
+    hfmt, code = (hip.BFP8B if fmt == 8 else hip.BFP4B), (hip.F32 if dtype == torch.float32 else hip.BF16)
+    shape = (1, 20500 if dtype == torch.float32 else 41000, 2051)
+    assert shape[1] * shape[2] * dtype.itemsize > 160 << 20
+    x = torch.randn(shape, device=dev, generator=torch.Generator(device=dev).manual_seed(4)).to(dtype)
+    got = {}
+    for variant in (0, 2):
+        hip.set_option("pack_variant", variant)
+        hip.set_option("unpack_variant", variant)
+        try:
+            p = pack_gpu(hip, dev, x, hfmt, shape, code, hip.ROW_MAJOR)
+            got[variant] = p, unpack_gpu(hip, dev, p, hfmt, shape, code, hip.ROW_MAJOR)
+        finally:
+            hip.set_option("pack_variant", 0)
+            hip.set_option("unpack_variant", 0)
+    assert torch.equal(got[0][0], got[2][0]) and torch.equal(got[0][1], got[2][1])
+
+
 @pytest.mark.parametrize("rows,cols", [(41000, 2051), (41024, 2048)])
 def test_large_tensors_take_strips(hip, dev, rows, cols):
     """Above the size up to which every shape goes chunk by chunk: whole strips and rows that start anywhere, against torch."""
@@ -265,8 +286,8 @@ def test_full_size_properties(hip, dev, orc, fmt):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("shape,shift", [((1, 1, 1), 0), ((2, 33, 129), 1), ((1, 64, 255), 3), ((3, 31, 257), 0), ((1, 95, 1023), 5), ((2, 40, 300), 2),
                                          ((1, 32, 512), 1), ((1, 500, 384), 0), ((2, 1100, 2081), 7)])
-def test_bfp_ragged_strips(hip, dev, orc, fmt, dtype, shape, shift):
-    """Strips whose rows start and end anywhere, on buffers that start at any element: packed bytes and read-back against the oracle
+def test_bfp_ragged(hip, dev, orc, fmt, dtype, shape, shift):
+    """Rows that start and end anywhere, on buffers that start at any element: packed bytes and read-back against the oracle
     and the generic kernel (random bit patterns: infinities, NaN and subnormal numbers among them), nothing written around them."""
     hfmt, code = (hip.BFP8B if fmt == 8 else hip.BFP4B), (hip.F32 if dtype == torch.float32 else hip.BF16)
     b, r, c = shape

@@ -13,6 +13,7 @@
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 chunk_any __attribute__((aligned(1)));   // 16 bytes at any address (the part takes them unaligned)
 
 #define TTM_EXPORT extern "C" __attribute__((visibility("default")))
 
@@ -92,6 +93,13 @@ bool ttm_rowwise_partials_supported(int64_t rows, int64_t cols);
 int ttm_rowwise_rmsnorm_from_partials(const float *partial, int slices, int64_t per, const void *residual, void *sum_out,
                                       const void *weight, int weight_layout, const void *bias, int bias_layout, void *out,
                                       int64_t rows, int64_t cols, float eps, hipStream_t s);
+
+// Workgroups are dealt to the eight XCDs in turn; this number gives neighbours to one XCD, whose L2 then puts the two parts of a
+// line at their common edge together.
+__device__ __forceinline__ uint32_t xcd_order() {
+  const uint32_t n8 = gridDim.x >> 3;
+  return blockIdx.x < n8 * 8 ? (blockIdx.x & 7) * n8 + (blockIdx.x >> 3) : blockIdx.x;
+}
 
 __host__ __device__ static inline int64_t ttm_round_up32(int64_t v) { return (v + 31) / 32 * 32; }
 static inline int64_t ttm_cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }

@@ -56,7 +56,6 @@ TTM_EXPORT int ttm_copy_kernel(const void *src, void *dst, size_t bytes, void *s
 // rows x 512 bytes through LDS with funnel shifts for odd rows: [3, 1000, 3001] bf16 tilize / untilize 9.0 / 10.6 -> 7.0 / 6.9 us,
 // [4000, 7001] fp32 42.0 / 37.2 -> 39.4 / 35.6, [2, 1266, 771] bf16 4.2 / 5.5 -> 3.1 / 3.2, [7, 33, 9000] fp32 7.7 / 6.2 -> 4.4 / 4.4,
 // [65536, 64] bf16 5.3 / 6.2 -> 3.1 / 3.6, [70000, 3, 100] bf16 590 / 528 -> 89 / 20.
-typedef chunk_t chunk_any __attribute__((aligned(1)));   // at any address
 template <int ELEM>
 using layout_elem = typename std::conditional<ELEM == 4, uint32_t, typename std::conditional<ELEM == 2, uint16_t, uint8_t>::type>::type;
 
@@ -68,8 +67,8 @@ __global__ __launch_bounds__(256) void ttm_tile_direct_k(const uint8_t *__restri
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ct = (cols + 31) >> 5, yt = (rows + 31) >> 5;
   // a wavefront's accesses are 1 << lw chunks wide, a workgroup 1 << wc wavefronts; its other wavefronts lie below
-  const uint32_t by = blockIdx.x / xu;
-  const int chunk = (int)((((blockIdx.x - by * xu) << wc) + (wave & ((1 << wc) - 1))) << lw) + (lane & ((1 << lw) - 1));
+  const uint32_t bid = xcd_order(), by = bid / xu;
+  const int chunk = (int)((((bid - by * xu) << wc) + (wave & ((1 << wc) - 1))) << lw) + (lane & ((1 << lw) - 1));
   const uint32_t row0 = ((by << (2 - wc)) + (wave >> wc)) * (64 >> lw) * U + (lane >> lw);   // of the rows of all matrices, padded ones for tilize
   const uint32_t per = TILIZE ? yt * 32 : rows;
   const int n = cols - chunk * V;                          // elements of the row from this chunk on
@@ -254,7 +253,7 @@ static int run_layout(const void *src, void *dst, int64_t batch, int64_t rows, i
   const bool aligned = rows == pr && cols == pc && ((uintptr_t)src & 15) == 0 && ((uintptr_t)dst & 15) == 0;
   // whole 16-byte chunks on the tile-order side, whole elements on the other
   const bool plain = pr < INT32_MAX && pc < INT32_MAX && ((uintptr_t)(TILIZE ? dst : src) & 15) == 0 && (uintptr_t)(TILIZE ? src : dst) % elem == 0;
-  const bool large = bytes > ((int64_t)(TILIZE ? 96 : 160) << 20) && ttm_option(TILIZE ? "tilize_variant" : "untilize_variant") == 0;
+  const bool large = bytes > ((int64_t)(aligned ? 64 : 160) << 20) && ttm_option(TILIZE ? "tilize_variant" : "untilize_variant") == 0;
   const int64_t strips = ttm_cdiv(pc * elem, 512);
   if (large && aligned && cols * elem % 512 == 0) {
     const int64_t blocks = batch * (pr / 32) * strips;
