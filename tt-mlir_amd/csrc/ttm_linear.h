@@ -109,19 +109,24 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   return *(uint32_t *)&h;
 }
 
-// Four consecutive outputs -> bf16, optionally followed by the element-wise tail.  The result is rounded to bf16 before the
-// tail and again after it, exactly as a separate binary op on the stored result would do.
-__device__ __forceinline__ u32x2 finish_quad(const LinearArgs &p, const uint8_t *cptr, const float (&v)[4]) {
+// Four consecutive bias values of column tile nt, from column n_in of the tile on
+__device__ __forceinline__ u32x2 bias_quad(const LinearArgs &p, int nt, int n_in) {
+  return *(const u32x2 *)(p.bias_tiled ? p.bias + (int64_t)nt * 1024 + (n_in >> 4) * 256 + (n_in & 15) : p.bias + nt * 32 + n_in);
+}
+// Bias and tail operands are loaded for many outputs in front of the first of them: requested one by one behind the store before (which
+// they might alias as far as the compiler knows), every quad waited for a memory round trip of its own.
+// Four consecutive outputs -> bf16, optionally followed by the element-wise tail with the quad `r`.  The result is rounded to bf16
+// before the tail and again after it, exactly as a separate binary op on the stored result would do.
+__device__ __forceinline__ u32x2 finish_quad(int tail, u32x2 r, const float (&v)[4]) {
   u32x2 o = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
-  if (p.tail != 0) {   // uniform
-    const u32x2 r = *(const u32x2 *)(cptr + p.tail_delta);
+  if (tail != 0) {   // uniform
     const float y[4] = {__uint_as_float(o.x << 16), __uint_as_float(o.x & 0xFFFF0000u), __uint_as_float(o.y << 16),
                         __uint_as_float(o.y & 0xFFFF0000u)};
     const float t[4] = {__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xFFFF0000u), __uint_as_float(r.y << 16),
                         __uint_as_float(r.y & 0xFFFF0000u)};
     float z[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) z[i] = p.tail == 1 ? y[i] + t[i] : y[i] * t[i];
+    for (int i = 0; i < 4; ++i) z[i] = tail == 1 ? y[i] + t[i] : y[i] * t[i];
     o = u32x2{pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3])};
   }
   return o;
@@ -153,6 +158,28 @@ __device__ __forceinline__ float linear_act_rt(int act, float x) {
   case TTM_ACT_RELU: return apply_act<TTM_ACT_RELU>(x);
   default: return x;
   }
+}
+// N values at once: the branches of a switch per value took longer than summing the wavefronts' shares of it
+template <int N>
+__device__ __forceinline__ void linear_act_rt(int act, float (&v)[N]) {
+  auto all = [&](auto a) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = apply_act<decltype(a)::value>(v[i]);
+  };
+  if (act == TTM_ACT_NONE) return;   // uniform
+  switch (act) {
+  case TTM_ACT_GELU: all(std::integral_constant<int, TTM_ACT_GELU>{}); break;
+  case TTM_ACT_SILU: all(std::integral_constant<int, TTM_ACT_SILU>{}); break;
+  case TTM_ACT_SIGMOID: all(std::integral_constant<int, TTM_ACT_SIGMOID>{}); break;
+  case TTM_ACT_RELU: all(std::integral_constant<int, TTM_ACT_RELU>{}); break;
+  }
+}
+// act0(a) x act1(b) of a gated pair, the factors rounded to bf16 as the two projections alone would store them
+__device__ __forceinline__ u32x2 glu_quad(const float *a, const float *b) {
+  const u32x2 g = {pack_bf16(a[0], a[1]), pack_bf16(a[2], a[3])}, u = {pack_bf16(b[0], b[1]), pack_bf16(b[2], b[3])};
+  const float z[4] = {__uint_as_float(g.x << 16) * __uint_as_float(u.x << 16), __uint_as_float(g.x & 0xFFFF0000u) * __uint_as_float(u.x & 0xFFFF0000u),
+                      __uint_as_float(g.y << 16) * __uint_as_float(u.y << 16), __uint_as_float(g.y & 0xFFFF0000u) * __uint_as_float(u.y & 0xFFFF0000u)};
+  return u32x2{pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3])};
 }
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 

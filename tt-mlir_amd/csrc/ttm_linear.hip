@@ -175,30 +175,36 @@ __device__ __forceinline__ void store_w(u32x4 *ldsW, int tid, const WRegs<WF> &r
 template <int ACT, int NA, int MB>
 __device__ __forceinline__ void linear_epilogue(const LinearArgs &p, uint8_t *C, f32x16 (&acc)[NA][MB], int mtw, int ntw, int nt_end, int lane) {
   const int m_in = lane & 31;
+  auto offset = [&](int a, int g, int b) __attribute__((always_inline)) {   // clamped to the last tile: tiles beyond it are not stored
+    const int n_in = g * 8 + (lane >> 5) * 4, mt = min(mtw + b, p.Mt - 1), nt = min(ntw + a, nt_end - 1);
+    return (((int64_t)mt * p.Nt + nt) * 1024 + ((m_in >> 4) * 2 + (n_in >> 4)) * 256 + (m_in & 15) * 16 + (n_in & 15)) * 2;
+  };
+  u32x2 bias[NA][4], tail[2][4][MB];
+  auto load_tail = [&](int a) __attribute__((always_inline)) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int b = 0; b < MB; ++b) tail[a & 1][g][b] = p.tail ? *(const u32x2 *)(C + offset(a, g, b) + p.tail_delta) : u32x2{0, 0};
+  };
+#pragma unroll
+  for (int a = 0; a < NA; ++a)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) bias[a][g] = p.bias ? bias_quad(p, min(ntw + a, nt_end - 1), g * 8 + (lane >> 5) * 4) : u32x2{0, 0};
+  load_tail(0);
 #pragma unroll
   for (int a = 0; a < NA; ++a) {
-    const int nt = ntw + a;
-    if (nt >= nt_end) continue;
+    if (a + 1 < NA) load_tail(a + 1);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      const int n_in = g * 8 + (lane >> 5) * 4;
-      float bv[4] = {0.f, 0.f, 0.f, 0.f};
-      if (p.bias) {
-        const int n = nt * 32 + n_in;
-        const uint16_t *bp = p.bias_tiled ? p.bias + (int64_t)nt * 1024 + (n_in >> 4) * 256 + (n_in & 15) : p.bias + n;
-        u32x2 raw = *(const u32x2 *)bp;
-        bv[0] = __uint_as_float(raw.x << 16); bv[1] = __uint_as_float(raw.x & 0xFFFF0000u);
-        bv[2] = __uint_as_float(raw.y << 16); bv[3] = __uint_as_float(raw.y & 0xFFFF0000u);
-      }
+      const u32x2 raw = bias[a][g];
+      const float bv[4] = {__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xFFFF0000u), __uint_as_float(raw.y << 16), __uint_as_float(raw.y & 0xFFFF0000u)};
 #pragma unroll
       for (int b = 0; b < MB; ++b) {
-        const int mt = mtw + b;
-        if (mt >= p.Mt) continue;
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = apply_act<ACT>(acc[a][b][g * 4 + r] + bv[r]);
-        int64_t off = ((int64_t)mt * p.Nt + nt) * 1024 + ((m_in >> 4) * 2 + (n_in >> 4)) * 256 + (m_in & 15) * 16 + (n_in & 15);
-        *(u32x2 *)(C + off * 2) = finish_quad(p, C + off * 2, v);
+        const u32x2 o = finish_quad(p.tail, tail[a & 1][g][b], v);
+        if (ntw + a < nt_end && mtw + b < p.Mt) *(u32x2 *)(C + offset(a, g, b)) = o;
       }
     }
   }
@@ -238,23 +244,19 @@ __device__ __forceinline__ void linear_epilogue_glu(const LinearArgs &p, uint8_t
     if (ntw + 2 * j >= nt_end) continue;
     const int nt = (ntw >> 1) + j;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int n_in = g * 8 + (lane >> 5) * 4;
+    for (int b = 0; b < MB; ++b) {
+      const int mt = mtw + b;
+      if (mt >= p.Mt) continue;
+      float x[16], y[16];
 #pragma unroll
-      for (int b = 0; b < MB; ++b) {
-        const int mt = mtw + b;
-        if (mt >= p.Mt) continue;
-        float x[4], y[4];
+      for (int r = 0; r < 16; ++r) { x[r] = acc[2 * j][b][r]; y[r] = acc[2 * j + 1][b][r]; }
+      linear_act_rt(act0, x);
+      linear_act_rt(act1, y);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          x[r] = linear_act_rt(act0, acc[2 * j][b][g * 4 + r]);
-          y[r] = linear_act_rt(act1, acc[2 * j + 1][b][g * 4 + r]);
-        }
-        const u32x2 gq = {pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3])}, uq = {pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3])};
-        const float z[4] = {__uint_as_float(gq.x << 16) * __uint_as_float(uq.x << 16), __uint_as_float(gq.x & 0xFFFF0000u) * __uint_as_float(uq.x & 0xFFFF0000u),
-                            __uint_as_float(gq.y << 16) * __uint_as_float(uq.y << 16), __uint_as_float(gq.y & 0xFFFF0000u) * __uint_as_float(uq.y & 0xFFFF0000u)};
+      for (int g = 0; g < 4; ++g) {
+        const int n_in = g * 8 + (lane >> 5) * 4;
         const int64_t off = ((int64_t)mt * NtR + nt) * 1024 + ((m_in >> 4) * 2 + (n_in >> 4)) * 256 + (m_in & 15) * 16 + (n_in & 15);
-        *(u32x2 *)(C + off * 2) = u32x2{pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3])};
+        *(u32x2 *)(C + off * 2) = glu_quad(&x[4 * g], &y[4 * g]);
       }
     }
   }
@@ -266,44 +268,24 @@ __global__ __launch_bounds__(256) void ttm_linear_reduce_k(LinearArgs p, int sli
   const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;   // group of four consecutive elements
   if (q * 4 >= per) return;
   const float *P = p.partial + (int64_t)blockIdx.z * slices * per + q * 4;
-  f32x4 sum = *(const f32x4 *)P;
-  for (int s = 1; s < slices; ++s) sum += *(const f32x4 *)(P + s * per);
   const int64_t off = q * 4;
   const int nt = (int)((off >> 10) % p.Nt), in = (int)(off & 1023);
   const int n_in = ((in >> 8) & 1) * 16 + (in & 15);
-  float bv[4] = {0.f, 0.f, 0.f, 0.f};
-  if (p.bias) {
-    const uint16_t *bp = p.bias_tiled ? p.bias + (int64_t)nt * 1024 + (n_in >> 4) * 256 + (n_in & 15) : p.bias + nt * 32 + n_in;
-    u32x2 raw = *(const u32x2 *)bp;
-    bv[0] = __uint_as_float(raw.x << 16); bv[1] = __uint_as_float(raw.x & 0xFFFF0000u);
-    bv[2] = __uint_as_float(raw.y << 16); bv[3] = __uint_as_float(raw.y & 0xFFFF0000u);
-  }
   GroupMember m = {};
   int act = p.act;
   if (p.group_n > 1) {   // tile nt of the concatenation belongs to one member
     m = group_member(p, nt, 1);
     act = m.act;
   }
-  float v[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    float x = sum[r] + bv[r];
-    switch (act) {
-    case TTM_ACT_GELU: x = apply_act<TTM_ACT_GELU>(x); break;
-    case TTM_ACT_SILU: x = apply_act<TTM_ACT_SILU>(x); break;
-    case TTM_ACT_SIGMOID: x = apply_act<TTM_ACT_SIGMOID>(x); break;
-    case TTM_ACT_RELU: x = apply_act<TTM_ACT_RELU>(x); break;
-    default: break;
-    }
-    v[r] = x;
-  }
-  if (p.group_n > 1) {
-    uint8_t *Cm = m.C + (((off >> 10) / p.Nt * m.Nt + m.local) * 1024 + in) * 2;
-    *(u32x2 *)Cm = finish_quad(p, Cm, v);
-    return;
-  }
-  uint8_t *C = p.C + (int64_t)blockIdx.z * p.c_batch;
-  *(u32x2 *)(C + off * 2) = finish_quad(p, C + off * 2, v);
+  uint8_t *C = p.group_n > 1 ? m.C + (((off >> 10) / p.Nt * m.Nt + m.local) * 1024 + in) * 2 : p.C + (int64_t)blockIdx.z * p.c_batch + off * 2;
+  const u32x2 raw = p.bias ? bias_quad(p, nt, n_in) : u32x2{0, 0}, tail = p.tail ? *(const u32x2 *)(C + p.tail_delta) : u32x2{0, 0};
+  f32x4 sum = *(const f32x4 *)P;
+#pragma unroll 4
+  for (int s = 1; s < slices; ++s) sum += *(const f32x4 *)(P + s * per);
+  float v[4] = {sum[0] + __uint_as_float(raw.x << 16), sum[1] + __uint_as_float(raw.x & 0xFFFF0000u), sum[2] + __uint_as_float(raw.y << 16),
+                sum[3] + __uint_as_float(raw.y & 0xFFFF0000u)};
+  linear_act_rt(act, v);
+  *(u32x2 *)C = finish_quad(p.tail, tail, v);
 }
 
 template <int NA, int MB>
@@ -322,28 +304,31 @@ __device__ __forceinline__ void linear_epilogue_act(const LinearArgs &p, uint8_t
 template <int ACT, int NU, int NV>
 __device__ __forceinline__ void linear_epilogue16(const LinearArgs &p, uint8_t *C, f32x4 (&acc)[NU][NV], int mtw, int ntw, int nt_end, int lane) {
   const int m16 = lane & 15, n4 = (lane >> 4) * 4;
+  static_assert(NU % 2 == 0, "whole column tiles");
+  auto offset = [&](int u, int v) __attribute__((always_inline)) {   // clamped to the last tile: tiles beyond it are not stored
+    const int n_in = (u & 1) * 16 + n4, m_in = (v & 1) * 16 + m16, mt = min(mtw + (v >> 1), p.Mt - 1), nt = min(ntw + (u >> 1), nt_end - 1);
+    return (((int64_t)mt * p.Nt + nt) * 1024 + ((m_in >> 4) * 2 + (n_in >> 4)) * 256 + (m_in & 15) * 16 + (n_in & 15)) * 2;
+  };
+  u32x2 bias[NU], tail[4][NV];
+  auto load_tail = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) tail[u & 3][v] = p.tail ? *(const u32x2 *)(C + offset(u, v) + p.tail_delta) : u32x2{0, 0};
+  };
+#pragma unroll
+  for (int u = 0; u < NU; ++u) bias[u] = p.bias ? bias_quad(p, min(ntw + (u >> 1), nt_end - 1), (u & 1) * 16 + n4) : u32x2{0, 0};
+  load_tail(0); load_tail(1);
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
-    const int nt = ntw + (u >> 1);
-    if (nt >= nt_end) continue;
-    const int n_in = (u & 1) * 16 + n4;
-    float bv[4] = {0.f, 0.f, 0.f, 0.f};
-    if (p.bias) {
-      const uint16_t *bp = p.bias_tiled ? p.bias + (int64_t)nt * 1024 + (n_in >> 4) * 256 + (n_in & 15) : p.bias + nt * 32 + n_in;
-      u32x2 raw = *(const u32x2 *)bp;
-      bv[0] = __uint_as_float(raw.x << 16); bv[1] = __uint_as_float(raw.x & 0xFFFF0000u);
-      bv[2] = __uint_as_float(raw.y << 16); bv[3] = __uint_as_float(raw.y & 0xFFFF0000u);
-    }
+    if (u + 2 < NU) load_tail(u + 2);
+    const u32x2 raw = bias[u];
+    const float bv[4] = {__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xFFFF0000u), __uint_as_float(raw.y << 16), __uint_as_float(raw.y & 0xFFFF0000u)};
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      const int mt = mtw + (v >> 1);
-      if (mt >= p.Mt) continue;
-      const int m_in = (v & 1) * 16 + m16;
       float x[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) x[r] = apply_act<ACT>(acc[u][v][r] + bv[r]);
-      const int64_t off = ((int64_t)mt * p.Nt + nt) * 1024 + ((m_in >> 4) * 2 + (n_in >> 4)) * 256 + (m_in & 15) * 16 + (n_in & 15);
-      *(u32x2 *)(C + off * 2) = finish_quad(p, C + off * 2, x);
+      const u32x2 o = finish_quad(p.tail, tail[u & 3][v], x);
+      if (ntw + (u >> 1) < nt_end && mtw + (v >> 1) < p.Mt) *(u32x2 *)(C + offset(u, v)) = o;
     }
   }
 }
@@ -1495,33 +1480,25 @@ __global__ __launch_bounds__(256) void ttm_linear_small_k(LinearArgs p) {
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] += red[0][r][lane] + red[1][r][lane] + red[2][r][lane];
   const int m_in = lane & 31;
+  u32x2 bias[4], tail[4];
+  auto offset = [&](int g) __attribute__((always_inline)) {
+    const int n_in = g * 8 + (lane >> 5) * 4;
+    return ((int64_t)nt * 1024 + ((m_in >> 4) * 2 + (n_in >> 4)) * 256 + (m_in & 15) * 16 + (n_in & 15)) * 2;
+  };
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    const int n_in = g * 8 + (lane >> 5) * 4;
-    float bv[4] = {0.f, 0.f, 0.f, 0.f};
-    if (p.bias) {
-      const uint16_t *bp = p.bias_tiled ? p.bias + (int64_t)nt * 1024 + (n_in >> 4) * 256 + (n_in & 15)
-                                        : p.bias + nt * 32 + n_in;
-      u32x2 raw = *(const u32x2 *)bp;
-      bv[0] = __uint_as_float(raw.x << 16); bv[1] = __uint_as_float(raw.x & 0xFFFF0000u);
-      bv[2] = __uint_as_float(raw.y << 16); bv[3] = __uint_as_float(raw.y & 0xFFFF0000u);
-    }
-    float v[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float x = acc[g * 4 + r] + bv[r];
-      switch (p.act) {
-      case TTM_ACT_GELU: x = apply_act<TTM_ACT_GELU>(x); break;
-      case TTM_ACT_SILU: x = apply_act<TTM_ACT_SILU>(x); break;
-      case TTM_ACT_SIGMOID: x = apply_act<TTM_ACT_SIGMOID>(x); break;
-      case TTM_ACT_RELU: x = apply_act<TTM_ACT_RELU>(x); break;
-      default: break;
-      }
-      v[r] = x;
-    }
-    int64_t off = (int64_t)nt * 1024 + ((m_in >> 4) * 2 + (n_in >> 4)) * 256 + (m_in & 15) * 16 + (n_in & 15);
-    *(u32x2 *)(C + off * 2) = finish_quad(p, C + off * 2, v);
+    bias[g] = p.bias ? bias_quad(p, nt, g * 8 + (lane >> 5) * 4) : u32x2{0, 0};
+    tail[g] = p.tail ? *(const u32x2 *)(C + offset(g) + p.tail_delta) : u32x2{0, 0};
   }
+  float v[16];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const uint32_t raw = e & 2 ? bias[e >> 2].y : bias[e >> 2].x;
+    v[e] = acc[e] + __uint_as_float(e & 1 ? raw & 0xFFFF0000u : raw << 16);
+  }
+  linear_act_rt(p.act, v);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) *(u32x2 *)(C + offset(g)) = finish_quad(p.tail, tail[g], {v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]});
 }
 
 // =============================================================================================
@@ -1721,89 +1698,58 @@ __global__ __launch_bounds__(512) void ttm_linear_decode_k(LinearArgs p) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[pr][h][j] -= accs[pr][h][j];
   }
-  // partial sums -> LDS as float4 (four consecutive n of one m): slot (((pr * 8 + wave) * 8 + h * 4 + i) * 64 + lane)
+  // partial sums -> LDS as float4 (four consecutive n of one m), then thread t finishes slot t of every tile pair's 512: (h, i, lane) =
+  // (t >> 8, (t >> 6) & 3, t & 63).  Its 8-byte stores lie 32 bytes apart; a face per wavefront instead, whose stores are 512 bytes
+  // in a row, took 1.5 us longer at [32, 4096] x [4096, 14336]: the sums then come out of LDS in another order than they went in.
   f32x4v *part = (f32x4v *)smem;
+  const int h = wave >> 2, fkg = lane >> 4, n_in = 16 * (fkg & 1) + 4 * (wave & 3);
+  const int in = (h * 2 + (fkg & 1)) * 256 + (lane & 15) * 16 + (n_in & 15);
+  u32x2 bias[NP], tail[NP];
+#pragma unroll
+  for (int pr = 0; pr < NP; ++pr) {
+    const int nt = min(2 * NP * cg + 2 * pr + (fkg >> 1), Nt - 1);
+    bias[pr] = !GLU && p.bias && !p.partial ? bias_quad(p, nt, n_in) : u32x2{0, 0};
+    tail[pr] = !GLU && p.tail && !p.partial ? *(const u32x2 *)(C + ((int64_t)nt * 1024 + in) * 2 + p.tail_delta) : u32x2{0, 0};
+  }
 #pragma unroll
   for (int pr = 0; pr < NP; ++pr)
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        part[((pr * 8 + wave) * 8 + h * 4 + i) * 64 + lane] = f32x4v{acc[pr][h][0][i], acc[pr][h][1][i], acc[pr][h][2][i], acc[pr][h][3][i]};
+        part[((pr * 8 + wave) * 8 + hh * 4 + i) * 64 + lane] = f32x4v{acc[pr][hh][0][i], acc[pr][hh][1][i], acc[pr][hh][2][i], acc[pr][hh][3][i]};
   __syncthreads();
-  const int h = tid >> 8, i = (tid >> 6) & 3;
   if constexpr (GLU) {
     // thread t holds the same four outputs of both matrices: out = bf16(bf16(act0(gate)) x bf16(act1(up))), the roundings
     // of the two projections stored by themselves and of the multiply that would read them
     f32x4v s0 = part[tid], s1 = part[4096 + tid];
 #pragma unroll
     for (int w = 1; w < 8; ++w) { s0 += part[w * 512 + tid]; s1 += part[4096 + w * 512 + tid]; }
-    const int nt = 2 * cg + (kg >> 1);
+    const int nt = 2 * cg + (fkg >> 1);
     if (nt >= Nt) return;
-    const int n_in = 16 * (kg & 1) + 4 * i;
-    const int64_t off = (int64_t)nt * 1024 + (h * 2 + (n_in >> 4)) * 256 + q16 * 16 + (n_in & 15);
-    float v0[4], v1[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float x = s0[r], y = s1[r];
-      switch (p.gAct[0]) {
-      case TTM_ACT_GELU: x = apply_act<TTM_ACT_GELU>(x); break;
-      case TTM_ACT_SILU: x = apply_act<TTM_ACT_SILU>(x); break;
-      case TTM_ACT_SIGMOID: x = apply_act<TTM_ACT_SIGMOID>(x); break;
-      case TTM_ACT_RELU: x = apply_act<TTM_ACT_RELU>(x); break;
-      default: break;
-      }
-      switch (p.gAct[1]) {
-      case TTM_ACT_GELU: y = apply_act<TTM_ACT_GELU>(y); break;
-      case TTM_ACT_SILU: y = apply_act<TTM_ACT_SILU>(y); break;
-      case TTM_ACT_SIGMOID: y = apply_act<TTM_ACT_SIGMOID>(y); break;
-      case TTM_ACT_RELU: y = apply_act<TTM_ACT_RELU>(y); break;
-      default: break;
-      }
-      v0[r] = x; v1[r] = y;
-    }
-    const u32x2 g = {pack_bf16(v0[0], v0[1]), pack_bf16(v0[2], v0[3])}, u = {pack_bf16(v1[0], v1[1]), pack_bf16(v1[2], v1[3])};
-    const float z[4] = {__uint_as_float(g.x << 16) * __uint_as_float(u.x << 16), __uint_as_float(g.x & 0xFFFF0000u) * __uint_as_float(u.x & 0xFFFF0000u),
-                        __uint_as_float(g.y << 16) * __uint_as_float(u.y << 16), __uint_as_float(g.y & 0xFFFF0000u) * __uint_as_float(u.y & 0xFFFF0000u)};
-    *(u32x2 *)(C + off * 2) = u32x2{pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3])};
+    float v0[4] = {s0[0], s0[1], s0[2], s0[3]}, v1[4] = {s1[0], s1[1], s1[2], s1[3]};
+    linear_act_rt(p.gAct[0], v0);
+    linear_act_rt(p.gAct[1], v1);
+    *(u32x2 *)(C + ((int64_t)nt * 1024 + in) * 2) = glu_quad(v0, v1);
     return;
   }
 #pragma unroll
   for (int pr = 0; pr < NP; ++pr) {
-  // thread t finishes slot t of the pair's 512: (h, i, lane) = (t >> 8, (t >> 6) & 3, t & 63)
-  f32x4v sum = part[pr * 4096 + tid];
+    f32x4v sum = part[pr * 4096 + tid];
 #pragma unroll
-  for (int w = 1; w < 8; ++w) sum += part[pr * 4096 + w * 512 + tid];
-  const int nt = 2 * NP * cg + 2 * pr + (kg >> 1);
-  if (nt >= Nt) continue;
-  const int n_in = 16 * (kg & 1) + 4 * i;
-  const int64_t off = (int64_t)nt * 1024 + (h * 2 + (n_in >> 4)) * 256 + q16 * 16 + (n_in & 15);
-  if (p.partial) {   // bias, activation and rounding happen in ttm_linear_reduce_k
-    const int64_t per = (int64_t)p.Nt * 1024;   // a group's partial sums are laid out as the concatenation
-    *(f32x4v *)(p.partial + ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * per + (int64_t)tile_base * 1024 + off) = sum;
-    continue;
-  }
-  float bv[4] = {0.f, 0.f, 0.f, 0.f};
-  if (p.bias) {
-    const uint16_t *bp = p.bias_tiled ? p.bias + (int64_t)nt * 1024 + (n_in >> 4) * 256 + (n_in & 15) : p.bias + nt * 32 + n_in;
-    u32x2 raw = *(const u32x2 *)bp;
-    bv[0] = __uint_as_float(raw.x << 16); bv[1] = __uint_as_float(raw.x & 0xFFFF0000u);
-    bv[2] = __uint_as_float(raw.y << 16); bv[3] = __uint_as_float(raw.y & 0xFFFF0000u);
-  }
-  float v[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    float x = sum[r] + bv[r];
-    switch (act) {
-    case TTM_ACT_GELU: x = apply_act<TTM_ACT_GELU>(x); break;
-    case TTM_ACT_SILU: x = apply_act<TTM_ACT_SILU>(x); break;
-    case TTM_ACT_SIGMOID: x = apply_act<TTM_ACT_SIGMOID>(x); break;
-    case TTM_ACT_RELU: x = apply_act<TTM_ACT_RELU>(x); break;
-    default: break;
+    for (int w = 1; w < 8; ++w) sum += part[pr * 4096 + w * 512 + tid];
+    const int nt = 2 * NP * cg + 2 * pr + (fkg >> 1);
+    if (nt >= Nt) continue;
+    const int64_t off = (int64_t)nt * 1024 + in;
+    if (p.partial) {   // bias, activation and rounding happen in ttm_linear_reduce_k
+      const int64_t per = (int64_t)p.Nt * 1024;   // a group's partial sums are laid out as the concatenation
+      *(f32x4v *)(p.partial + ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * per + (int64_t)tile_base * 1024 + off) = sum;
+      continue;
     }
-    v[r] = x;
-  }
-  *(u32x2 *)(C + off * 2) = finish_quad(p, C + off * 2, v);
+    float v[4] = {sum[0] + __uint_as_float(bias[pr].x << 16), sum[1] + __uint_as_float(bias[pr].x & 0xFFFF0000u),
+                  sum[2] + __uint_as_float(bias[pr].y << 16), sum[3] + __uint_as_float(bias[pr].y & 0xFFFF0000u)};
+    linear_act_rt(act, v);
+    *(u32x2 *)(C + off * 2) = finish_quad(p.tail, tail[pr], v);
   }
 }
 

@@ -203,9 +203,18 @@ __global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(Line
   }
   // one row tile at a time: the wavefronts' sums -> LDS as float4 (four consecutive n of one m), then the threads finish the 512
   // slots, (h, i, lane) = (t >> 8, (t >> 6) & 3, t & 63)
+  constexpr int T = THREADS < 512 ? 512 / THREADS : 1;
+  const int n_in = 16 * (kg & 1) + 4 * (wave & 3), nt = 2 * cg + (kg >> 1), ntc = min(nt, Nt - 1);
+  const u32x2 bias = !GLU && p.bias && !p.partial ? bias_quad(p, ntc, n_in) : u32x2{0, 0};
+  const float bv[4] = {__uint_as_float(bias.x << 16), __uint_as_float(bias.x & 0xFFFF0000u), __uint_as_float(bias.y << 16), __uint_as_float(bias.y & 0xFFFF0000u)};
+  auto element = [&](int t) __attribute__((always_inline)) { return (((wave + 4 * t) >> 2) * 2 + (n_in >> 4)) * 256 + q16 * 16 + (n_in & 15); };
 #pragma unroll
   for (int r = 0; r < MT; ++r) {
     if (mt0 + r >= p.Mt) break;      // workgroup-uniform
+    u32x2 tail[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+      tail[t] = !GLU && p.tail && !p.partial ? *(const u32x2 *)(C + (((int64_t)(mt0 + r) * Nt + ntc) * 1024 + element(t)) * 2 + p.tail_delta) : u32x2{0, 0};
     if (r > 0) __syncthreads();
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh)
@@ -214,41 +223,30 @@ __global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(Line
         part[(wave * 8 + hh * 4 + ii) * 64 + lane] = f32x4v{acc[2 * r + hh][0][ii], acc[2 * r + hh][1][ii], acc[2 * r + hh][2][ii], acc[2 * r + hh][3][ii]};
     __syncthreads();
 #pragma unroll
-    for (int t0 = 0; t0 < 512; t0 += THREADS) {
-      const int t = t0 + tid, h = t >> 8, i = (t >> 6) & 3;
-      const int n_in = 16 * (kg & 1) + 4 * i, nt = 2 * cg + (kg >> 1);
+    for (int t = 0; t < T; ++t) {
+      const int in = element(t), slot = t * THREADS + tid;
       if (nt >= Nt) continue;
-      const int in = (h * 2 + (n_in >> 4)) * 256 + q16 * 16 + (n_in & 15);
       f32x4v sums[WN];
 #pragma unroll
       for (int q = 0; q < WN; ++q) {
-        sums[q] = part[q * WK * 512 + t];
+        sums[q] = part[q * WK * 512 + slot];
 #pragma unroll
-        for (int w = 1; w < WK; ++w) sums[q] += part[(q * WK + w) * 512 + t];
+        for (int w = 1; w < WK; ++w) sums[q] += part[(q * WK + w) * 512 + slot];
       }
       uint8_t *c = C + (((int64_t)(mt0 + r) * Nt + nt) * 1024 + in) * 2;
+      float v[4] = {sums[0][0], sums[0][1], sums[0][2], sums[0][3]};
       if constexpr (GLU) {
-        float v0[4], v1[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) { v0[e] = linear_act_rt(p.gAct[0], sums[0][e]); v1[e] = linear_act_rt(p.gAct[1], sums[WN - 1][e]); }
-        const u32x2 g = {pack_bf16(v0[0], v0[1]), pack_bf16(v0[2], v0[3])}, u = {pack_bf16(v1[0], v1[1]), pack_bf16(v1[2], v1[3])};
-        const float z[4] = {__uint_as_float(g.x << 16) * __uint_as_float(u.x << 16), __uint_as_float(g.x & 0xFFFF0000u) * __uint_as_float(u.x & 0xFFFF0000u),
-                            __uint_as_float(g.y << 16) * __uint_as_float(u.y << 16), __uint_as_float(g.y & 0xFFFF0000u) * __uint_as_float(u.y & 0xFFFF0000u)};
-        *(u32x2 *)c = u32x2{pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3])};
+        float v1[4] = {sums[WN - 1][0], sums[WN - 1][1], sums[WN - 1][2], sums[WN - 1][3]};
+        linear_act_rt(p.gAct[0], v);
+        linear_act_rt(p.gAct[1], v1);
+        *(u32x2 *)c = glu_quad(v, v1);
       } else if (p.partial) {   // bias, activation and rounding happen in ttm_linear_reduce_k
         *(f32x4v *)(p.partial + (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * p.Mt + mt0 + r) * p.Nt * 1024 + (int64_t)(tile_base + nt) * 1024 + in) = sums[0];
       } else {
-        float bv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (p.bias) {
-          const uint16_t *bp = p.bias_tiled ? p.bias + (int64_t)nt * 1024 + (n_in >> 4) * 256 + (n_in & 15) : p.bias + nt * 32 + n_in;
-          const u32x2 raw = *(const u32x2 *)bp;
-          bv[0] = __uint_as_float(raw.x << 16); bv[1] = __uint_as_float(raw.x & 0xFFFF0000u);
-          bv[2] = __uint_as_float(raw.y << 16); bv[3] = __uint_as_float(raw.y & 0xFFFF0000u);
-        }
-        float v[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = linear_act_rt(act, sums[0][e] + bv[e]);
-        *(u32x2 *)c = finish_quad(p, c, v);
+        for (int e = 0; e < 4; ++e) v[e] += bv[e];
+        linear_act_rt(act, v);
+        *(u32x2 *)c = finish_quad(p.tail, tail[t], v);
       }
     }
   }
