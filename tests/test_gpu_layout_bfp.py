@@ -73,7 +73,8 @@ def test_tilize_ragged_zero_padded(hip, dev, orc, shape, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.uint16, np.uint8])
-@pytest.mark.parametrize("shape,offset", [((70, 1002), 1), ((3, 33, 129), 3), ((5, 3, 8), 1), ((40, 4, 17), 5), ((1, 1), 1), ((2, 65, 515), 7)])
+@pytest.mark.parametrize("shape,offset", [((70, 1002), 1), ((3, 33, 129), 3), ((5, 3, 8), 1), ((40, 4, 17), 5), ((1, 1), 1), ((2, 65, 515), 7),
+                                          ((2, 1000, 1003), 1), ((2, 1000, 1027), 3)])   # bf16: 4 MiB, and beyond it
 def test_tilize_untilize_at_any_element(hip, dev, orc, shape, dtype, offset):
     """The row-major side starts at any element of its buffer and nothing in front of it or behind it is written; rows narrower
     than a wavefront's access, matrices shorter than a workgroup's."""

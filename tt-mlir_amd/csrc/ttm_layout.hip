@@ -47,7 +47,7 @@ TTM_EXPORT int ttm_copy_kernel(const void *src, void *dst, size_t bytes, void *s
 }
 
 // ------------------------------------------------------------------------------------ direct
-// A wavefront's access covers 8 / ELEM rows x 8 ELEM chunks (more rows of narrower tensors): 8 / ELEM face rows of 16 ELEM bytes are one 128-byte line of the tiled
+// A wavefront's access covers 8 / ELEM rows x 8 ELEM chunks (more rows of narrower tensors, fewer and longer ones of small tensors): 8 / ELEM face rows of 16 ELEM bytes are one 128-byte line of the tiled
 // side, and a row's W chunks are 128 ELEM contiguous bytes of the row-major side, which starts and ends at any element: 16-byte
 // accesses at their own alignment (a lane whose chunk crosses the end of a row takes elements), so nothing outside the tensor is read
 // and nothing is shifted or exchanged.  U accesses per lane.  What bounds it is bytes in flight against the number of
@@ -283,8 +283,14 @@ static int run_layout(const void *src, void *dst, int64_t batch, int64_t rows, i
   }
   const int u = TILIZE && bytes <= ((int64_t)32 << 20) ? 2 : 1;   // accesses per lane
   const int64_t across = ttm_cdiv((TILIZE ? pc : cols) * elem, 16);   // chunks of a row
+  // Chunks of a row that a wavefront's access covers: whole lines of the tiled side, and for tilize up to 4 MiB at least 512 bytes, as these are
+  // mostly uploads whose rows a kernel reads from page-locked memory, while on the device the launch hides the partial lines of the
+  // tiled side (3.6 us either way).  512 against 256 bytes there: a program of [256, 512] x [512, 256] bf16 70.1 -> 68.7 us, [250, 520] x
+  // [520, 264] 71.4 -> 70.9; tilize alone [700, 264] bf16 10.2 -> 9.4, [500, 712] 17.1 -> 16.0, [512, 1024] of one byte 15.0 -> 12.9,
+  // [1024, 1024] bf16 42.9 -> 42.8; 1024 bytes are no better ([256, 512] fp32 12.8 -> 13.9).
+  const int widest = TILIZE && bytes <= ((int64_t)4 << 20) && elem < 4 ? 32 : 8 * elem;
   int lw = 0, wc = 0;
-  while ((1 << lw) < 8 * elem && (1 << lw) < across) ++lw;
+  while ((1 << lw) < widest && (1 << lw) < across) ++lw;
   while (wc < 2 && ((int64_t)1 << (lw + wc)) < across) ++wc;
   const int64_t xu = ttm_cdiv(across, 1 << (lw + wc)), rows_all = batch * (TILIZE ? pr : rows), groups = ttm_cdiv(rows_all, ((64 >> lw) * u) << (2 - wc));
   if (plain && rows_all < INT32_MAX && groups * xu < INT32_MAX) {
