@@ -101,6 +101,14 @@ __device__ __forceinline__ uint32_t xcd_order() {
   return blockIdx.x < n8 * 8 ? (blockIdx.x & 7) * n8 + (blockIdx.x >> 3) : blockIdx.x;
 }
 
+// HIP refuses a grid of 2^32 lanes or more in a dimension: workgroups 0 .. groups - 1 of 256 lanes as launches of up to 2^23 of them,
+// launch(first workgroup, grid).
+template <class F>
+static inline void ttm_launches(int64_t groups, F &&launch) {
+  constexpr int64_t kMost = (int64_t)1 << 23;
+  for (int64_t first = 0; first < groups; first += kMost) launch((uint32_t)first, dim3((unsigned)(groups - first < kMost ? groups - first : kMost)));
+}
+
 __host__ __device__ static inline int64_t ttm_round_up32(int64_t v) { return (v + 31) / 32 * 32; }
 static inline int64_t ttm_cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
