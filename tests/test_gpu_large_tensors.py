@@ -18,7 +18,8 @@ def fill(t, seed):
         p.copy_(torch.randint(1, 256, (p.numel(),), dtype=torch.uint8, device=t.device, generator=torch.Generator(device=t.device).manual_seed(seed + i)))
 
 
-def test_tilize_of_a_row_of_2_31_elements(hip, large):
+def test_tilize_and_untilize_of_a_row_of_2_31_elements(hip, large):
+    """The row's last lanes lie beyond it, at columns that an int no longer holds."""
     cols = 2**31 - 77
     pc = -(-cols // 32) * 32
     x = torch.empty(cols, dtype=torch.uint8, device=large)
@@ -31,6 +32,11 @@ def test_tilize_of_a_row_of_2_31_elements(hip, large):
         row = got[:, 0, :, 0, :].reshape(-1)
         assert torch.equal(row[:want.numel()], want) and not bool(row[want.numel():].any())
         assert not bool(got[:, 1].any()) and not bool(got[:, 0, :, 1:].any())
+    back = torch.full((cols + 64,), 7, dtype=torch.uint8, device=large)
+    hip.call("ttm_untilize", hip.ptr(t), hip.ptr(back), 1, 1, cols, 1, hip.current_stream())
+    for got, want in zip(back[:cols].split(1 << 28), x.split(1 << 28)):
+        assert torch.equal(got, want)
+    assert bool((back[cols:] == 7).all())
 
 
 def test_unpack_of_more_rows_than_a_grid_holds(hip, large):
@@ -48,3 +54,18 @@ def test_unpack_of_more_rows_than_a_grid_holds(hip, large):
         hip.call("ttm_bfp_unpack", hip.ptr(packed[b * matrix:]), hip.BFP4B, hip.ptr(want), hip.BF16, hip.ROW_MAJOR, n, rows, cols, s)
         assert torch.equal(out[b * rows:(b + n) * rows].view(torch.int16), want.view(torch.int16))
     assert bool((out[batch * rows:] == 7).all())
+
+
+def test_unpack_of_a_row_of_2_31_elements(hip, large):
+    cols, part = 2**31 - 77, 1 << 20   # tiles
+    packed = torch.empty(-(-cols // 32) * 576, dtype=torch.uint8, device=large)
+    fill(packed, 3)
+    out = torch.full((cols + 64,), 7, dtype=torch.bfloat16, device=large)
+    s = hip.current_stream()
+    hip.call("ttm_bfp_unpack", hip.ptr(packed), hip.BFP4B, hip.ptr(out), hip.BF16, hip.ROW_MAJOR, 1, 1, cols, s)
+    for tile in range(0, -(-cols // 32), part):
+        n = min(part * 32, cols - tile * 32)
+        want = torch.empty(n, dtype=torch.bfloat16, device=large)
+        hip.call("ttm_bfp_unpack", hip.ptr(packed[tile * 576:]), hip.BFP4B, hip.ptr(want), hip.BF16, hip.ROW_MAJOR, 1, 1, n, s)
+        assert torch.equal(out[tile * 32:tile * 32 + n].view(torch.int16), want.view(torch.int16))
+    assert bool((out[cols:] == 7).all())

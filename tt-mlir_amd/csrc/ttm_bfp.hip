@@ -318,7 +318,7 @@ __global__ __launch_bounds__(256) void ttm_bfp_direct_k(const uint8_t *__restric
   const int chunk = (int)((((bid - by * xu) << wc) + (wave & ((1 << wc) - 1))) << lw) + (lane & ((1 << lw) - 1));
   const uint32_t row0 = ((by << (2 - wc)) + (wave >> wc)) * (64 >> lw) * U + (lane >> lw);   // of the rows of all matrices, padded ones for pack
   const uint32_t per = PACK ? yt * 32 : rows;
-  const int n = cols - chunk * EPT;                        // elements of the row from this chunk on
+  const int n = (int)((uint32_t)cols - (uint32_t)chunk * EPT);   // elements of the row from this chunk on; a lane past a row of almost 2^31 elements goes beyond int
   if (PACK ? chunk >= ct * 2 * ELEM : n <= 0) return;      // a face row is ELEM chunks: its lanes stay or go together
   const int tc = chunk / (2 * ELEM), f = chunk / ELEM & 1, q = chunk % ELEM;
   u32x4 v[U];

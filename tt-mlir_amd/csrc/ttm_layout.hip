@@ -71,7 +71,7 @@ __global__ __launch_bounds__(256) void ttm_tile_direct_k(const uint8_t *__restri
   const int chunk = (int)((((bid - by * xu) << wc) + (wave & ((1 << wc) - 1))) << lw) + (lane & ((1 << lw) - 1));
   const uint32_t row0 = ((by << (2 - wc)) + (wave >> wc)) * (64 >> lw) * U + (lane >> lw);   // of the rows of all matrices, padded ones for tilize
   const uint32_t per = TILIZE ? yt * 32 : rows;
-  const int n = cols - chunk * V;                          // elements of the row from this chunk on
+  const int n = (int)((uint32_t)cols - (uint32_t)chunk * V);   // elements of the row from this chunk on; a lane past a row of almost 2^31 elements goes beyond int
   if (TILIZE ? chunk >= ct * 2 * ELEM : n <= 0) return;
   const int tc = chunk / (2 * ELEM), in = (chunk / ELEM & 1) * (16 * ELEM) + chunk % ELEM;   // tile column, face column and chunk of a face row
   chunk_t v[U];
