@@ -320,6 +320,7 @@ def test_relu_epilogue_keeps_nan(hip, dev, orc, wfmt_name, M, K, N, option, valu
     ("bfp4", 330, 232, 677, "linear_split_k", 2),     # split-K main kernel
     ("bf16", 288, 160, 320, None, 0),                 # register-staged kernel
     ("bfp8", 96, 96, 160, "linear_variant", 1),       # 64-bit-addressed fallback
+    ("bf16", 330, 232, 677, "linear_variant", 1),     # the same, ragged: row and column tiles past the last one
 ])
 def test_linear_with_fused_tail_equals_two_ops(hip, dev, orc, metrics, tail, wfmt_name, M, K, N, option, value):
     """ttm_linear_tail (add / multiply with a second tensor in the epilogue) against ttm_linear followed by the oracle's

@@ -168,12 +168,47 @@ __device__ __forceinline__ void store_w(u32x4 *ldsW, int tid, const WRegs<WF> &r
   }
 }
 
-// bias, activation, bf16, 8-byte stores into the output face rows.  acc[a][b]: n tile a, m tile b of the
-// wavefront; a lane holds m = lane % 32 and n = 8 g + 4 (lane / 32) + r in register g * 4 + r.
-// bias, activation, bf16, and 8-byte stores into the output face rows for a wavefront's NA x MB accumulator tiles;
-// column tiles at or beyond nt_end are left alone
+// bias, activation, bf16, 8-byte stores into the output face rows for a wavefront's NA x MB accumulator tiles.  acc[a][b]: n tile a, m
+// tile b of the wavefront; a lane holds m = lane % 32 and n = 8 g + 4 (lane / 32) + r in register g * 4 + r.  Column tiles at or beyond
+// nt_end are left alone.
+// Without a tail, bias values quad by quad: what 4 x 4 tiles have registers for.  Requested in front of all outputs, 6 to 8 registers
+// spilled and [2048, 4096] x [4096, 4096] bfp8_b took 167.4 us (165.3 this way), [4096, 1024] x [1024, 8192] bf16 100.1 (97.1); with a tail
+// the requests in front win all the same, 184.1 quad by quad and 170.2, 122.1 and 97.5.
+template <int ACT, int NA, int MB>
+__device__ __forceinline__ void linear_epilogue_quads(const LinearArgs &p, uint8_t *C, f32x16 (&acc)[NA][MB], int mtw, int ntw, int nt_end, int lane) {
+  const int m_in = lane & 31;
+#pragma unroll
+  for (int a = 0; a < NA; ++a) {
+    const int nt = ntw + a;
+    if (nt >= nt_end) continue;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int n_in = g * 8 + (lane >> 5) * 4;
+      float bv[4] = {0.f, 0.f, 0.f, 0.f};
+      if (p.bias) {
+        const u32x2 raw = bias_quad(p, nt, n_in);
+        bv[0] = __uint_as_float(raw.x << 16); bv[1] = __uint_as_float(raw.x & 0xFFFF0000u);
+        bv[2] = __uint_as_float(raw.y << 16); bv[3] = __uint_as_float(raw.y & 0xFFFF0000u);
+      }
+#pragma unroll
+      for (int b = 0; b < MB; ++b) {
+        const int mt = mtw + b;
+        if (mt >= p.Mt) continue;
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = apply_act<ACT>(acc[a][b][g * 4 + r] + bv[r]);
+        uint8_t *c = C + (((int64_t)mt * p.Nt + nt) * 1024 + ((m_in >> 4) * 2 + (n_in >> 4)) * 256 + (m_in & 15) * 16 + (n_in & 15)) * 2;
+        *(u32x2 *)c = u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+      }
+    }
+  }
+}
 template <int ACT, int NA, int MB>
 __device__ __forceinline__ void linear_epilogue(const LinearArgs &p, uint8_t *C, f32x16 (&acc)[NA][MB], int mtw, int ntw, int nt_end, int lane) {
+  if (NA * MB > 8 && !p.tail) {
+    linear_epilogue_quads<ACT>(p, C, acc, mtw, ntw, nt_end, lane);
+    return;
+  }
   const int m_in = lane & 31;
   auto offset = [&](int a, int g, int b) __attribute__((always_inline)) {   // clamped to the last tile: tiles beyond it are not stored
     const int n_in = g * 8 + (lane >> 5) * 4, mt = min(mtw + b, p.Mt - 1), nt = min(ntw + a, nt_end - 1);
