@@ -47,11 +47,11 @@ TTM_EXPORT int ttm_copy_kernel(const void *src, void *dst, size_t bytes, void *s
 }
 
 // ------------------------------------------------------------------------------------ direct
-// A wavefront's access covers 8 / ELEM rows x 8 ELEM chunks (more rows of narrower tensors, fewer and longer ones of small tensors): 8 / ELEM face rows of 16 ELEM bytes are one 128-byte line of the tiled
-// side, and a row's W chunks are 128 ELEM contiguous bytes of the row-major side, which starts and ends at any element: 16-byte
-// accesses at their own alignment (a lane whose chunk crosses the end of a row takes elements), so nothing outside the tensor is read
-// and nothing is shifted or exchanged.  U accesses per lane.  What bounds it is bytes in flight against the number of
-// workgroups: two loads per lane are best for tilize up to some 16 MiB, one beyond and for untilize (a store needs no more).
+// A wavefront's access covers 8 / ELEM rows x 8 ELEM chunks (more rows of narrower tensors, fewer and longer ones of small tensors):
+// 8 / ELEM face rows of 16 ELEM bytes are one 128-byte line of the tiled side, and a row's 8 ELEM chunks are 128 ELEM contiguous bytes
+// of the row-major side, which starts and ends at any element: 16-byte accesses at their own alignment (a lane whose chunk crosses the
+// end of a row takes elements), so nothing outside the tensor is read and nothing is shifted or exchanged.  U accesses per lane.  What bounds it is bytes in flight against the number of
+// workgroups: two loads per lane are best for tilize up to 32 MiB, one beyond and for untilize (a store needs no more).
 // Tilize streams its stores past the caches, untilize does not (partial lines at the ends of rows meet in L2).  Against strips of 32
 // rows x 512 bytes through LDS with funnel shifts for odd rows: [3, 1000, 3001] bf16 tilize / untilize 9.0 / 10.6 -> 7.0 / 6.9 us,
 // [4000, 7001] fp32 42.0 / 37.2 -> 39.4 / 35.6, [2, 1266, 771] bf16 4.2 / 5.5 -> 3.1 / 3.2, [7, 33, 9000] fp32 7.7 / 6.2 -> 4.4 / 4.4,
@@ -233,13 +233,16 @@ __global__ __launch_bounds__(256) void ttm_untilize_ragged_k(const uint8_t *__re
   }
 }
 
-// The kernel of a shape.  `bytes` is one side; both together stay in the 256 MB last-level cache up to some 128 MiB each.
-//   aligned whole strips: direct up to there, strips beyond ([2048, 4096] bf16 tilize / untilize 6.6 / 6.5 strips, 6.0 / 6.1 us direct,
-//     [4096, 4096] fp32 21.6 / 22.2, 19.9 / 19.9, [8192, 8192] bf16 41.3 / 42.0, 38.8 / 41.2, fp32 80.6 / 82.2, 87 / 87)
-//   other shapes: tilize direct ([8192, 8191] fp32 93 strips, 88 direct, [3, 4000, 8001] fp32 136, 127); untilize direct up to there
-//     ([4000, 7001] fp32 36.8 strips, 35.1 direct), strips where a strip is mostly real rows and columns beyond ([3, 4096, 8190] bf16
-//     64 strips, 73 direct, [8192, 8191] fp32 78, 96)
-// To page-locked host memory the direct form, whose stores go through L2, is the faster one too ([2048, 8192] bf16 669 -> 631 us).
+// The kernel of a shape, by `bytes`, one side with its padding.  Times in us, tilize / untilize, of the same tensors over and over | of
+// tensors that left the 256 MB last-level cache in between:
+//   whole strips: direct up to 64 MiB, where neither form wins everywhere: [4096, 4096] bf16 direct 10.6 / 11.0 | 14.1 / 14.3, strips
+//     11.8 / 11.2 | 12.5 / 12.4, right behind the kernel that wrote the input 10.5 / 11.2 and 10.9 / 10.7; into page-locked host memory
+//     direct is the faster one ([2048, 4096] bf16 310, strips 355).  Strips beyond: [6144, 8192] bf16 30.7 / 32.4 | 31.5 / 32.4, direct
+//     24.1 / 24.2 | 34.8 / 36.9, [8192, 8192] fp32 79.8 / 82.6 | 79.6 / 82.5, direct 61.3 / 91.2 | 87.9 / 91.3, [12288, 8192] fp32
+//     120 / 123, direct 133 / 139.
+//   other shapes: tilize direct.  Untilize direct up to 160 MiB ([4096, 8160] fp32 37.7 | 52.8, shifted strips 43.2 | 53.3; [10240, 8160]
+//     bf16 53.7 | 59.7, 56.2 | 61.2), shifted strips where a strip is mostly real rows and columns beyond ([8192, 8191] fp32 69.2 | 96.0,
+//     direct 91.1 | 91.6, [2, 8192, 8191] bf16 72.4 | 97.0, 90.9 | 91.2).
 template <bool TILIZE>
 static int run_layout(const void *src, void *dst, int64_t batch, int64_t rows, int64_t cols, int elem,
                       void *stream, const char *who) {
@@ -253,9 +256,10 @@ static int run_layout(const void *src, void *dst, int64_t batch, int64_t rows, i
   const bool aligned = rows == pr && cols == pc && ((uintptr_t)src & 15) == 0 && ((uintptr_t)dst & 15) == 0;
   // whole 16-byte chunks on the tile-order side, whole elements on the other
   const bool plain = pr < INT32_MAX && pc < INT32_MAX && ((uintptr_t)(TILIZE ? dst : src) & 15) == 0 && (uintptr_t)(TILIZE ? src : dst) % elem == 0;
-  const bool large = bytes > ((int64_t)(aligned ? 64 : 160) << 20) && ttm_option(TILIZE ? "tilize_variant" : "untilize_variant") == 0;
+  const bool whole = aligned && cols * elem % 512 == 0;   // strips, all of them
+  const bool large = bytes > ((int64_t)(whole ? 64 : 160) << 20) && ttm_option(TILIZE ? "tilize_variant" : "untilize_variant") == 0;
   const int64_t strips = ttm_cdiv(pc * elem, 512);
-  if (large && aligned && cols * elem % 512 == 0) {
+  if (large && whole) {
     const int64_t blocks = batch * (pr / 32) * strips;
     TTM_REQUIRE(blocks < (1ll << 31), "%s: tensor too large", who);
 #define STRIP(E) \
