@@ -74,7 +74,8 @@ def test_tilize_ragged_zero_padded(hip, dev, orc, shape, dtype):
 
 @pytest.mark.parametrize("dtype", [np.float32, np.uint16, np.uint8])
 @pytest.mark.parametrize("shape,offset", [((70, 1002), 1), ((3, 33, 129), 3), ((5, 3, 8), 1), ((40, 4, 17), 5), ((1, 1), 1), ((2, 65, 515), 7),
-                                          ((2, 1000, 1003), 1), ((2, 1000, 1027), 3)])   # bf16: 4 MiB, and beyond it
+                                          ((2, 1000, 1003), 1), ((2, 1000, 1027), 3),   # bf16: 4 MiB, and beyond it
+                                          ((2, 70, 283), 1), ((2, 70, 570), 3), ((3, 40, 1140), 1)])   # one and two wavefronts side by side
 def test_tilize_untilize_at_any_element(hip, dev, orc, shape, dtype, offset):
     """The row-major side starts at any element of its buffer and nothing in front of it or behind it is written; rows narrower
     than a wavefront's access, matrices shorter than a workgroup's."""
@@ -286,7 +287,7 @@ def test_full_size_properties(hip, dev, orc, fmt):
 @pytest.mark.parametrize("fmt", [8, 4])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("shape,shift", [((1, 1, 1), 0), ((2, 33, 129), 1), ((1, 64, 255), 3), ((3, 31, 257), 0), ((1, 95, 1023), 5), ((2, 40, 300), 2),
-                                         ((1, 32, 512), 1), ((1, 500, 384), 0), ((2, 1100, 2081), 7)])
+                                         ((1, 32, 512), 1), ((1, 500, 384), 0), ((2, 1100, 2081), 7), ((2, 50, 83), 1), ((3, 70, 167), 5)])
 def test_bfp_ragged(hip, dev, orc, fmt, dtype, shape, shift):
     """Rows that start and end anywhere, on buffers that start at any element: packed bytes and read-back against the oracle
     and the generic kernel (random bit patterns: infinities, NaN and subnormal numbers among them), nothing written around them."""

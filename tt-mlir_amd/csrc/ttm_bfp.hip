@@ -576,8 +576,7 @@ static int run_bfp(const void *src, void *dst, int fmt, int dtype, int layout, i
   // bfp4_b 6.2 us by chunks, 4.8).
   const int64_t across = ttm_cdiv((PACK ? pc : cols) * elem, 16), rows_all = batch * (PACK ? pr : rows);   // chunks of a row; rows of all matrices
   const int lw = across > 4 ? 3 : 2, u = PACK && batch * rows * cols * elem > ((int64_t)16 << 20) ? 2 : 1;
-  int wc = 0;
-  while (wc < 2 && ((int64_t)1 << (lw + wc)) < across) ++wc;
+  const int wc = ttm_wavefronts_across(across, lw);
   const int64_t xu = ttm_cdiv(across, 1 << (lw + wc)), groups = ttm_cdiv(rows_all, ((64 >> lw) * u) << (2 - wc));
   if (plain && (!PACK || rows >= 24 || variant == 2) && pc < INT32_MAX && rows_all < INT32_MAX && groups * xu < INT32_MAX) {
 #define DIRECT(Wv, EL, U)                                                                                                                       \

@@ -293,9 +293,9 @@ static int run_layout(const void *src, void *dst, int64_t batch, int64_t rows, i
   // [520, 264] 71.4 -> 70.9; tilize alone [700, 264] bf16 10.2 -> 9.4, [500, 712] 17.1 -> 16.0, [512, 1024] of one byte 15.0 -> 12.9,
   // [1024, 1024] bf16 42.9 -> 42.8; 1024 bytes are no better ([256, 512] fp32 12.8 -> 13.9).
   const int widest = TILIZE && bytes <= ((int64_t)4 << 20) && elem < 4 ? 32 : 8 * elem;
-  int lw = 0, wc = 0;
+  int lw = 0;
   while ((1 << lw) < widest && (1 << lw) < across) ++lw;
-  while (wc < 2 && ((int64_t)1 << (lw + wc)) < across) ++wc;
+  const int wc = ttm_wavefronts_across(across, lw);
   const int64_t xu = ttm_cdiv(across, 1 << (lw + wc)), rows_all = batch * (TILIZE ? pr : rows), groups = ttm_cdiv(rows_all, ((64 >> lw) * u) << (2 - wc));
   if (plain && rows_all < INT32_MAX && groups * xu < INT32_MAX) {
 #define DIRECT(E, U)                                                                                                                            \
