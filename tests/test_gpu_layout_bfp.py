@@ -287,7 +287,7 @@ def test_full_size_properties(hip, dev, orc, fmt):
 @pytest.mark.parametrize("fmt", [8, 4])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("shape,shift", [((1, 1, 1), 0), ((2, 33, 129), 1), ((1, 64, 255), 3), ((3, 31, 257), 0), ((1, 95, 1023), 5), ((2, 40, 300), 2),
-                                         ((1, 32, 512), 1), ((1, 500, 384), 0), ((2, 1100, 2081), 7), ((2, 50, 83), 1), ((3, 70, 167), 5)])
+                                         ((1, 32, 512), 1), ((1, 500, 384), 0), ((2, 1100, 2081), 7), ((2, 50, 83), 1), ((3, 70, 167), 5), ((2, 90, 16), 1), ((1, 70, 17), 3)])
 def test_bfp_ragged(hip, dev, orc, fmt, dtype, shape, shift):
     """Rows that start and end anywhere, on buffers that start at any element: packed bytes and read-back against the oracle
     and the generic kernel (random bit patterns: infinities, NaN and subnormal numbers among them), nothing written around them."""
@@ -304,7 +304,7 @@ def test_bfp_ragged(hip, dev, orc, fmt, dtype, shape, shift):
         src = torch.zeros(n + 2 * pad, dtype=dtype, device=dev)
         src[pad + shift:pad + shift + n] = x.to(dev)
         got = {}
-        for variant in (2, 1):
+        for variant in (0, 2, 1):
             hip.set_option("pack_variant", variant)
             hip.set_option("unpack_variant", variant)
             try:
@@ -319,6 +319,7 @@ def test_bfp_ragged(hip, dev, orc, fmt, dtype, shape, shift):
             got[variant] = p.cpu(), back.cpu()
         (p, back), (gp, gback) = got[2], got[1]
         assert torch.equal(p, gp) and torch.equal(back, gback)
+        assert torch.equal(got[0][0], gp) and torch.equal(got[0][1], gback)
         assert (p[packed:] == 9).all() and (back[:pad + shift] == 5).all() and (back[pad + shift + n:] == 5).all()
         if oracle:
             want = orc.bfp_pack(x.float().numpy().reshape(shape), fmt)

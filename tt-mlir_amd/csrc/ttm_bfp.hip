@@ -572,13 +572,14 @@ static int run_bfp(const void *src, void *dst, int fmt, int dtype, int layout, i
     TTM_LAUNCH_CHECK();
     return TTM_OK;
   }
-  // Chunk by chunk: rows of any width and start.  Matrices that are mostly padding are packed a tile per workgroup ([1000, 3, 100] fp32
-  // bfp4_b 6.2 us by chunks, 4.8).
+  // Chunk by chunk: rows of any width and start.  Matrices that are mostly padding are packed a tile per workgroup: few rows ([1000, 3, 100]
+  // fp32 bfp4_b 6.2 us by chunks, 4.8), and fp32 of up to half a tile's columns ([64, 5093, 4] bfp8_b 11.9 by chunks, 9.2, [64, 5093, 16] 10.9
+  // and 9.5, out of cache 11.6 and 11.0; [64, 5093, 25] 13.6 and 13.7; bf16 [64, 5093, 4] 9.1 and 9.9).
   const int64_t across = ttm_cdiv((PACK ? pc : cols) * elem, 16), rows_all = batch * (PACK ? pr : rows);   // chunks of a row; rows of all matrices
   const int lw = across > 4 ? 3 : 2, u = PACK && batch * rows * cols * elem > ((int64_t)16 << 20) ? 2 : 1;
   const int wc = ttm_wavefronts_across(across, lw);
   const int64_t xu = ttm_cdiv(across, 1 << (lw + wc)), groups = ttm_cdiv(rows_all, ((64 >> lw) * u) << (2 - wc));
-  if (plain && (!PACK || rows >= 24 || variant == 2) && pc < INT32_MAX && rows_all < INT32_MAX && groups * xu < INT32_MAX) {
+  if (plain && (!PACK || (rows >= 24 && (bf16 || cols > 16)) || variant == 2) && pc < INT32_MAX && rows_all < INT32_MAX && groups * xu < INT32_MAX) {
 #define DIRECT(Wv, EL, U)                                                                                                                       \
   ttm_launches(groups * xu, [&](uint32_t first, dim3 grid) {                                                                                    \
     hipLaunchKernelGGL((ttm_bfp_direct_k<Wv, EL, U, PACK>), grid, dim3(256), 0, s, (const uint8_t *)src, (uint8_t *)dst, (int)rows, (int)cols,  \
