@@ -118,6 +118,42 @@ def test_bfp_large_tensors_take_strips(hip, dev, fmt, dtype):
     assert torch.equal(got[0][0], got[2][0]) and torch.equal(got[0][1], got[2][1])
 
 
+@pytest.mark.parametrize("fmt", [8, 4])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_bfp_of_host_memory(hip, dev, fmt, dtype):
+    """Either side in page-locked host memory, at a size from which that is packed and unpacked by strips: what the generic kernel makes of
+    the same bits on the device, and nothing around it."""
+    hfmt, code = (hip.BFP8B if fmt == 8 else hip.BFP4B), (hip.F32 if dtype == torch.float32 else hip.BF16)
+    b, r, c = shape = (2, 1100, 2081)
+    ints = torch.int32 if dtype == torch.float32 else torch.int16
+    n, at, s = b * r * c, 3, hip.current_stream()
+    bits = torch.randint(-2**15, 2**15 - 1, (n,), generator=torch.Generator().manual_seed(n)).to(ints)
+    x = (bits << 16 if ints == torch.int32 else bits).to(dev)
+    hip.set_option("pack_variant", 1)
+    hip.set_option("unpack_variant", 1)
+    try:
+        packed = pack_gpu(hip, dev, x.view(dtype), hfmt, shape, code, hip.ROW_MAJOR)
+        back = unpack_gpu(hip, dev, packed, hfmt, shape, code, hip.ROW_MAJOR).view(ints).reshape(-1)
+        torch.cuda.synchronize()
+    finally:
+        hip.set_option("pack_variant", 0)
+        hip.set_option("unpack_variant", 0)
+    hx, hp = torch.full((n + 32,), 5, dtype=ints).pin_memory(), torch.full((packed.numel() + 32,), 9, dtype=torch.uint8).pin_memory()
+    hx[at:at + n] = x.cpu()
+    got = torch.zeros_like(packed)
+    hip.call("ttm_bfp_pack", hip.ptr(hx[at:]), code, hip.ROW_MAJOR, hip.ptr(got), hfmt, b, r, c, s)
+    hip.call("ttm_bfp_pack", hip.ptr(x), code, hip.ROW_MAJOR, hip.ptr(hp), hfmt, b, r, c, s)
+    torch.cuda.synchronize()
+    assert torch.equal(got, packed) and torch.equal(hp[:packed.numel()], packed.cpu()) and bool((hp[packed.numel():] == 9).all())
+    dx = torch.full((n + 32,), 5, dtype=ints, device=dev)
+    hip.call("ttm_bfp_unpack", hip.ptr(hp), hfmt, hip.ptr(dx[at:]), code, hip.ROW_MAJOR, b, r, c, s)
+    hx.fill_(5)
+    hip.call("ttm_bfp_unpack", hip.ptr(packed), hfmt, hip.ptr(hx[at:]), code, hip.ROW_MAJOR, b, r, c, s)
+    torch.cuda.synchronize()
+    for o in (dx.cpu(), hx):
+        assert torch.equal(o[at:at + n], back.cpu()) and bool((o[:at] == 5).all()) and bool((o[at + n:] == 5).all())
+
+
 @pytest.mark.parametrize("rows,cols", [(41000, 2051), (41024, 2048)])
 def test_large_tensors_take_strips(hip, dev, rows, cols):
     """Above the size up to which every shape goes chunk by chunk: whole strips and rows that start anywhere, against torch."""

@@ -15,7 +15,7 @@
 // fully contiguous 512-byte row segments and permuted through a padded LDS image, exactly like
 // the tilize kernel; the packed side of a strip is one contiguous run of tiles.
 // Row-major shapes whose rows are not a multiple of 512 bytes, or that need zero padding, are moved chunk by chunk at any
-// address without LDS; tile-ordered tensors that are no whole number of strips take a generic kernel with one face row quad
+// address without LDS, large ones and those of host memory by strips that start anywhere; tile-ordered tensors that are no whole number of strips take a generic kernel with one face row quad
 // per lane group and bounds-checked scalar accesses.
 #include <type_traits>
 
@@ -383,8 +383,8 @@ __global__ __launch_bounds__(256) void ttm_bfp_direct_k(const uint8_t *__restric
 }
 
 // ------------------------------------------------------------------------------------ ragged shapes, large
-// Where the two sides no longer meet in the last-level cache: the row-major side in strips of 32 rows x 512 bytes that start and end
-// anywhere, moved in shifted aligned chunks (ttm_ragged.h), the packed side as in the strip kernel.  HBM-bound.
+// Where the two sides no longer meet in the last-level cache, or one is host memory: the row-major side in strips of 32 rows x 512 bytes
+// that start and end anywhere, moved in shifted aligned chunks (ttm_ragged.h), the packed side as in the strip kernel.  HBM-bound.
 template <int W, int ELEM, bool PACK>
 __global__ __launch_bounds__(256) void ttm_bfp_ragged_k(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int rows, int cols, int strips) {
   constexpr int EPT = 16 / ELEM, CPT = 64 * ELEM, TPS = 16 / ELEM;   // elements per chunk, chunks per tile, tiles per strip
@@ -497,6 +497,14 @@ __global__ __launch_bounds__(256) void ttm_bfp_generic_k(const void *__restrict_
 
 TTM_EXPORT int64_t ttm_bfp_tile_bytes(int fmt) { return fmt == TTM_BFP8B ? 1088 : (fmt == TTM_BFP4B ? 576 : -1); }
 
+// Page-locked host memory or not: 0.1 us.  A pointer that HIP does not know counts as device memory.
+static bool on_host(const void *p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeHost;
+  (void)hipGetLastError();
+  return false;
+}
+
 template <bool PACK>
 static int run_bfp(const void *src, void *dst, int fmt, int dtype, int layout, int64_t batch, int64_t rows,
                    int64_t cols, void *stream, const char *who) {
@@ -555,19 +563,23 @@ static int run_bfp(const void *src, void *dst, int fmt, int dtype, int layout, i
   // 8190] bf16 72 / 58, [3, 4096, 4000] bf16 30 to 36 / 32, [4096, 8190] bf16 18 / 24),
   // packing fp32 above 96 MiB ([3, 4096, 4000] 48 / 44, [2, 4096, 4000] 34 / 31, [3, 4000, 8001] 88 / 86; [4096, 4000] 16.1 / 17.4),
   // packing bf16 never ([3, 4096, 8190] 59 / 68).
+  // To and from page-locked host memory, where every piece of a line is an access of its own, strips from 2304 tiles packed, 1536 unpacked
+  // on (us, chunk by chunk / strips: pack [1500, 2001] fp32 bfp8_b from the host 261 / 244, to it 82 / 74, [4096, 4000] bf16 752 / 678,
+  // 435 / 371; unpack from the host [2, 700, 1500] bf16 bfp8_b 66 / 57, [2000, 3001] bfp4_b 89 / 84).  Chunk by chunk is the better one for
+  // bfp4_b packed to the host (190 / 205), unpacked from it to fp32 (193 / 206) and for unpacking to it (165 / 168).
   const int64_t strips = ttm_cdiv(pc * elem, 512);
-  if (plain && variant == 0 && !(PACK && bf16) && batch * pr * pc * elem > ((int64_t)(PACK ? 96 : bf16 ? 80 : 160) << 20) && pr * pc < ((int64_t)1 << 31) &&
-      rows >= 24 && cols * elem * 4 >= strips * 512 * 3) {
+  const bool large = !(PACK && bf16) && batch * pr * pc * elem > ((int64_t)(PACK ? 96 : bf16 ? 80 : 160) << 20);
+  const auto host_side = [&] {
+    if (ntiles < (PACK ? 2304 : 1536)) return false;
+    if (PACK) return on_host(src) || (fmt == TTM_BFP8B && on_host(dst));
+    return (fmt == TTM_BFP8B || bf16) && on_host(src);
+  };
+  if (plain && variant == 0 && pr * pc < ((int64_t)1 << 31) && rows >= 24 && cols * elem * 4 >= strips * 512 * 3 && (large || host_side())) {
     const dim3 grid((unsigned)(strips * yt), (unsigned)batch);
 #define RAGGED(Wv, EL) \
   hipLaunchKernelGGL((ttm_bfp_ragged_k<Wv, EL, PACK>), grid, dim3(256), 0, s, (const uint8_t *)src, (uint8_t *)dst, (int)rows, (int)cols, (int)strips)
-    if constexpr (PACK) {
-      if (fmt == TTM_BFP8B) RAGGED(7, 4);
-      else RAGGED(3, 4);
-    } else {
-      if (fmt == TTM_BFP8B) { if (bf16) RAGGED(7, 2); else RAGGED(7, 4); }
-      else { if (bf16) RAGGED(3, 2); else RAGGED(3, 4); }
-    }
+    if (fmt == TTM_BFP8B) { if (bf16) RAGGED(7, 2); else RAGGED(7, 4); }
+    else { if (bf16) RAGGED(3, 2); else RAGGED(3, 4); }
 #undef RAGGED
     TTM_LAUNCH_CHECK();
     return TTM_OK;
