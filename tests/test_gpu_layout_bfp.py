@@ -13,6 +13,16 @@ NP2T = {np.dtype(np.float32): torch.float32, np.dtype(np.uint16): torch.int16, n
         np.dtype(np.int32): torch.int32}
 
 
+@pytest.fixture(autouse=True)
+def by_the_rule(request):
+    """Every test leaves the kernel choice to the rules, whatever it sets and however it ends."""
+    h = request.getfixturevalue("hip") if "hip" in request.fixturenames else None
+    yield
+    if h is not None:
+        for option in ("tilize_variant", "untilize_variant", "pack_variant", "unpack_variant"):
+            h.set_option(option, 0)
+
+
 def to_dev(x, dev):
     return torch.from_numpy(x.view(np.int16) if x.dtype == np.uint16 else x).to(dev)
 
@@ -29,7 +39,7 @@ def run_tilize(hip, dev, x, variant=0, untilize_shape=None):
     return out
 
 
-@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("variant", [0, 1, 2])
 @pytest.mark.parametrize("shape,dtype", [((256, 512), np.uint16), ((512, 256), np.uint16), ((64, 128), np.float32),
                                          ((3, 64, 256), np.float32), ((2, 2, 32, 32), np.uint8),
                                          ((96, 1536), np.uint8), ((1024, 1024), np.float32)])
@@ -76,13 +86,16 @@ def test_tilize_ragged_zero_padded(hip, dev, orc, shape, dtype):
 @pytest.mark.parametrize("shape,offset", [((70, 1002), 1), ((3, 33, 129), 3), ((5, 3, 8), 1), ((40, 4, 17), 5), ((1, 1), 1), ((2, 65, 515), 7),
                                           ((2, 1000, 1003), 1), ((2, 1000, 1027), 3),   # bf16: 4 MiB, and beyond it
                                           ((2, 70, 283), 1), ((2, 70, 570), 3), ((3, 40, 1140), 1)])   # one and two wavefronts side by side
-def test_tilize_untilize_at_any_element(hip, dev, orc, shape, dtype, offset):
-    """The row-major side starts at any element of its buffer and nothing in front of it or behind it is written; rows narrower
-    than a wavefront's access, matrices shorter than a workgroup's."""
+@pytest.mark.parametrize("variant", [0, 2])
+def test_tilize_untilize_at_any_element(hip, dev, orc, shape, dtype, offset, variant):
+    """Chunk by chunk, and untilized by strips: the row-major side starts at any element of its buffer and nothing in front of it or
+    behind it is written; rows narrower than a wavefront's access, matrices shorter than a workgroup's."""
     rng = np.random.default_rng(2)
     x = rng.standard_normal(shape).astype(np.float32) if dtype == np.float32 else rng.integers(1, 250, shape).astype(dtype)
     n = x.size
     b, r, c = orc._split3(shape)
+    hip.set_option("tilize_variant", variant)
+    hip.set_option("untilize_variant", variant)
     buf = torch.full((n + 64,), 7, dtype=NP2T[np.dtype(dtype)], device=dev)
     rm = buf[offset:offset + n]
     rm.copy_(to_dev(x, dev).reshape(-1))
@@ -97,16 +110,25 @@ def test_tilize_untilize_at_any_element(hip, dev, orc, shape, dtype, offset):
     assert np.all(got[:offset] == seven) and np.all(got[offset + n:] == seven)
 
 
+def test_untilize_by_strips_of_more_matrices_than_a_grid_has_rows(hip, dev):
+    batch, r, c = 65600, 3, 5
+    t = torch.randint(0, 255, (batch, 2, 2, 16, 16), dtype=torch.uint8, device=dev)
+    out = torch.full((batch * r * c + 64,), 7, dtype=torch.uint8, device=dev)
+    hip.set_option("untilize_variant", 2)
+    hip.call("ttm_untilize", hip.ptr(t), hip.ptr(out), batch, r, c, 1, hip.current_stream())
+    assert torch.equal(out[:batch * r * c].view(batch, r, c), t[:, 0, 0, :r, :c]) and bool((out[batch * r * c:] == 7).all())
+
+
 @pytest.mark.parametrize("fmt", [8, 4])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-def test_bfp_large_tensors_take_strips(hip, dev, fmt, dtype):
-    """Above the size up to which odd shapes go chunk by chunk, packed and unpacked by strips: the same bytes and values."""
+def test_bfp_large_tensors(hip, dev, fmt, dtype):
+    """Above the size up to which odd shapes go chunk by chunk (bf16 packs at any): what the generic kernel packs and unpacks."""
     hfmt, code = (hip.BFP8B if fmt == 8 else hip.BFP4B), (hip.F32 if dtype == torch.float32 else hip.BF16)
     shape = (1, 20500 if dtype == torch.float32 else 41000, 2051)
     assert shape[1] * shape[2] * dtype.itemsize > 160 << 20
     x = torch.randn(shape, device=dev, generator=torch.Generator(device=dev).manual_seed(4)).to(dtype)
     got = {}
-    for variant in (0, 2):
+    for variant in (0, 1):
         hip.set_option("pack_variant", variant)
         hip.set_option("unpack_variant", variant)
         try:
@@ -115,7 +137,7 @@ def test_bfp_large_tensors_take_strips(hip, dev, fmt, dtype):
         finally:
             hip.set_option("pack_variant", 0)
             hip.set_option("unpack_variant", 0)
-    assert torch.equal(got[0][0], got[2][0]) and torch.equal(got[0][1], got[2][1])
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
 @pytest.mark.parametrize("fmt", [8, 4])
@@ -325,8 +347,8 @@ def test_full_size_properties(hip, dev, orc, fmt):
 @pytest.mark.parametrize("shape,shift", [((1, 1, 1), 0), ((2, 33, 129), 1), ((1, 64, 255), 3), ((3, 31, 257), 0), ((1, 95, 1023), 5), ((2, 40, 300), 2),
                                          ((1, 32, 512), 1), ((1, 500, 384), 0), ((2, 1100, 2081), 7), ((2, 50, 83), 1), ((3, 70, 167), 5), ((2, 90, 16), 1), ((1, 70, 17), 3)])
 def test_bfp_ragged(hip, dev, orc, fmt, dtype, shape, shift):
-    """Rows that start and end anywhere, on buffers that start at any element: packed bytes and read-back against the oracle
-    and the generic kernel (random bit patterns: infinities, NaN and subnormal numbers among them), nothing written around them."""
+    """Rows that start and end anywhere, on buffers that start at any element: packed bytes and read-back of the rule's choice, the chunk
+    kernel and the strips against the generic kernel, and of that against the oracle (random bit patterns: infinities, NaN and subnormal numbers among them), nothing written around them."""
     hfmt, code = (hip.BFP8B if fmt == 8 else hip.BFP4B), (hip.F32 if dtype == torch.float32 else hip.BF16)
     b, r, c = shape
     n, pad, s = b * r * c, 64, hip.current_stream()
@@ -340,7 +362,7 @@ def test_bfp_ragged(hip, dev, orc, fmt, dtype, shape, shift):
         src = torch.zeros(n + 2 * pad, dtype=dtype, device=dev)
         src[pad + shift:pad + shift + n] = x.to(dev)
         got = {}
-        for variant in (0, 2, 1):
+        for variant in (0, 1, 2, 3):
             hip.set_option("pack_variant", variant)
             hip.set_option("unpack_variant", variant)
             try:
@@ -353,9 +375,9 @@ def test_bfp_ragged(hip, dev, orc, fmt, dtype, shape, shift):
                 hip.set_option("pack_variant", 0)
                 hip.set_option("unpack_variant", 0)
             got[variant] = p.cpu(), back.cpu()
-        (p, back), (gp, gback) = got[2], got[1]
-        assert torch.equal(p, gp) and torch.equal(back, gback)
-        assert torch.equal(got[0][0], gp) and torch.equal(got[0][1], gback)
+        p, back = got[1]
+        for variant in (0, 2, 3):
+            assert torch.equal(got[variant][0], p) and torch.equal(got[variant][1], back), variant
         assert (p[packed:] == 9).all() and (back[:pad + shift] == 5).all() and (back[pad + shift + n:] == 5).all()
         if oracle:
             want = orc.bfp_pack(x.float().numpy().reshape(shape), fmt)

@@ -526,8 +526,8 @@ static int run_bfp(const void *src, void *dst, int fmt, int dtype, int layout, i
   const bool padded = rm && (rows != pr || cols != pc);
   hipStream_t s = (hipStream_t)stream;
   const int tiles_per_wg = 16 / elem;
-  const int variant = ttm_option(PACK ? "pack_variant" : "unpack_variant");   // 0 by the rules below, 1 generic, 2 chunk by chunk
-  bool strip = aligned && !padded && variant == 0;
+  const int variant = ttm_option(PACK ? "pack_variant" : "unpack_variant");   // 0 by the rules below, 1 generic, 2 chunk by chunk, 3 strips of any size
+  bool strip = aligned && !padded && (variant == 0 || variant == 3);
   int64_t strips_per_row = 0, blocks = 0;
   if (strip) {
     if (rm) {
@@ -574,7 +574,8 @@ static int run_bfp(const void *src, void *dst, int fmt, int dtype, int layout, i
     if (PACK) return on_host(src) || (fmt == TTM_BFP8B && on_host(dst));
     return (fmt == TTM_BFP8B || bf16) && on_host(src);
   };
-  if (plain && variant == 0 && pr * pc < ((int64_t)1 << 31) && rows >= 24 && cols * elem * 4 >= strips * 512 * 3 && (large || host_side())) {
+  if (plain && pr * pc < ((int64_t)1 << 31) &&
+      (variant == 3 || (variant == 0 && rows >= 24 && cols * elem * 4 >= strips * 512 * 3 && (large || host_side())))) {
     const dim3 grid((unsigned)(strips * yt), (unsigned)batch);
 #define RAGGED(Wv, EL) \
   hipLaunchKernelGGL((ttm_bfp_ragged_k<Wv, EL, PACK>), grid, dim3(256), 0, s, (const uint8_t *)src, (uint8_t *)dst, (int)rows, (int)cols, (int)strips)

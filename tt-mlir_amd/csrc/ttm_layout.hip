@@ -7,7 +7,7 @@
 //   strips: a workgroup owns a strip of 32 rows x 512 bytes (16/elem tiles).  Global reads and writes are both contiguous (512 B
 //           per row segment on the row-major side, 16 KiB on the tiled side); the face permutation happens between a padded LDS
 //           image and registers.  Tensors that pass through the last-level cache.
-// ttm_set_option("tilize_variant" / "untilize_variant"): 0 by the rule, 1 direct.
+// ttm_set_option("tilize_variant" / "untilize_variant"): 0 by the rule, 1 direct, 2 strips of any size where a strip kernel takes the shape.
 #include "ttm_common.h"
 #include "ttm_ragged.h"
 
@@ -257,7 +257,8 @@ static int run_layout(const void *src, void *dst, int64_t batch, int64_t rows, i
   // whole 16-byte chunks on the tile-order side, whole elements on the other
   const bool plain = pr < INT32_MAX && pc < INT32_MAX && ((uintptr_t)(TILIZE ? dst : src) & 15) == 0 && (uintptr_t)(TILIZE ? src : dst) % elem == 0;
   const bool whole = aligned && cols * elem % 512 == 0;   // strips, all of them
-  const bool large = bytes > ((int64_t)(whole ? 64 : 160) << 20) && ttm_option(TILIZE ? "tilize_variant" : "untilize_variant") == 0;
+  const int variant = ttm_option(TILIZE ? "tilize_variant" : "untilize_variant");
+  const bool large = variant == 2 || (variant == 0 && bytes > ((int64_t)(whole ? 64 : 160) << 20));
   const int64_t strips = ttm_cdiv(pc * elem, 512);
   if (large && whole) {
     const int64_t blocks = batch * (pr / 32) * strips;
@@ -273,7 +274,7 @@ static int run_layout(const void *src, void *dst, int64_t batch, int64_t rows, i
     return TTM_OK;
   }
   if constexpr (!TILIZE) {
-    if (large && plain && pr * pc < ((int64_t)1 << 31) && rows >= 24 && cols * elem * 4 >= strips * 512 * 3) {
+    if (large && plain && pr * pc < ((int64_t)1 << 31) && (variant == 2 || (rows >= 24 && cols * elem * 4 >= strips * 512 * 3))) {
       const dim3 grid((unsigned)(strips * (pr / 32)), (unsigned)(batch > 65535 ? 65535 : batch));
 #define RAGGED(E) \
   hipLaunchKernelGGL((ttm_untilize_ragged_k<E>), grid, dim3(256), 0, s, (const uint8_t *)src, (uint8_t *)dst, (int)rows, (int)cols, (int)strips, batch)
