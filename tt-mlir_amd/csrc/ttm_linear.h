@@ -150,16 +150,7 @@ __device__ __forceinline__ uint32_t pack_hi(float a, float b) {
   return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
 
-__device__ __forceinline__ float linear_act_rt(int act, float x) {
-  switch (act) {
-  case TTM_ACT_GELU: return apply_act<TTM_ACT_GELU>(x);
-  case TTM_ACT_SILU: return apply_act<TTM_ACT_SILU>(x);
-  case TTM_ACT_SIGMOID: return apply_act<TTM_ACT_SIGMOID>(x);
-  case TTM_ACT_RELU: return apply_act<TTM_ACT_RELU>(x);
-  default: return x;
-  }
-}
-// N values at once: the branches of a switch per value took longer than summing the wavefronts' shares of it
+// The activation of N values at once: the branches of a switch per value took longer than summing the wavefronts' shares of it
 template <int N>
 __device__ __forceinline__ void linear_act_rt(int act, float (&v)[N]) {
   auto all = [&](auto a) __attribute__((always_inline)) {

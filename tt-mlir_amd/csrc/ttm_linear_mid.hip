@@ -203,7 +203,8 @@ __global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(Line
   }
   // one row tile at a time: the wavefronts' sums -> LDS as float4 (four consecutive n of one m), then the threads finish the 512
   // slots, (h, i, lane) = (t >> 8, (t >> 6) & 3, t & 63)
-  constexpr int T = THREADS < 512 ? 512 / THREADS : 1;
+  static_assert(THREADS == 256 || THREADS == 512, "element() counts four wavefronts per pass");
+  constexpr int T = 512 / THREADS;
   const int n_in = 16 * (kg & 1) + 4 * (wave & 3), nt = 2 * cg + (kg >> 1), ntc = min(nt, Nt - 1);
   const u32x2 bias = !GLU && p.bias && !p.partial ? bias_quad(p, ntc, n_in) : u32x2{0, 0};
   const float bv[4] = {__uint_as_float(bias.x << 16), __uint_as_float(bias.x & 0xFFFF0000u), __uint_as_float(bias.y << 16), __uint_as_float(bias.y & 0xFFFF0000u)};
