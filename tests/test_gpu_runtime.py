@@ -83,6 +83,18 @@ def test_to_layout_round_trip(device, orc, shape, dtype):
     assert not loop_in.is_allocated() and not r3.get_retain()
 
 
+@pytest.mark.parametrize("shape", [(3, 33, 77), (1, 65), (2009, 463)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.uint8])
+def test_rows_of_any_width_change_layout_on_the_way(device, orc, shape, dtype):
+    """Tilized while they are uploaded and untilized while they are read back, in one launch each: rows that start at any element."""
+    x = torch.randint(1, 120, shape, generator=torch.Generator().manual_seed(5)).to(dtype)
+    bits = x.view(torch.int16).numpy().view(np.uint16) if dtype == torch.bfloat16 else x.numpy()
+    h = rt.from_torch(x)
+    d = rt.to_layout(h, device, rt.Layout(ST.Device, TL.Tile, h.layout.dtype), retain=True)
+    assert np.array_equal(rt.to_numpy(rt.to_host(d, untilize=False)[0]).view(np.uint8).reshape(-1), orc.tilize(bits).view(np.uint8).reshape(-1))
+    assert np.array_equal(rt.to_numpy(rt.to_host(d, untilize=True)[0]).reshape(shape), bits)
+
+
 def test_c3_linear_program_and_const_eval_cache(device, orc, metrics):
     M, K, N = 96, 256, 320
     a, w, bias = datagen.c3_linear(M, K, N, seed=2)
