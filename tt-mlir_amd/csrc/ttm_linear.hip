@@ -336,34 +336,40 @@ __device__ __forceinline__ void linear_epilogue_act(const LinearArgs &p, uint8_t
 
 // The same three steps for accumulators of v_mfma_f32_16x16x32_bf16: acc[u][v] is the 16 (n) x 16 (m) tile u of the
 // wavefront's columns and v of its rows; a lane holds m = lane % 16 and n = 4 (lane / 16) + r in register r.
-template <int ACT, int NU, int NV>
+// TAIL: the tail operands are requested two column halves ahead of the outputs ([2048, 4096] x [4096, 14336] bfp8_b 237.9 us one by one,
+// 214.0 ahead).  A kernel of its own for products without one: one code for both, with the addresses clamped, took 44.9 us for [1665, 376] x
+// [376, 12055] bfp8_b with SiLU and 34.4 without, where these take 43.0 and 33.4.
+template <int ACT, bool TAIL, int NU, int NV>
 __device__ __forceinline__ void linear_epilogue16(const LinearArgs &p, uint8_t *C, f32x4 (&acc)[NU][NV], int mtw, int ntw, int nt_end, int lane) {
   const int m16 = lane & 15, n4 = (lane >> 4) * 4;
   static_assert(NU % 2 == 0, "whole column tiles");
-  auto offset = [&](int u, int v) __attribute__((always_inline)) {   // clamped to the last tile: tiles beyond it are not stored
-    const int n_in = (u & 1) * 16 + n4, m_in = (v & 1) * 16 + m16, mt = min(mtw + (v >> 1), p.Mt - 1), nt = min(ntw + (u >> 1), nt_end - 1);
+  auto offset = [&](int u, int v) __attribute__((always_inline)) {   // TAIL: clamped to the last tile, tiles beyond it are not stored
+    const int n_in = (u & 1) * 16 + n4, m_in = (v & 1) * 16 + m16;
+    const int mt = TAIL ? min(mtw + (v >> 1), p.Mt - 1) : mtw + (v >> 1), nt = TAIL ? min(ntw + (u >> 1), nt_end - 1) : ntw + (u >> 1);
     return (((int64_t)mt * p.Nt + nt) * 1024 + ((m_in >> 4) * 2 + (n_in >> 4)) * 256 + (m_in & 15) * 16 + (n_in & 15)) * 2;
   };
   u32x2 bias[NU], tail[4][NV];
   auto load_tail = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
-    for (int v = 0; v < NV; ++v) tail[u & 3][v] = p.tail ? *(const u32x2 *)(C + offset(u, v) + p.tail_delta) : u32x2{0, 0};
+    for (int v = 0; v < NV; ++v) tail[u & 3][v] = *(const u32x2 *)(C + offset(u, v) + p.tail_delta);
   };
 #pragma unroll
   for (int u = 0; u < NU; ++u) bias[u] = p.bias ? bias_quad(p, min(ntw + (u >> 1), nt_end - 1), (u & 1) * 16 + n4) : u32x2{0, 0};
-  load_tail(0); load_tail(1);
+  if (TAIL) { load_tail(0); load_tail(1); }
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
-    if (u + 2 < NU) load_tail(u + 2);
+    if (TAIL && u + 2 < NU) load_tail(u + 2);
+    if (!TAIL && ntw + (u >> 1) >= nt_end) continue;
     const u32x2 raw = bias[u];
     const float bv[4] = {__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xFFFF0000u), __uint_as_float(raw.y << 16), __uint_as_float(raw.y & 0xFFFF0000u)};
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
+      if (!TAIL && mtw + (v >> 1) >= p.Mt) continue;
       float x[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) x[r] = apply_act<ACT>(acc[u][v][r] + bv[r]);
-      const u32x2 o = finish_quad(p.tail, tail[u & 3][v], x);
-      if (ntw + (u >> 1) < nt_end && mtw + (v >> 1) < p.Mt) *(u32x2 *)(C + offset(u, v)) = o;
+      const u32x2 o = finish_quad(TAIL ? p.tail : TTM_TAIL_NONE, TAIL ? tail[u & 3][v] : u32x2{0, 0}, x);
+      if (!TAIL || (ntw + (u >> 1) < nt_end && mtw + (v >> 1) < p.Mt)) *(u32x2 *)(C + offset(u, v)) = o;
     }
   }
 }
@@ -385,14 +391,14 @@ __device__ __forceinline__ void linear_store_partial16(const LinearArgs &p, floa
     }
   }
 }
-template <int NU, int NV>
+template <bool TAIL, int NU, int NV>
 __device__ __forceinline__ void linear_epilogue_act16(const LinearArgs &p, uint8_t *C, f32x4 (&acc)[NU][NV], int mtw, int ntw, int nt_end, int lane) {
   switch (p.act) {   // uniform
-  case TTM_ACT_GELU: linear_epilogue16<TTM_ACT_GELU>(p, C, acc, mtw, ntw, nt_end, lane); break;
-  case TTM_ACT_SILU: linear_epilogue16<TTM_ACT_SILU>(p, C, acc, mtw, ntw, nt_end, lane); break;
-  case TTM_ACT_SIGMOID: linear_epilogue16<TTM_ACT_SIGMOID>(p, C, acc, mtw, ntw, nt_end, lane); break;
-  case TTM_ACT_RELU: linear_epilogue16<TTM_ACT_RELU>(p, C, acc, mtw, ntw, nt_end, lane); break;
-  default: linear_epilogue16<TTM_ACT_NONE>(p, C, acc, mtw, ntw, nt_end, lane); break;
+  case TTM_ACT_GELU: linear_epilogue16<TTM_ACT_GELU, TAIL>(p, C, acc, mtw, ntw, nt_end, lane); break;
+  case TTM_ACT_SILU: linear_epilogue16<TTM_ACT_SILU, TAIL>(p, C, acc, mtw, ntw, nt_end, lane); break;
+  case TTM_ACT_SIGMOID: linear_epilogue16<TTM_ACT_SIGMOID, TAIL>(p, C, acc, mtw, ntw, nt_end, lane); break;
+  case TTM_ACT_RELU: linear_epilogue16<TTM_ACT_RELU, TAIL>(p, C, acc, mtw, ntw, nt_end, lane); break;
+  default: linear_epilogue16<TTM_ACT_NONE, TAIL>(p, C, acc, mtw, ntw, nt_end, lane); break;
   }
 }
 
@@ -1073,7 +1079,7 @@ __device__ __forceinline__ void linear_dma_block(const LinearArgs &p, int bid, i
 // fragments of the chunk; weight fragments are requested two tiles ahead.  The block barrier sits after n tile 3 of the
 // second chunk: tiles 4 .. 7 of that chunk multiply from fragments requested before the barrier, and the first fragments
 // of the next step are requested right behind it, so the matrix core does not drain at the barrier.
-template <int WF, int NTW, int BN_ = 2 * NTW>
+template <int WF, int NTW, bool TAIL, int BN_ = 2 * NTW>
 __device__ __forceinline__ void linear_img16_block(const LinearArgs &p, int bid, int nblk, int nt_first, int nt_end) {
   static_assert(BN_ == 2 * NTW || (BN_ == 7 && (NTW == 4 || NTW == 3)), "block of 2 NTW column tiles, or the uneven seven");
   constexpr int MB = 2, BN = BN_, NU = 2 * NTW, NV = 2 * MB;
@@ -1230,7 +1236,7 @@ __device__ __forceinline__ void linear_img16_block(const LinearArgs &p, int bid,
 
   if (p.partial) linear_store_partial16(p, p.partial + ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * ((int64_t)p.Mt * p.Nt * 1024), acc,
                                         mt0 + wm * MB, nt0 + wcol, nt_end, lane);
-  else linear_epilogue_act16(p, C, acc, mt0 + wm * MB, nt0 + wcol, nt_end, lane);
+  else linear_epilogue_act16<TAIL>(p, C, acc, mt0 + wm * MB, nt0 + wcol, nt_end, lane);
 }
 
 // group launch: the block's member becomes an ordinary single launch over that member's columns (p is rebound); the
@@ -1263,7 +1269,7 @@ __global__ __launch_bounds__(512) void ttm_linear_dma_glu_k(LinearArgs p) {
   linear_dma_block<WF_BFP8, 4, false, 8, true>(p, blockIdx.x, gridDim.x, 0, p.Nt);
 }
 
-template <int WF, bool M16 = true>   // M16: v_mfma_f32_16x16x32_bf16 (linear_img16_block); else 32x32x16
+template <int WF, bool M16, bool TAIL>   // M16: v_mfma_f32_16x16x32_bf16 (linear_img16_block), with or without a tail; else 32x32x16, either
 __global__ __launch_bounds__(512) void ttm_linear_img_k(LinearArgs p) {
   int bid = blockIdx.x, nblk = gridDim.x, first = 0, end = p.Nt, ntw = p.ntw;
   if (p.group_n > 1) linear_group_rebind(p, bid, nblk, end);   // workgroup-uniform
@@ -1274,11 +1280,11 @@ __global__ __launch_bounds__(512) void ttm_linear_img_k(LinearArgs p) {
   if constexpr (M16) {
     if (ntw == 7) {   // seven tiles wide: wide and narrow wavefronts (wavefront-uniform branch)
       const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-      if ((((wave & 3) & 1) ^ (wave >> 2)) == 0) linear_img16_block<WF, 4, 7>(p, bid, nblk, first, end);
-      else linear_img16_block<WF, 3, 7>(p, bid, nblk, first, end);
-    } else if (ntw == 4) linear_img16_block<WF, 4>(p, bid, nblk, first, end);
-    else if (ntw == 3) linear_img16_block<WF, 3>(p, bid, nblk, first, end);
-    else linear_img16_block<WF, 2>(p, bid, nblk, first, end);
+      if ((((wave & 3) & 1) ^ (wave >> 2)) == 0) linear_img16_block<WF, 4, TAIL, 7>(p, bid, nblk, first, end);
+      else linear_img16_block<WF, 3, TAIL, 7>(p, bid, nblk, first, end);
+    } else if (ntw == 4) linear_img16_block<WF, 4, TAIL>(p, bid, nblk, first, end);
+    else if (ntw == 3) linear_img16_block<WF, 3, TAIL>(p, bid, nblk, first, end);
+    else linear_img16_block<WF, 2, TAIL>(p, bid, nblk, first, end);
   } else {
     if (ntw == 7) {
       const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2130,7 +2136,8 @@ static int launch_linear(const LinearArgs &a, int64_t batch, hipStream_t s) {
       if (two_pass) {
         static bool attr2 = false;
         if (!attr2) {
-          if (int rc = set_lds_limit(ttm_linear_img_k<WI>, 131072)) return rc;
+          if (int rc = set_lds_limit(ttm_linear_img_k<WI, true, false>, 131072)) return rc;
+          if (int rc = set_lds_limit(ttm_linear_img_k<WI, true, true>, 131072)) return rc;
           attr2 = true;
         }
         if constexpr (!BFP) {
@@ -2154,10 +2161,12 @@ static int launch_linear(const LinearArgs &a, int64_t batch, hipStream_t s) {
         p.w_batch = a.w_batch == 0 ? 0 : img_set;
         p.img_zero_step = ksteps;
         if (ttm_option("linear_img_variant") == 1) {   // the 32x32x16 form of the second pass, for comparison
-          if (int rc = set_lds_limit(ttm_linear_img_k<WI, false>, 131072)) return rc;
-          hipLaunchKernelGGL((ttm_linear_img_k<WI, false>), dim3(p.n_blocks, slices, (unsigned)batch), dim3(512), 131072, s, p);
+          if (int rc = set_lds_limit(ttm_linear_img_k<WI, false, false>, 131072)) return rc;
+          hipLaunchKernelGGL((ttm_linear_img_k<WI, false, false>), dim3(p.n_blocks, slices, (unsigned)batch), dim3(512), 131072, s, p);
+        } else if (p.tail && !p.partial) {
+          hipLaunchKernelGGL((ttm_linear_img_k<WI, true, true>), dim3(p.n_blocks, slices, (unsigned)batch), dim3(512), 131072, s, p);
         } else {
-          hipLaunchKernelGGL((ttm_linear_img_k<WI>), dim3(p.n_blocks, slices, (unsigned)batch), dim3(512), 131072, s, p);
+          hipLaunchKernelGGL((ttm_linear_img_k<WI, true, false>), dim3(p.n_blocks, slices, (unsigned)batch), dim3(512), 131072, s, p);
         }
       } else if constexpr (BFP) {
         hipLaunchKernelGGL((ttm_linear_dma_k<WF>), dim3(p.n_blocks, slices, (unsigned)batch), dim3(512), lds6, s, p);
