@@ -50,8 +50,10 @@ TTM_EXPORT int ttm_copy_kernel(const void *src, void *dst, size_t bytes, void *s
 // A wavefront's access covers 8 / ELEM rows x 8 ELEM chunks (more rows of narrower tensors, fewer and longer ones of small tensors):
 // 8 / ELEM face rows of 16 ELEM bytes are one 128-byte line of the tiled side, and a row's 8 ELEM chunks are 128 ELEM contiguous bytes
 // of the row-major side, which starts and ends at any element: 16-byte accesses at their own alignment (a lane whose chunk crosses the
-// end of a row takes elements), so nothing outside the tensor is read and nothing is shifted or exchanged.  U accesses per lane.  What bounds it is bytes in flight against the number of
-// workgroups: two loads per lane are best for tilize up to 32 MiB, one beyond and for untilize (a store needs no more).
+// end of a row takes elements), so nothing outside the tensor is read and nothing is shifted or exchanged.  U accesses per lane.  What
+// bounds it is bytes in flight against the number of workgroups: two loads per lane are best for tilize from 192 KiB to 32 MiB, one beyond
+// and for untilize (a store needs no more).  Below, a lane's second load is no shorter than the launch (kernel alone, two / one: [49, 8]
+// bytes 2.7 / 2.2 us, [2, 19, 444] bf16 2.8 / 2.35, from page-locked memory [256, 264] bytes 6.5 / 5.2, but [256, 512] bf16 7.9 / 8.2).
 // Tilize streams its stores past the caches, untilize does not (partial lines at the ends of rows meet in L2).  Against strips of 32
 // rows x 512 bytes through LDS with funnel shifts for odd rows: [3, 1000, 3001] bf16 tilize / untilize 9.0 / 10.6 -> 7.0 / 6.9 us,
 // [4000, 7001] fp32 42.0 / 37.2 -> 39.4 / 35.6, [2, 1266, 771] bf16 4.2 / 5.5 -> 3.1 / 3.2, [7, 33, 9000] fp32 7.7 / 6.2 -> 4.4 / 4.4,
@@ -286,7 +288,7 @@ static int run_layout(const void *src, void *dst, int64_t batch, int64_t rows, i
       return TTM_OK;
     }
   }
-  const int u = TILIZE && bytes <= ((int64_t)32 << 20) ? 2 : 1;   // accesses per lane
+  const int u = TILIZE && bytes > 192 << 10 && bytes <= ((int64_t)32 << 20) ? 2 : 1;   // accesses per lane
   const int64_t across = ttm_cdiv((TILIZE ? pc : cols) * elem, 16);   // chunks of a row
   // Chunks of a row that a wavefront's access covers: whole lines of the tiled side, and for tilize up to 4 MiB at least 512 bytes, as these are
   // mostly uploads whose rows a kernel reads from page-locked memory, while on the device the launch hides the partial lines of the
