@@ -176,6 +176,25 @@ def test_bfp_of_host_memory(hip, dev, fmt, dtype):
         assert torch.equal(o[at:at + n], back.cpu()) and bool((o[:at] == 5).all()) and bool((o[at + n:] == 5).all())
 
 
+def test_bfp_of_shapes_that_strips_could_serve_can_be_captured(hip, dev):
+    """Which memory the pointers name is asked of such shapes, under capture as well."""
+    b, r, c = shape = (2, 1100, 2081)
+    x = torch.randn(b * r * c, device=dev)
+    want = pack_gpu(hip, dev, x, hip.BFP8B, shape, hip.F32, hip.ROW_MAJOR)
+    back = unpack_gpu(hip, dev, want, hip.BFP8B, shape, hip.F32, hip.ROW_MAJOR)
+    p, y = torch.zeros_like(want), torch.zeros_like(back)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        hip.call("ttm_bfp_pack", hip.ptr(x), hip.F32, hip.ROW_MAJOR, hip.ptr(p), hip.BFP8B, b, r, c, hip.current_stream())
+        hip.call("ttm_bfp_unpack", hip.ptr(p), hip.BFP8B, hip.ptr(y), hip.F32, hip.ROW_MAJOR, b, r, c, hip.current_stream())
+    for _ in range(3):
+        p.zero_()
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(p, want) and torch.equal(y, back)
+
+
 @pytest.mark.parametrize("rows,cols", [(41000, 2051), (41024, 2048)])
 def test_large_tensors_take_strips(hip, dev, rows, cols):
     """Above the size up to which every shape goes chunk by chunk: whole strips and rows that start anywhere, against torch."""
