@@ -217,6 +217,34 @@ def test_softmax_and_reduce_lastdim(hip, dev, orc, dtype, shape, rowwise_variant
             assert np.max(bf16_ulps(got, orc.round_bf16(w))) <= 1.0, op
         assert np.all(np.isfinite(o.float().cpu().numpy()))
 
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("rows,cols", [(1000, 1024), (993, 1030), (1000, 2056), (512, 2100), (480, 4096), (512, 4100), (1025, 4100), (97, 8192), (481, 8192), (1030, 8100), (8200, 3100)])
+def test_rowwise_lanes_by_width(hip, dev, dtype, rows, cols):
+    """Every width at which a row-wise launch takes more lanes per workgroup, either side of the row counts at which it takes four rows
+    per workgroup, and an input read past the caches; against float64.  fp32: a sum of n terms in any tree of 256 to 1024 lanes and up
+    to 16 terms per lane is off by at most 30 roundings of its magnitude."""
+    tdt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    hdt = hip.BF16 if dtype == "bf16" else hip.F32
+    x = datagen.randn((rows, cols), seed=61, std=2.0, dtype=tdt)
+    w = (1.0 + 0.02 * datagen.randn((cols,), seed=62)).to(tdt)
+    xt, x64 = tilize_dev(hip, x, dev), x.to(dev).double()
+    s, out = hip.current_stream(), torch.full_like(xt, float("nan"))
+    ulp = 2.0 ** -8 if dtype == "bf16" else 2.0 ** -20
+    hip.call("ttm_rms_norm", hip.ptr(xt), hip.ptr(w.to(dev)), hip.ROW_MAJOR, None, hip.ROW_MAJOR, hip.ptr(out), hdt, 1, rows, cols, 1e-5, s)
+    want = x64 / (x64.square().mean(-1, keepdim=True) + 1e-5).sqrt() * w.to(dev).double()
+    assert torch.all((untilize_dev(hip, out, (rows, cols), dev).double() - want).abs() <= ulp * want.abs() + 1e-30)
+    hip.call("ttm_softmax_lastdim", hip.ptr(xt), hip.ptr(out.fill_(float("nan"))), hdt, 1, rows, cols, s)
+    want = torch.softmax(x64, -1)
+    assert torch.all((untilize_dev(hip, out, (rows, cols), dev).double() - want).abs() <= (ulp + 2.0 ** -17) * want + 1e-30)
+    assert bool(torch.isfinite(out.float()).all())
+    sums = torch.full(((rows + 31) // 32 * 1024,), float("nan"), dtype=tdt, device=dev)
+    hip.call("ttm_reduce_lastdim", 0, hip.ptr(xt), hip.ptr(sums), hdt, 1, rows, cols, s)
+    want = x64.sum(-1, keepdim=True)
+    assert torch.all((untilize_dev(hip, sums, (rows, 1), dev).double() - want).abs() <= ulp * want.abs() + 30 * 2.0 ** -24 * x64.abs().sum(-1, keepdim=True))
+    assert bool(torch.isfinite(sums.float()).all())
+
+
 def _same_specials(got, want, what):
     """NaN in the same places, the same infinities, and equal values elsewhere up to `tol` bf16 / fp32 handling by the caller."""
     assert np.array_equal(np.isnan(got), np.isnan(want)), what + ": NaN in other places than in the oracle's result"

@@ -19,6 +19,7 @@ struct RowArgs {
   int64_t rows, cols;  // logical extent of the last two dims
   int rt, ct;          // tiles per batch entry
   float eps;
+  int stream;          // band kernel: the input is read past the caches
   int out_ct;          // reductions: column tiles of the output (1), keepdim layout [.., rows, 1]
   // ttm_rowwise_row_k<.., PRE = true>: x is not read but made on the way in from the fp32 partial sums of a split-K
   // projection of one row tile, x = bf16(bf16(sum over slices) + residual), and also stored to sum_out
@@ -282,16 +283,16 @@ __global__ __launch_bounds__(256) void ttm_rowwise_resident_k(RowArgs p) {
   }
 }
 
-// RMSNorm / softmax with one row per workgroup, for rows of up to NK = 2, 4 or 8 chunks per lane (at most 16384 bf16 or
-// 8192 fp32 columns).
+// RMSNorm / softmax with one row per workgroup of NT = 256, 512 or 1024 lanes, NK = 2 chunks per lane (at most 16384 bf16 or
+// 8192 fp32 columns).  Wide rows on more lanes instead of more chunks per lane: [238, 5184] fp32 RMSNorm 7.6 -> 4.4 us, softmax 8.0 -> 5.2.
 // The row stays in registers between the reduction and the output pass, weights are fetched while the reduction is in
 // flight, and a workgroup issues all its loads at once: a [32, 4096] input is 32 short workgroups instead of 4 long ones.
 // Consecutive rows of a face share 128-byte lines, so the row -> workgroup map gives every XCD (workgroup id mod 8)
 // a contiguous range of rows and its L2 sees each line of that range whole.
-template <int MODE, int ELEM, int NK, bool PRE = false>
-__global__ __launch_bounds__(256) void ttm_rowwise_row_k(RowArgs p, int total_rows) {
-  constexpr int EPC = 16 / ELEM;
-  __shared__ float red[4], red2[4];
+template <int MODE, int ELEM, bool PRE, int NT>
+__global__ __launch_bounds__(NT) void ttm_rowwise_row_k(RowArgs p, int total_rows) {
+  constexpr int EPC = 16 / ELEM, NW = NT / 64, NK = 2;
+  __shared__ float red[NW], red2[NW];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int per_xcd = total_rows / 8;                    // total_rows is a multiple of 32
   const int lrow = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
@@ -304,7 +305,7 @@ __global__ __launch_bounds__(256) void ttm_rowwise_row_k(RowArgs p, int total_ro
   u32x4 v[NK];
 #pragma unroll
   for (int k = 0; k < NK; ++k) {
-    const int q = tid + k * 256;
+    const int q = tid + k * NT;
     v[k] = u32x4{0, 0, 0, 0};
     if constexpr (PRE) {   // bf16 rows made from partial sums: the projection's rounding, then the residual add's
       static_assert(!PRE || ELEM == 2, "partial sums finish as bf16");
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(256) void ttm_rowwise_row_k(RowArgs p, int total_ro
   if (MODE == RW_RMSNORM) {
 #pragma unroll
     for (int k = 0; k < NK; ++k) {
-      const int q = tid + k * 256;
+      const int q = tid + k * NT;
       if (q < nq) {
         const int c0 = chunk_pos<ELEM>(r, q).c0;
         const int64_t tiled = (int64_t)(c0 >> 5) * 1024 + ((c0 >> 4) & 1) * 256 + (c0 & 15);
@@ -343,7 +344,7 @@ __global__ __launch_bounds__(256) void ttm_rowwise_row_k(RowArgs p, int total_ro
   float acc = MODE == RW_SOFTMAX ? -INFINITY : 0.0f;
 #pragma unroll
   for (int k = 0; k < NK; ++k) {
-    const int q = tid + k * 256;
+    const int q = tid + k * NT;
     if (q < nq) {
       const int c0 = chunk_pos<ELEM>(r, q).c0;
       float f[EPC];
@@ -360,7 +361,9 @@ __global__ __launch_bounds__(256) void ttm_rowwise_row_k(RowArgs p, int total_ro
   for (int s = 32; s > 0; s >>= 1) acc = MODE == RW_SOFTMAX ? ttm_max(acc, __shfl_xor(acc, s)) : acc + __shfl_xor(acc, s);
   if (lane == 0) red[wave] = acc;
   __syncthreads();
-  const float stat = MODE == RW_SOFTMAX ? ttm_max(ttm_max(red[0], red[1]), ttm_max(red[2], red[3])) : red[0] + red[1] + red[2] + red[3];
+  float stat = red[0];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) stat = MODE == RW_SOFTMAX ? ttm_max(stat, red[w]) : stat + red[w];
   float mul;
   if (MODE == RW_RMSNORM) {
     mul = 1.0f / sqrtf(stat / (float)cols + p.eps);
@@ -368,7 +371,7 @@ __global__ __launch_bounds__(256) void ttm_rowwise_row_k(RowArgs p, int total_ro
     float sum = 0.0f;
 #pragma unroll
     for (int k = 0; k < NK; ++k) {
-      const int q = tid + k * 256;
+      const int q = tid + k * NT;
       if (q < nq) {
         const int c0 = chunk_pos<ELEM>(r, q).c0;
         float f[EPC];
@@ -381,11 +384,14 @@ __global__ __launch_bounds__(256) void ttm_rowwise_row_k(RowArgs p, int total_ro
     for (int s = 32; s > 0; s >>= 1) sum += __shfl_xor(sum, s);
     if (lane == 0) red2[wave] = sum;
     __syncthreads();
-    mul = 1.0f / (red2[0] + red2[1] + red2[2] + red2[3]);
+    float den = red2[0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) den += red2[w];
+    mul = 1.0f / den;
   }
 #pragma unroll
   for (int k = 0; k < NK; ++k) {
-    const int q = tid + k * 256;
+    const int q = tid + k * NT;
     if (q < nq) {
       const ChunkPos<ELEM> cp = chunk_pos<ELEM>(r, q);
       float f[EPC], w[EPC], b[EPC];
@@ -421,20 +427,18 @@ __global__ __launch_bounds__(256) void ttm_rowwise_row_k(RowArgs p, int total_ro
 #ifndef TTM_BAND_EXP
 #define TTM_BAND_EXP expf
 #endif
-// Workgroups per CU by mode and band size (NK x 4 KiB per workgroup), measured at 65536 rows: reductions 4 at 16 KiB
-// (44 -> 40 us for 1024 fp32 columns) and 3 from 32 KiB up (89 -> 82 us for 2048); fp32 softmax 4 at 16 KiB (94 -> 88 us)
-// and 2 from 32 KiB up (195 -> 185 us); RMSNorm 3 at 16 KiB (96 -> 90 us); everything else runs best without a cap.
-template <int MODE, int ELEM, int NK>
+// Workgroups per CU of 256-lane bands of 16 KiB, measured at 65536 rows: reductions 4 (44 -> 40 us for 1024 fp32 columns), fp32 softmax
+// 4 (94 -> 88 us); everything else runs best without a cap.
+template <int MODE, int ELEM, int NK, int NT>
 constexpr int band_max_waves() {
-  if (MODE == RW_SUM || MODE == RW_MEAN || MODE == RW_MAX || MODE == RW_MIN) return NK == 4 ? 4 : (NK >= 8 ? 3 : 8);
-  if (MODE == RW_SOFTMAX && ELEM == 4) return NK == 4 ? 4 : (NK >= 8 ? 2 : 8);
-  if (MODE == RW_RMSNORM) return NK == 4 ? 3 : 8;
-  return 8;
+  return NT == 256 && NK == 4 && (MODE >= RW_SUM || (MODE == RW_SOFTMAX && ELEM == 4)) ? 4 : 8;
 }
-// NT = 512 lanes take bands of up to 32 chunks per 256 lanes (16384 bf16 or 8192 fp32 columns) with sixteen chunks per lane:
-// one such workgroup per CU (128 KiB).
-template <int MODE, int ELEM, int NK, int NT = 256>
-__global__ __launch_bounds__(NT) TTM_MAX_WAVES((NT == 512 ? 2 : band_max_waves<MODE, ELEM, NK>())) void ttm_rowwise_band_k(RowArgs p) {
+// NT lanes, up to eight chunks each: bands wider than a few chunks per 256 lanes take 512 or 1024 lanes instead of more chunks per
+// lane, whose unrolled code is executed once and mostly waits for its own instructions.  In turn over three tensors (us, sixteen or
+// eight chunks per lane before, now): RMSNorm [2048, 4096] bf16 9.1 -> 7.5, [843, 5952] fp32 29.3 -> 8.7, [2048, 8192] bf16 17.4 -> 14.1;
+// softmax [2048, 4096] bf16 11.0 -> 9.3, [843, 5952] fp32 18.5 -> 11.6; sum [560, 8000] bf16 14.1 -> 3.6, [2048, 8192] fp32 13.3 -> 11.7.
+template <int MODE, int ELEM, int NK, int NT>
+__global__ __launch_bounds__(NT) TTM_MAX_WAVES((band_max_waves<MODE, ELEM, NK, NT>())) void ttm_rowwise_band_k(RowArgs p) {
   constexpr int EPC = 16 / ELEM, RUN = 4 * ELEM;         // chunks per run of four face rows
   constexpr bool IS_MAX = MODE == RW_SOFTMAX || MODE == RW_MAX;
   constexpr bool REDUCE = MODE == RW_SUM || MODE == RW_MEAN || MODE == RW_MAX || MODE == RW_MIN;
@@ -454,30 +458,36 @@ __global__ __launch_bounds__(NT) TTM_MAX_WAVES((NT == 512 ? 2 : band_max_waves<M
   auto off_of = [&](int run) { return (int64_t)(run >> 1) * 1024 + ((r >> 4) * 2 + (run & 1)) * 256 + (r & 15) * 16 + part * EPC; };
   auto col_of = [&](int run) { return (run >> 1) * 32 + (run & 1) * 16 + part * EPC; };
   u32x4 v[NK];
+  // unconditional (a run past the end repeats the last one and is masked where it is used): a branch around a load
+  // makes the compiler wait for each load before it issues the next
+  auto at = [&](int k) { return (const u32x4 *)(x + off_of(min(run_of(k), nruns - 1)) * ELEM); };
+  if (p.stream) {   // uniform; the empty asm keeps the compiler from merging the two forms of a load
+    asm volatile("");
 #pragma unroll
-  for (int k = 0; k < NK; ++k) {
-    // unconditional (a run past the end repeats the last one and is masked where it is used): a branch around a load
-    // makes the compiler wait for each load before it issues the next
-    const int run = min(run_of(k), nruns - 1);
-    v[k] = __builtin_nontemporal_load((const u32x4 *)(x + off_of(run) * ELEM));
+    for (int k = 0; k < NK; ++k) v[k] = __builtin_nontemporal_load(at(k));
+    asm volatile("");
+  } else {
+#pragma unroll
+    for (int k = 0; k < NK; ++k) v[k] = *at(k);
   }
-  // RMSNorm: the weight and bias chunks of this lane's columns.  Up to eight chunks per lane they are loaded up front, beside
-  // the input; with sixteen that would take every register of a SIMD for a single wavefront (measured 3.2 TB/s at 8192 bf16
-  // columns), so there they are loaded four chunks at a time where they are used (they come from the L2: every row shares them)
-  constexpr bool WB_EARLY = MODE == RW_RMSNORM && NK <= 8;
-  auto wb_load = [&](int k, u32x4 &wv, u32x4 &bv) {
-    const int c0 = col_of(min(run_of(k), nruns - 1));
-    const int64_t tiled = (int64_t)(c0 >> 5) * 1024 + ((c0 >> 4) & 1) * 256 + (c0 & 15);
-    // a null vector reads the input instead (the value is not used): no branch around the loads
-    const uint8_t *wsrc = p.w ? (const uint8_t *)p.w + (p.w_tiled ? tiled : c0) * ELEM : x;
-    const uint8_t *bsrc = p.b ? (const uint8_t *)p.b + (p.b_tiled ? tiled : c0) * ELEM : x;
-    wv = *(const u32x4 *)wsrc;
-    bv = *(const u32x4 *)bsrc;
+  // RMSNorm: the weight and bias chunks of this lane's columns, beside the input where the registers allow it ([2048, 4096] fp32 11.2 us,
+  // 14.2 at the use), else four chunks at a time where they are used (they come from the L2: every row shares them; [2048, 4096] bf16 7.4
+  // us, 7.8 up front)
+  constexpr bool WB_EARLY = MODE == RW_RMSNORM && NK * NT <= (ELEM == 4 ? 4096 : 1024);
+  auto vec_load = [&](const void *vec, int tiled, int k) {
+    const int c0 = min(col_of(run_of(k)), (cols - 1) / EPC * EPC);   // the padding of the last tile has no weight: a valid chunk again
+    return *(const u32x4 *)((const uint8_t *)vec + (tiled ? (int64_t)(c0 >> 5) * 1024 + ((c0 >> 4) & 1) * 256 + (c0 & 15) : (int64_t)c0) * ELEM);
   };
   u32x4 wraw[WB_EARLY ? NK : 1], braw[WB_EARLY ? NK : 1];
   if constexpr (WB_EARLY) {
+    if (p.w) {   // uniform
 #pragma unroll
-    for (int k = 0; k < NK; ++k) wb_load(k, wraw[k], braw[k]);
+      for (int k = 0; k < NK; ++k) wraw[k] = vec_load(p.w, p.w_tiled, k);
+    }
+    if (p.b) {
+#pragma unroll
+      for (int k = 0; k < NK; ++k) braw[k] = vec_load(p.b, p.b_tiled, k);
+    }
   }
   // the lanes of a wavefront that share a row differ in the chunk-part bits (below ELEM) and the run bits (RUN and up)
   auto wave_combine = [&](float a, bool is_max, bool is_min) {
@@ -516,8 +526,9 @@ __global__ __launch_bounds__(NT) TTM_MAX_WAVES((NT == 512 ? 2 : band_max_waves<M
       return IS_MAX ? ttm_max(ttm_max(a0, a1), ttm_max(a2, a3)) : (MODE == RW_MIN ? ttm_min(ttm_min(a0, a1), ttm_min(a2, a3)) : (a0 + a1) + (a2 + a3));
     };
     stat = four(0);
-    if constexpr (NW == 8) {
-      const float hi = four(4);
+#pragma unroll
+    for (int w0 = 4; w0 < NW; w0 += 4) {
+      const float hi = four(w0);
       stat = IS_MAX ? ttm_max(stat, hi) : (MODE == RW_MIN ? ttm_min(stat, hi) : stat + hi);
     }
   }
@@ -556,7 +567,8 @@ __global__ __launch_bounds__(NT) TTM_MAX_WAVES((NT == 512 ? 2 : band_max_waves<M
       if ((lane & ~(RUN - ELEM)) == 0) red2[wave][rl] = sum;
       __syncthreads();
       float den = (red2[0][rl] + red2[1][rl]) + (red2[2][rl] + red2[3][rl]);
-      if constexpr (NW == 8) den += (red2[4][rl] + red2[5][rl]) + (red2[6][rl] + red2[7][rl]);
+#pragma unroll
+      for (int w0 = 4; w0 < NW; w0 += 4) den += (red2[w0][rl] + red2[w0 + 1][rl]) + (red2[w0 + 2][rl] + red2[w0 + 3][rl]);
       mul = 1.0f / den;
     }
     u32x4 wlate[4], blate[4];
@@ -565,8 +577,14 @@ __global__ __launch_bounds__(NT) TTM_MAX_WAVES((NT == 512 ? 2 : band_max_waves<M
       if constexpr (MODE == RW_RMSNORM && !WB_EARLY) {
         if (k % 4 == 0) {
           __builtin_amdgcn_sched_barrier(0);   // the loads of one batch only: the scheduler would hoist all sixteen
+          if (p.w) {
 #pragma unroll
-          for (int u = 0; u < 4; ++u) wb_load(min(k + u, NK - 1), wlate[u], blate[u]);
+            for (int u = 0; u < 4; ++u) wlate[u] = vec_load(p.w, p.w_tiled, min(k + u, NK - 1));
+          }
+          if (p.b) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) blate[u] = vec_load(p.b, p.b_tiled, min(k + u, NK - 1));
+          }
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -794,27 +812,36 @@ template <int MODE>
 static int launch_rowwise(const RowArgs &p, int dtype, int64_t trows, hipStream_t s) {
   TTM_REQUIRE(trows < (1ll << 29), "row-wise kernel: tensor too large");
   {
-    // four rows per workgroup, whole lines, the band in registers: from one workgroup per CU upwards, rows of up to 16
-    // chunks per lane (16384 bf16 or 8192 fp32 columns).  rowwise_variant: 2 forces it, 1 and 3 exclude it.
     const int elem = dtype == TTM_BF16 ? 2 : 4, variant = ttm_option("rowwise_variant");
-    const int nk = (int)ttm_cdiv((int64_t)p.ct * 2 * 4 * elem, 256);
-    if (nk > 16 && nk <= 32 && trows * 8 < (1ll << 31) && (variant == 2 || (variant == 0 && trows * 8 >= 256))) {
-      // twice the lanes for bands of 17 - 32 chunks per 256 lanes
-      const dim3 grid((unsigned)(trows * 8)), block(512);
-      if (dtype == TTM_BF16) hipLaunchKernelGGL((ttm_rowwise_band_k<MODE, 2, 16, 512>), grid, block, 0, s, p);
-      else hipLaunchKernelGGL((ttm_rowwise_band_k<MODE, 4, 16, 512>), grid, block, 0, s, p);
-      TTM_LAUNCH_CHECK();
-      return TTM_OK;
-    }
-    if (nk <= 16 && trows * 8 < (1ll << 31) && (variant == 2 || (variant == 0 && trows * 8 >= 256))) {
-      const dim3 grid((unsigned)(trows * 8)), block(256);
-#define TTM_BAND_LAUNCH(E, N) hipLaunchKernelGGL((ttm_rowwise_band_k<MODE, E, N>), grid, block, 0, s, p)
-#define TTM_BAND_NK(E) \
-      do { if (nk <= 1) TTM_BAND_LAUNCH(E, 1); else if (nk <= 2) TTM_BAND_LAUNCH(E, 2); else if (nk <= 4) TTM_BAND_LAUNCH(E, 4); \
-           else if (nk <= 8) TTM_BAND_LAUNCH(E, 8); else TTM_BAND_LAUNCH(E, 16); } while (0)
-      if (dtype == TTM_BF16) TTM_BAND_NK(2); else TTM_BAND_NK(4);
-#undef TTM_BAND_NK
-#undef TTM_BAND_LAUNCH
+    const int64_t bands = trows * 8;
+    const int nk = (int)ttm_cdiv((int64_t)p.ct * 2 * 4 * elem, 256);   // chunks per lane of a 256-lane workgroup
+    // Four rows per workgroup, whole lines, the band in registers: rows of up to 32 chunks per 256 lanes (16384 bf16 or 8192 fp32
+    // columns).  RMSNorm and softmax take it from one workgroup per CU upwards, wide rows from half of that (fp32 [500, 4096] 4.9 us, one
+    // row per workgroup 5.3; fewer rows are faster that way: [238, 5184] 4.4, as bands 7.5); reductions, whose other kernel gives a lane
+    // of 32 per row, always ([238, 5184] bf16 6.8 -> 3.5 us), but for the rows that ttm_rowwise_wide_* spreads over the device.
+    // rowwise_variant: 2 forces it, 1 and 3 exclude it.
+    bool band = nk <= 32 && bands < (1ll << 31) && variant != 1 && variant != 3;
+    if constexpr (MODE == RW_RMSNORM || MODE == RW_SOFTMAX) band = band && (variant == 2 || bands >= 256 || (nk > 8 && bands >= 128));
+    else band = band && (variant == 2 || p.ct < 256 || bands >= 64);
+    if (band) {
+      const dim3 grid((unsigned)bands);
+      RowArgs q = p;
+      // Plain loads find what the producer left in the last-level cache (RMSNorm [8192, 4096] bf16 30.9 -> 23.1 us); an input of which little
+      // can be there is read past it (sum [8192, 8192] fp32 42.7 us, 47.6 plain)
+      q.stream = (int64_t)p.ct * 1024 * elem * trows > 100000000;
+#define TTM_BAND(N, T) \
+      do { if (dtype == TTM_BF16) hipLaunchKernelGGL((ttm_rowwise_band_k<MODE, 2, N, T>), grid, dim3(T), 0, s, q); \
+           else hipLaunchKernelGGL((ttm_rowwise_band_k<MODE, 4, N, T>), grid, dim3(T), 0, s, q); } while (0)
+      // lanes by width: measured per mode at 500 to 8192 rows.  RMSNorm of 3 and 4 chunks: [6738, 1920] bf16 10.4 us, 11.4 with 256 lanes
+      // (softmax 11.5 / 11.1); 9 to 16 chunks: softmax [4000, 6000] bf16 26.8 with 512 lanes, 31.3 with 1024 (843 rows 9.5 / 8.4, RMSNorm
+      // 26.5 / 23.1)
+      if (nk <= 1) TTM_BAND(1, 256);
+      else if (nk <= 2) TTM_BAND(2, 256);
+      else if (nk <= 4) { if (MODE == RW_RMSNORM) TTM_BAND(2, 512); else TTM_BAND(4, 256); }
+      else if (nk <= 8) TTM_BAND(4, 512);
+      else if (nk <= 16) { if (MODE == RW_SOFTMAX && bands >= 256) TTM_BAND(8, 512); else TTM_BAND(4, 1024); }
+      else TTM_BAND(8, 1024);
+#undef TTM_BAND
       TTM_LAUNCH_CHECK();
       return TTM_OK;
     }
@@ -850,17 +877,13 @@ static int launch_rowwise(const RowArgs &p, int dtype, int64_t trows, hipStream_
     const int elem = dtype == TTM_BF16 ? 2 : 4;
     if (p.ct * 2 * elem <= 8 * 256 && trows * 32 < (1 << 24) && ttm_option("rowwise_variant") != 1) {   // one row per workgroup
       const int total = (int)(trows * 32), nq = p.ct * 2 * elem;
-      const dim3 grid((unsigned)total), block(256);
-#define TTM_ROW_LAUNCH(E, N) hipLaunchKernelGGL((ttm_rowwise_row_k<MODE, E, N>), grid, block, 0, s, p, total)
-      if (dtype == TTM_BF16) {
-        if (nq <= 512) TTM_ROW_LAUNCH(2, 2);
-        else if (nq <= 1024) TTM_ROW_LAUNCH(2, 4);
-        else TTM_ROW_LAUNCH(2, 8);
-      } else {
-        if (nq <= 512) TTM_ROW_LAUNCH(4, 2);
-        else if (nq <= 1024) TTM_ROW_LAUNCH(4, 4);
-        else TTM_ROW_LAUNCH(4, 8);
-      }
+      const dim3 grid((unsigned)total);
+#define TTM_ROW_LAUNCH(T) \
+      do { if (dtype == TTM_BF16) hipLaunchKernelGGL((ttm_rowwise_row_k<MODE, 2, false, T>), grid, dim3(T), 0, s, p, total); \
+           else hipLaunchKernelGGL((ttm_rowwise_row_k<MODE, 4, false, T>), grid, dim3(T), 0, s, p, total); } while (0)
+      if (nq <= 512) TTM_ROW_LAUNCH(256);
+      else if (nq <= 1024) TTM_ROW_LAUNCH(512);
+      else TTM_ROW_LAUNCH(1024);
 #undef TTM_ROW_LAUNCH
       TTM_LAUNCH_CHECK();
       return TTM_OK;
@@ -892,7 +915,7 @@ static int fill_args(RowArgs &p, const void *x, void *out, int dtype, int64_t ba
   p.x = x; p.out = out; p.w = p.b = nullptr; p.w_tiled = p.b_tiled = 0;
   p.rows = rows; p.cols = cols;
   p.rt = (int)ttm_cdiv(rows, 32); p.ct = (int)ttm_cdiv(cols, 32);
-  p.eps = 0.0f; p.out_ct = 1;
+  p.eps = 0.0f; p.stream = 0; p.out_ct = 1;
   p.partial = nullptr; p.slices = 0; p.per = 0; p.residual = nullptr; p.sum_out = nullptr;
   return TTM_OK;
 }
@@ -915,10 +938,10 @@ int ttm_rowwise_rmsnorm_from_partials(const float *partial, int slices, int64_t 
   p.w = weight; p.b = bias; p.w_tiled = weight_layout == TTM_TILE; p.b_tiled = bias_layout == TTM_TILE; p.eps = eps;
   p.partial = partial; p.slices = slices; p.per = per; p.residual = residual; p.sum_out = sum_out;
   const int nq = p.ct * 4;
-  const dim3 grid(32), block(256);
-  if (nq <= 512) hipLaunchKernelGGL((ttm_rowwise_row_k<RW_RMSNORM, 2, 2, true>), grid, block, 0, s, p, 32);
-  else if (nq <= 1024) hipLaunchKernelGGL((ttm_rowwise_row_k<RW_RMSNORM, 2, 4, true>), grid, block, 0, s, p, 32);
-  else hipLaunchKernelGGL((ttm_rowwise_row_k<RW_RMSNORM, 2, 8, true>), grid, block, 0, s, p, 32);
+  const dim3 grid(32);
+  if (nq <= 512) hipLaunchKernelGGL((ttm_rowwise_row_k<RW_RMSNORM, 2, true, 256>), grid, dim3(256), 0, s, p, 32);
+  else if (nq <= 1024) hipLaunchKernelGGL((ttm_rowwise_row_k<RW_RMSNORM, 2, true, 512>), grid, dim3(512), 0, s, p, 32);
+  else hipLaunchKernelGGL((ttm_rowwise_row_k<RW_RMSNORM, 2, true, 1024>), grid, dim3(1024), 0, s, p, 32);
   TTM_LAUNCH_CHECK();
   return TTM_OK;
 }
