@@ -309,12 +309,12 @@ __global__ __launch_bounds__(256) TTM_MAX_WAVES((PACK && ROWMAJOR && W == 7 && E
 // [1024, 1056] fp32 4.2 / 4.6 -> 2.9 / 3.1.
 template <int W, int ELEM, int U, bool PACK>
 __global__ __launch_bounds__(256) void ttm_bfp_direct_k(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int rows, int cols, int lw, int wc,
-                                                        uint32_t xu, uint32_t matrices, uint32_t first) {
+                                                        uint32_t xu, uint32_t matrices, uint32_t first, uint32_t groups) {
   typedef typename std::conditional<ELEM == 4, uint32_t, uint16_t>::type T;
   constexpr int EPT = 16 / ELEM, TILE_BYTES = 64 + (W == 7 ? 1024 : 512), CHUNK_OUT = EPT * (W + 1) / 8;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ct = (cols + 31) >> 5, yt = (rows + 31) >> 5;
-  const uint32_t bid = first + xcd_order(), by = bid / xu;
+  const uint32_t bid = first + xcd_order(groups), by = bid / xu;
   const int chunk = (int)((((bid - by * xu) << wc) + (wave & ((1 << wc) - 1))) << lw) + (lane & ((1 << lw) - 1));
   const uint32_t row0 = ((by << (2 - wc)) + (wave >> wc)) * (64 >> lw) * U + (lane >> lw);   // of the rows of all matrices, padded ones for pack
   const uint32_t per = PACK ? yt * 32 : rows;
@@ -596,7 +596,7 @@ static int run_bfp(const void *src, void *dst, int fmt, int dtype, int layout, i
 #define DIRECT(Wv, EL, U)                                                                                                                       \
   ttm_launches(groups * xu, [&](uint32_t first, dim3 grid) {                                                                                    \
     hipLaunchKernelGGL((ttm_bfp_direct_k<Wv, EL, U, PACK>), grid, dim3(256), 0, s, (const uint8_t *)src, (uint8_t *)dst, (int)rows, (int)cols,  \
-                       lw, wc, (uint32_t)xu, (uint32_t)batch, first);                                                                           \
+                       lw, wc, (uint32_t)xu, (uint32_t)batch, first, grid.x);                                                                   \
   })
 #define DIRECT_U(Wv, EL)            \
   do {                              \

@@ -49,7 +49,7 @@ __global__ __launch_bounds__(256) void ttm_rotary_k(const T *__restrict__ x, con
                                                     const T *__restrict__ sinc, T *__restrict__ out, int64_t rows_pad,
                                                     int64_t cols, int64_t per_batch, int64_t total8, int64_t token_index,
                                                     int64_t rows, int64_t src_cols) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total8) return;
   const int64_t ct = cols >> 5, half = cols >> 1;
   const int64_t e = i * 8, b = e / per_batch, o = e % per_batch;
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(256) void ttm_update_cache_k(T *__restrict__ cache,
                                                           const int32_t *__restrict__ index, int64_t heads, int64_t seq_pad,
                                                           int64_t max_seq, int64_t dim, int64_t in_users, int64_t in_users_pad,
                                                           int64_t batch_offset, int64_t total8) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total8) return;
   const int64_t pos = index[0];
   if (pos < 0 || pos >= max_seq) return;          // out of range positions write nothing
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256) void ttm_update_cache_k(T *__restrict__ cache,
 __global__ __launch_bounds__(256) void ttm_fill_cache_k(u32x4 *__restrict__ cache, const u32x4 *__restrict__ input,
                                                         int64_t head_stride_cache16, int64_t head_stride_in16, int64_t base16,
                                                         int64_t total16) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total16) return;
   const int64_t h = i / head_stride_in16, o = i % head_stride_in16;
   cache[base16 + h * head_stride_cache16 + o] = input[i];
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(256) void ttm_paged_update_cache_k(T *__restrict__ 
                                                                 const int32_t *__restrict__ index, const int32_t *__restrict__ table,
                                                                 int64_t blocks, int64_t heads, int64_t block_size, int64_t dim,
                                                                 int64_t users, int64_t pages, int shared, int64_t total8) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total8) return;
   const int64_t d8 = dim >> 3, ct = dim >> 5;
   const int64_t c = (i % d8) * 8, h = (i / d8) % heads, u = i / (d8 * heads);
@@ -156,7 +156,7 @@ __global__ __launch_bounds__(256) void ttm_paged_fill_cache_k(T *__restrict__ ca
                                                               const int32_t *__restrict__ table, const int32_t *__restrict__ batch_idx,
                                                               int64_t blocks, int64_t heads, int64_t block_size, int64_t dim,
                                                               int64_t seq, int64_t table_rows, int64_t pages, int64_t total8) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total8) return;
   const int64_t d8 = dim >> 3, ct = dim >> 5;
   const int64_t c = (i % d8) * 8, s = (i / d8) % seq, h = (i / (d8 * seq)) % heads, b = i / (d8 * seq * heads);
@@ -178,7 +178,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void ttm_paged_gather_k(const T *__restrict__ cache, const int32_t *__restrict__ table, T *__restrict__ out,
                                                           int64_t blocks, int64_t heads, int64_t block_size, int64_t dim, int64_t pages,
                                                           int64_t total8) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total8) return;
   const int64_t d8 = dim >> 3, ct = dim >> 5, seq = pages * block_size;
   const int64_t c = (i % d8) * 8, s = (i / d8) % seq, h = (i / (d8 * seq)) % heads, b = i / (d8 * seq * heads);
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(256) void ttm_paged_gather_k(const T *__restrict__ 
 // memory, so the launch can be recorded into a graph and replayed for the next chunk
 __global__ __launch_bounds__(256) void ttm_chunk_mask_k(uint16_t *__restrict__ mask, const int32_t *__restrict__ start, int64_t rows_pad,
                                                         int64_t cols_pad, int64_t total8) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total8) return;
   const int64_t c8 = cols_pad >> 3, r = i / c8, c = (i % c8) * 8;
   const int64_t limit = (int64_t)start[0] + r;
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(256) void ttm_rotary_llama_k(const uint16_t *__rest
   __shared__ float T[32][33];
   for (int e = threadIdx.x; e < 1024; e += 256) T[e >> 5][e & 31] = ttm_bf16_to_f32(tmat[ttm_tiled_offset(e >> 5, e & 31, 1)]);
   __syncthreads();
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total) return;
   const int64_t c = i % cols, r = (i / cols) % rows_pad, b = i / (cols * rows_pad), ct = cols >> 5;
   const int64_t off = b * rows_pad * cols + ttm_tiled_offset(r, c, ct);
@@ -268,7 +268,31 @@ struct DecodeArgs {
   int window;         // >= 0: only the last `window` keys up to the decode position are visible
   const uint16_t *sink;   // [H, 32] in tiles, column 0: one more logit per head (times scale) with a zero value row; or null
   float scale;
+  __device__ __forceinline__ const DecodeArgs &full() const { return *this; }
 };
+// The same without mask and sink, in the 112 bytes that launch quickly (ttm_common.h)
+struct DecodeLean {
+  const uint16_t *q, *k, *v;
+  const int32_t *cur_pos, *page_table;
+  float *part;
+  uint16_t *out;
+  int B, Hkv, S, shares, block, pages_per_user, blocks, Gt, g0, window;
+  float scale;
+  uint16_t D;
+  uint8_t G, flags;
+  explicit DecodeLean(const DecodeArgs &a)
+      : q(a.q), k(a.k), v(a.v), cur_pos(a.cur_pos), page_table(a.page_table), part(a.part), out(a.out), B(a.B), Hkv(a.Hkv), S(a.S), shares(a.shares),
+        block(a.block), pages_per_user(a.pages_per_user), blocks(a.blocks), Gt(a.Gt), g0(a.g0), window(a.window), scale(a.scale), D((uint16_t)a.D),
+        G((uint8_t)a.G), flags((uint8_t)((a.is_causal ? 1 : 0) | (a.concat_heads ? 2 : 0))) {}
+  __device__ __forceinline__ DecodeArgs full() const {
+    DecodeArgs p = {};
+    p.q = q; p.k = k; p.v = v; p.cur_pos = cur_pos; p.page_table = page_table; p.part = part; p.out = out;
+    p.B = B; p.H = Hkv * Gt; p.Hkv = Hkv; p.G = G; p.S = S; p.D = D; p.shares = shares; p.block = block; p.pages_per_user = pages_per_user;
+    p.is_causal = flags & 1; p.blocks = blocks; p.concat_heads = flags >> 1; p.Gt = Gt; p.g0 = g0; p.window = window; p.scale = scale;
+    return p;
+  }
+};
+static_assert(sizeof(DecodeLean) <= 112, "the size up to which a launch is quick");
 
 constexpr int kMaxG = 8;
 // K is read by streaming (nontemporal) loads: each line once per launch, by one instruction.  STREAM = false when several launches
@@ -359,8 +383,9 @@ __device__ __forceinline__ void store_padding(const DecodeArgs &p, int b, int hk
 }
 
 // GM: most query heads, DM: most column tiles (1, 2, 4, 8), NW: wavefronts
-template <bool STREAM, int GM, int DM, bool EXACT, int NW, bool DIRECT>
-__global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void ttm_sdpa_decode_k(DecodeArgs p) {
+template <bool STREAM, int GM, int DM, bool EXACT, int NW, bool DIRECT, class ARGS>
+__global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void ttm_sdpa_decode_k(ARGS args) {
+  const DecodeArgs p = args.full();
   constexpr int KS = DM >= 4 ? 1 : 4 / DM;   // lanes of a column pair that share the tile's keys
   constexpr int NP = DM > 4 ? 2 : 1;         // column pairs of a lane
   constexpr int KEYS = 32 / KS;              // keys of a tile a lane multiplies
@@ -609,7 +634,9 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void ttm_sdpa_decode_k(D
 // hundred KiB in all), so there are two: the users' positions, then a lane's maxima and sums together with its first eight
 // numerators, which do not wait for the weights.  5 users x 4 heads of 4 kv heads, 1300 keys on average (about 20 slots each):
 // both launches 27.4 us with a workgroup per 256 outputs, one head after the other and numerators behind the weights -> 13.9 us.
-__global__ __launch_bounds__(256) void ttm_sdpa_decode_combine_k(DecodeArgs p) {
+template <class ARGS>
+__global__ __launch_bounds__(256) void ttm_sdpa_decode_combine_k(ARGS args) {
+  const DecodeArgs p = args.full();
   __shared__ float wgt[kDecodeBlocks];   // a user's slots lie in at most that many shares
   __shared__ float red[256];
   __shared__ float tops[4], sums[4];
@@ -846,7 +873,8 @@ static int decode_scratch_ptr(void **ptr) {
 template <bool STREAM, int GM, int DM, bool EXACT, int NW, bool DIRECT>
 static void launch_decode(const DecodeArgs &p, dim3 grid, hipStream_t s) {
   const size_t lds = (size_t)NW * p.G * p.D * sizeof(float);   // at most 32 KiB
-  hipLaunchKernelGGL((ttm_sdpa_decode_k<STREAM, GM, DM, EXACT, NW, DIRECT>), grid, dim3(NW * 64), lds, s, p);
+  if (p.mask || p.sink) hipLaunchKernelGGL((ttm_sdpa_decode_k<STREAM, GM, DM, EXACT, NW, DIRECT, DecodeArgs>), grid, dim3(NW * 64), lds, s, p);
+  else hipLaunchKernelGGL((ttm_sdpa_decode_k<STREAM, GM, DM, EXACT, NW, DIRECT, DecodeLean>), grid, dim3(NW * 64), lds, s, DecodeLean(p));
 }
 // The head dims 32, 64, 128 and 256 have kernels of their own; others, and heads in several launches, the next larger one's loops
 // with a bound.  Up to four heads (and 128 columns) the direct form holds its state in 128 registers and takes 16 wavefronts.
@@ -944,7 +972,9 @@ static int sdpa_decode_entry(const void *q, const void *k, const void *v, const 
     }
     launch_decode<false>(p, dim3((unsigned)shares, (unsigned)kv_heads), s);
     TTM_LAUNCH_CHECK();
-    hipLaunchKernelGGL(ttm_sdpa_decode_combine_k, dim3((unsigned)(batch * kv_heads), (unsigned)p.G), dim3(256), 0, s, p);
+    const dim3 heads_of_users((unsigned)(batch * kv_heads), (unsigned)p.G);
+    if (p.mask || p.sink) hipLaunchKernelGGL(ttm_sdpa_decode_combine_k<DecodeArgs>, heads_of_users, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL(ttm_sdpa_decode_combine_k<DecodeLean>, heads_of_users, dim3(256), 0, s, DecodeLean(p));
     TTM_LAUNCH_CHECK();
   }
   return TTM_OK;

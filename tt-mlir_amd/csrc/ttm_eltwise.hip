@@ -89,6 +89,21 @@ __device__ __forceinline__ float binary_op(int op, float a, float b) {
   }
 }
 
+// x = x op y for N values: one branch for all of them ([58, 429] bf16 add 3.4 -> 2.7 us against one per value)
+template <int N>
+__device__ __forceinline__ void binary_all(int op, float (&x)[N], const float (&y)[N]) {
+  auto all = [&](auto o) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = binary_op(decltype(o)::value, x[i], y[i]);
+  };
+#define B(OP) case OP: all(std::integral_constant<int, OP>{}); break;
+  switch (op) {   // uniform
+    B(B_ADD) B(B_MUL) B(B_SUB) B(B_EQ) B(B_NE) B(B_GE) B(B_GT) B(B_LE) B(B_LT) B(B_DIV) B(B_AND) B(B_OR) B(B_XOR) B(B_MAXIMUM) B(B_MINIMUM)
+    B(B_REMAINDER) B(B_POW) B(B_ATAN2)
+  }
+#undef B
+}
+
 template <bool BF16>
 __device__ __forceinline__ void chunk_load(const void *p, int64_t chunk, float (&f)[BF16 ? 8 : 4]) {
   u32x4 v = ((const u32x4 *)p)[chunk];
@@ -118,9 +133,9 @@ __device__ __forceinline__ void chunk_store(void *p, int64_t chunk, const float 
 
 template <int OP, bool BF16>
 __global__ __launch_bounds__(256) void ttm_unary_k(const void *__restrict__ in, void *__restrict__ out, int64_t nchunks,
-                                                   int64_t n, float param, float param2) {
+                                                   int64_t n, float param, float param2, int64_t stride) {
   constexpr int EPC = BF16 ? 8 : 4;
-  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < nchunks; c += (int64_t)gridDim.x * 256) {
+  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < nchunks; c += stride) {
     if ((c + 1) * EPC <= n) {
       float f[EPC];
       chunk_load<BF16>(in, c, f);
@@ -158,7 +173,7 @@ __global__ __launch_bounds__(256) void ttm_unary_masked_k(const void *__restrict
   }
 }
 
-typedef void (*unary_fn)(const void *, void *, int64_t, int64_t, float, float);
+typedef void (*unary_fn)(const void *, void *, int64_t, int64_t, float, float, int64_t);
 typedef void (*unary_masked_fn)(const void *, void *, int64_t, int64_t, int64_t, float, float);
 
 template <bool BF16>
@@ -190,11 +205,11 @@ static unary_masked_fn pick_unary_masked(int op) {
 // padding; grid.y numbers the matrices
 template <int OP, bool BF16>
 __global__ __launch_bounds__(256) void ttm_unary_masked_chunk_k(const void *__restrict__ in, void *__restrict__ out, uint32_t chunks_per_plane,
-                                                                uint32_t rows, uint32_t cols, float param, float param2) {
+                                                                uint32_t rows, uint32_t cols, float param, float param2, uint32_t stride) {
   constexpr int EPC = BF16 ? 8 : 4;
   const uint32_t tcols = (cols + 31) >> 5;
   const int64_t base = (int64_t)blockIdx.y * chunks_per_plane;
-  for (uint32_t ci = blockIdx.x * 256 + threadIdx.x; ci < chunks_per_plane; ci += gridDim.x * 256) {
+  for (uint32_t ci = blockIdx.x * 256 + threadIdx.x; ci < chunks_per_plane; ci += stride) {
     const uint32_t w = ci * EPC, tile = w >> 10, e = w & 1023, face = e >> 8;
     const uint32_t r = (tile / tcols) * 32 + (face >> 1) * 16 + ((e >> 4) & 15), c0 = (tile % tcols) * 32 + (face & 1) * 16 + (e & 15);
     float f[EPC];
@@ -208,7 +223,7 @@ __global__ __launch_bounds__(256) void ttm_unary_masked_chunk_k(const void *__re
     chunk_store<BF16>(out, base + ci, f);
   }
 }
-typedef void (*unary_chunk_fn)(const void *, void *, uint32_t, uint32_t, uint32_t, float, float);
+typedef void (*unary_chunk_fn)(const void *, void *, uint32_t, uint32_t, uint32_t, float, float, uint32_t);
 template <bool BF16>
 static unary_chunk_fn pick_unary_masked_chunk(int op) {
 #define U(OP) case OP: return ttm_unary_masked_chunk_k<OP, BF16>;
@@ -243,7 +258,7 @@ static int unary_entry(int op, const void *in, void *out, int dtype, int layout,
     if (!fn) return ttm_set_error(TTM_ERR_UNSUPPORTED, "ttm_eltwise_unary: unsupported op %d", op);
     const uint32_t cpp = (uint32_t)(pr * pc * (dtype == TTM_BF16 ? 2 : 4) / 16);
     hipLaunchKernelGGL(fn, dim3(grid_for(cpp), (unsigned)batch), dim3(256), 0, (hipStream_t)stream, in, out, cpp, (uint32_t)rows, (uint32_t)cols,
-                       param, param2);
+                       param, param2, grid_for(cpp) * 256u);
     TTM_LAUNCH_CHECK();
     return TTM_OK;
   }
@@ -259,7 +274,8 @@ static int unary_entry(int op, const void *in, void *out, int dtype, int layout,
   if (!fn) return ttm_set_error(TTM_ERR_UNSUPPORTED, "ttm_eltwise_unary: unsupported op %d", op);
   const int epc = dtype == TTM_BF16 ? 8 : 4;
   int64_t nchunks = ttm_cdiv(n, epc);
-  hipLaunchKernelGGL(fn, dim3(grid_for(nchunks)), dim3(256), 0, (hipStream_t)stream, in, out, nchunks, n, param, param2);
+  hipLaunchKernelGGL(fn, dim3(grid_for(nchunks)), dim3(256), 0, (hipStream_t)stream, in, out, nchunks, n, param, param2,
+                     (int64_t)grid_for(nchunks) * 256);
   TTM_LAUNCH_CHECK();
   return TTM_OK;
 }
@@ -280,14 +296,13 @@ TTM_EXPORT int ttm_clamp(const void *in, void *out, int dtype, int layout, int64
 // ---- binary, same shape: flat
 template <bool BF16>
 __global__ __launch_bounds__(256) void ttm_binary_flat_k(int op, const void *__restrict__ a, const void *__restrict__ b,
-                                                         void *__restrict__ out, int64_t nchunks) {
+                                                         void *__restrict__ out, int64_t nchunks, int64_t stride) {
   constexpr int EPC = BF16 ? 8 : 4;
-  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < nchunks; c += (int64_t)gridDim.x * 256) {
+  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < nchunks; c += stride) {
     float x[EPC], y[EPC];
     chunk_load<BF16>(a, c, x);
     chunk_load<BF16>(b, c, y);
-#pragma unroll
-    for (int i = 0; i < EPC; ++i) x[i] = binary_op(op, x[i], y[i]);
+    binary_all(op, x, y);
     chunk_store<BF16>(out, c, x);
   }
 }
@@ -297,14 +312,21 @@ struct BcastArgs {
   int64_t oshape[4], ashape[4], bshape[4];
   int tiled;
 };
+// the chunk kernels' shapes: extents of at most 2^31 elements a plane (chunkable), N operands behind the output
+template <int N>
+struct ChunkShapes {
+  uint32_t out[4], in[N][4];
+  int tiled;
+};
 
-__device__ __forceinline__ int64_t bcast_offset(const int64_t (&shape)[4], int64_t i0, int64_t i1, int64_t r, int64_t c,
+template <typename S>
+__device__ __forceinline__ int64_t bcast_offset(const S (&shape)[4], int64_t i0, int64_t i1, int64_t r, int64_t c,
                                                 int tiled) {
   i0 = shape[0] == 1 ? 0 : i0; i1 = shape[1] == 1 ? 0 : i1;
   r = shape[2] == 1 ? 0 : r; c = shape[3] == 1 ? 0 : c;
   int64_t batch = i0 * shape[1] + i1;
   if (tiled) {
-    int64_t pr = (shape[2] + 31) / 32 * 32, pc = (shape[3] + 31) / 32 * 32;
+    int64_t pr = ((int64_t)shape[2] + 31) / 32 * 32, pc = ((int64_t)shape[3] + 31) / 32 * 32;
     return batch * pr * pc + ttm_tiled_offset(r, c, pc / 32);
   }
   return (batch * shape[2] + r) * shape[3] + c;
@@ -350,11 +372,11 @@ struct ChunkPos {
   int valid;    // how many of its EPC columns do (fewer than EPC only in the last tile column of a ragged tile tensor)
 };
 template <int EPC>
-__device__ __forceinline__ ChunkPos chunk_pos(const int64_t (&oshape)[4], int tiled, uint32_t ci, uint32_t chunks_per_plane) {
-  const uint32_t R = (uint32_t)oshape[2], C = (uint32_t)oshape[3];
+__device__ __forceinline__ ChunkPos chunk_pos(const uint32_t (&oshape)[4], int tiled, uint32_t ci, uint32_t chunks_per_plane) {
+  const uint32_t R = oshape[2], C = oshape[3];
   ChunkPos q;
   const uint32_t batch = blockIdx.y;
-  q.i0 = batch / (uint32_t)oshape[1]; q.i1 = batch % (uint32_t)oshape[1];
+  q.i0 = batch / oshape[1]; q.i1 = batch % oshape[1];
   uint32_t r, c0;
   if (tiled) {
     const uint32_t w = ci * EPC, tile = w >> 10, e = w & 1023, face = e >> 8, tcols = (C + 31) >> 5;
@@ -371,7 +393,7 @@ __device__ __forceinline__ ChunkPos chunk_pos(const int64_t (&oshape)[4], int ti
   return q;
 }
 template <bool BF16, typename F>
-__device__ __forceinline__ void operand_chunk(const void *base, const int64_t (&shape)[4], const ChunkPos &q, int tiled, F (&v)[BF16 ? 8 : 4]) {
+__device__ __forceinline__ void operand_chunk(const void *base, const uint32_t (&shape)[4], const ChunkPos &q, int tiled, F (&v)[BF16 ? 8 : 4]) {
   constexpr int EPC = BF16 ? 8 : 4;
   const int64_t off = bcast_offset(shape, q.i0, q.i1, q.r, q.c0, tiled);
   if (shape[3] != 1) {
@@ -404,18 +426,19 @@ __device__ __forceinline__ void operand_chunk(const void *base, const int64_t (&
 
 template <bool BF16>
 __global__ __launch_bounds__(256) void ttm_binary_chunk_k(int op, const void *__restrict__ a, const void *__restrict__ b,
-                                                          void *__restrict__ out, BcastArgs p, uint32_t chunks_per_plane) {
+                                                          void *__restrict__ out, ChunkShapes<2> p, uint32_t chunks_per_plane, uint32_t stride) {
   constexpr int EPC = BF16 ? 8 : 4;
-  for (uint32_t ci = blockIdx.x * 256 + threadIdx.x; ci < chunks_per_plane; ci += gridDim.x * 256) {
-    const ChunkPos q = chunk_pos<EPC>(p.oshape, p.tiled, ci, chunks_per_plane);
+  for (uint32_t ci = blockIdx.x * 256 + threadIdx.x; ci < chunks_per_plane; ci += stride) {
+    const ChunkPos q = chunk_pos<EPC>(p.out, p.tiled, ci, chunks_per_plane);
     float x[EPC], y[EPC];
 #pragma unroll
     for (int i = 0; i < EPC; ++i) x[i] = 0.0f;
     if (q.live) {
-      operand_chunk<BF16>(a, p.ashape, q, p.tiled, x);
-      operand_chunk<BF16>(b, p.bshape, q, p.tiled, y);
+      operand_chunk<BF16>(a, p.in[0], q, p.tiled, x);
+      operand_chunk<BF16>(b, p.in[1], q, p.tiled, y);
+      binary_all(op, x, y);
 #pragma unroll
-      for (int i = 0; i < EPC; ++i) x[i] = i < q.valid ? binary_op(op, x[i], y[i]) : 0.0f;
+      for (int i = 0; i < EPC; ++i) x[i] = i < q.valid ? x[i] : 0.0f;
     }
     chunk_store<BF16>(out, q.out_chunk, x);
   }
@@ -476,14 +499,17 @@ TTM_EXPORT int ttm_eltwise_binary(int op, const void *a, const int64_t *a_shape,
   if (same && al && !ragged) {
     int64_t nchunks = total * es / 16;
     if (dtype == TTM_BF16)
-      hipLaunchKernelGGL(ttm_binary_flat_k<true>, dim3(grid_for(nchunks)), dim3(256), 0, s, op, a, b, out, nchunks);
+      hipLaunchKernelGGL(ttm_binary_flat_k<true>, dim3(grid_for(nchunks)), dim3(256), 0, s, op, a, b, out, nchunks, (int64_t)grid_for(nchunks) * 256);
     else
-      hipLaunchKernelGGL(ttm_binary_flat_k<false>, dim3(grid_for(nchunks)), dim3(256), 0, s, op, a, b, out, nchunks);
+      hipLaunchKernelGGL(ttm_binary_flat_k<false>, dim3(grid_for(nchunks)), dim3(256), 0, s, op, a, b, out, nchunks, (int64_t)grid_for(nchunks) * 256);
   } else if (chunkable(p.oshape, p.tiled, es, {a, b, out})) {
     const uint32_t cpp = (uint32_t)(pr * pc * es / 16);
     const dim3 grid(grid_for(cpp), (unsigned)(p.oshape[0] * p.oshape[1]));
-    if (dtype == TTM_BF16) hipLaunchKernelGGL(ttm_binary_chunk_k<true>, grid, dim3(256), 0, s, op, a, b, out, p, cpp);
-    else hipLaunchKernelGGL(ttm_binary_chunk_k<false>, grid, dim3(256), 0, s, op, a, b, out, p, cpp);
+    ChunkShapes<2> q;
+    for (int d = 0; d < 4; ++d) { q.out[d] = (uint32_t)p.oshape[d]; q.in[0][d] = (uint32_t)p.ashape[d]; q.in[1][d] = (uint32_t)p.bshape[d]; }
+    q.tiled = p.tiled;
+    if (dtype == TTM_BF16) hipLaunchKernelGGL(ttm_binary_chunk_k<true>, grid, dim3(256), 0, s, op, a, b, out, q, cpp, grid.x * 256);
+    else hipLaunchKernelGGL(ttm_binary_chunk_k<false>, grid, dim3(256), 0, s, op, a, b, out, q, cpp, grid.x * 256);
   } else {
     if (dtype == TTM_BF16)
       hipLaunchKernelGGL(ttm_binary_bcast_k<true>, dim3(grid_for(total)), dim3(256), 0, s, op, a, b, out, p, total);
@@ -530,17 +556,17 @@ __global__ __launch_bounds__(256) void ttm_where_k(const void *__restrict__ cond
 
 template <bool BF16>
 __global__ __launch_bounds__(256) void ttm_where_chunk_k(const void *__restrict__ cond, const void *__restrict__ a, const void *__restrict__ b,
-                                                         void *__restrict__ out, WhereArgs p, uint32_t chunks_per_plane) {
+                                                         void *__restrict__ out, ChunkShapes<3> p, uint32_t chunks_per_plane, uint32_t stride) {
   constexpr int EPC = BF16 ? 8 : 4;
-  for (uint32_t ci = blockIdx.x * 256 + threadIdx.x; ci < chunks_per_plane; ci += gridDim.x * 256) {
-    const ChunkPos q = chunk_pos<EPC>(p.oshape, p.tiled, ci, chunks_per_plane);
+  for (uint32_t ci = blockIdx.x * 256 + threadIdx.x; ci < chunks_per_plane; ci += stride) {
+    const ChunkPos q = chunk_pos<EPC>(p.out, p.tiled, ci, chunks_per_plane);
     uint32_t cv[EPC], av[EPC], bv[EPC];
 #pragma unroll
     for (int i = 0; i < EPC; ++i) av[i] = 0u;
     if (q.live) {
-      operand_chunk<BF16>(cond, p.cshape, q, p.tiled, cv);
-      operand_chunk<BF16>(a, p.ashape, q, p.tiled, av);
-      operand_chunk<BF16>(b, p.bshape, q, p.tiled, bv);
+      operand_chunk<BF16>(cond, p.in[0], q, p.tiled, cv);
+      operand_chunk<BF16>(a, p.in[1], q, p.tiled, av);
+      operand_chunk<BF16>(b, p.in[2], q, p.tiled, bv);
 #pragma unroll
       for (int i = 0; i < EPC; ++i)   // +-0 is false, NaN is true; columns in the padding stay zero
         av[i] = i >= q.valid ? 0u : ((cv[i] & (BF16 ? 0x7FFFu : 0x7FFFFFFFu)) != 0 ? av[i] : bv[i]);
@@ -586,8 +612,14 @@ TTM_EXPORT int ttm_where(const void *cond, const int64_t *cond_shape, const void
   if (chunkable(p.oshape, p.tiled, es, {cond, a, b, out})) {
     const uint32_t cpp = (uint32_t)(pr * pc * es / 16);
     const dim3 grid(grid_for(cpp), (unsigned)(p.oshape[0] * p.oshape[1]));
-    if (dtype == TTM_BF16) hipLaunchKernelGGL(ttm_where_chunk_k<true>, grid, dim3(256), 0, (hipStream_t)stream, cond, a, b, out, p, cpp);
-    else hipLaunchKernelGGL(ttm_where_chunk_k<false>, grid, dim3(256), 0, (hipStream_t)stream, cond, a, b, out, p, cpp);
+    ChunkShapes<3> q;
+    for (int d = 0; d < 4; ++d) {
+      q.out[d] = (uint32_t)p.oshape[d];
+      q.in[0][d] = (uint32_t)p.cshape[d]; q.in[1][d] = (uint32_t)p.ashape[d]; q.in[2][d] = (uint32_t)p.bshape[d];
+    }
+    q.tiled = p.tiled;
+    if (dtype == TTM_BF16) hipLaunchKernelGGL(ttm_where_chunk_k<true>, grid, dim3(256), 0, (hipStream_t)stream, cond, a, b, out, q, cpp, grid.x * 256);
+    else hipLaunchKernelGGL(ttm_where_chunk_k<false>, grid, dim3(256), 0, (hipStream_t)stream, cond, a, b, out, q, cpp, grid.x * 256);
     TTM_LAUNCH_CHECK();
     return TTM_OK;
   }
@@ -636,8 +668,8 @@ __global__ __launch_bounds__(256) void ttm_typecast_k(const void *__restrict__ i
 // bf16 <-> fp32 in groups of four elements per lane: 8 bytes of bf16 against 16 of fp32, every instruction of a wavefront
 // touching one contiguous run (the element-wise kernel above moves 2 + 4 bytes per lane and reaches half the bandwidth)
 template <bool WIDEN>
-__global__ __launch_bounds__(256) void ttm_typecast4_k(const void *__restrict__ in, void *__restrict__ out, int64_t groups) {
-  for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < groups; g += (int64_t)gridDim.x * 256) {
+__global__ __launch_bounds__(256) void ttm_typecast4_k(const void *__restrict__ in, void *__restrict__ out, int64_t groups, int64_t stride) {
+  for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < groups; g += stride) {
     if (WIDEN) {
       const u32x2 v = __builtin_nontemporal_load((const u32x2 *)in + g);
       const u32x4 w = {v.x << 16, v.x & 0xFFFF0000u, v.y << 16, v.y & 0xFFFF0000u};
@@ -684,8 +716,8 @@ TTM_EXPORT int ttm_typecast(const void *in, int src_dtype, void *out, int dst_dt
   TTM_REQUIRE(in && out, "ttm_typecast: null pointer");
   const bool widen = src_dtype == TTM_BF16 && dst_dtype == TTM_F32, narrow = src_dtype == TTM_F32 && dst_dtype == TTM_BF16;
   if ((widen || narrow) && n % 4 == 0 && (((uintptr_t)in | (uintptr_t)out) & 15) == 0) {
-    if (widen) hipLaunchKernelGGL(ttm_typecast4_k<true>, dim3(grid_for(n / 4)), dim3(256), 0, (hipStream_t)stream, in, out, n / 4);
-    else hipLaunchKernelGGL(ttm_typecast4_k<false>, dim3(grid_for(n / 4)), dim3(256), 0, (hipStream_t)stream, in, out, n / 4);
+    if (widen) hipLaunchKernelGGL(ttm_typecast4_k<true>, dim3(grid_for(n / 4)), dim3(256), 0, (hipStream_t)stream, in, out, n / 4, (int64_t)grid_for(n / 4) * 256);
+    else hipLaunchKernelGGL(ttm_typecast4_k<false>, dim3(grid_for(n / 4)), dim3(256), 0, (hipStream_t)stream, in, out, n / 4, (int64_t)grid_for(n / 4) * 256);
     TTM_LAUNCH_CHECK();
     return TTM_OK;
   }

@@ -63,13 +63,13 @@ using layout_elem = typename std::conditional<ELEM == 4, uint32_t, typename std:
 
 template <int ELEM, int U, bool TILIZE>
 __global__ __launch_bounds__(256) void ttm_tile_direct_k(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int rows, int cols, int lw, int wc,
-                                                         uint32_t xu, uint32_t matrices, uint32_t first) {
+                                                         uint32_t xu, uint32_t matrices, uint32_t first, uint32_t groups) {
   typedef layout_elem<ELEM> T;
   constexpr int V = 16 / ELEM;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ct = (cols + 31) >> 5, yt = (rows + 31) >> 5;
   // a wavefront's accesses are 1 << lw chunks wide, a workgroup 1 << wc wavefronts; its other wavefronts lie below
-  const uint32_t bid = first + xcd_order(), by = bid / xu;
+  const uint32_t bid = first + xcd_order(groups), by = bid / xu;
   const int chunk = (int)((((bid - by * xu) << wc) + (wave & ((1 << wc) - 1))) << lw) + (lane & ((1 << lw) - 1));
   const uint32_t row0 = ((by << (2 - wc)) + (wave >> wc)) * (64 >> lw) * U + (lane >> lw);   // of the rows of all matrices, padded ones for tilize
   const uint32_t per = TILIZE ? yt * 32 : rows;
@@ -304,7 +304,7 @@ static int run_layout(const void *src, void *dst, int64_t batch, int64_t rows, i
 #define DIRECT(E, U)                                                                                                                            \
   ttm_launches(groups * xu, [&](uint32_t first, dim3 grid) {                                                                                    \
     hipLaunchKernelGGL((ttm_tile_direct_k<E, U, TILIZE>), grid, dim3(256), 0, s, (const uint8_t *)src, (uint8_t *)dst, (int)rows, (int)cols, lw, wc, \
-                       (uint32_t)xu, (uint32_t)batch, first);                                                                                   \
+                       (uint32_t)xu, (uint32_t)batch, first, grid.x);                                                                           \
   })
 #define DIRECT_U(E)                                       \
   do {                                                    \

@@ -23,6 +23,7 @@ struct LinearArgs {
   int nt_split, n_blocks1, ntw2;      // two-part grid: blocks [0, n_blocks1) cover column tiles [0, nt_split) at width ntw,
                                       // the rest cover [nt_split, Nt) at width ntw2; nt_split = 0: one part
   int k_slice;                        // k-tiles per grid.y slice (split-K); Kt when the reduction is not split
+  int slices;                         // of K (grid.y) in a launch that leaves partial sums
   float *partial;                     // split-K: fp32 partial sums [slices][Mt * Nt * 1024] in output tile order
   int img_zero_step;                  // two-pass launch: W points at the dequantised images, this step index holds zeros
   // group launch (group_n >= 2): several weight matrices [K, N_i] applied to the same activations, each with its own
@@ -39,7 +40,33 @@ struct LinearArgs {
   int plan_batch;                     // host side only: batch entries the launch plan counts (a pair of matrices plans as one alone)
   const struct QkvFinishArgs *qkv;    // host side only: the decode launch leaves partial sums and ttm_qkv_finish_k ends it
   const struct NormFinishArgs *norm;  // host side only: ... and the RMSNorm kernel ends it (residual add, then the norm)
+  __device__ __forceinline__ const LinearArgs &full() const { return *this; }
 };
+
+// The same for a launch that is neither a group nor a gated pair, in the 112 bytes that launch quickly (ttm_common.h)
+struct LinearPlain {
+  const uint8_t *A, *W;
+  const uint16_t *bias;
+  uint8_t *C;
+  int Mt, Nt, Kt;
+  uint8_t act, bias_tiled, tail;
+  int n_blocks, k_slice, slices;
+  int64_t a_batch, w_batch, c_batch;
+  float *partial;
+  int64_t tail_delta;
+  explicit LinearPlain(const LinearArgs &a)
+      : A(a.A), W(a.W), bias(a.bias), C(a.C), Mt(a.Mt), Nt(a.Nt), Kt(a.Kt), act((uint8_t)a.act), bias_tiled((uint8_t)a.bias_tiled), tail((uint8_t)a.tail),
+        n_blocks(a.n_blocks), k_slice(a.k_slice), slices(a.slices), a_batch(a.a_batch), w_batch(a.w_batch), c_batch(a.c_batch), partial(a.partial),
+        tail_delta(a.tail_delta) {}
+  __device__ __forceinline__ LinearArgs full() const {
+    LinearArgs p = {};
+    p.A = A; p.W = W; p.bias = bias; p.C = C; p.Mt = Mt; p.Nt = Nt; p.Kt = Kt; p.act = act; p.bias_tiled = bias_tiled; p.tail = tail;
+    p.n_blocks = n_blocks; p.k_slice = k_slice; p.slices = slices; p.a_batch = a_batch; p.w_batch = w_batch; p.c_batch = c_batch;
+    p.partial = partial; p.tail_delta = tail_delta;
+    return p;
+  }
+};
+static_assert(sizeof(LinearPlain) <= 112, "the size up to which a launch is quick");
 
 // x1 = residual + projection (stored to sum_out), then out = rms_norm(x1): the operands of the second launch
 struct NormFinishArgs {
@@ -214,7 +241,7 @@ static inline int column_units(const LinearArgs &p, int unit_tiles) {
 
 
 // Split-K partial sums -> output (ttm_linear.hip): grid ((per / 4 + 255) / 256, 1, batch) of 256 lanes, per = Mt * Nt * 1024
-void ttm_linear_launch_reduce(const LinearArgs &p, int slices, int64_t batch, hipStream_t s);
+void ttm_linear_launch_reduce(const LinearArgs &p, int64_t batch, hipStream_t s);
 
 // The mid-size kernel (ttm_linear_mid.hip).  Launch plan: row tiles per workgroup, shares of K in a workgroup (wavefronts), slices
 // of K over grid.y, modelled time.

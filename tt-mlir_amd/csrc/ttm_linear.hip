@@ -298,7 +298,10 @@ __device__ __forceinline__ void linear_epilogue_glu(const LinearArgs &p, uint8_t
 }
 
 // split-K: sums the slices, then bias, activation and bf16 as in the fused epilogue; one lane per four elements
-__global__ __launch_bounds__(256) void ttm_linear_reduce_k(LinearArgs p, int slices) {
+template <class ARGS>
+__global__ __launch_bounds__(256) void ttm_linear_reduce_k(ARGS args) {
+  const LinearArgs p = args.full();
+  const int slices = p.slices;
   const int64_t per = (int64_t)p.Mt * p.Nt * 1024;
   const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;   // group of four consecutive elements
   if (q * 4 >= per) return;
@@ -1423,7 +1426,8 @@ __global__ __launch_bounds__(256) void ttm_linear_image_group_k(ImageGroup g, in
 // resident).  Partial sums are reduced through LDS.
 // =============================================================================================
 template <int WF>
-__global__ __launch_bounds__(256) void ttm_linear_small_k(LinearArgs p) {
+__global__ __launch_bounds__(256) void ttm_linear_small_k(LinearPlain args) {
+  const LinearArgs p = args.full();
   __shared__ u32x4 smem[4 * 512];  // per wave: 32 rows x 16 chunks (128 k)
   __shared__ float red[3][16][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1563,8 +1567,9 @@ __global__ __launch_bounds__(256) void ttm_linear_small_k(LinearArgs p) {
 // or steps, V and S go through the matrix cores into two accumulators, and the result is their difference: twice the
 // MFMAs (which were idle) for less than half the vector instructions.  The two sums are each a few times larger than
 // their difference, so the fp32 rounding error grows by that factor - still four decimal orders below a bf16 result.
-template <bool BFP4, bool TWO_TERM, int NP, bool GLU>
-__global__ __launch_bounds__(512) void ttm_linear_decode_k(LinearArgs p) {
+template <bool BFP4, bool TWO_TERM, int NP, bool GLU, class ARGS>
+__global__ __launch_bounds__(512) void ttm_linear_decode_k(ARGS args) {
+  const LinearArgs p = args.full();
   extern __shared__ u32x4 smem[];   // partial sums: NP x 8 wavefronts x 8 x 64 float4 = NP x 64 KiB
   constexpr int D = 2;
   constexpr bool WL = !BFP4;   // whole-row loads and a transpose within lane quads (bfp8_b)
@@ -1784,7 +1789,7 @@ __global__ __launch_bounds__(512) void ttm_linear_decode_k(LinearArgs p) {
     const int64_t off = (int64_t)nt * 1024 + in;
     if (p.partial) {   // bias, activation and rounding happen in ttm_linear_reduce_k
       const int64_t per = (int64_t)p.Nt * 1024;   // a group's partial sums are laid out as the concatenation
-      *(f32x4v *)(p.partial + ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * per + (int64_t)tile_base * 1024 + off) = sum;
+      *(f32x4v *)(p.partial + ((int64_t)blockIdx.z * p.slices + blockIdx.y) * per + (int64_t)tile_base * 1024 + off) = sum;
       continue;
     }
     float v[4] = {sum[0] + __uint_as_float(bias[pr].x << 16), sum[1] + __uint_as_float(bias[pr].x & 0xFFFF0000u),
@@ -1911,9 +1916,28 @@ static int set_lds_limit(K kernel, int bytes) {
   return 0;
 }
 
-void ttm_linear_launch_reduce(const LinearArgs &p, int slices, int64_t batch, hipStream_t s) {
+void ttm_linear_launch_reduce(const LinearArgs &p, int64_t batch, hipStream_t s) {
   const int64_t per = (int64_t)p.Mt * p.Nt * 1024;
-  hipLaunchKernelGGL(ttm_linear_reduce_k, dim3((unsigned)((per / 4 + 255) / 256), 1, (unsigned)batch), dim3(256), 0, s, p, slices);
+  const dim3 grid((unsigned)((per / 4 + 255) / 256), 1, (unsigned)batch);
+  if (p.group_n > 1) hipLaunchKernelGGL(ttm_linear_reduce_k<LinearArgs>, grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL(ttm_linear_reduce_k<LinearPlain>, grid, dim3(256), 0, s, LinearPlain(p));
+}
+
+template <bool BFP4, bool TWO_TERM, int NP, bool GLU, class ARGS>
+static int launch_decode(const ARGS &p, dim3 grid, hipStream_t s) {
+  if constexpr (NP == 2) {
+    static bool attr = false;
+    if (!attr) {
+      if (int rc = set_lds_limit(ttm_linear_decode_k<BFP4, TWO_TERM, NP, GLU, ARGS>, 131072)) return rc;
+      attr = true;
+    }
+  }
+  hipLaunchKernelGGL((ttm_linear_decode_k<BFP4, TWO_TERM, NP, GLU, ARGS>), grid, dim3(512), NP * 65536, s, p);
+  return 0;
+}
+template <bool BFP4, bool TWO_TERM, class ARGS>
+static int launch_decode(const ARGS &p, int np, dim3 grid, hipStream_t s) {
+  return np == 2 ? launch_decode<BFP4, TWO_TERM, 2, false, ARGS>(p, grid, s) : launch_decode<BFP4, TWO_TERM, 1, false, ARGS>(p, grid, s);
 }
 
 // The mid-size kernel is the library's own choice: an option that pins another kernel or its plan rules it out.
@@ -2016,6 +2040,7 @@ static int launch_linear(const LinearArgs &a, int64_t batch, hipStream_t s) {
       void *ws = nullptr;
       if (int rc = ttm_stream_workspace(s, (size_t)(per * slices * batch) * sizeof(float), &ws)) return rc;
       p.partial = (float *)ws;
+      p.slices = slices;
       p.Mt = 1;   // the reduction sees one row tile per launch
     }
     for (int mt = 0; mt < a.Mt; ++mt) {
@@ -2026,24 +2051,13 @@ static int launch_linear(const LinearArgs &a, int64_t batch, hipStream_t s) {
       const bool two_term = ttm_option("linear_decode_variant") != 1;   // 1 = operands by int -> float conversion
       if (decode) {
         constexpr bool B4 = WF == WF_BFP4;
-        if (np == 2) {
-          static bool attr = false;
-          if (!attr) {
-            if (int rc = set_lds_limit(ttm_linear_decode_k<B4, true, 2, false>, 131072)) return rc;
-            if (int rc = set_lds_limit(ttm_linear_decode_k<B4, false, 2, false>, 131072)) return rc;
-            if (int rc = set_lds_limit(ttm_linear_decode_k<B4, true, 2, true>, 131072)) return rc;
-            if (int rc = set_lds_limit(ttm_linear_decode_k<B4, false, 2, true>, 131072)) return rc;
-            attr = true;
-          }
-          if (a.glu) {
-            if (two_term) hipLaunchKernelGGL((ttm_linear_decode_k<B4, true, 2, true>), grid, dim3(512), 131072, s, p);
-            else hipLaunchKernelGGL((ttm_linear_decode_k<B4, false, 2, true>), grid, dim3(512), 131072, s, p);
-          } else if (two_term) hipLaunchKernelGGL((ttm_linear_decode_k<B4, true, 2, false>), grid, dim3(512), 131072, s, p);
-          else hipLaunchKernelGGL((ttm_linear_decode_k<B4, false, 2, false>), grid, dim3(512), 131072, s, p);
-        } else if (two_term) hipLaunchKernelGGL((ttm_linear_decode_k<B4, true, 1, false>), grid, dim3(512), 65536, s, p);
-        else hipLaunchKernelGGL((ttm_linear_decode_k<B4, false, 1, false>), grid, dim3(512), 65536, s, p);
+        if (a.glu) {
+          if (int rc = two_term ? launch_decode<B4, true, 2, true, LinearArgs>(p, grid, s) : launch_decode<B4, false, 2, true, LinearArgs>(p, grid, s)) return rc;
+        } else if (a.group_n > 1) {
+          if (int rc = two_term ? launch_decode<B4, true, LinearArgs>(p, np, grid, s) : launch_decode<B4, false, LinearArgs>(p, np, grid, s)) return rc;
+        } else if (int rc = two_term ? launch_decode<B4, true>(LinearPlain(p), np, grid, s) : launch_decode<B4, false>(LinearPlain(p), np, grid, s)) return rc;
       }
-      else hipLaunchKernelGGL((ttm_linear_small_k<WF>), dim3(a.Nt, 1, (unsigned)batch), dim3(256), 0, s, p);
+      else hipLaunchKernelGGL((ttm_linear_small_k<WF>), dim3(a.Nt, 1, (unsigned)batch), dim3(256), 0, s, LinearPlain(p));
       if (a.qkv) {
         QkvFinishArgs f = *a.qkv;
         f.partial = p.partial; f.slices = slices; f.per = per;
@@ -2054,8 +2068,7 @@ static int launch_linear(const LinearArgs &a, int64_t batch, hipStream_t s) {
         if (int rc = ttm_rowwise_rmsnorm_from_partials(p.partial, slices, per, f.residual, f.sum_out, f.weight, f.weight_layout, f.bias,
                                                        f.bias_layout, f.out, f.rows, f.cols, f.eps, s))
           return rc;
-      } else if (slices > 1)
-        hipLaunchKernelGGL(ttm_linear_reduce_k, dim3((unsigned)((per / 4 + 255) / 256), 1, (unsigned)batch), dim3(256), 0, s, p, slices);
+      } else if (slices > 1) ttm_linear_launch_reduce(p, batch, s);
     }
     return 0;
   }
@@ -2123,6 +2136,7 @@ static int launch_linear(const LinearArgs &a, int64_t batch, hipStream_t s) {
       if (img_bytes + part_bytes > 0)
         if (int rc = ttm_stream_workspace(s, img_bytes + part_bytes, (void **)&ws)) return rc;
       if (slices > 1) p.partial = (float *)(ws + img_bytes);
+      p.slices = slices;
       if (two_pass && slices == 1 && p.nt_split == 0) {
         // without the conversion a block may be seven tiles wide (the wavefronts of a SIMD take 4 + 3): worth it when
         // that fills the last round, e.g. 8 x 448 tiles = 448 blocks of 8 (1.75 rounds on 256 CUs, paid as 2) against 512
@@ -2171,8 +2185,7 @@ static int launch_linear(const LinearArgs &a, int64_t batch, hipStream_t s) {
       } else if constexpr (BFP) {
         hipLaunchKernelGGL((ttm_linear_dma_k<WF>), dim3(p.n_blocks, slices, (unsigned)batch), dim3(512), lds6, s, p);
       }
-      if (slices > 1)
-        hipLaunchKernelGGL(ttm_linear_reduce_k, dim3((unsigned)((per / 4 + 255) / 256), 1, (unsigned)batch), dim3(256), 0, s, p, slices);
+      if (slices > 1) ttm_linear_launch_reduce(p, batch, s);
       return 0;
     }
   }
@@ -2237,7 +2250,7 @@ static int linear_entry(const void *a, int a_dtype, const void *w, int w_dtype, 
   p.c_batch = (int64_t)p.Mt * p.Nt * 2048;
   p.m_blocks = (p.Mt + 7) / 8; p.n_blocks = (p.Nt + 7) / 8;
   p.ntw = 4;
-  p.k_slice = p.Kt; p.partial = nullptr;
+  p.k_slice = p.Kt; p.slices = 1; p.partial = nullptr;
   p.nt_split = p.n_blocks1 = p.ntw2 = 0;
   p.img_zero_step = 0;
   p.group_n = 0; p.glu = 0;
@@ -2361,7 +2374,7 @@ TTM_EXPORT int ttm_linear_glu(const void *a, const void *w_gate, const void *w_u
   p.a_batch = p.w_batch = p.c_batch = 0;
   p.m_blocks = 1; p.n_blocks = (p.Nt + 7) / 8;
   p.ntw = 4;
-  p.k_slice = p.Kt; p.partial = nullptr;
+  p.k_slice = p.Kt; p.slices = 1; p.partial = nullptr;
   p.nt_split = p.n_blocks1 = p.ntw2 = 0;
   p.img_zero_step = 0;
   p.tail = TTM_TAIL_NONE; p.tail_delta = 0;
@@ -2431,7 +2444,7 @@ static int linear_group_entry(const void *a, int n, const void *const *w, int w_
   p.a_batch = p.w_batch = p.c_batch = 0;
   p.m_blocks = (p.Mt + 7) / 8; p.n_blocks = (p.Nt + 7) / 8;
   p.ntw = 4;
-  p.k_slice = p.Kt; p.partial = nullptr;
+  p.k_slice = p.Kt; p.slices = 1; p.partial = nullptr;
   p.nt_split = p.n_blocks1 = p.ntw2 = 0;
   p.img_zero_step = 0;
   p.tail = TTM_TAIL_NONE; p.tail_delta = 0;

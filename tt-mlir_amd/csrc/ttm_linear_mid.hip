@@ -12,8 +12,9 @@
 // weights: 64), 128 MT of the matrix core, 32 + 32 MT of L1; MT = 2 balances them for short launches, MT = 4 halves the weight
 // traffic and conversions where the row count fills it.
 // =============================================================================================
-template <int WF, int MT, int WK, bool TT, bool GLU>
-__global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(LinearArgs p) {
+template <int WF, int MT, int WK, bool TT, bool GLU, class ARGS>
+__global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(ARGS args) {
+  const LinearArgs p = args.full();
   constexpr int WN = GLU ? 2 : 1;    // column pairs of the workgroup
   constexpr int THREADS = WN * WK * 64, D = 2;
   __shared__ f32x4v part[WN * WK * 512];   // partial sums of one row tile: per wavefront 8 x 64 float4 = 8 KiB
@@ -242,7 +243,7 @@ __global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(Line
         linear_act_rt(p.gAct[1], v1);
         *(u32x2 *)c = glu_quad(v, v1);
       } else if (p.partial) {   // bias, activation and rounding happen in ttm_linear_reduce_k
-        *(f32x4v *)(p.partial + (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * p.Mt + mt0 + r) * p.Nt * 1024 + (int64_t)(tile_base + nt) * 1024 + in) = sums[0];
+        *(f32x4v *)(p.partial + (((int64_t)blockIdx.z * p.slices + blockIdx.y) * p.Mt + mt0 + r) * p.Nt * 1024 + (int64_t)(tile_base + nt) * 1024 + in) = sums[0];
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] += bv[e];
@@ -294,7 +295,8 @@ MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu, int max_slice
 template <int WF, int MT, int WK, bool TT>
 static void launch_mid_mt(const LinearArgs &p, dim3 grid, hipStream_t s) {
   constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
-  hipLaunchKernelGGL((ttm_linear_mid_k<WF, MT, WK, TT && BFP, false>), grid, dim3(WK * 64), 0, s, p);
+  if (p.group_n > 1) hipLaunchKernelGGL((ttm_linear_mid_k<WF, MT, WK, TT && BFP, false, LinearArgs>), grid, dim3(WK * 64), 0, s, p);
+  else hipLaunchKernelGGL((ttm_linear_mid_k<WF, MT, WK, TT && BFP, false, LinearPlain>), grid, dim3(WK * 64), 0, s, LinearPlain(p));
 }
 template <int WF>
 static int launch_mid(const LinearArgs &a, const MidPlan &plan, int64_t batch, bool glu, hipStream_t s) {
@@ -312,12 +314,13 @@ static int launch_mid(const LinearArgs &a, const MidPlan &plan, int64_t batch, b
     if (int rc = ttm_stream_workspace(s, (size_t)(per * slices * batch) * sizeof(float), &ws)) return rc;
     p.partial = (float *)ws;
   }
+  p.slices = slices;
   p.n_blocks = mid_units(a, glu);
   const dim3 grid((unsigned)((p.n_blocks + 7) / 8 * 8 * ((p.Mt + plan.mt - 1) / plan.mt)), (unsigned)slices, (unsigned)batch);
   if (glu) {
     if constexpr (WF == WF_BFP8) {
-      if (plan.mt == 2) hipLaunchKernelGGL((ttm_linear_mid_k<WF_BFP8, 2, 4, false, true>), grid, dim3(512), 0, s, p);
-      else hipLaunchKernelGGL((ttm_linear_mid_k<WF_BFP8, 4, 4, false, true>), grid, dim3(512), 0, s, p);
+      if (plan.mt == 2) hipLaunchKernelGGL((ttm_linear_mid_k<WF_BFP8, 2, 4, false, true, LinearArgs>), grid, dim3(512), 0, s, p);
+      else hipLaunchKernelGGL((ttm_linear_mid_k<WF_BFP8, 4, 4, false, true, LinearArgs>), grid, dim3(512), 0, s, p);
       return 0;
     }
     return ttm_set_error(TTM_ERR_INVALID, "ttm_linear_glu: the mid-size kernel's gated form takes bfp8_b weights");
@@ -334,7 +337,7 @@ static int launch_mid(const LinearArgs &a, const MidPlan &plan, int64_t batch, b
   default: launch_mid_mt<WF, 2, 4, false>(p, grid, s);   // 42: ttm_linear_plan_mid has no others
   }
   if (slices > 1)
-    ttm_linear_launch_reduce(p, slices, batch, s);
+    ttm_linear_launch_reduce(p, batch, s);
   return 0;
 }
 

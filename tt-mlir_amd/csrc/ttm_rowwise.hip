@@ -15,16 +15,16 @@ struct RowArgs {
   const void *x;
   void *out;
   const void *w, *b;   // rmsnorm weight / bias (same dtype as x) or null
-  int w_tiled, b_tiled;
-  int64_t rows, cols;  // logical extent of the last two dims
+  int64_t rows;        // logical extent of the last two dims
+  int cols;
   int rt, ct;          // tiles per batch entry
   float eps;
-  int stream;          // band kernel: the input is read past the caches
-  int out_ct;          // reductions: column tiles of the output (1), keepdim layout [.., rows, 1]
+  uint8_t w_tiled, b_tiled;
+  uint8_t stream;      // band kernel: the input is read past the caches
   // ttm_rowwise_row_k<.., PRE = true>: x is not read but made on the way in from the fp32 partial sums of a split-K
   // projection of one row tile, x = bf16(bf16(sum over slices) + residual), and also stored to sum_out
-  const float *partial;
   int slices;
+  const float *partial;
   int64_t per;         // floats per slice
   const void *residual;
   void *sum_out;
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256) void ttm_rowwise_k(RowArgs p) {
   const bool row_ok = row < p.rows;
   const int nq = p.ct * 2 * ELEM;                        // chunks per row
   const uint8_t *x = (const uint8_t *)p.x + trow * p.ct * 1024 * ELEM;
-  const int cols = (int)p.cols;
+  const int cols = p.cols;
 
   constexpr bool IS_MAX = MODE == RW_SOFTMAX || MODE == RW_MAX;
   float acc = IS_MAX ? -INFINITY : (MODE == RW_MIN ? INFINITY : 0.0f);
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256) void ttm_rowwise_resident_k(RowArgs p) {
   const int nq = p.ct * 2 * ELEM;
   const uint8_t *x = (const uint8_t *)p.x + (int64_t)trow * p.ct * 1024 * ELEM;
   uint8_t *o = (uint8_t *)p.out + (int64_t)trow * p.ct * 1024 * ELEM;
-  const int cols = (int)p.cols;
+  const int cols = p.cols;
   const int nk = (nq - j + J - 1) / J;   // chunks of this lane
   float acc = MODE == RW_SOFTMAX ? -INFINITY : 0.0f;
 #pragma unroll 8
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(NT) void ttm_rowwise_row_k(RowArgs p, int total_row
   const int r = lrow & 31, trow = lrow >> 5;
   const int row = (trow % p.rt) * 32 + r;
   const bool row_ok = row < p.rows;
-  const int nq = p.ct * 2 * ELEM, cols = (int)p.cols;
+  const int nq = p.ct * 2 * ELEM, cols = p.cols;
   const uint8_t *x = (const uint8_t *)p.x + (int64_t)trow * p.ct * 1024 * ELEM;
   uint8_t *o = (uint8_t *)p.out + (int64_t)trow * p.ct * 1024 * ELEM;
   u32x4 v[NK];
@@ -451,7 +451,7 @@ __global__ __launch_bounds__(NT) TTM_MAX_WAVES((band_max_waves<MODE, ELEM, NK, N
   const int r = g4 * 4 + rl;
   const int64_t row = (trow % p.rt) * 32 + r;
   const bool row_ok = row < p.rows;
-  const int nruns = p.ct * 2, cols = (int)p.cols;        // runs per band: one per (tile, face column)
+  const int nruns = p.ct * 2, cols = p.cols;        // runs per band: one per (tile, face column)
   const uint8_t *x = (const uint8_t *)p.x + trow * p.ct * 1024 * ELEM;
   // chunk k of this lane: run tid / RUN + k * (NT / RUN)
   auto run_of = [&](int k) { return tid / RUN + k * (NT / RUN); };
@@ -657,7 +657,7 @@ __global__ __launch_bounds__(256) void ttm_rowwise_wide_stats_k(RowArgs p, float
   constexpr int EPC = L::EPC;
   constexpr bool IS_MAX = MODE == RW_SOFTMAX || MODE == RW_MAX;
   __shared__ float sa[256], sb[256];
-  const int tid = threadIdx.x, slice = blockIdx.x, cols = (int)p.cols;
+  const int tid = threadIdx.x, slice = blockIdx.x, cols = p.cols;
   const int64_t trow = blockIdx.y;
   const L ln(tid);
   const uint8_t *x = (const uint8_t *)p.x + trow * p.ct * 1024 * ELEM;
@@ -748,7 +748,7 @@ __global__ __launch_bounds__(256) void ttm_rowwise_wide_apply_k(RowArgs p, const
   using L = WideLane<ELEM>;
   constexpr int EPC = L::EPC;
   __shared__ float ga[32], gb[32], ta[256], tb[256];
-  const int tid = threadIdx.x, slice = blockIdx.x, cols = (int)p.cols;
+  const int tid = threadIdx.x, slice = blockIdx.x, cols = p.cols;
   const int64_t trow = blockIdx.y;
   wide_totals<MODE>(stats + trow * 32 * slices * 2, slices, ga, gb, ta, tb);
   const L ln(tid);
@@ -913,9 +913,9 @@ static int fill_args(RowArgs &p, const void *x, void *out, int dtype, int64_t ba
   TTM_REQUIRE(x && out, "%s: null pointer", who);
   TTM_REQUIRE(((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0, "%s: pointers must be 16-byte aligned", who);
   p.x = x; p.out = out; p.w = p.b = nullptr; p.w_tiled = p.b_tiled = 0;
-  p.rows = rows; p.cols = cols;
+  p.rows = rows; p.cols = (int)cols;
   p.rt = (int)ttm_cdiv(rows, 32); p.ct = (int)ttm_cdiv(cols, 32);
-  p.eps = 0.0f; p.stream = 0; p.out_ct = 1;
+  p.eps = 0.0f; p.stream = 0;
   p.partial = nullptr; p.slices = 0; p.per = 0; p.residual = nullptr; p.sum_out = nullptr;
   return TTM_OK;
 }
