@@ -2,6 +2,7 @@
 
   lib/libttmlir_amd_hip.so   gfx950 kernels + C ABI (csrc/*.hip, hipcc)
   lib/libttmlir_amd_rt.so    C++ host runtime in the tt::runtime style (runtime/*.cpp, g++)
+  lib/_ttm_call.so           the kernel library's entry points as Python calls (runtime/py_call.cpp, g++)
 
 Usage: python build.py [--force] [--jobs N]
 """
@@ -10,8 +11,10 @@ import concurrent.futures
 import glob
 import os
 import shutil
+import re
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -23,6 +26,8 @@ INCLUDE = os.path.join(ROOT, "include")
 
 HIP_LIB = os.path.join(LIBDIR, "libttmlir_amd_hip.so")
 RT_LIB = os.path.join(LIBDIR, "libttmlir_amd_rt.so")
+CALL_LIB = os.path.join(LIBDIR, "_ttm_call.so")
+CALL_SRC = os.path.join(RTSRC, "py_call.cpp")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = [
@@ -77,7 +82,7 @@ def build_hip(force=False, jobs=8, verbose=True):
 
 
 def build_runtime(force=False, jobs=8, verbose=True):
-    srcs = sorted(glob.glob(os.path.join(RTSRC, "*.cpp")))
+    srcs = [s for s in sorted(glob.glob(os.path.join(RTSRC, "*.cpp"))) if s != CALL_SRC]
     if not srcs:
         return None
     os.makedirs(LIBDIR, exist_ok=True)
@@ -96,13 +101,30 @@ def build_runtime(force=False, jobs=8, verbose=True):
     return RT_LIB
 
 
+def build_call(force=False):
+    """The Python binding: a stub per function that the C header declares, their names in a list made from it."""
+    os.makedirs(LIBDIR, exist_ok=True)
+    os.makedirs(OBJDIR, exist_ok=True)
+    header = os.path.join(INCLUDE, "ttmlir_amd_hip.h")
+    if not force and _newer(CALL_LIB, [CALL_SRC, header]):
+        return CALL_LIB
+    text = re.sub(r"/\*.*?\*/", "", open(header).read(), flags=re.S)
+    names = re.findall(r"^\s*(?:const char \*|int64_t |int )\s*(ttm_\w+)\s*\(", text, flags=re.M)
+    with open(os.path.join(OBJDIR, "ttm_entries.inc"), "w") as f:
+        f.writelines("TTM_ENTRY(%s)\n" % n for n in names)
+    out = _run([CXX] + CXX_FLAGS + ["-I", OBJDIR, "-I", sysconfig.get_paths()["include"], "-shared", CALL_SRC, "-o", CALL_LIB])
+    if out.strip():
+        print(out)
+    return CALL_LIB
+
+
 def build_all(force=False, jobs=8, verbose=True):
-    return build_hip(force, jobs, verbose), build_runtime(force, jobs, verbose)
+    return build_hip(force, jobs, verbose), build_runtime(force, jobs, verbose), build_call(force)
 
 
 def clean():
     shutil.rmtree(OBJDIR, ignore_errors=True)
-    for p in (HIP_LIB, RT_LIB):
+    for p in (HIP_LIB, RT_LIB, CALL_LIB):
         if os.path.exists(p):
             os.remove(p)
 

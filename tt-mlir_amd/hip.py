@@ -12,6 +12,7 @@ ROOT = os.path.dirname(_HERE)
 # TTMLIR_AMD_HIP_LIB names another build of the library (a kernel variant under measurement)
 LIB_PATH = os.environ.get("TTMLIR_AMD_HIP_LIB") or os.path.join(_HERE, "lib", "libttmlir_amd_hip.so")
 HEADER = os.path.join(ROOT, "include", "ttmlir_amd_hip.h")
+CALL_PATH = os.path.join(_HERE, "lib", "_ttm_call.so")   # call() and ptr() as compiled code (runtime/py_call.cpp)
 
 F32, F16, BF16, BFP8B, BFP4B, U32, U16, U8, I32 = 0, 1, 2, 4, 6, 9, 10, 11, 12
 ROW_MAJOR, TILE = 0, 1
@@ -59,11 +60,14 @@ def lib():
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise TTMError("native kernel library missing: %s (run `python tt-mlir_amd/build.py`)" % LIB_PATH)
+        if _native is None:
+            raise TTMError("native binding missing: %s (run `python tt-mlir_amd/build.py`)" % CALL_PATH)
         l = ctypes.CDLL(LIB_PATH)
         for name, res, argtypes in declared_functions():
             fn = getattr(l, name)
             fn.restype, fn.argtypes = res, argtypes
         _lib = l
+        _native.bind({n: ctypes.cast(getattr(l, n), ctypes.c_void_p).value for n in _native.names()})
         if _check_buffers:   # switched on by the environment before the library was loaded: the library's own check goes with it
             l.ttm_set_option(b"check_extents", 1)
     return _lib
@@ -153,6 +157,8 @@ def check_buffers(on=True):
     of any call whose buffers were sized by hand."""
     global _check_buffers
     _check_buffers = bool(on)
+    if _native is not None:
+        _native.check(_check_buffers)
     # the library's own check covers every entry point (the rules above cover the common ones, against the tensor's size,
     # which is tighter than the allocation the library can see)
     set_option("check_extents", 1 if on else 0)
@@ -180,34 +186,57 @@ def _verify_extents(name, args):
                            "padded to whole 32 x 32 tiles)" % (name, what, idx, p.nbytes, need))
 
 
-def call(name, *args):
-    if _check_buffers:
-        _verify_extents(name, args)
+def _call(name, *args):
+    """call() through ctypes: before the library is loaded, and for arguments that py_call.cpp does not convert."""
     status = getattr(_lib or lib(), name)(*args)
     if status:
         check(status, name)
 
 
-def ptr(t):
-    """Device address of a torch tensor (must be contiguous); it carries the tensor's size for check_buffers."""
+def _ptr(t):
+    """ptr() for tensors that are not contiguous."""
     assert t.is_contiguous()
     p = _Ptr(t.data_ptr())
     p.nbytes = t.nbytes
     return p
 
 
-_raw_stream = None
+def _load_native():
+    import importlib.machinery
+    import importlib.util
+    if not os.path.exists(CALL_PATH):
+        return None
+    loader = importlib.machinery.ExtensionFileLoader("_ttm_call", CALL_PATH)
+    m = importlib.util.module_from_spec(importlib.util.spec_from_loader("_ttm_call", loader))
+    loader.exec_module(m)
+    m.setup(ctypes.c_void_p, _Ptr, _call, _ptr, check, _verify_extents)
+    m.check(_check_buffers)
+    return m
+
+
+_native = _load_native()
+if _native is not None:
+    call, ptr = _native.call, _native.ptr
+else:   # nothing is built yet: lib() says so
+    call, ptr = _call, _ptr
+
+_raw_stream = _device_of_thread = None
+
+
+def _torch_streams():
+    global _raw_stream, _device_of_thread
+    import torch
+    torch.cuda.current_stream()     # initialises torch's side of the device
+    _device_of_thread = torch._C._cuda_getDevice
+    _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", lambda device: torch.cuda.current_stream(device).cuda_stream)
 
 
 def current_stream():
     """Raw hipStream_t of torch's current stream, so kernels order with torch work."""
-    global _raw_stream
-    import torch
     if _raw_stream is None:
-        torch.cuda.current_stream()     # initialises torch's side of the device
-        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", lambda device: torch.cuda.current_stream(device).cuda_stream)
+        _torch_streams()
     # the handle itself, without torch's Stream object around it: 3.3 us of the 8.3 us a small call took
-    return ctypes.c_void_p(_raw_stream(torch._C._cuda_getDevice()))
+    return ctypes.c_void_p(_raw_stream(_device_of_thread()))
 
 
 def set_option(name, value):
