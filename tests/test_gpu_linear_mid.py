@@ -146,3 +146,33 @@ def test_infinite_activations_up_to_64_rows(hip, dev, wfmt_name, M):
         assert torch.isnan(got[hit]).all() and torch.isfinite(got[~hit]).all()
         if option == 0:
             assert torch.equal(got[~hit], clean[~hit])
+
+
+@pytest.mark.parametrize("M,option", [(1, 0), (32, 0), (64, 8101), (100, 4201), (130, 8202), (128, 8401)])
+def test_bfp4_operands_of_every_exponent(hip, dev, M, option):
+    """Every nibble under every exponent as the kernels that keep weights in registers turn it into bf16: rows of the identity times such
+    weights give them back, exactly from exponent 3 on and, below (values under 2^-123), either as they are or as zero."""
+    K, N = 320, 96
+    g = torch.Generator().manual_seed(M)
+    kt, nt = K // 32, N // 32
+    tiles = torch.randint(0, 256, (kt, nt, 576), generator=g, dtype=torch.uint8)
+    tiles[:, :, :64] = (torch.arange(kt * nt * 64) % 254).reshape(kt, nt, 64).to(torch.uint8)
+    face = tiles[:, :, 64:].reshape(kt, nt, 2, 2, 16, 8)
+    nibbles = torch.stack([face & 15, face >> 4], -1).reshape(kt, nt, 2, 2, 16, 16).double()
+    value = torch.where(nibbles >= 8, 8 - nibbles, nibbles) * 2.0 ** (tiles[:, :, :64].reshape(kt, nt, 2, 2, 16, 1).double() - 129)
+    w = value.permute(0, 2, 4, 1, 3, 5).reshape(K, N)
+    rows = torch.randperm(K, generator=g)[:M]
+    a = torch.zeros(M, K, dtype=torch.bfloat16)
+    a[torch.arange(M), rows] = 1.0
+    at, wd = tilize_dev(hip, a, dev), tiles.reshape(-1).to(dev)
+    out = torch.full(((M + 31) // 32 * 32 * N,), float("nan"), dtype=torch.bfloat16, device=dev)
+    hip.set_option("linear_mid", option)
+    try:
+        hip.call("ttm_linear", hip.ptr(at), hip.BF16, hip.ptr(wd), hip.BFP4B, 0, None, hip.BF16, hip.TILE, hip.ptr(out), hip.BF16, 1, 1, M, N, K, 0,
+                 hip.current_stream())
+    finally:
+        hip.set_option("linear_mid", 0)
+    got, want = untilize_dev(hip, out, (M, N), dev).cpu().double(), w[rows]
+    tiny = want.abs() < 2.0 ** -123
+    assert torch.equal(got[~tiny], want[~tiny])
+    assert ((got - want).abs() <= want.abs() + 2.0 ** -133)[tiny].all()

@@ -221,6 +221,36 @@ __device__ __forceinline__ void quad_transpose(uint32_t *v, int lane) {
 }
 
 
+// ---- bfp4_b operands of the kernels that keep weights in registers (decode and mid-size): a lane's 8 (k) x 4 (n) block
+// Load: the four lanes of a quad need 8 k rows x 8 bytes, one 64-byte half of a face; each fetches two whole rows with one 16-byte load (eight
+// 2-byte words took 8 loads and 128 line look-ups per tile pair) and the quad transposes: pk[i] = the lane's four nibbles of the rows 2 i and 2 i + 1.
+__device__ __forceinline__ void bfp4_rows(const u32x4 &x, int lane, uint32_t (&pk)[4]) {
+  pk[0] = __builtin_amdgcn_perm(x.z, x.x, 0x05040100u); pk[1] = __builtin_amdgcn_perm(x.z, x.x, 0x07060302u);
+  pk[2] = __builtin_amdgcn_perm(x.w, x.y, 0x05040100u); pk[3] = __builtin_amdgcn_perm(x.w, x.y, 0x07060302u);
+  quad_transpose(pk, lane);
+}
+// (257 - E) << 7 of the rows 2 i and 2 i + 1 in the halves of a word
+__device__ __forceinline__ void bfp4_exponents(const u32x2 &ex, uint32_t (&sub)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) sub[i] = (0x01010101u - __builtin_amdgcn_perm(0u, i < 2 ? ex.x : ex.y, (i & 1) ? 0x0c030c02u : 0x0c010c00u)) << 7;
+}
+// The columns n and n + 2 (n = 0, 1) as bf16 pairs along k.  A magnitude of 1 .. 7 has four fractions and three exponents: v_perm looks the
+// two bytes of 0x7F80 + (its bf16 less that of 1) up for four elements at once, 0 for a magnitude of 0; less (257 - E) << 7, saturating at zero, that
+// is the bf16 of magnitude x 2^(E - 129) (exponents below 3 give zero or what bf16 holds of the value).  100 vector instructions for a block, where
+// two conversions to float per element took 205 and the two-term operand 100 with twice the matrix instructions.
+__device__ __forceinline__ void bfp4_columns(const uint32_t (&pk)[4], const uint32_t (&sub)[4], int n, u32x4 &w0, u32x4 &w2) {
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t sel = (n ? pk[i] >> 4 : pk[i]) & 0x07070707u;
+    const uint32_t lo = __builtin_amdgcn_perm(0xE0C0A080u, 0x40008000u, sel), hi = __builtin_amdgcn_perm(0x80808080u, 0x80807F00u, sel);
+    const uint32_t a = __builtin_amdgcn_perm(hi, lo, 0x06020400u), b = __builtin_amdgcn_perm(hi, lo, 0x07030501u);
+    const u16x2 x = __builtin_elementwise_sub_sat(*(const u16x2 *)&a, *(const u16x2 *)&sub[i]), y = __builtin_elementwise_sub_sat(*(const u16x2 *)&b, *(const u16x2 *)&sub[i]);
+    w0[i] = *(const uint32_t *)&x | (n ? (pk[i] & 0x00800080u) << 8 : (pk[i] & 0x00080008u) << 12);
+    w2[i] = *(const uint32_t *)&y | (n ? pk[i] & 0x80008000u : (pk[i] & 0x08000800u) << 4);
+  }
+}
+
 static inline int device_cu_count() {
   static int cus = 0;
   if (cus == 0) {

@@ -1551,18 +1551,17 @@ __global__ __launch_bounds__(256) void ttm_linear_small_k(LinearPlain args) {
 // A workgroup owns 64 output columns (two weight tiles); its 8 wavefronts take every 8th k-tile and are
 // summed through LDS at the end.  Per k-tile a lane needs an 8 (k) x 4 (n) block as eight 4-byte words (bfp8_b: the four
 // lanes of a quad fetch the 128-byte line that holds their four blocks as two whole 16-byte rows each and transpose
-// it between them with DPP moves; bfp4_b: eight 2-byte loads), dequantises it in registers and feeds byte j of the words to MFMA j: with
+// it between them with DPP moves; bfp4_b: bfp4_rows), dequantises it in registers and feeds byte j of the words to MFMA j: with
 // v_mfma_f32_16x16x32_bf16 lane l supplies row l % 16 and k = 8 (l / 16) .. + 7 of the 16 x 32 weight
 // operand, and MFMA j's row r stands for column n = 4 r + j, so one accumulator register of the four
 // MFMAs is four consecutive n again.  Loads run two k-tiles ahead (register ring): with eight wavefronts that is
 // 74 KiB in flight per CU; four ahead measured 5 % slower ([4096, 14336] at M = 32: 17.4 -> 16.5 us), one or five slower still.
 // =============================================================================================
 // BFP4 = true reads bfp4_b tiles (576 bytes, two elements per byte, low nibble first): a lane's 4 (n) of a k row are one
-// 16-bit word, whose nibbles are spread into the bytes of a word before the same sign-magnitude -> offset-binary step.
+// 16-bit word (bfp4_columns).
 //
-// TWO_TERM = true builds the bf16 operands with bit operations alone instead of int -> float conversions.  A weight is
-// +-mag x 2^(E - 133) (bfp8_b; mag x 2^(E - 129) for bfp4_b).  The bf16 number with the sign, exponent field E + 1 and
-// mantissa field mag (mag << 4 for bfp4_b) is V = +-(1 + mag / 128) x 2^(E - 126) = weight + S with S = +-2^(E - 126),
+// TWO_TERM = true (bfp8_b) builds the bf16 operands with bit operations alone instead of int -> float conversions.  A weight is
+// +-mag x 2^(E - 133).  The bf16 number with the sign, exponent field E + 1 and mantissa field mag is V = +-(1 + mag / 128) x 2^(E - 126) = weight + S with S = +-2^(E - 126),
 // the same bits with a zero mantissa.  Both are made for two k rows at a time with a byte permute and three mask / shift /
 // or steps, V and S go through the matrix cores into two accumulators, and the result is their difference: twice the
 // MFMAs (which were idle) for less than half the vector instructions.  The two sums are each a few times larger than
@@ -1572,8 +1571,8 @@ __global__ __launch_bounds__(512) void ttm_linear_decode_k(ARGS args) {
   const LinearArgs p = args.full();
   extern __shared__ u32x4 smem[];   // partial sums: NP x 8 wavefronts x 8 x 64 float4 = NP x 64 KiB
   constexpr int D = 2;
-  constexpr bool WL = !BFP4;   // whole-row loads and a transpose within lane quads (bfp8_b)
-  constexpr uint32_t TB = BFP4 ? 576u : 1088u, FACE = BFP4 ? 128u : 256u, ROW = BFP4 ? 8u : 16u;
+  static_assert(!(BFP4 && TWO_TERM), "bfp4_b has one operand");
+  constexpr uint32_t TB = BFP4 ? 576u : 1088u, FACE = BFP4 ? 128u : 256u;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int cg = blockIdx.x, Nt = p.Nt, tile_base = 0, act = p.act;   // column pair, column tiles of the matrix, its first tile in a group's concatenation
@@ -1594,12 +1593,15 @@ __global__ __launch_bounds__(512) void ttm_linear_decode_k(ARGS args) {
 #pragma unroll
   for (int pr = 0; pr < NP; ++pr) {
     const uint32_t nt_l = (uint32_t)min(GLU ? 2 * cg + (q16 >> 3) : 2 * NP * cg + 2 * pr + (q16 >> 3), Nt - 1);
-    offW[pr] = nt_l * TB + 64u + (fr * 2 + fc) * FACE + half * (FACE / 2) + quad * (WL ? ROW : ROW / 4);   // + ROW i (WL: row quad, + 4 ROW)
+    offW[pr] = nt_l * TB + 64u + (fr * 2 + fc) * FACE + half * (FACE / 2) + quad * 16;   // bfp8_b: row quad, + 64: row quad + 4; bfp4_b: rows 2 quad and 2 quad + 1
     offE[pr] = nt_l * TB + (fr * 2 + fc) * 16 + half * 8;
   }
   const uint32_t offA = fr * 512 + q16 * 32 + half * 16;                                     // + 1024 h
 
   f32x4v acc[NP][2][4], accs[NP][2][4];   // accs: the sum over the S terms (TWO_TERM)
+  // bfp4_b: the activations times zero, NaN in a row with an infinite one and added to it at the end: such a row is NaN in every column, as the
+  // two terms of bfp8_b leave it (inf - inf)
+  f32x4v zero[2] = {f32x4v{0.f, 0.f, 0.f, 0.f}, f32x4v{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
   for (int pr = 0; pr < NP; ++pr)
 #pragma unroll
@@ -1607,7 +1609,8 @@ __global__ __launch_bounds__(512) void ttm_linear_decode_k(ARGS args) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[pr][h][j] = accs[pr][h][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
 
-  uint32_t rows[D][NP][8], keeps[D];
+  uint32_t rows[D][NP][BFP4 ? 1 : 8], keeps[D];
+  u32x4 raw[D][NP];   // bfp4_b
   u32x2 ex[D][NP];
   u32x4 af[D][2];
   // split-K: workgroup y of the grid takes k-tiles [y k_slice, (y + 1) k_slice) and leaves fp32 partial sums
@@ -1623,17 +1626,15 @@ __global__ __launch_bounds__(512) void ttm_linear_decode_k(ARGS args) {
 #pragma unroll
     for (int pr = 0; pr < NP; ++pr) {
       const uint8_t *Wk = pr == 0 ? Wk0 : Wk1;
-      if constexpr (WL) {
+      if constexpr (BFP4) {
+        raw[s][pr] = *(const u32x4 *)(Wk + offW[pr]);
+      } else {
         // the four lanes of a quad need one 128-byte line between them (8 k rows x 16 n bytes, a dword column each): every
         // lane fetches two whole rows of it (rows quad and quad + 4) and the quad transposes in registers when the slot is
         // consumed - 2 loads and 32 cache-line look-ups per wavefront and tile pair instead of 8 and 128
         const u32x4 x = *(const u32x4 *)(Wk + offW[pr]), y = *(const u32x4 *)(Wk + offW[pr] + 64);
         rows[s][pr][0] = x.x; rows[s][pr][1] = x.y; rows[s][pr][2] = x.z; rows[s][pr][3] = x.w;
         rows[s][pr][4] = y.x; rows[s][pr][5] = y.y; rows[s][pr][6] = y.z; rows[s][pr][7] = y.w;
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i)   // the eight loads share their cache lines: cached loads
-          rows[s][pr][i] = BFP4 ? (uint32_t) * (const uint16_t *)(Wk + offW[pr] + i * ROW) : *(const uint32_t *)(Wk + offW[pr] + i * ROW);
       }
       ex[s][pr] = *(const u32x2 *)(Wk + offE[pr]);
     }
@@ -1642,9 +1643,30 @@ __global__ __launch_bounds__(512) void ttm_linear_decode_k(ARGS args) {
     for (int h = 0; h < 2; ++h) af[s][h] = *(const u32x4 *)(Ak + offA + h * 1024);
   };
   auto process_pair = [&](int s, int pr) __attribute__((always_inline)) {
-    if constexpr (WL) {
-      if (!TWO_TERM || keeps[s] != 0u) { quad_transpose(&rows[s][pr][0], lane); quad_transpose(&rows[s][pr][4], lane); }
+    if constexpr (BFP4) {
+      if (keeps[s] == 0u) return;   // wavefront-uniform: a k-tile past the end contributes nothing
+      uint32_t pk[4], sub[4];
+      bfp4_rows(raw[s][pr], lane, pk);
+      bfp4_exponents(ex[s][pr], sub);
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        u32x4 w0, w2;
+        bfp4_columns(pk, sub, n, w0, w2);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          acc[pr][h][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(bf16x8 *)&w0, *(bf16x8 *)&af[s][h], acc[pr][h][n], 0, 0, 0);
+          acc[pr][h][n + 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(bf16x8 *)&w2, *(bf16x8 *)&af[s][h], acc[pr][h][n + 2], 0, 0, 0);
+        }
+      }
+      if (pr == 0) {
+        const u32x4 none = {0, 0, 0, 0};
+#pragma unroll
+        for (int h = 0; h < 2; ++h) zero[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8 *)&none, *(bf16x8 *)&af[s][h], zero[h], 0, 0, 0);
+      }
+      return;
     }
+    if constexpr (!BFP4) {
+    if (!TWO_TERM || keeps[s] != 0u) { quad_transpose(&rows[s][pr][0], lane); quad_transpose(&rows[s][pr][4], lane); }
     if constexpr (TWO_TERM) {
       if (keeps[s] == 0u) return;   // wavefront-uniform: a k-tile past the end contributes nothing
       // (E + 1) << 7 for the rows 2 ip and 2 ip + 1, in the two halves of a word; E is capped so that the field stays 8 bits
@@ -1658,28 +1680,14 @@ __global__ __launch_bounds__(512) void ttm_linear_decode_k(ARGS args) {
         e2 = *(const uint32_t *)&capped;
         epk[ip] = (e2 + 0x00010001u) << 7;
       }
-      uint32_t pk[4] = {0u, 0u, 0u, 0u};
-      if constexpr (BFP4) {
-#pragma unroll
-        for (int ip = 0; ip < 4; ++ip) pk[ip] = rows[s][pr][2 * ip] | (rows[s][pr][2 * ip + 1] << 16);   // four nibbles per row
-      }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         u32x4 wv, ws;
 #pragma unroll
         for (int ip = 0; ip < 4; ++ip) {
-          uint32_t sb, v;
-          if constexpr (BFP4) {
-            const uint32_t q = pk[ip] >> (4 * j);            // nibble j of either row in bits 0..3 and 16..19
-            sb = ((q & 0x00080008u) << 12) | epk[ip];
-            v = ((q & 0x00070007u) << 4) | sb;
-          } else {
-            const uint32_t q = __builtin_amdgcn_perm(rows[s][pr][2 * ip + 1], rows[s][pr][2 * ip], 0x0c040c00u + 0x00010001u * j);
-            sb = ((q & 0x00800080u) << 8) | epk[ip];
-            v = (q & 0x007F007Fu) | sb;
-          }
-          wv[ip] = v;
-          ws[ip] = sb;
+          const uint32_t q = __builtin_amdgcn_perm(rows[s][pr][2 * ip + 1], rows[s][pr][2 * ip], 0x0c040c00u + 0x00010001u * j);
+          ws[ip] = ((q & 0x00800080u) << 8) | epk[ip];
+          wv[ip] = (q & 0x007F007Fu) | ws[ip];
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -1693,17 +1701,11 @@ __global__ __launch_bounds__(512) void ttm_linear_decode_k(ARGS args) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       uint32_t E = (((i < 4 ? ex[s][pr].x : ex[s][pr].y) & keeps[s]) >> (8 * (i & 3))) & 0xFFu;
-      // value = magnitude x 2^(E - 127 - 6) (bfp8_b) or 2^(E - 127 - 2) (bfp4_b); smaller exponents flush to zero
-      constexpr uint32_t EB = BFP4 ? 2u : 6u, SIGN = BFP4 ? 0x08080808u : 0x80808080u, SH = BFP4 ? 3u : 7u;
-      E = max(E, EB);
-      const float scale = __uint_as_float((E - EB) << 23), nscale = (BFP4 ? -8.0f : -128.0f) * scale;
-      uint32_t d = rows[s][pr][i];
-      if (BFP4) {   // nibbles n3 n2 n1 n0 of the low half -> one per byte
-        d = (d | (d << 8)) & 0x00FF00FFu;
-        d = (d | (d << 4)) & 0x0F0F0F0Fu;
-      }
-      const uint32_t sg = d & SIGN, sb = sg >> SH;
-      const uint32_t t = (d ^ SIGN ^ (sg - sb)) + sb;
+      // value = magnitude x 2^(E - 127 - 6); smaller exponents flush to zero
+      E = max(E, 6u);
+      const float scale = __uint_as_float((E - 6u) << 23), nscale = -128.0f * scale;
+      const uint32_t d = rows[s][pr][i], sg = d & 0x80808080u, sb = sg >> 7;
+      const uint32_t t = (d ^ 0x80808080u ^ (sg - sb)) + sb;
 #pragma unroll
       for (int b = 0; b < 4; ++b) f[i][b] = fmaf((float)((t >> (8 * b)) & 0xFFu), scale, nscale);
     }
@@ -1713,6 +1715,7 @@ __global__ __launch_bounds__(512) void ttm_linear_decode_k(ARGS args) {
 #pragma unroll
       for (int h = 0; h < 2; ++h)
         acc[pr][h][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(bf16x8 *)&w, *(bf16x8 *)&af[s][h], acc[pr][h][j], 0, 0, 0);
+    }
     }
   };
   auto process = [&](int s) __attribute__((always_inline)) {
@@ -1736,13 +1739,13 @@ __global__ __launch_bounds__(512) void ttm_linear_decode_k(ARGS args) {
     }
   }
 
-  if constexpr (TWO_TERM) {
+  if constexpr (TWO_TERM || BFP4) {
 #pragma unroll
     for (int pr = 0; pr < NP; ++pr)
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[pr][h][j] -= accs[pr][h][j];
+        for (int j = 0; j < 4; ++j) acc[pr][h][j] -= BFP4 ? zero[h] : accs[pr][h][j];
   }
   // partial sums -> LDS as float4 (four consecutive n of one m), then thread t finishes slot t of every tile pair's 512: (h, i, lane) =
   // (t >> 8, (t >> 6) & 3, t & 63).  Its 8-byte stores lie 32 bytes apart; a face per wavefront instead, whose stores are 512 bytes
@@ -2048,14 +2051,14 @@ static int launch_linear(const LinearArgs &a, int64_t batch, hipStream_t s) {
       p.C = a.C + (int64_t)mt * a.Nt * 2048;
       for (int j = 0; j < a.group_n; ++j) p.gC[j] = a.gC[j] + (int64_t)mt * a.gNt[j] * 2048;
       const dim3 grid((unsigned)units, slices, (unsigned)batch);
-      const bool two_term = ttm_option("linear_decode_variant") != 1;   // 1 = operands by int -> float conversion
+      const bool two_term = ttm_option("linear_decode_variant") != 1;   // 1 = bfp8_b operands by int -> float conversion
       if (decode) {
         constexpr bool B4 = WF == WF_BFP4;
         if (a.glu) {
-          if (int rc = two_term ? launch_decode<B4, true, 2, true, LinearArgs>(p, grid, s) : launch_decode<B4, false, 2, true, LinearArgs>(p, grid, s)) return rc;
+          if (int rc = two_term ? launch_decode<B4, !B4, 2, true, LinearArgs>(p, grid, s) : launch_decode<B4, false, 2, true, LinearArgs>(p, grid, s)) return rc;
         } else if (a.group_n > 1) {
-          if (int rc = two_term ? launch_decode<B4, true, LinearArgs>(p, np, grid, s) : launch_decode<B4, false, LinearArgs>(p, np, grid, s)) return rc;
-        } else if (int rc = two_term ? launch_decode<B4, true>(LinearPlain(p), np, grid, s) : launch_decode<B4, false>(LinearPlain(p), np, grid, s)) return rc;
+          if (int rc = two_term ? launch_decode<B4, !B4, LinearArgs>(p, np, grid, s) : launch_decode<B4, false, LinearArgs>(p, np, grid, s)) return rc;
+        } else if (int rc = two_term ? launch_decode<B4, !B4>(LinearPlain(p), np, grid, s) : launch_decode<B4, false>(LinearPlain(p), np, grid, s)) return rc;
       }
       else hipLaunchKernelGGL((ttm_linear_small_k<WF>), dim3(a.Nt, 1, (unsigned)batch), dim3(256), 0, s, LinearPlain(p));
       if (a.qkv) {

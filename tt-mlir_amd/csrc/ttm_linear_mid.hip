@@ -21,7 +21,8 @@ __global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(ARGS
   constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
   constexpr uint32_t TB = WF == WF_BFP8 ? 1088u : WF == WF_BFP4 ? 576u : 2048u;
   constexpr uint32_t FACE = WF == WF_BFP8 ? 256u : WF == WF_BFP4 ? 128u : 512u, ROW = FACE / 16;
-  constexpr int RW = BFP ? 8 : 16;   // dwords of weights per lane, k-tile and column pair
+  constexpr int RW = WF == WF_BFP8 ? 8 : WF == WF_BFP4 ? 4 : 16;   // dwords of weights per lane, k-tile and column pair
+  static_assert(!TT || BFP, "block-float weights");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wn = GLU ? wave / WK : 0, wk = wave & (WK - 1);
   // row blocks of one column unit are neighbours on one XCD: its L2 serves the weights to all but the first of them
@@ -43,23 +44,24 @@ __global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(ARGS
   const int fc = (q16 >> 2) & 1, quad = q16 & 3, fr = kg >> 1, half = kg & 1;
   if (GLU) W = wn ? p.gW[1] : p.gW[0];
   const uint32_t nt_l = (uint32_t)min(2 * cg + (q16 >> 3), Nt - 1);
-  // bfp8_b: two whole 16-byte rows of the quad's 128-byte line; bfp4_b: eight 2-byte words; bf16 [K, N]: eight 8-byte words;
+  // bfp8_b: two whole 16-byte rows of the quad's 128-byte line; bfp4_b: two whole 8-byte rows of its 64; bf16 [K, N]: eight 8-byte words;
   // bf16 [N, K]: the 8 k of each of the four columns
   const uint32_t offW = WF == WF_BF16_NK ? (uint32_t)(fc * 1024 + quad * 128 + fr * 512 + half * 16)
-                                         : (BFP ? 64u : 0u) + (fr * 2 + fc) * FACE + half * (FACE / 2) + quad * (WF == WF_BFP8 ? ROW : ROW / 4);
-  const uint32_t offE = (fr * 2 + fc) * 16 + half * 8;
+                                         : nt_l * TB + (BFP ? 64u : 0u) + (fr * 2 + fc) * FACE + half * (FACE / 2) + quad * (BFP ? 16 : ROW / 4);
+  const uint32_t offE = nt_l * TB + (fr * 2 + fc) * 16 + half * 8;
   const uint32_t offA = fr * 512 + q16 * 32 + half * 16;
   int64_t rowA[MT];
 #pragma unroll
-  for (int r = 0; r < MT; ++r) rowA[r] = (int64_t)min(mt0 + r, p.Mt - 1) * p.Kt * 2048 + offA;
+  for (int r = 0; r < MT; ++r) rowA[r] = (int64_t)min(mt0 + r, p.Mt - 1) * p.Kt * 2048;
 
-  f32x4v acc[2 * MT][4], accs[TT ? 2 * MT : 1][4];   // accs: the sums over the S terms
+  // accs: the sums over the S terms; bfp4_b, whose operand is one term: of the activations times zero (see launch_mid)
+  f32x4v acc[2 * MT][4], accs[TT ? 2 * MT : 1][WF == WF_BFP4 ? 1 : 4];
 #pragma unroll
   for (int h = 0; h < 2 * MT; ++h)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       acc[h][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
-      if (TT) accs[h][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
+      if (TT && (j == 0 || WF != WF_BFP4)) accs[h][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
     }
   uint32_t rows[D][RW];
   u32x2 ex[D];
@@ -80,14 +82,14 @@ __global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(ARGS
         rw[4 * j] = x.x; rw[4 * j + 1] = x.y; rw[4 * j + 2] = x.z; rw[4 * j + 3] = x.w;
       }
     } else {
-      const uint8_t *Wt = W + ((int64_t)ktc * Nt + nt_l) * TB, *Wk = Wt + offW;
+      const uint8_t *Wt = W + (int64_t)ktc * Nt * TB, *Wk = Wt + offW;
       if constexpr (WF == WF_BFP8) {
         const u32x4 x = *(const u32x4 *)Wk, y = *(const u32x4 *)(Wk + 64);
         rw[0] = x.x; rw[1] = x.y; rw[2] = x.z; rw[3] = x.w;
         rw[4] = y.x; rw[5] = y.y; rw[6] = y.z; rw[7] = y.w;
       } else if constexpr (WF == WF_BFP4) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) rw[i] = *(const uint16_t *)(Wk + i * ROW);
+        const u32x4 x = *(const u32x4 *)Wk;
+        rw[0] = x.x; rw[1] = x.y; rw[2] = x.z; rw[3] = x.w;
       } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -98,15 +100,37 @@ __global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(ARGS
       if constexpr (BFP) ex[s] = *(const u32x2 *)(Wt + offE);
     }
 #pragma unroll
-    for (int h = 0; h < 2 * MT; ++h) af[s][h] = *(const u32x4 *)(A + rowA[h >> 1] + (int64_t)ktc * 2048 + (h & 1) * 1024);
+    for (int h = 0; h < 2 * MT; ++h) af[s][h] = *(const u32x4 *)(A + rowA[h >> 1] + (int64_t)ktc * 2048 + offA + (h & 1) * 1024);
   };
   auto process = [&](int s) __attribute__((always_inline)) {
     if (!live[s]) return;   // wavefront-uniform: a k-tile past the end contributes nothing
     uint32_t *rw = rows[s];
-    if constexpr (TT && BFP) {
-      if constexpr (WF == WF_BFP8) { quad_transpose(rw, lane); quad_transpose(rw + 4, lane); }
+    if constexpr (WF == WF_BFP4) {
+      uint32_t pk[4], sub[4];
+      bfp4_rows(u32x4{rw[0], rw[1], rw[2], rw[3]}, lane, pk);
+      bfp4_exponents(ex[s], sub);
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        u32x4 w[2];
+        bfp4_columns(pk, sub, n, w[0], w[1]);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int h = 0; h < 2 * MT; ++h)
+            acc[h][n + 2 * j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(bf16x8 *)&w[j], *(bf16x8 *)&af[s][h], acc[h][n + 2 * j], 0, 0, 0);
+        if constexpr (MT > 2) __builtin_amdgcn_sched_barrier(0);   // two columns' operands at a time: more of them do not fit the registers
+      }
+      if constexpr (TT) {
+        const u32x4 none = {0, 0, 0, 0};
+#pragma unroll
+        for (int h = 0; h < 2 * MT; ++h) accs[h][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8 *)&none, *(bf16x8 *)&af[s][h], accs[h][0], 0, 0, 0);
+      }
+      return;
+    }
+    if constexpr (TT && WF == WF_BFP8) {
+      quad_transpose(rw, lane); quad_transpose(rw + 4, lane);
       // (E + 1) << 7 for the rows 2 ip and 2 ip + 1, in the two halves of a word; E is capped so that the field stays 8 bits
-      uint32_t epk[4], pk[4] = {0u, 0u, 0u, 0u};
+      uint32_t epk[4];
 #pragma unroll
       for (int ip = 0; ip < 4; ++ip) {
         uint32_t e2 = __builtin_amdgcn_perm(0u, ip < 2 ? ex[s].x : ex[s].y, (ip & 1) ? 0x0c030c02u : 0x0c010c00u);
@@ -114,22 +138,15 @@ __global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(ARGS
         const u16x2 capped = __builtin_elementwise_min(*(const u16x2 *)&e2, u16x2{0xFD, 0xFD});
         e2 = *(const uint32_t *)&capped;
         epk[ip] = (e2 + 0x00010001u) << 7;
-        if constexpr (WF == WF_BFP4) pk[ip] = rw[2 * ip] | (rw[2 * ip + 1] << 16);   // four nibbles per row
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         u32x4 wv, ws;
 #pragma unroll
         for (int ip = 0; ip < 4; ++ip) {
-          if constexpr (WF == WF_BFP4) {
-            const uint32_t q = pk[ip] >> (4 * j);            // nibble j of either row in bits 0..3 and 16..19
-            ws[ip] = ((q & 0x00080008u) << 12) | epk[ip];
-            wv[ip] = ((q & 0x00070007u) << 4) | ws[ip];
-          } else {
-            const uint32_t q = __builtin_amdgcn_perm(rw[2 * ip + 1], rw[2 * ip], 0x0c040c00u + 0x00010001u * j);
-            ws[ip] = ((q & 0x00800080u) << 8) | epk[ip];
-            wv[ip] = (q & 0x007F007Fu) | ws[ip];
-          }
+          const uint32_t q = __builtin_amdgcn_perm(rw[2 * ip + 1], rw[2 * ip], 0x0c040c00u + 0x00010001u * j);
+          ws[ip] = ((q & 0x00800080u) << 8) | epk[ip];
+          wv[ip] = (q & 0x007F007Fu) | ws[ip];
         }
 #pragma unroll
         for (int h = 0; h < 2 * MT; ++h) {
@@ -141,29 +158,23 @@ __global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(ARGS
     }
     float scale[8], nscale[8];
     uint32_t t[8];
-    if constexpr (BFP) {
-      if constexpr (WF == WF_BFP8) { quad_transpose(rw, lane); quad_transpose(rw + 4, lane); }
+    if constexpr (WF == WF_BFP8) {
+      quad_transpose(rw, lane); quad_transpose(rw + 4, lane);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         uint32_t E = ((i < 4 ? ex[s].x : ex[s].y) >> (8 * (i & 3))) & 0xFFu;
-        // value = magnitude x 2^(E - 127 - 6) (bfp8_b) or 2^(E - 127 - 2) (bfp4_b); smaller exponents flush to zero
-        constexpr uint32_t EB = WF == WF_BFP4 ? 2u : 6u, SIGN = WF == WF_BFP4 ? 0x08080808u : 0x80808080u, SH = WF == WF_BFP4 ? 3u : 7u;
-        E = max(E, EB);
-        scale[i] = __uint_as_float((E - EB) << 23);
-        nscale[i] = (WF == WF_BFP4 ? -8.0f : -128.0f) * scale[i];
-        uint32_t d = rw[i];
-        if (WF == WF_BFP4) {   // nibbles n3 n2 n1 n0 of the low half -> one per byte
-          d = (d | (d << 8)) & 0x00FF00FFu;
-          d = (d | (d << 4)) & 0x0F0F0F0Fu;
-        }
-        const uint32_t sg = d & SIGN, sb = sg >> SH;
-        t[i] = (d ^ SIGN ^ (sg - sb)) + sb;
+        // value = magnitude x 2^(E - 127 - 6); smaller exponents flush to zero
+        E = max(E, 6u);
+        scale[i] = __uint_as_float((E - 6u) << 23);
+        nscale[i] = -128.0f * scale[i];
+        const uint32_t d = rw[i], sg = d & 0x80808080u, sb = sg >> 7;
+        t[i] = (d ^ 0x80808080u ^ (sg - sb)) + sb;
       }
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       u32x4 w;
-      if constexpr (BFP) {
+      if constexpr (WF == WF_BFP8) {
         float f[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) f[i] = fmaf((float)((t[i] >> (8 * j)) & 0xFFu), scale[i], nscale[i]);
@@ -196,11 +207,11 @@ __global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(ARGS
     }
   }
 
-  if constexpr (TT && BFP) {
+  if constexpr (TT) {
 #pragma unroll
     for (int h = 0; h < 2 * MT; ++h)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[h][j] -= accs[h][j];
+      for (int j = 0; j < 4; ++j) acc[h][j] -= accs[h][WF == WF_BFP4 ? 0 : j];
   }
   // one row tile at a time: the wavefronts' sums -> LDS as float4 (four consecutive n of one m), then the threads finish the 512
   // slots, (h, i, lane) = (t >> 8, (t >> 6) & 3, t & 63)
@@ -267,6 +278,8 @@ MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu, int max_slice
   MidPlan best;
   best.us = 1e30;
   const int cus = device_cu_count(), units = mid_units(p, glu);
+  // a lane's place in a k row of weights is a 32-bit offset
+  if (wf != WF_BF16_NK && (int64_t)(glu ? p.gNt[0] : p.Nt) * 2048 >= (int64_t)1 << 32) return best;
   const int f = wf == WF_BFP8 || wf == WF_BFP4 ? 0 : 1;
   // us per k-tile of a wavefront at 1 / 2 / 4 row tiles (wavefronts of a SIMD share it, so they add up)
   static const double kChunk[2][5] = {{0, 0.25, 0.44, 0, 0.57}, {0, 0.32, 0.45, 0, 0.68}};
@@ -294,9 +307,8 @@ MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu, int max_slice
 
 template <int WF, int MT, int WK, bool TT>
 static void launch_mid_mt(const LinearArgs &p, dim3 grid, hipStream_t s) {
-  constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
-  if (p.group_n > 1) hipLaunchKernelGGL((ttm_linear_mid_k<WF, MT, WK, TT && BFP, false, LinearArgs>), grid, dim3(WK * 64), 0, s, p);
-  else hipLaunchKernelGGL((ttm_linear_mid_k<WF, MT, WK, TT && BFP, false, LinearPlain>), grid, dim3(WK * 64), 0, s, LinearPlain(p));
+  if (p.group_n > 1) hipLaunchKernelGGL((ttm_linear_mid_k<WF, MT, WK, TT && (WF == WF_BFP8 || WF == WF_BFP4), false, LinearArgs>), grid, dim3(WK * 64), 0, s, p);
+  else hipLaunchKernelGGL((ttm_linear_mid_k<WF, MT, WK, TT && (WF == WF_BFP8 || WF == WF_BFP4), false, LinearPlain>), grid, dim3(WK * 64), 0, s, LinearPlain(p));
 }
 template <int WF>
 static int launch_mid(const LinearArgs &a, const MidPlan &plan, int64_t batch, bool glu, hipStream_t s) {
@@ -327,8 +339,9 @@ static int launch_mid(const LinearArgs &a, const MidPlan &plan, int64_t batch, b
   }
   switch (plan.wk * 10 + plan.mt) {
   case 81:
-    // The two-term operand (1.m and 1.0 products, subtracted at the end) saves conversion work, but an infinite activation leaves
-    // inf - inf: only up to 64 rows, where the decode kernel multiplies the same way.
+    // The two-term operand of bfp8_b (1.m and 1.0 products, subtracted at the end) saves conversion work, but an infinite activation leaves
+    // inf - inf: only up to 64 rows, where the decode kernel multiplies the same way.  bfp4_b has one term and adds the activations times zero there,
+    // so that such a row is NaN in every column whatever the format.
     if (a.Mt <= 2) launch_mid_mt<WF, 1, 8, true>(p, grid, s);
     else launch_mid_mt<WF, 1, 8, false>(p, grid, s);
     break;
