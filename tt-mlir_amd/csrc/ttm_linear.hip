@@ -1960,7 +1960,13 @@ static double other_us(const LinearArgs &a, bool measured = false) {
   constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
   const int cus = device_cu_count(), ksteps = (a.Kt + 1) / 2;
   if (BFP && a.Mt * 32 <= 64) return 1e30;
-  if (!BFP && a.Mt == 1) return 3.5 + (a.Nt * a.plan_batch + cus - 1) / cus * ((a.Kt + 15) / 16) * 1.9;
+  if (!BFP && a.Mt == 1) {
+    // fitted to 107 shapes of 1 .. 32 rows, 7 % rms: the better one where K is short ([7, 544] x [544, 992] 4.9 us, mid-size kernel 6.1; [1, 704] x
+    // [704, 1824] 5.0 / 6.0; [5, 2432] x [2432, 5248] 12.0 / 9.9)
+    const int64_t tiles = (int64_t)a.Nt * a.plan_batch;
+    const double share = std::min(1.0, (double)tiles / cus);
+    return 2.0 + (a.Kt + 15) / 16 * (1.7 * (double)((tiles + cus - 1) / cus) + 0.75 * share * share);
+  }
   LinearArgs p = a;
   double us = 0;
   const int slices = plan_dma_grid(p, cus, 0, a.group_n > 1 ? 1 : 0, 0, &us);
@@ -1971,19 +1977,17 @@ static double other_us(const LinearArgs &a, bool measured = false) {
   if (measured) return !BFP ? 0.77 * two : us <= two ? 0.97 * us : 0.82 * two;
   return BFP ? std::min(us, two) : two;
 }
-// Whether the mid-size kernel's plan beats it.  Its own model is 3 % low for block-float and 5 % high for bf16 weights (10 % at
-// these sizes, less where K is long: 14336 x 4096 bf16 at 700 rows 140 / 148).  4096 x 6144 bf16, image route / mid-size kernel: 520
-// rows 60.5 / 48.3 us, 661 rows 61.7 / 71.3; 5120 x 2880 bfp8_b, 400 rows 38.6 / 28.1, 661 rows 52.3 / 49.6, 930 rows 56.0 / 54.1, 1600
-// rows 71.5 / 85.8.  Of 2900 random shapes (33 .. 2048 rows, weights of 512 .. 8192 x 512 .. 14336, all formats) it is taken at 2116, on
-// average in 0.62 of the other's time, and is the slower one at 46 of them: by 5 % at the median, at worst 28.5 / 23.1 us at 897
-// rows x 518 x 8653 bf16 and 79.9 / 68.0 at 1514 rows x 3072 x 5024 bfp4_b, two in five of them with K below 850.  The models scatter by
-// 4 .. 10 %: lines that leave out more of the 46 (refitted models, an extra charge for short K) take away as much elsewhere, up
-// to 30 % a shape.
+// Whether the mid-size kernel's plan beats it.  4096 x 6144 bf16, image route / mid-size kernel: 520 rows 60.5 / 48.3 us, 661 rows 61.7 / 71.3;
+// 5120 x 2880 bfp8_b, 400 rows 38.6 / 28.1, 661 rows 52.3 / 49.6, 930 rows 56.0 / 54.1, 1600 rows 71.5 / 85.8.  Of 600 random shapes (33 .. 2048 rows,
+// weights of 512 .. 8192 x 512 .. 14336, all formats) it is taken at 473, on average in 0.60 of the other's time; it is the slower one at 3 of
+// them, by 4 .. 8 %, and is left out at 19 where it would be more than 5 % faster, at worst 29 % (787 rows x 7392 x 9202 bfp8_b).  The worst shape seen with
+// the lines as they are is 1952 rows x 3872 x 3298 bfp4_b, 90.7 us against 71 on the other route.  The models scatter by 5 .. 8 %: a line
+// that is right at one of those shapes is wrong at others.
 template <int WF>
 static bool mid_beats_other(const LinearArgs &a, const MidPlan &plan) {
   constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
   if (!BFP && a.Mt == 1) return plan.us < 0.93 * other_us<WF>(a);
-  return (BFP ? 1.03 : 0.95) * plan.us < other_us<WF>(a, true);
+  return (BFP ? 1.0 : 0.97) * plan.us < other_us<WF>(a, true);
 }
 
 template <int WF>

@@ -1,4 +1,6 @@
 // Dense contraction at row counts between decode and prefill, and small products (see ttm_linear.hip for the operands).
+#include <algorithm>
+
 #include "ttm_linear.h"
 
 // =============================================================================================
@@ -8,9 +10,11 @@
 // memory to registers and become the MFMA operand there as in the decode kernel (byte j of eight row words feeds MFMA j, whose
 // row r stands for column 4 r + j), activation fragments are 16-byte loads of whole face-row halves.  That leaves no barrier in the loop and nothing to fill before it: a launch costs 3 us + its k-tiles, where
 // the LDS-direct kernels' blocks cost 12 k-steps (20 us) before and after theirs - what bounded every product below some
-// 10 GFLOP.  Bounds inside the loop, per 32 k of a wavefront: about 480 cycles of vector issue for the conversion (bf16
+// 10 GFLOP.  Bounds inside the loop, per 32 k of a wavefront: about 670 cycles of vector issue for the conversion of bfp8_b (bfp4_b: 400, bf16
 // weights: 64), 128 MT of the matrix core, 32 + 32 MT of L1; MT = 2 balances them for short launches, MT = 4 halves the weight
-// traffic and conversions where the row count fills it.
+// traffic and conversions where the row count fills it.  Vector issue and products mostly add up (512 rows x 14336 x 4096 bfp4_b, when its
+// conversion took 820: 106k and 57k of 160k cycles per SIMD; interleaving one column's products with the next one's conversion gave nothing).
+// bfp4_b by table look-up: 74.9 -> 63.4 us there, 113 rows x 5515 x 5253 28.8 -> 21.2, 259 x 576 x 8256 12.5 -> 10.7.
 // =============================================================================================
 template <int WF, int MT, int WK, bool TT, bool GLU, class ARGS>
 __global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(ARGS args) {
@@ -268,10 +272,11 @@ __global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(ARGS
 // ---- the mid-size kernel's launch plan
 static int mid_units(const LinearArgs &p, bool glu) { return glu ? (p.gNt[0] + 1) / 2 : column_units(p, 2); }
 
-// The model was fitted to 36 shapes of 3 .. 1236 rows, 296 .. 7488 x 265 .. 14336 weights of all formats under every plan (11 % rms
-// over 380 timings; the plan it picks is 1 % slower than the best one on average): 3.3 us for launch, first loads and the last
-// wavefronts, the k-tiles that the wavefronts of a SIMD take, 0.2 + 0.95 us per row tile for the sums through LDS of each
-// round of workgroups, and for a split K the reduction's launch and its traffic at 2.5 TB/s.
+// The model was fitted to 2700 random shapes (33 .. 2048 rows, weights of 512 .. 8192 x 512 .. 14336, all formats) under every plan: 6 % rms
+// over 15000 timings, and the plan it picks is 0.4 % slower than the best one on average, 3 % at the 95th percentile (one without figures of their
+// own for the formats and wavefront counts 2 - 3 %, 15 %: 113 rows x 5515 x 5253 bfp4_b 21.2 / 18.4 us, 64 x 4096 x 14336
+// bfp8_b 19.8 / 17.8).  us = 3.0 for launch, first loads and the last wavefronts; per round of workgroups the k-tiles that
+// the wavefronts of a SIMD take and the sums through LDS; for a split K the reduction's launch and its traffic.
 MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu, int max_slices) {
   // option linear_mid: 0 by the model, 1 never, 1000 * shares + 100 * row tiles + slices pins a plan
   const int force = ttm_option("linear_mid");
@@ -280,26 +285,42 @@ MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu, int max_slice
   const int cus = device_cu_count(), units = mid_units(p, glu);
   // a lane's place in a k row of weights is a 32-bit offset
   if (wf != WF_BF16_NK && (int64_t)(glu ? p.gNt[0] : p.Nt) * 2048 >= (int64_t)1 << 32) return best;
-  const int f = wf == WF_BFP8 || wf == WF_BFP4 ? 0 : 1;
-  // us per k-tile of a wavefront at 1 / 2 / 4 row tiles (wavefronts of a SIMD share it, so they add up)
-  static const double kChunk[2][5] = {{0, 0.25, 0.44, 0, 0.57}, {0, 0.32, 0.45, 0, 0.68}};
-  for (int mt = 1; mt <= 4; mt *= 2) {
+  const int f = wf == WF_BFP8 ? 0 : wf == WF_BFP4 ? 1 : 2;
+  // row tiles, shares of K; us of the sums of a round; how whole a last round counts (two or three of the smaller workgroups share a CU), and every
+  // round behind the first; us per k-tile of a wavefront of bfp8_b / bfp4_b / bf16 weights (wavefronts of a SIMD share it, so they add up)
+  static const struct { int mt, wk; double sums, whole, further, chunk[3]; } kPlain[] = {{2, 4, 1.57, 0.75, 0.87, {0.440, 0.356, 0.466}},
+                                                                                         {1, 8, 0.64, 0.87, 1.00, {0.297, 0.242, 0.345}},
+                                                                                         {2, 8, 2.15, 0.89, 1.25, {0.355, 0.285, 0.391}},
+                                                                                         {4, 8, 4.74, 0.84, 1.17, {0.491, 0.414, 0.565}}};
+  // the gated form: eight wavefronts, four shares of K of either matrix (36 shapes)
+  static const struct { int mt, wk; double sums, chunk; } kGated[] = {{2, 4, 2.1, 0.44}, {4, 4, 4.0, 0.57}};
+  static const double kAlone[3] = {1.08, 1.0, 0.8};   // of a k-tile where a SIMD has one wavefront
+  const auto consider = [&](int mt, int wk, double sums, double whole, double further, double chunk) {
     const int blocks = (units + 7) / 8 * 8 * ((p.Mt + mt - 1) / mt) * p.plan_batch;   // a column unit's row blocks run on one XCD
-    for (int wk = 4; wk <= 8; wk += 4) {
-      if (glu ? wk != 4 || mt == 1 : (wk == 4 && mt != 2)) continue;
-      for (int slices = 1; slices <= (glu ? 1 : max_slices); slices *= 2) {
-        if (force >= 1000) {
-          if (force / 1000 != wk || force % 1000 / 100 != mt || force % 100 != slices) continue;
-        } else if ((mt > 1 && mt >= 2 * p.Mt) || (slices > 1 && p.Kt < 2 * wk * slices)) {
-          continue;
-        }
-        const int kt = (p.Kt + slices - 1) / slices, chunks = (kt + wk - 1) / wk, rounds = (blocks * slices + cus - 1) / cus;
-        if (force < 1000 && rounds > 8) continue;   // beyond what was measured; larger blocks amortise their ends better
-        const int waves = rounds * wk / 4 * (glu ? 2 : 1);            // per SIMD
-        double us = 3.3 + waves * chunks * kChunk[f][mt] + (wk == 8 || glu ? rounds : 1) * (0.2 + 0.95 * mt);
-        if (slices > 1) us += 2.7 + (slices + 0.5) * (double)p.Mt * p.Nt * p.plan_batch * 4096.0 / 2.5e6;
-        if (us < best.us) { best.us = us; best.mt = mt; best.wk = wk; best.slices = slices; }
+    for (int slices = 1; slices <= (glu ? 1 : max_slices); slices *= 2) {
+      if (force >= 1000) {
+        if (force / 1000 != wk || force % 1000 / 100 != mt || force % 100 != slices) continue;
+      } else if ((mt > 1 && mt >= 2 * p.Mt) || (slices > 1 && p.Kt < 2 * wk * slices)) {
+        continue;
       }
+      const int kt = (p.Kt + slices - 1) / slices, chunks = (kt + wk - 1) / wk, rounds = (blocks * slices + cus - 1) / cus;
+      if (force < 1000 && rounds > 8) continue;   // beyond what was measured; larger blocks amortise their ends better
+      const double r = rounds > 1 ? 1 + further * (whole * rounds + (1 - whole) * blocks * slices / cus - 1) : 1.0;
+      double us;
+      if (glu) us = 3.3 + r * 2 * chunks * chunk + r * sums;
+      else us = 3.0 + r * (wk / 4) * chunks * chunk * (wk == 4 && rounds == 1 ? kAlone[f] : 1.0) + (wk == 8 ? r : 0.5 + 0.5 * r) * sums;
+      if (slices > 1) us += 2.65 + (slices + 0.5) * (double)p.Mt * p.Nt * p.plan_batch * 4096.0 / 3.8e6;
+      if (us < best.us) { best.us = us; best.mt = mt; best.wk = wk; best.slices = slices; }
+    }
+  };
+  if (glu) {
+    for (const auto &k : kGated) consider(k.mt, k.wk, k.sums, 1.0, 1.0, k.chunk);
+  } else {
+    for (const auto &k : kPlain) {
+      // every column unit passes all activations by; from twice an XCD's L2 on the workgroups of 64 rows wait for them (1952 rows x 3872 x 3298 bfp4_b,
+      // 15 MB: 111 us, 77 by the rounds, with 128 rows 90 and 82; 1656 x 7136 x 1344 73 / 62)
+      if (k.wk == 4 && force < 1000 && (int64_t)p.Mt * p.Kt * 2048 > 8000000) continue;
+      consider(k.mt, k.wk, k.sums, k.whole, k.further, k.chunk[f]);
     }
   }
   return best;
