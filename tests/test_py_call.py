@@ -1,4 +1,4 @@
-"""call() and ptr() as compiled code (runtime/py_call.cpp) against the ctypes functions they stand for: the same conversions, the same
+"""call() and ptr() as compiled code (binding/py_call.cpp) against the ctypes functions they stand for: the same conversions, the same
 errors.  What an argument arrived as shows in the entry points' own messages; nothing is launched."""
 import ctypes
 

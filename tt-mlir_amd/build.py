@@ -2,7 +2,7 @@
 
   lib/libttmlir_amd_hip.so   gfx950 kernels + C ABI (csrc/*.hip, hipcc)
   lib/libttmlir_amd_rt.so    C++ host runtime in the tt::runtime style (runtime/*.cpp, g++)
-  lib/_ttm_call.so           the kernel library's entry points as Python calls (runtime/py_call.cpp, g++)
+  lib/_ttm_call.so           the kernel library's entry points as Python calls (binding/py_call.cpp, g++)
 
 Usage: python build.py [--force] [--jobs N]
 """
@@ -27,7 +27,7 @@ INCLUDE = os.path.join(ROOT, "include")
 HIP_LIB = os.path.join(LIBDIR, "libttmlir_amd_hip.so")
 RT_LIB = os.path.join(LIBDIR, "libttmlir_amd_rt.so")
 CALL_LIB = os.path.join(LIBDIR, "_ttm_call.so")
-CALL_SRC = os.path.join(RTSRC, "py_call.cpp")
+CALL_SRC = os.path.join(HERE, "binding", "py_call.cpp")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = [
@@ -82,7 +82,7 @@ def build_hip(force=False, jobs=8, verbose=True):
 
 
 def build_runtime(force=False, jobs=8, verbose=True):
-    srcs = [s for s in sorted(glob.glob(os.path.join(RTSRC, "*.cpp"))) if s != CALL_SRC]
+    srcs = sorted(glob.glob(os.path.join(RTSRC, "*.cpp")))
     if not srcs:
         return None
     os.makedirs(LIBDIR, exist_ok=True)

@@ -12,7 +12,7 @@ ROOT = os.path.dirname(_HERE)
 # TTMLIR_AMD_HIP_LIB names another build of the library (a kernel variant under measurement)
 LIB_PATH = os.environ.get("TTMLIR_AMD_HIP_LIB") or os.path.join(_HERE, "lib", "libttmlir_amd_hip.so")
 HEADER = os.path.join(ROOT, "include", "ttmlir_amd_hip.h")
-CALL_PATH = os.path.join(_HERE, "lib", "_ttm_call.so")   # call() and ptr() as compiled code (runtime/py_call.cpp)
+CALL_PATH = os.path.join(_HERE, "lib", "_ttm_call.so")   # call() and ptr() as compiled code (binding/py_call.cpp)
 
 F32, F16, BF16, BFP8B, BFP4B, U32, U16, U8, I32 = 0, 1, 2, 4, 6, 9, 10, 11, 12
 ROW_MAJOR, TILE = 0, 1
