@@ -96,6 +96,18 @@ int ttm_tilize(const void *src, void *dst, int64_t batch, int64_t rows, int64_t 
 int ttm_untilize(const void *src, void *dst, int64_t batch, int64_t rows, int64_t cols, int elem_bytes,
                  void *stream);
 
+/* Up to TTM_GROUP_MAX small tensors in one launch, as ttm_tilize of [rows, cols] (elem_bytes in {1, 2, 4}) or, with elem_bytes 0, a copy of
+ * `cols` bytes (rows 1; a multiple of 16, both addresses too) would bring each: the inputs of a step that come from the host
+ * (runtime/lib/ttnn/operations/trace/capture_or_execute_trace.cpp).  Destinations must not overlap anything else of the group. */
+#define TTM_GROUP_MAX 8
+typedef struct {
+  const void *src;
+  void *dst;
+  int64_t rows, cols;
+  int elem_bytes;
+} ttm_tilize_item;
+int ttm_tilize_group(const ttm_tilize_item *items, int n, void *stream);
+
 /* ---- block-float pack / unpack: ::ttnn::typecast to / from BFLOAT8_B, BFLOAT4_B
  * (runtime/lib/ttnn/operations/layout/typecast.cpp:14-31, types/layout_converter.cpp:47-52,
  * host readback runtime/lib/ttnn/runtime.cpp:450-466).  fmt is TTM_BFP8B or TTM_BFP4B.

@@ -364,6 +364,23 @@ EXPORT int ttm_tilize(const void *src, void *dst, int64_t batch, int64_t rows, i
   EXT(tilize, src, dst, batch, rows, cols, elem);
   return launch([=] { orc_tilize(src, dst, batch, rows, cols, elem); });
 }
+EXPORT int ttm_tilize_group(const ttm_tilize_item *items, int n, void *) {
+  if (n < 0 || n > TTM_GROUP_MAX) return fail("ttm_tilize_group: count");
+  std::vector<ttm_tilize_item> list;
+  for (int i = 0; i < n; ++i) {
+    const ttm_tilize_item &t = items[i];
+    if (t.rows * t.cols == 0) continue;
+    if (t.elem_bytes) EXT(tilize, t.src, t.dst, 1, t.rows, t.cols, t.elem_bytes);
+    else EXT(copy_kernel, t.src, t.dst, (size_t)t.cols);
+    list.push_back(t);
+  }
+  return launch([=] {
+    for (const ttm_tilize_item &t : list) {
+      if (t.elem_bytes) orc_tilize(t.src, t.dst, 1, t.rows, t.cols, t.elem_bytes);
+      else memmove(t.dst, t.src, (size_t)t.cols);
+    }
+  }, true);
+}
 EXPORT int ttm_untilize(const void *src, void *dst, int64_t batch, int64_t rows, int64_t cols, int elem, void *) {
   if (batch * rows * cols == 0) return TTM_OK;
   EXT(untilize, src, dst, batch, rows, cols, elem);

@@ -403,3 +403,56 @@ def test_bfp_ragged(hip, dev, orc, fmt, dtype, shape, shift):
             assert np.array_equal(p[:packed].numpy(), want)
             vals = orc.bfp_unpack(want, shape, fmt).reshape(-1)
             assert np.array_equal(back[pad + shift:pad + shift + n].view(dtype).float().numpy(), vals)
+
+
+@pytest.mark.parametrize("shapes", [
+    [(32, 4096, 2), (1, 128, 2), (1, 128, 2), (1, 16, 0), (1, 128, 0)],                       # a decode step's inputs
+    [(33, 65, 4), (1, 1, 1), (31, 31, 2), (64, 1000, 1), (5, 7, 4), (200, 3, 2), (1, 1040, 0), (17, 129, 2)],
+    [(0, 5, 2), (257, 9, 1)],
+])
+def test_tilize_group(hip, dev, shapes):
+    """Several tensors in one launch against each by itself: every element size, ragged extents, copies, empty ones; from device and from
+    page-locked memory, at odd element offsets too."""
+    import ctypes
+
+    class Item(ctypes.Structure):
+        _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p), ("rows", ctypes.c_int64), ("cols", ctypes.c_int64), ("elem", ctypes.c_int)]
+
+    g = torch.Generator().manual_seed(len(shapes))
+    for pinned in (False, True):
+        items, want, got, keep = (Item * len(shapes))(), [], [], []
+        for i, (rows, cols, elem) in enumerate(shapes):
+            shift = 0 if elem == 0 else (i % 3) * elem      # rows that start at any element
+            raw = torch.randint(0, 256, (shift + rows * cols * max(elem, 1) + 64,), generator=g, dtype=torch.uint8)
+            raw = raw.pin_memory() if pinned else raw.to(dev)
+            keep.append(raw)
+            data = raw[shift:shift + rows * cols * max(elem, 1)].clone()
+            n = rows * cols if elem == 0 else (rows + 31) // 32 * 32 * ((cols + 31) // 32 * 32) * elem
+            out = torch.full((n,), 0xA5, dtype=torch.uint8, device=dev)
+            if elem and n:
+                ref, src = torch.full_like(out, 0x5A), data.to(dev)
+                hip.call("ttm_tilize", hip.ptr(src), hip.ptr(ref), 1, rows, cols, elem, hip.current_stream())
+            else:
+                ref = data.to(dev)
+            items[i] = Item(raw.data_ptr() + shift, out.data_ptr(), rows, cols, elem)
+            want.append(ref)
+            got.append(out)
+        hip.call("ttm_tilize_group", items, len(shapes), hip.current_stream())
+        torch.cuda.synchronize()
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
+
+
+def test_tilize_group_refuses(hip, dev):
+    import ctypes
+
+    class Item(ctypes.Structure):
+        _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p), ("rows", ctypes.c_int64), ("cols", ctypes.c_int64), ("elem", ctypes.c_int)]
+
+    t = torch.zeros(4096, dtype=torch.uint8, device=dev)
+    p = t.data_ptr()
+    for bad in (Item(p, p, 1, 8, 3), Item(p, p + 8, 1, 8, 2), Item(p + 1, p, 1, 8, 2), Item(p, p, 1, 24, 0), Item(None, p, 1, 16, 0), Item(p, p, -1, 8, 2), Item(p, p, 2, 16, 0)):
+        with pytest.raises(hip.TTMError):
+            hip.call("ttm_tilize_group", (Item * 1)(bad), 1, hip.current_stream())
+    with pytest.raises(hip.TTMError):
+        hip.call("ttm_tilize_group", (Item * 9)(), 9, hip.current_stream())

@@ -340,6 +340,87 @@ TTM_EXPORT int ttm_tilize(const void *src, void *dst, int64_t batch, int64_t row
   return run_layout<true>(src, dst, batch, rows, cols, elem_bytes, stream, "ttm_tilize");
 }
 
+// ---- several small tensors in one launch
+// A lane per 16-byte chunk of the tiled side (of a copy's bytes), chunks numbered along the rows, so that a wavefront reads 1 KiB of a row.  Bound
+// by the way to the host and back: five inputs of a decode step (256 KiB and four of a few bytes) in launches of their own 18 us one behind
+// the other, of which the large one 7.9; in one launch the small ones come along.
+struct TilizeGroup {
+  struct Item {
+    const uint8_t *src;
+    uint8_t *dst;
+    uint32_t rows, cols, elem, groups;   // workgroups of this and the items before it
+  } item[TTM_GROUP_MAX];
+};
+template <typename T>
+__device__ __forceinline__ void tilize_chunk(const TilizeGroup::Item &t, uint32_t i) {
+  constexpr uint32_t EPT = 16 / sizeof(T);
+  const uint32_t ct = (t.cols + 31) >> 5, across = ct * (32 / EPT), r = i / across, c = (i - r * across) * EPT;
+  if (r >= ((t.rows + 31) & ~31u)) return;
+  const T *src = (const T *)t.src + (uint64_t)r * t.cols + c;
+  union { T e[EPT]; u32x4 v; } x;
+  x.v = u32x4{0, 0, 0, 0};
+  if (r < t.rows) {
+    if (c + EPT <= t.cols && ((uintptr_t)src & 15) == 0) {
+      x.v = *(const u32x4 *)src;
+    } else {
+#pragma unroll
+      for (uint32_t k = 0; k < EPT; ++k) x.e[k] = c + k < t.cols ? src[k] : (T)0;
+    }
+  }
+  const uint64_t tile = (uint64_t)(r >> 5) * ct + (c >> 5);
+  *(u32x4 *)((T *)t.dst + tile * 1024 + (((r >> 4) & 1) * 2 + ((c >> 4) & 1)) * 256 + (r & 15) * 16 + (c & 15)) = x.v;
+}
+__global__ __launch_bounds__(256) void ttm_tilize_group_k(TilizeGroup p) {
+  uint32_t first = 0;
+  int i = 0;
+  while (blockIdx.x >= p.item[i].groups) first = p.item[i++].groups;   // uniform; the last item's is the size of the grid
+  const TilizeGroup::Item t = p.item[i];
+  const uint32_t chunk = (blockIdx.x - first) * 256 + threadIdx.x;
+  if (t.elem == 0) {
+    if (chunk < t.cols / 16) ((u32x4 *)t.dst)[chunk] = ((const u32x4 *)t.src)[chunk];
+  } else if (t.elem == 1) {
+    tilize_chunk<uint8_t>(t, chunk);
+  } else if (t.elem == 2) {
+    tilize_chunk<uint16_t>(t, chunk);
+  } else {
+    tilize_chunk<uint32_t>(t, chunk);
+  }
+}
+TTM_EXPORT int ttm_tilize_group(const ttm_tilize_item *items, int n, void *stream) {
+  TTM_REQUIRE(n >= 0 && n <= TTM_GROUP_MAX, "ttm_tilize_group: 0 to %d tensors (got %d)", TTM_GROUP_MAX, n);
+  TTM_REQUIRE(items || n == 0, "ttm_tilize_group: null pointer");
+  TilizeGroup p = {};
+  int64_t groups = 0;
+  int used = 0;
+  for (int i = 0; i < n; ++i) {
+    const ttm_tilize_item &t = items[i];
+    TTM_REQUIRE(t.elem_bytes == 0 || t.elem_bytes == 1 || t.elem_bytes == 2 || t.elem_bytes == 4, "ttm_tilize_group: unsupported element size %d", t.elem_bytes);
+    TTM_REQUIRE(t.rows >= 0 && t.cols >= 0, "ttm_tilize_group: negative dimension");
+    if (t.rows == 0 || t.cols == 0) continue;
+    TTM_REQUIRE(t.src && t.dst, "ttm_tilize_group: null pointer");
+    TTM_REQUIRE(((uintptr_t)t.dst & 15) == 0, "ttm_tilize_group: the destination must be 16-byte aligned");
+    TTM_REQUIRE(t.rows < (1 << 24) && t.cols < (1 << 30), "ttm_tilize_group: tensor %d is too large", i);
+    int64_t chunks;
+    if (t.elem_bytes == 0) {
+      TTM_REQUIRE(t.rows == 1 && t.cols % 16 == 0 && ((uintptr_t)t.src & 15) == 0, "ttm_tilize_group: a copy takes multiples of 16 bytes");
+      TTM_EXTENTS(copy_kernel, t.src, t.dst, (size_t)t.cols);
+      chunks = t.cols / 16;
+    } else {
+      TTM_REQUIRE(((uintptr_t)t.src & (uintptr_t)(t.elem_bytes - 1)) == 0, "ttm_tilize_group: the source is not aligned to its elements");
+      TTM_EXTENTS(tilize, t.src, t.dst, 1, t.rows, t.cols, t.elem_bytes);
+      chunks = ttm_round_up32(t.rows) * ttm_round_up32(t.cols) * t.elem_bytes / 16;
+    }
+    TTM_REQUIRE(chunks < (1ll << 31), "ttm_tilize_group: tensor %d is too large", i);   // the kernel counts them in 32 bits
+    groups += ttm_cdiv(chunks, 256);
+    TTM_REQUIRE(groups < (1ll << 31), "ttm_tilize_group: too large");
+    p.item[used++] = {(const uint8_t *)t.src, (uint8_t *)t.dst, (uint32_t)t.rows, (uint32_t)t.cols, (uint32_t)t.elem_bytes, (uint32_t)groups};
+  }
+  if (groups == 0) return TTM_OK;
+  hipLaunchKernelGGL(ttm_tilize_group_k, dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream, p);
+  TTM_LAUNCH_CHECK();
+  return TTM_OK;
+}
+
 TTM_EXPORT int ttm_untilize(const void *src, void *dst, int64_t batch, int64_t rows, int64_t cols,
                             int elem_bytes, void *stream) {
   TTM_EXTENTS(untilize, src, dst, batch, rows, cols, elem_bytes);

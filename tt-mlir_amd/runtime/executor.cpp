@@ -2247,15 +2247,24 @@ bool inDeviceMemory(const fb::Table &ref) { return layoutFromTensorRef(ref).stor
 void updateTraceInputSlots(const fb::Table &op, ProgramContext &ctx, std::vector<Tensor> &slots, bool deviceResidentOnly) {
   auto ins = op.tables(schema::CaptureOrExecuteTraceOp::f_inputs);
   TTRT_ASSERT(ins.size() == slots.size(), "capture_or_execute_trace: mismatched number of input slots");
+  UploadBatch batch(ctx.dev);   // the small host inputs of a step go up in one launch
+  std::vector<std::pair<std::uint32_t, std::uint64_t>> batched;   // slot, version
   for (std::uint32_t i = 0; i < ins.size(); ++i) {
     const bool resident = inDeviceMemory(ins[i]);
     if (deviceResidentOnly && !resident) continue;
     Tensor &in = ctx.get(ins[i], "trace input");
     if (in.handle->data.get() == slots[i].handle->data.get()) continue;
     if (in.handle->version == slots[i].handle->version) continue;
+    if (batch.add(in, slots[i])) {
+      batched.push_back({i, in.handle->version});
+      continue;
+    }
+    batch.flush();   // the staging block may be started over below
     overwriteTensor(ctx, slots[i], in, "trace input slot");
     slots[i].handle->version = in.handle->version;
   }
+  batch.flush();
+  for (const auto &b : batched) slots[b.first].handle->version = b.second;
 }
 void publishTraceOutputs(const fb::Table &op, ProgramContext &ctx, const std::vector<Tensor> &slots) {
   auto outs = op.tables(schema::CaptureOrExecuteTraceOp::f_outputs);

@@ -881,6 +881,45 @@ bool uploadInto(const Tensor &h, const Tensor &d) {
   return true;
 }
 
+UploadBatch::UploadBatch(const std::shared_ptr<DeviceState> &device) : dev(device), lock(device->mu) {}
+
+bool UploadBatch::add(const Tensor &h, const Tensor &d) {
+  const TensorImpl &s = *h.handle, &t = *d.handle;
+  if (s.storage != StorageType::Host || t.storage != StorageType::Device || t.device != dev || s.dtype != t.dtype || s.shape != t.shape) return false;
+  const bool copied = s.layout == t.layout;
+  if (!copied && (t.layout != TensorLayout::Tile || utils::isBlockFormatDataType(s.dtype) || utils::dataTypeElementSize(s.dtype) > 4 || dims3(s.shape).batch != 1))
+    return false;
+  if (s.bytes == 0 || s.bytes > kKernelCopyMax || !dev->kernelsReachHost) return false;
+  requireNotCapturing(dev, "a host to device transfer");
+  const size_t room = (s.bytes + 511) / 512 * 512;
+  if (items.size() == TTM_GROUP_MAX || dev->stagingHead + room > kStagingBytes) flush();
+  const void *p = stage(*dev, s.data.get(), s.bytes);
+  if (!p) return false;
+  items.push_back({d, p, s.shape, s.dtype, s.layout});
+  return true;
+}
+
+void UploadBatch::flush() {
+  if (items.empty()) return;
+  std::vector<Item> now;
+  now.swap(items);
+  if (now.size() == 1) {
+    const Item &i = now[0];
+    convertInOneLaunch(i.staged, i.layout, i.dtype, i.device.handle->data.get(), i.device.handle->layout, i.dtype, i.shape, dev->stream);
+  } else {
+    std::vector<ttm_tilize_item> list;
+    for (const Item &i : now) {
+      const Dims3 e = dims3(i.shape);
+      const bool copied = i.layout == i.device.handle->layout;
+      const size_t bytes = tensorBytes(i.shape, i.dtype, i.layout);
+      list.push_back({i.staged, i.device.handle->data.get(), copied ? 1 : e.rows, copied ? static_cast<std::int64_t>((bytes + 15) / 16 * 16) : e.cols,
+                      copied ? 0 : static_cast<int>(utils::dataTypeElementSize(i.dtype))});
+    }
+    TTM_CALL(ttm_tilize_group(list.data(), static_cast<int>(list.size()), dev->stream));
+  }
+  finishUpload(*dev);
+}
+
 Tensor uploadAs(const Tensor &h, const std::shared_ptr<DeviceState> &dev, TensorLayout layout, DataType dtype) {
   if (h.handle->layout != layout || h.handle->dtype != dtype) {
     Tensor d = makeDeviceTensor(dev, h.handle->shape, dtype, layout);

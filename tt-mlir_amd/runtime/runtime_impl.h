@@ -144,6 +144,28 @@ Tensor fetchAs(const Tensor &deviceTensor, TensorLayout layout, DataType dtype);
 // (and nothing done) when that takes more than one launch
 bool uploadInto(const Tensor &hostTensor, const Tensor &deviceTensor);
 
+// Small host tensors into device tensors of one handle, several in a launch.  Holds the handle's lock: between the copy into the staging
+// block and the launch that reads it nothing else may start the block over.
+class UploadBatch {
+public:
+  explicit UploadBatch(const std::shared_ptr<DeviceState> &device);
+  // As uploadInto, but left for the next flush(), which this calls when it has to; false (and nothing done) for what a group does not take.
+  bool add(const Tensor &hostTensor, const Tensor &deviceTensor);
+  void flush();
+
+private:
+  struct Item {
+    Tensor device;   // held until the launch
+    const void *staged;
+    std::vector<std::uint32_t> shape;
+    DataType dtype;
+    TensorLayout layout;   // of the staged values
+  };
+  std::shared_ptr<DeviceState> dev;
+  std::unique_lock<std::recursive_mutex> lock;
+  std::vector<Item> items;
+};
+
 Layout layoutFromTensorRef(const fb::Table &tensorRef);
 std::vector<std::uint32_t> shapeFromTensorRef(const fb::Table &tensorRef);
 
