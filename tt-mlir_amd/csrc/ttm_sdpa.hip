@@ -1306,8 +1306,21 @@ static int sdpa_entry(const void *q, const void *k, const void *v, const void *m
       // overlap the other's middle.  It pays for many short query-block columns (several sequences of up to ~3000 tokens,
       // 128 columns: [2..8, 32 / 8, 2048, 128] causal 5..13 % faster, [1, 32 / 8, 3000, 128] 12 %); a single sequence of 2048
       // tokens has only two blocks per CU, of very different length, and is 8 % slower that way, 4096 tokens 4 % slower,
-      // 8192 the same.  sdpa_variant 7 forces it, 8 keeps the eight-wavefront form.
-      const bool four = variant == 7 || (variant == 0 && D == 128 && blocks >= 3 * (int64_t)cus && nqb <= 24);
+      // 8192 the same.  Under a causal mask over as many keys as queries the lines are those of 2000 random shapes (batches of 1 .. 4, 8 to 32
+      // heads, 64 .. 4096 tokens, 64 and 128 columns, a quarter of them with a window of an eighth): the more blocks there are for a CU,
+      // and the less they differ in length, the more is won by two side by side; how far, follows the rounds that either form
+      // takes (chosen so, 0.5 % slower than the better one on average, before 3.3 %).  Eight / four wavefronts, us: [4, 32 / 8, 616, 128] 42.4 / 28.7, [4, 32 / 8, 559, 64] 30.9 / 22.5, [4, 32 / 8, 3145, 128] 435 / 362, one
+      // block column per matrix [1, 8 / 8, 66, 128] 8.3 / 7.4; not [1, 32 / 8, 1700, 128] (448 blocks in columns of 14) 38 / 43.  Under a window all blocks
+      // are as long: from one per CU on ([4, 16 / 4, 3300, 128] window 412 113 / 83, [1, 32 / 8, 1103, 64] window 137 18.1 / 15.0; [1, 32 / 8,
+      // 508, 128] window 63 10.9 / 12.2).  sdpa_variant 7 forces it, 8 keeps the eight-wavefront form.
+      bool four = D == 128 && blocks >= 3 * (int64_t)cus && nqb <= 24;
+      if (is_causal && Sq == Sk) {
+        const int64_t half_rounds = ttm_cdiv(2 * blocks, cus);
+        const int most = half_rounds <= 2 ? (D == 128 ? 2 : 1) : half_rounds == 3 ? 8 : half_rounds == 4 ? 4 : half_rounds == 5 ? 16 : half_rounds == 6 ? 8 :
+                         half_rounds == 7 ? 16 : half_rounds == 8 ? 14 : INT32_MAX;
+        four = p.lo_off < Sq / 2 ? blocks > cus : nqb <= most;
+      }
+      four = variant == 7 || (variant == 0 && four);
       const int ring = (int)D / 32 * (four ? 20480 : 40960);   // five stages of 32 or 64 keys of K and V
       const void *fn = four ? (D == 128 ? (const void *)ttm_sdpa_pipe_k<4, 1> : (const void *)ttm_sdpa_pipe_k<2, 1>)
                             : (D == 128 ? (const void *)ttm_sdpa_pipe_k<4, 2> : (const void *)ttm_sdpa_pipe_k<2, 2>);
