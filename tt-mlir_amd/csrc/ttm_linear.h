@@ -230,24 +230,33 @@ __device__ __forceinline__ void bfp4_rows(const u32x4 &x, int lane, uint32_t (&p
   quad_transpose(pk, lane);
 }
 // (257 - E) << 7 of the rows 2 i and 2 i + 1 in the halves of a word
+__device__ __forceinline__ uint32_t bfp4_exponent_pair(const u32x2 &ex, int i) {
+  return (0x01010101u - __builtin_amdgcn_perm(0u, i < 2 ? ex.x : ex.y, (i & 1) ? 0x0c030c02u : 0x0c010c00u)) << 7;
+}
 __device__ __forceinline__ void bfp4_exponents(const u32x2 &ex, uint32_t (&sub)[4]) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) sub[i] = (0x01010101u - __builtin_amdgcn_perm(0u, i < 2 ? ex.x : ex.y, (i & 1) ? 0x0c030c02u : 0x0c010c00u)) << 7;
+  for (int i = 0; i < 4; ++i) sub[i] = bfp4_exponent_pair(ex, i);
 }
 // The columns n and n + 2 (n = 0, 1) as bf16 pairs along k.  A magnitude of 1 .. 7 has four fractions and three exponents: v_perm looks the
 // two bytes of 0x7F80 + (its bf16 less that of 1) up for four elements at once, 0 for a magnitude of 0; less (257 - E) << 7, saturating at zero, that
 // is the bf16 of magnitude x 2^(E - 129) (exponents below 3 give zero or what bf16 holds of the value).  100 vector instructions for a block, where
 // two conversions to float per element took 205 and the two-term operand 100 with twice the matrix instructions.
-__device__ __forceinline__ void bfp4_columns(const uint32_t (&pk)[4], const uint32_t (&sub)[4], int n, u32x4 &w0, u32x4 &w2) {
+__device__ __forceinline__ void bfp4_pair(uint32_t pk, uint32_t sub, int n, uint32_t &w0, uint32_t &w2) {
   typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+  const uint32_t sel = (n ? pk >> 4 : pk) & 0x07070707u;
+  const uint32_t lo = __builtin_amdgcn_perm(0xE0C0A080u, 0x40008000u, sel), hi = __builtin_amdgcn_perm(0x80808080u, 0x80807F00u, sel);
+  const uint32_t a = __builtin_amdgcn_perm(hi, lo, 0x06020400u), b = __builtin_amdgcn_perm(hi, lo, 0x07030501u);
+  const u16x2 x = __builtin_elementwise_sub_sat(*(const u16x2 *)&a, *(const u16x2 *)&sub), y = __builtin_elementwise_sub_sat(*(const u16x2 *)&b, *(const u16x2 *)&sub);
+  w0 = *(const uint32_t *)&x | (n ? (pk & 0x00800080u) << 8 : (pk & 0x00080008u) << 12);
+  w2 = *(const uint32_t *)&y | (n ? pk & 0x80008000u : (pk & 0x08000800u) << 4);
+}
+__device__ __forceinline__ void bfp4_columns(const uint32_t (&pk)[4], const uint32_t (&sub)[4], int n, u32x4 &w0, u32x4 &w2) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const uint32_t sel = (n ? pk[i] >> 4 : pk[i]) & 0x07070707u;
-    const uint32_t lo = __builtin_amdgcn_perm(0xE0C0A080u, 0x40008000u, sel), hi = __builtin_amdgcn_perm(0x80808080u, 0x80807F00u, sel);
-    const uint32_t a = __builtin_amdgcn_perm(hi, lo, 0x06020400u), b = __builtin_amdgcn_perm(hi, lo, 0x07030501u);
-    const u16x2 x = __builtin_elementwise_sub_sat(*(const u16x2 *)&a, *(const u16x2 *)&sub[i]), y = __builtin_elementwise_sub_sat(*(const u16x2 *)&b, *(const u16x2 *)&sub[i]);
-    w0[i] = *(const uint32_t *)&x | (n ? (pk[i] & 0x00800080u) << 8 : (pk[i] & 0x00080008u) << 12);
-    w2[i] = *(const uint32_t *)&y | (n ? pk[i] & 0x80008000u : (pk[i] & 0x08000800u) << 4);
+    uint32_t a, b;
+    bfp4_pair(pk[i], sub[i], n, a, b);
+    w0[i] = a;
+    w2[i] = b;
   }
 }
 

@@ -950,12 +950,12 @@ __device__ __forceinline__ void linear_dma_block(const LinearArgs &p, int bid, i
   auto quarter = [&](int c, uint32_t raw_off, uint32_t w_off) {
     if constexpr (IMG) return;
     if (!converts) return;
-    float f[2][4];
+    if constexpr (WF == WF_BFP8) {
+      float f[2][4];
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int i = 2 * c + r;
-      uint32_t E = ((i < 4 ? exps.x : exps.y) >> (8 * (i & 3))) & 0xFFu;
-      if constexpr (WF == WF_BFP8) {
+      for (int r = 0; r < 2; ++r) {
+        const int i = 2 * c + r;
+        uint32_t E = ((i < 4 ? exps.x : exps.y) >> (8 * (i & 3))) & 0xFFu;
         E = max(E, 6u);   // rows below 2^-120, and the zeroed exponents of the k tail, dequantise to zero
         const float scale = __uint_as_float((E - 6u) << 23), nscale = -128.0f * scale;
         const uint32_t d = *(const uint32_t *)(lds + (rawRd ^ (i << 4)) + raw_off);
@@ -963,18 +963,20 @@ __device__ __forceinline__ void linear_dma_block(const LinearArgs &p, int bid, i
         const uint32_t t = (d ^ 0x80808080u ^ (sg - sb)) + sb;   // per byte: 128 + mag or 128 - mag
 #pragma unroll
         for (int b = 0; b < 4; ++b) f[r][b] = fmaf((float)((t >> (8 * b)) & 0xFFu), scale, nscale);
-      } else {
-        E = max(E, 2u);
-        const float scale = __uint_as_float((E - 2u) << 23), nscale = -8.0f * scale;
-        const uint32_t d = *(const uint16_t *)(lds + rawRd + i * 8 + raw_off);
-        const uint32_t sg = d & 0x8888u, sb = sg >> 3;
-        const uint32_t t = (d ^ 0x8888u ^ (sg - sb)) + sb;       // per nibble: 8 + mag or 8 - mag
+      }
 #pragma unroll
-        for (int b = 0; b < 4; ++b) f[r][b] = fmaf((float)((t >> (4 * b)) & 0xFu), scale, nscale);
+      for (int j = 0; j < 4; ++j) out[j][c] = pack_hi(f[0][j], f[1][j]);
+    } else {   // (the zeroed exponents of the k tail: at most 7 x 2^-129)
+      const uint8_t *raw = (const uint8_t *)lds + rawRd + c * 16 + raw_off;
+      const uint32_t pk = (uint32_t) * (const uint16_t *)raw | (uint32_t) * (const uint16_t *)(raw + 8) << 16, sub = bfp4_exponent_pair(exps, c);
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        uint32_t a, b;
+        bfp4_pair(pk, sub, n, a, b);
+        out[n][c] = a;
+        out[n + 2][c] = b;
       }
     }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) out[j][c] = pack_hi(f[0][j], f[1][j]);
     // the block is stored in two halves (k 0..3 after quarter 1, k 4..7 after quarter 3) to halve the store burst
     if (c == 1) {
 #pragma unroll
