@@ -1982,13 +1982,14 @@ static double other_us(const LinearArgs &a, bool measured = false) {
 // Whether the mid-size kernel's plan beats it.  4096 x 6144 bf16, image route / mid-size kernel: 520 rows 60.5 / 48.3 us, 661 rows 61.7 / 71.3;
 // 5120 x 2880 bfp8_b, 400 rows 38.6 / 28.1, 661 rows 52.3 / 49.6, 930 rows 56.0 / 54.1, 1600 rows 71.5 / 85.8.  Of 600 random shapes (33 .. 2048 rows,
 // weights of 512 .. 8192 x 512 .. 14336, all formats) it is taken at 473, on average in 0.60 of the other's time; it is the slower one at 3 of
-// them, by 4 .. 8 %, and is left out at 19 where it would be more than 5 % faster, at worst 29 % (787 rows x 7392 x 9202 bfp8_b).  The worst shape seen with
-// the lines as they are is 1952 rows x 3872 x 3298 bfp4_b, 90.7 us against 71 on the other route.  The models scatter by 5 .. 8 %: a line
-// that is right at one of those shapes is wrong at others.
+// them, by 4 .. 8 %, and is left out at 19 where it would be more than 5 % faster, at worst 29 % (787 rows x 7392 x 9202 bfp8_b).  The models scatter
+// by 5 .. 8 %: a line that is right at one of those shapes is wrong at others.
 template <int WF>
 static bool mid_beats_other(const LinearArgs &a, const MidPlan &plan) {
   constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
-  if (!BFP && a.Mt == 1) return plan.us < 0.93 * other_us<WF>(a);
+  // one row tile of bf16 weights: the kernel without shares of K only where K is short ([18, 1120] x [1120, 1258] 6.1 us, mid-size 7.1; [27, 1472] x [1472,
+  // 3552] 7.9 / 7.4, [13, 1856] x [1856, 3008] 9.7 / 8.5)
+  if (!BFP && a.Mt == 1) return plan.us < (a.Kt > 40 ? 1.1 : 0.93) * other_us<WF>(a);
   return (BFP ? 1.0 : 0.97) * plan.us < other_us<WF>(a, true);
 }
 

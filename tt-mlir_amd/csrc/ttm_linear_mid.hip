@@ -317,11 +317,15 @@ MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu, int max_slice
     for (const auto &k : kGated) consider(k.mt, k.wk, k.sums, 1.0, 1.0, k.chunk);
   } else {
     for (const auto &k : kPlain) {
-      // every column unit passes all activations by; from twice an XCD's L2 on the workgroups of 64 rows wait for them (1952 rows x 3872 x 3298 bfp4_b,
-      // 15 MB: 111 us, 77 by the rounds, with 128 rows 90 and 82; 1656 x 7136 x 1344 73 / 62)
-      if (k.wk == 4 && force < 1000 && (int64_t)p.Mt * p.Kt * 2048 > 8000000) continue;
+      // every column unit passes all activations by; from three times an XCD's L2 on the workgroups of 64 rows wait for them (1952 rows x 3872 x 3298 bfp4_b,
+      // 15 MB: 111 us, 77 by the rounds, with 128 rows 90 and 82; 1656 x 7136 x 1344 73 / 62; but 1292 x 3424 x 1376 bfp8_b, 8.8 MB, 28 / 31)
+      if (k.wk == 4 && force < 1000 && (int64_t)p.Mt * p.Kt * 2048 > 12000000) continue;
       consider(k.mt, k.wk, k.sums, k.whole, k.further, k.chunk[f]);
     }
+    // and from two rounds on, whose workgroups are not at the same k, their bytes bound the launch: 2048 rows x 4096 x 4096 bfp4_b, 16.8 MB for 64
+    // units, 102 us (84 by the rounds; the fused kernel 88), 2000 x 5000 x 3000 89 (83); in one round 512 x 14336 x 4096 takes 63
+    const double activations = (double)p.Mt * p.Kt * 2048.0;
+    if (activations > 10e6 && best.mt && (int64_t)units * ((p.Mt + best.mt - 1) / best.mt) * best.slices * p.plan_batch >= 2 * cus) best.us = std::max(best.us, 3.0 + units * activations * p.plan_batch / 10.5e6);
   }
   return best;
 }
