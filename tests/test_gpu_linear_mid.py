@@ -148,31 +148,90 @@ def test_infinite_activations_up_to_64_rows(hip, dev, wfmt_name, M):
             assert torch.equal(got[~hit], clean[~hit])
 
 
-@pytest.mark.parametrize("M,option", [(1, 0), (32, 0), (64, 8101), (100, 4201), (130, 8202), (128, 8401)])
-def test_bfp4_operands_of_every_exponent(hip, dev, M, option):
-    """Every nibble under every exponent as the kernels that keep weights in registers turn it into bf16: rows of the identity times such
-    weights give them back, exactly from exponent 3 on and, below (values under 2^-123), either as they are or as zero."""
-    K, N = 320, 96
-    g = torch.Generator().manual_seed(M)
-    kt, nt = K // 32, N // 32
-    tiles = torch.randint(0, 256, (kt, nt, 576), generator=g, dtype=torch.uint8)
-    tiles[:, :, :64] = (torch.arange(kt * nt * 64) % 254).reshape(kt, nt, 64).to(torch.uint8)
+def _bfp4_weights(tiles):
+    """float64 values of bfp4_b tiles [K / 32, N / 32, 576]."""
+    kt, nt = tiles.shape[:2]
     face = tiles[:, :, 64:].reshape(kt, nt, 2, 2, 16, 8)
     nibbles = torch.stack([face & 15, face >> 4], -1).reshape(kt, nt, 2, 2, 16, 16).double()
     value = torch.where(nibbles >= 8, 8 - nibbles, nibbles) * 2.0 ** (tiles[:, :, :64].reshape(kt, nt, 2, 2, 16, 1).double() - 129)
-    w = value.permute(0, 2, 4, 1, 3, 5).reshape(K, N)
-    rows = torch.randperm(K, generator=g)[:M]
-    a = torch.zeros(M, K, dtype=torch.bfloat16)
-    a[torch.arange(M), rows] = 1.0
+    return value.permute(0, 2, 4, 1, 3, 5).reshape(kt * 32, nt * 32)
+
+
+def _bfp4_product(hip, dev, a, tiles, options):
+    M, K, N = a.shape[0], a.shape[1], tiles.shape[1] * 32
     at, wd = tilize_dev(hip, a, dev), tiles.reshape(-1).to(dev)
     out = torch.full(((M + 31) // 32 * 32 * N,), float("nan"), dtype=torch.bfloat16, device=dev)
-    hip.set_option("linear_mid", option)
+    for name, v in options.items():
+        hip.set_option(name, v)
     try:
         hip.call("ttm_linear", hip.ptr(at), hip.BF16, hip.ptr(wd), hip.BFP4B, 0, None, hip.BF16, hip.TILE, hip.ptr(out), hip.BF16, 1, 1, M, N, K, 0,
                  hip.current_stream())
     finally:
-        hip.set_option("linear_mid", 0)
-    got, want = untilize_dev(hip, out, (M, N), dev).cpu().double(), w[rows]
-    tiny = want.abs() < 2.0 ** -123
-    assert torch.equal(got[~tiny], want[~tiny])
-    assert ((got - want).abs() <= want.abs() + 2.0 ** -133)[tiny].all()
+        for name in options:
+            hip.set_option(name, 0)
+    return untilize_dev(hip, out, (M, N), dev).cpu().double()
+
+
+# the kernels that keep weights in registers, the decode kernel and the mid-size one under every kind of plan; the fused kernel, whose last step of two
+# k-tiles reaches past an odd number of them, whole and in slices of K; and weights as images first
+BFP4_FORMS = [(1, {}), (32, {}), (32, {"linear_decode_wide": 2}), (32, {"linear_decode_split": 3}), (64, {"linear_mid": 8101}), (100, {"linear_mid": 4201}),
+              (130, {"linear_mid": 8202}), (128, {"linear_mid": 8401}), (352, {"linear_mid": 1, "linear_two_pass": 1}),
+              (352, {"linear_mid": 1, "linear_two_pass": 1, "linear_split_k": 2}), (352, {"linear_mid": 1, "linear_two_pass": 2})]
+
+
+@pytest.mark.parametrize("M,options", BFP4_FORMS)
+def test_bfp4_operands_of_every_exponent(hip, dev, M, options):
+    """Every nibble under every exponent as these kernels turn it into bf16: rows of the identity times such weights give them back, exactly from
+    exponent 3 on and below at most 2^-127 too small, or as zeros by way of images.  (Those take 254 for an overflow.)"""
+    K, N = 352, 96
+    images = options.get("linear_two_pass") == 2
+    g = torch.Generator().manual_seed(M)
+    tiles = torch.randint(0, 256, (K // 32, N // 32, 576), generator=g, dtype=torch.uint8)
+    tiles[:, :, :64] = (torch.arange(K // 32 * N // 32 * 64) % (254 if images else 255)).reshape(K // 32, N // 32, 64).to(torch.uint8)
+    w = _bfp4_weights(tiles)
+    small = tiles.clone()
+    small[:, :, 64:] = torch.where(tiles[:, :, :64].repeat_interleave(8, -1) < 3, tiles[:, :, 64:], 0)
+    small = _bfp4_weights(small)      # the weights below exponent 3, zeros elsewhere
+    for rows in torch.randperm(K, generator=g).split(M)[:12]:
+        a = torch.zeros(M, K, dtype=torch.bfloat16)
+        a[torch.arange(len(rows)), rows] = 1.0
+        got, want, below = _bfp4_product(hip, dev, a, tiles, options)[:len(rows)], w[rows], small[rows]
+        assert torch.equal(got[below == 0], want[below == 0])
+        if images:
+            assert not got[below != 0].any()
+        off = (want - got)[below != 0] * below[below != 0].sign()
+        assert (off >= 0).all() and (images or (off <= 2.0 ** -127).all())
+
+
+@pytest.mark.parametrize("options", [{}, {"linear_split_k": 2}])
+def test_bfp4_fused_ends_with_its_k_tiles(hip, dev, options):
+    """The last step of the fused kernel multiplies two k-tiles; where their number is odd the second is the last one again, under weights of
+    zero: with the smallest exponents and activations of 2^100 nothing of it shows."""
+    M, K, N = 352, 352, 96
+    tiles = torch.randint(0, 256, (K // 32, N // 32, 576), generator=torch.Generator().manual_seed(7), dtype=torch.uint8)
+    tiles[:, :, :64] = 3
+    a = torch.zeros(M, K, dtype=torch.bfloat16)
+    a[torch.arange(M), torch.arange(M)] = 2.0 ** 100
+    got = _bfp4_product(hip, dev, a, tiles, {"linear_mid": 1, "linear_two_pass": 1, **options})
+    assert torch.equal(got, _bfp4_weights(tiles) * 2.0 ** 100)
+
+
+@pytest.mark.parametrize("M,options", BFP4_FORMS[:-1])
+def test_bfp4_rows_of_exponent_255(hip, dev, M, options):
+    """A row of weights that had an infinity or a NaN, under activations of 1: magnitude 4 is an infinity again, 5 to 7 are NaN, the others values like
+    any."""
+    K, N, k = 352, 96, 331
+    tiles = torch.zeros(K // 32, N // 32, 576, dtype=torch.uint8)
+    tiles[:, :, :64] = 120
+    r = k % 32
+    for half in (0, 1):
+        f = (r >> 4) * 2 + half
+        tiles[k // 32, :, f * 16 + (r & 15)] = 255
+        tiles[k // 32, :, 64 + f * 128 + (r & 15) * 8:][:, :8] = torch.tensor([0x10 + 0x22 * j for j in range(8)], dtype=torch.uint8)   # 0 .. 15
+    want = _bfp4_weights(tiles)[k]
+    mag = want.abs() / 2.0 ** 126
+    want[mag == 4] *= float("inf")
+    want[mag > 4] = float("nan")
+    assert want.isinf().sum() == 12 and want.isnan().sum() == 36
+    got = _bfp4_product(hip, dev, torch.ones(M, K, dtype=torch.bfloat16), tiles, options)
+    assert torch.equal(got.nan_to_num(1.0, 2.0 ** 200, -2.0 ** 200), want.nan_to_num(1.0, 2.0 ** 200, -2.0 ** 200).expand(M, N))
