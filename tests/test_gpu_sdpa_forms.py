@@ -21,6 +21,12 @@ pytestmark = pytest.mark.gpu
     (4, 32, 8, 616, 128, -1, True),      # 2.5, columns of five
     (1, 32, 8, 1100, 64, 130, True),     # a window, more blocks than CUs
     (1, 32, 8, 500, 128, 60, False),     # a window, fewer
+    (1, 16, 4, 8200, 128, -1, False),    # more than 4096 tokens, too few matrices for nine half rounds of blocks
+    (1, 32, 32, 5125, 64, -1, False),    # enough of them, five blocks per CU
+    (1, 32, 8, 7000, 64, -1, False),     # just under seven
+    (2, 32, 8, 4200, 64, -1, True),      # 8.25
+    (1, 16, 4, 4120, 128, 1024, False),  # a window, two rounds
+    (2, 16, 4, 4120, 64, 500, True),     # a window, four
 ])
 def test_form_by_the_rule(hip, dev, B, H, Hkv, S, D, window, four):
     q, k, v = (datagen.randn((B, n, S, D), seed=i, dtype=torch.bfloat16) for i, n in enumerate((H, Hkv, Hkv)))

@@ -1319,6 +1319,11 @@ static int sdpa_entry(const void *q, const void *k, const void *v, const void *m
         const int most = half_rounds <= 2 ? (D == 128 ? 2 : 1) : half_rounds == 3 ? 8 : half_rounds == 4 ? 4 : half_rounds == 5 ? 16 : half_rounds == 6 ? 8 :
                          half_rounds == 7 ? 16 : half_rounds == 8 ? 14 : INT32_MAX;
         four = p.lo_off < Sq / 2 ? blocks > cus : nqb <= most;
+        // Longer ones (250 shapes of 4097 .. 16384 tokens): four wavefronts where 32 or more matrices share 256 CUs, from seven blocks per CU on ([1, 32 / 8,
+        // 9117, 64] 476 / 453, [2, 32 / 8, 11822, 128] 2277 / 2204; with 16 matrices [1, 16 / 4, 8405, 128] 300 / 370, [1, 16 / 4, 15393, 64] 639 / 721; with
+        // fewer blocks [1, 32 / 32, 5125, 128] 235 / 247); under a window of less than a quarter from three on ([2, 32 / 32, 8668, 128] window 1024 431 /
+        // 344; with two [1, 16 / 4, 4120, 128] window 1024 52 / 64)
+        if (nqb > 32) four = blocks >= (p.lo_off < Sq / 4 ? 3 : 7) * (int64_t)cus && (p.lo_off < Sq / 4 || (int64_t)Hq * B * 8 >= cus);
       }
       four = variant == 7 || (variant == 0 && four);
       const int ring = (int)D / 32 * (four ? 20480 : 40960);   // five stages of 32 or 64 keys of K and V
