@@ -245,6 +245,23 @@ def test_rowwise_lanes_by_width(hip, dev, dtype, rows, cols):
     assert bool(torch.isfinite(sums.float()).all())
 
 
+@pytest.mark.parametrize("rows,cols", [(2, 2048), (2, 4096), (2, 8192), (1024, 2048), (1024, 8192)])
+def test_sums_of_many_wavefronts_keep_their_precision(hip, dev, rows, cols):
+    """RMSNorm where one wavefront's sum of squares is 2^24 and every other's 1: added one behind the other they were lost, one rounding of 2^-24
+    for each.  A chain of four and the pairs of at most four such make 5 roundings, of which the square root halves the effect; square root, reciprocal and
+    product add one each (the mean over 2^n columns is exact): 5.5 in all."""
+    x = torch.zeros(rows, cols)
+    lanes = 1024 if cols > 4096 else 512 if cols > 2048 else 256    # of the kernel with a row per workgroup: 4 columns a lane
+    step = 256 if rows == 2 else 64                                 # four rows per workgroup: a wavefront has 64 columns of each
+    x[:, 0] = 4096.0
+    x[:, step:lanes * 4 if rows == 2 else lanes:step] = 1.0
+    xt, out = tilize_dev(hip, x, dev), torch.zeros((rows + 31) // 32 * 32 * cols, device=dev)
+    hip.call("ttm_rms_norm", hip.ptr(xt), None, hip.TILE, None, hip.TILE, hip.ptr(out), hip.F32, 1, rows, cols, 0.0, hip.current_stream())
+    got, x64 = untilize_dev(hip, out, (rows, cols), dev).cpu().double(), x.double()
+    want = x64 / x64.square().mean(-1, keepdim=True).sqrt()
+    assert torch.all((got - want).abs() <= 5.5 * 2.0 ** -24 * want)
+
+
 def _same_specials(got, want, what):
     """NaN in the same places, the same infinities, and equal values elsewhere up to `tol` bf16 / fp32 handling by the caller."""
     assert np.array_equal(np.isnan(got), np.isnan(want)), what + ": NaN in other places than in the oracle's result"
