@@ -580,7 +580,7 @@ __global__ __launch_bounds__(NT) TTM_MAX_WAVES((band_max_waves<MODE, ELEM, NK, N
     for (int k = 0; k < NK; ++k) {
       if constexpr (MODE == RW_RMSNORM && !WB_EARLY) {
         if (k % 4 == 0) {
-          __builtin_amdgcn_sched_barrier(0);   // the loads of one batch only: the scheduler would hoist all sixteen
+          __builtin_amdgcn_sched_barrier(0);   // the loads of one batch only: the scheduler would hoist all of them
           if (p.w) {
 #pragma unroll
             for (int u = 0; u < 4; ++u) wlate[u] = vec_load(p.w, p.w_tiled, min(k + u, NK - 1));
@@ -598,9 +598,6 @@ __global__ __launch_bounds__(NT) TTM_MAX_WAVES((band_max_waves<MODE, ELEM, NK, N
         float f[EPC];
         if constexpr (MODE == RW_RMSNORM) {
           float w[EPC], b[EPC];
-          // bf16: unpacked again from the raw chunk; without the empty asm the compiler keeps the floats of the first pass
-          // alive across the barrier, twice the registers of the raw chunks
-          if constexpr (ELEM == 2 && NK >= 16) asm volatile("" : "+v"(v[k]));
           unpack_vals<ELEM>(v[k], f);
           if (p.w) unpack_vals<ELEM>(WB_EARLY ? wraw[WB_EARLY ? k : 0] : wlate[k % 4], w);
           if (p.b) unpack_vals<ELEM>(WB_EARLY ? braw[WB_EARLY ? k : 0] : blate[k % 4], b);
