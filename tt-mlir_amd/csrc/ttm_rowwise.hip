@@ -468,7 +468,7 @@ __global__ __launch_bounds__(NT) TTM_MAX_WAVES((band_max_waves<MODE, ELEM, NK, N
   // unconditional (a run past the end repeats the last one and is masked where it is used): a branch around a load
   // makes the compiler wait for each load before it issues the next
   auto at = [&](int k) { return (const u32x4 *)(x + off_of(min(run_of(k), nruns - 1)) * ELEM); };
-  if (p.stream) {   // uniform; the empty asm keeps the compiler from merging the two forms of a load
+  if (REDUCE || p.stream) {   // uniform; the empty asm keeps the compiler from merging the two forms of a load
     asm volatile("");
 #pragma unroll
     for (int k = 0; k < NK; ++k) v[k] = __builtin_nontemporal_load(at(k));
@@ -828,7 +828,8 @@ static int launch_rowwise(const RowArgs &p, int dtype, int64_t trows, hipStream_
       const dim3 grid((unsigned)bands);
       RowArgs q = p;
       // Plain loads find what the producer left in the last-level cache (RMSNorm [8192, 4096] bf16 30.9 -> 23.1 us); an input of which little
-      // can be there is read past it (sum [8192, 8192] fp32 42.7 us, 47.6 plain)
+      // can be there is read past it, and that of a reduction always, whose short workgroups the choice itself delays (sum over twelve tensors, us: plain /
+      // past the caches, bf16 [8192, 2048] 7.6 / 7.1, [2048, 8192] 7.7 / 7.2, fp32 [4096, 2048] 7.4 / 6.9, [500, 8000] 4.9 / 5.5, [8192, 8192] 47.6 / 42.7)
       q.stream = (int64_t)p.ct * 1024 * elem * trows > 100000000;
 #define TTM_BAND(N, T) \
       do { if (dtype == TTM_BF16) hipLaunchKernelGGL((ttm_rowwise_band_k<MODE, 2, N, T>), grid, dim3(T), 0, s, q); \
