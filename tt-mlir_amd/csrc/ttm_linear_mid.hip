@@ -289,12 +289,15 @@ MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu, int max_slice
   // row tiles, shares of K; us of the sums of a round; how whole a last round counts (two or three of the smaller workgroups share a CU), and every
   // round behind the first; us per k-tile of a wavefront of bfp8_b / bfp4_b / bf16 weights (wavefronts of a SIMD share it, so they add up)
   static const struct { int mt, wk; double sums, whole, further, chunk[3]; } kPlain[] = {{2, 4, 1.57, 0.75, 0.87, {0.440, 0.356, 0.466}},
-                                                                                         {1, 8, 0.64, 0.87, 1.00, {0.297, 0.242, 0.335}},
+                                                                                         {1, 8, 0.64, 0.87, 1.00, {0.297, 0.242, 0.345}},
                                                                                          {2, 8, 2.15, 0.89, 1.25, {0.355, 0.285, 0.391}},
                                                                                          {4, 8, 4.74, 0.84, 1.17, {0.491, 0.414, 0.565}}};
   // the gated form: eight wavefronts, four shares of K of either matrix (36 shapes)
   static const struct { int mt, wk; double sums, chunk; } kGated[] = {{2, 4, 2.1, 0.44}, {4, 4, 4.0, 0.57}};
-  static const double kAlone[3] = {1.08, 1.0, 0.84};   // of a k-tile where a SIMD has one wavefront
+  static const double kAlone[3] = {1.08, 1.0, 0.80};   // of a k-tile where a SIMD has one wavefront
+  // us per slice of K beside the reduction's launch and traffic: with bf16 weights alone (1085 shapes of 1 .. 2048 rows: the plan picked is 0.36 % slower
+  // than the best one, without the term 0.69 %, [36, 2432] x [2432, 3424] 11.6 us in four slices, 9.8 in one)
+  static const double kSlice[3] = {0.0, 0.0, 0.3};
   const auto consider = [&](int mt, int wk, double sums, double whole, double further, double chunk) {
     const int blocks = (units + 7) / 8 * 8 * ((p.Mt + mt - 1) / mt) * p.plan_batch;   // a column unit's row blocks run on one XCD
     for (int slices = 1; slices <= (glu ? 1 : max_slices); slices *= 2) {
@@ -309,7 +312,7 @@ MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu, int max_slice
       double us;
       if (glu) us = 3.3 + r * 2 * chunks * chunk + r * sums;
       else us = 3.0 + r * (wk / 4) * chunks * chunk * (wk == 4 && rounds == 1 ? kAlone[f] : 1.0) + (wk == 8 ? r : 0.5 + 0.5 * r) * sums;
-      if (slices > 1) us += 2.65 + (slices + 0.5) * (double)p.Mt * p.Nt * p.plan_batch * 4096.0 / 3.8e6;
+      if (slices > 1) us += 2.65 + kSlice[f] * slices + (slices + 0.5) * (double)p.Mt * p.Nt * p.plan_batch * 4096.0 / 3.8e6;
       if (us < best.us) { best.us = us; best.mt = mt; best.wk = wk; best.slices = slices; }
     }
   };
