@@ -1,6 +1,10 @@
 """call() and ptr() as compiled code (binding/py_call.cpp) against the ctypes functions they stand for: the same conversions, the same
 errors.  What an argument arrived as shows in the entry points' own messages; nothing is launched."""
 import ctypes
+import os
+import shutil
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -70,6 +74,52 @@ def test_ptr(hip):
         assert type(a) is type(b) and a.value == b.value and a.nbytes == b.nbytes == t.nbytes
     assert outcome(hip.ptr, torch.zeros(4, 4).t()) == outcome(hip._ptr, torch.zeros(4, 4).t())
     assert outcome(hip.ptr, 5)[0] is AttributeError
+    assert hip.ptr(t=t).value == t.data_ptr() and outcome(hip.ptr)[0] is TypeError and outcome(hip.ptr, t, t)[0] is TypeError
+
+
+def test_keywords(hip):
+    assert outcome(lambda: hip.call(name="ttm_fill_u32"))[0] == outcome(lambda: hip._call(name="ttm_fill_u32"))[0]
+    assert outcome(lambda: hip.call("ttm_fill_u32", None, 0, 4, stream=None))[0] is TypeError
+
+
+@pytest.mark.parametrize("built", [False, True])
+def test_a_binding_built_after_the_import(hip, tmp_path, built):
+    """A process that imports the module, then builds, then calls: it uses the binding that is there by the first call, and without one makes its
+    calls through ctypes, with the check of extents."""
+    lib = tmp_path / "tt-mlir_amd" / "lib"
+    lib.mkdir(parents=True)
+    shutil.copy(os.path.join(hip._HERE, "hip.py"), lib.parent)
+    os.symlink(os.path.join(hip.ROOT, "include"), tmp_path / "include")
+    for f in os.listdir(os.path.dirname(hip.LIB_PATH)):
+        if not f.startswith("_ttm_call"):
+            os.symlink(os.path.join(os.path.dirname(hip.LIB_PATH), f), lib / f)
+    code = """
+import shutil, sys, torch
+sys.path.insert(0, %r)
+import hip
+assert hip._native is None
+if %r:
+    shutil.copy(%r, hip.CALL_PATH)
+hip.lib()
+assert (hip._native is not None) == %r and (type(hip.call) is type(len)) == %r
+t = torch.zeros(16)
+for on in (False, True):
+    hip.check_buffers(on)
+    try:
+        hip.call("ttm_tilize", hip.ptr(t), hip.ptr(t), 1, 32, 32, 4 if on else 3, None)
+    except hip.TTMError as e:
+        print(e)
+    else:
+        raise SystemExit("accepted")
+""" % (str(lib.parent), built, hip.CALL_PATH, built, built)
+    done = subprocess.run([sys.executable, "-c", code], env={**os.environ, "TTMLIR_AMD_CHECK_BUFFERS": "0"}, capture_output=True, text=True)
+    assert done.returncode == 0, done.stderr
+    assert "elem_bytes" in done.stdout and "row-major input" in done.stdout
+
+
+def test_the_binding_is_one_for_this_python(hip):
+    import sysconfig
+    assert hip.CALL_PATH.endswith(sysconfig.get_config_var("EXT_SUFFIX")) and type(hip.call) is type(len)
 
 
 def test_sizes_are_checked_before_the_call(hip):

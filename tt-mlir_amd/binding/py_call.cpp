@@ -1,7 +1,8 @@
 // The kernel library's entry points as Python calls: what hip.call() and hip.ptr() do, with the argument types known at compile time.
 // A call through ctypes converts each argument by a look-up and an object of its own and took 1.1 (8 arguments) to 2.1 us (18), a
 // device address 0.5 us: more than a small kernel.  Only ints, floats, None and ctypes.c_void_p objects are converted here; a
-// call with anything else in it (byref, arrays, bytes, a wrong number of arguments) goes to the ctypes function as it is.
+// call with anything else in it (byref, arrays, bytes, keywords, a wrong number of arguments) goes to the ctypes function as it is, and so does every
+// call while buffer extents are checked.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -16,7 +17,7 @@
 namespace {
 
 PyTypeObject *voidPointer = nullptr;   // ctypes.c_void_p
-PyObject *addressType = nullptr, *slowCall = nullptr, *slowPtr = nullptr, *raiseStatus = nullptr, *verify = nullptr;   // hip.py's
+PyObject *addressType = nullptr, *slowCall = nullptr, *slowPtr = nullptr, *raiseStatus = nullptr;   // hip.py's
 PyObject *entries = nullptr;           // {name: capsule of an Entry}
 PyObject *sContiguous, *sDataPtr, *sBytes;
 bool checking = false;
@@ -135,13 +136,13 @@ PyObject *bind(PyObject *, PyObject *addresses) {
   Py_RETURN_NONE;
 }
 
-// setup(c_void_p, address type, call, ptr, check, verify)
+// setup(c_void_p, address type, call, ptr, check)
 PyObject *setup(PyObject *, PyObject *args) {
-  PyObject *vp, *at, *sc, *sp, *rs, *ve;
-  if (!PyArg_ParseTuple(args, "O!OOOOO", &PyType_Type, &vp, &at, &sc, &sp, &rs, &ve)) return nullptr;
-  for (PyObject *o : {vp, at, sc, sp, rs, ve}) Py_INCREF(o);   // for good: the module lives as long as the process
+  PyObject *vp, *at, *sc, *sp, *rs;
+  if (!PyArg_ParseTuple(args, "O!OOOO", &PyType_Type, &vp, &at, &sc, &sp, &rs)) return nullptr;
+  for (PyObject *o : {vp, at, sc, sp, rs}) Py_INCREF(o);   // for good: the module lives as long as the process
   voidPointer = reinterpret_cast<PyTypeObject *>(vp);
-  addressType = at; slowCall = sc; slowPtr = sp; raiseStatus = rs; verify = ve;
+  addressType = at; slowCall = sc; slowPtr = sp; raiseStatus = rs;
   Py_RETURN_NONE;
 }
 
@@ -152,24 +153,12 @@ PyObject *check(PyObject *, PyObject *on) {
   Py_RETURN_NONE;
 }
 
-PyObject *call(PyObject *, PyObject *const *args, Py_ssize_t n) {
+PyObject *call(PyObject *, PyObject *const *args, Py_ssize_t n, PyObject *keywords) {
   if (!slowCall) {
     PyErr_SetString(PyExc_RuntimeError, "call before setup");
     return nullptr;
   }
-  if (n < 1) return PyObject_Vectorcall(slowCall, args, static_cast<size_t>(n), nullptr);
-  if (checking) {
-    PyObject *rest = PyTuple_New(n - 1);
-    if (!rest) return nullptr;
-    for (Py_ssize_t i = 1; i < n; ++i) {
-      Py_INCREF(args[i]);
-      PyTuple_SET_ITEM(rest, i - 1, args[i]);
-    }
-    PyObject *r = PyObject_CallFunctionObjArgs(verify, args[0], rest, nullptr);
-    Py_DECREF(rest);
-    if (!r) return nullptr;
-    Py_DECREF(r);
-  }
+  if (n < 1 || keywords || checking) return PyObject_Vectorcall(slowCall, args, static_cast<size_t>(n), keywords);
   PyObject *c = entries ? PyDict_GetItemWithError(entries, args[0]) : nullptr;
   if (!c && PyErr_Occurred()) PyErr_Clear();
   const Entry *e = c ? static_cast<const Entry *>(PyCapsule_GetPointer(c, nullptr)) : nullptr;
@@ -184,7 +173,13 @@ PyObject *call(PyObject *, PyObject *const *args, Py_ssize_t n) {
   Py_RETURN_NONE;
 }
 
-PyObject *ptr(PyObject *, PyObject *t) {
+PyObject *ptr(PyObject *, PyObject *const *args, Py_ssize_t n_args, PyObject *keywords) {
+  if (!slowPtr) {
+    PyErr_SetString(PyExc_RuntimeError, "ptr before setup");
+    return nullptr;
+  }
+  if (n_args != 1 || keywords) return PyObject_Vectorcall(slowPtr, args, static_cast<size_t>(n_args), keywords);
+  PyObject *t = args[0];
   PyObject *dense = PyObject_CallMethodNoArgs(t, sContiguous);
   if (!dense) return nullptr;
   const bool yes = dense == Py_True;
@@ -203,9 +198,10 @@ PyMethodDef methods[] = {
     {"names", names, METH_NOARGS, "The entry points that can be bound."},
     {"bind", bind, METH_O, nullptr},
     {"check", check, METH_O, nullptr},
-    {"call", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(call)), METH_FASTCALL,
+    {"call", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(call)), METH_FASTCALL | METH_KEYWORDS,
      "call(name, *args): the entry point `name` of the kernel library; raises TTMError if it fails."},
-    {"ptr", ptr, METH_O, "Device address of a torch tensor (must be contiguous); it carries the tensor's size for check_buffers."},
+    {"ptr", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(ptr)), METH_FASTCALL | METH_KEYWORDS,
+     "Device address of a torch tensor (must be contiguous); it carries the tensor's size for check_buffers."},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ttm_call", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

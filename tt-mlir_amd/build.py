@@ -2,7 +2,7 @@
 
   lib/libttmlir_amd_hip.so   gfx950 kernels + C ABI (csrc/*.hip, hipcc)
   lib/libttmlir_amd_rt.so    C++ host runtime in the tt::runtime style (runtime/*.cpp, g++)
-  lib/_ttm_call.so           the kernel library's entry points as Python calls (binding/py_call.cpp, g++)
+  lib/_ttm_call.<ABI>.so     the kernel library's entry points as Python calls (binding/py_call.cpp, g++)
 
 Usage: python build.py [--force] [--jobs N]
 """
@@ -26,7 +26,7 @@ INCLUDE = os.path.join(ROOT, "include")
 
 HIP_LIB = os.path.join(LIBDIR, "libttmlir_amd_hip.so")
 RT_LIB = os.path.join(LIBDIR, "libttmlir_amd_rt.so")
-CALL_LIB = os.path.join(LIBDIR, "_ttm_call.so")
+CALL_LIB = os.path.join(LIBDIR, "_ttm_call" + sysconfig.get_config_var("EXT_SUFFIX"))   # one per Python
 CALL_SRC = os.path.join(HERE, "binding", "py_call.cpp")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

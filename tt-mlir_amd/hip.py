@@ -6,13 +6,15 @@ plain integer addresses (e.g. torch_tensor.data_ptr()); streams are raw hipStrea
 import ctypes
 import os
 import re
+import sysconfig
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(_HERE)
 # TTMLIR_AMD_HIP_LIB names another build of the library (a kernel variant under measurement)
 LIB_PATH = os.environ.get("TTMLIR_AMD_HIP_LIB") or os.path.join(_HERE, "lib", "libttmlir_amd_hip.so")
 HEADER = os.path.join(ROOT, "include", "ttmlir_amd_hip.h")
-CALL_PATH = os.path.join(_HERE, "lib", "_ttm_call.so")   # call() and ptr() as compiled code (binding/py_call.cpp)
+# call() and ptr() as compiled code (binding/py_call.cpp), for this Python; without it they go through ctypes
+CALL_PATH = os.path.join(_HERE, "lib", "_ttm_call" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 F32, F16, BF16, BFP8B, BFP4B, U32, U16, U8, I32 = 0, 1, 2, 4, 6, 9, 10, 11, 12
 ROW_MAJOR, TILE = 0, 1
@@ -60,14 +62,12 @@ def lib():
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise TTMError("native kernel library missing: %s (run `python tt-mlir_amd/build.py`)" % LIB_PATH)
-        if _native is None:
-            raise TTMError("native binding missing: %s (run `python tt-mlir_amd/build.py`)" % CALL_PATH)
         l = ctypes.CDLL(LIB_PATH)
         for name, res, argtypes in declared_functions():
             fn = getattr(l, name)
             fn.restype, fn.argtypes = res, argtypes
         _lib = l
-        _native.bind({n: ctypes.cast(getattr(l, n), ctypes.c_void_p).value for n in _native.names()})
+        _use_native()   # what was built since the import, too
         if _check_buffers:   # switched on by the environment before the library was loaded: the library's own check goes with it
             l.ttm_set_option(b"check_extents", 1)
     return _lib
@@ -187,14 +187,16 @@ def _verify_extents(name, args):
 
 
 def _call(name, *args):
-    """call() through ctypes: before the library is loaded, and for arguments that py_call.cpp does not convert."""
+    """call() through ctypes: before the library is loaded, while extents are checked, and for arguments that py_call.cpp does not convert."""
+    if _check_buffers:
+        _verify_extents(name, args)
     status = getattr(_lib or lib(), name)(*args)
     if status:
         check(status, name)
 
 
 def _ptr(t):
-    """ptr() for tensors that are not contiguous."""
+    """Device address of a torch tensor (must be contiguous); it carries the tensor's size for check_buffers."""
     assert t.is_contiguous()
     p = _Ptr(t.data_ptr())
     p.nbytes = t.nbytes
@@ -209,16 +211,26 @@ def _load_native():
     loader = importlib.machinery.ExtensionFileLoader("_ttm_call", CALL_PATH)
     m = importlib.util.module_from_spec(importlib.util.spec_from_loader("_ttm_call", loader))
     loader.exec_module(m)
-    m.setup(ctypes.c_void_p, _Ptr, _call, _ptr, check, _verify_extents)
+    m.setup(ctypes.c_void_p, _Ptr, _call, _ptr, check)
     m.check(_check_buffers)
     return m
 
 
-_native = _load_native()
-if _native is not None:
-    call, ptr = _native.call, _native.ptr
-else:   # nothing is built yet: lib() says so
-    call, ptr = _call, _ptr
+_native = None
+call, ptr = _call, _ptr
+
+
+def _use_native():
+    global _native, call, ptr
+    if _native is None:
+        _native = _load_native()
+    if _native is not None:
+        call, ptr = _native.call, _native.ptr
+        if _lib is not None:
+            _native.bind({n: ctypes.cast(getattr(_lib, n), ctypes.c_void_p).value for n in _native.names()})
+
+
+_use_native()
 
 _raw_stream = _device_of_thread = None
 
