@@ -81,8 +81,10 @@ std::vector<Launch> *g_recording = nullptr;
 // TTMLIR_AMD_NULL_DEVICE_COMPUTE=0: arithmetic launches are counted and recorded but do nothing (programs at benchmark
 // sizes, where only the extents matter); copies and fills always run
 const bool g_compute = !(getenv("TTMLIR_AMD_NULL_DEVICE_COMPUTE") && std::string(getenv("TTMLIR_AMD_NULL_DEVICE_COMPUTE")) == "0");
+// option null_device_fail_in: n > 0 makes the n-th launch from there on fail once
 int launch(Launch f, bool cheap = false) {
   ++g_kernel_calls;
+  if (int &n = g_options["null_device_fail_in"]; n > 0 && --n == 0) return fail("a launch that was to fail");
   if (!g_compute && !cheap) f = [] {};
   if (g_recording) g_recording->push_back(std::move(f)); else f();
   return TTM_OK;

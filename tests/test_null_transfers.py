@@ -144,3 +144,82 @@ def test_transfers_on_both_routes(null_env, pageable):  # noqa: F811
     r = subprocess.run([sys.executable, "-m", "pytest", os.path.join(ROOT, "tests", "test_gpu_transfers.py"), "-q", "-m", "gpu", "-p", "no:cacheprovider",
                         "-k", skip], env=dict(null_env, TTMLIR_AMD_NULL_DEVICE_PAGEABLE=pageable), capture_output=True, text=True, timeout=600, cwd=ROOT)
     assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-1000:]
+
+
+TRACE = """
+class Builder(rt.ProgramBuilder):    # host tensors of [64, 96] are fp32, their slots bf16
+    def input(self, shape, dtype, layout=TL.Tile, storage=ST.Device):
+        return super().input(shape, DT.Float32 if storage == ST.Host and tuple(shape) == (64, 96) else dtype, layout, storage)
+small = [((33, 70), DT.BFloat16), ((1, 128), DT.Float32), ((17,), DT.Float32, TL.RowMajor), ((5, 7), DT.BFloat16)]
+large = [((450, 500 + i), DT.Float32) for i in range(11)]     # 0.9 MB each: more than the staging block holds
+args = small + large[:6] + [((3, 40, 33), DT.BFloat16), ((600, 1000), DT.Float32), ((64, 96), DT.BFloat16)] + large[6:] + small + [((2, 40), DT.Float32)]
+if ALONE: args = args[:1]
+args = [(a[0], a[1], False) + a[2:] for a in args]
+def body(pb, ids):
+    tiled = [pb.to_layout(i, TL.Tile) if len(a) > 3 else i for a, i in zip(args, ids)]
+    return [pb.binary(programs.BINARY["add"], t, t) for t in tiled]
+pb = Builder()
+emit = programs.add_traced(pb, "sums", args, body, [(a[0], rt.Layout(ST.Device, TL.Tile, a[1])) for a in args])
+pb.begin_program("sums")
+for y in emit(pb, [pb.input(a[0], a[1], TL.RowMajor, ST.Host) for a in args]):
+    pb.output(y)
+pb.end_program()
+binary = rt.Binary.load_from_memory(pb.finish())
+torch_type = {DT.BFloat16: torch.bfloat16, DT.Float32: torch.float32}
+def values(step):
+    g = torch.Generator().manual_seed(step)
+    return [torch.randn(a[0], generator=g).to(torch.float32 if a[0] == (64, 96) else torch_type[a[1]]) for a in args]
+def step(tensors):
+    return [rt.to_torch(rt.to_host(y, untilize=True)[0]) for y in rt.submit(device, binary, binary.get_num_programs() - 1, tensors)]
+def check(got, xs):
+    for a, y, x in zip(args, got, xs):
+        assert torch.equal(y, x.to(torch_type[a[1]]) * 2), a
+"""
+
+
+def test_host_inputs_of_a_traced_step(null_env):  # noqa: F811
+    """More of them than a launch takes and than the staging block holds at once, between them one with a change of type, a batch of matrices
+    and one over 1 MiB; then some of them new, none, and a step with one input."""
+    run(null_env, "ALONE = False" + TRACE + """
+assert len(args) == 23 and sum(a[0][0] * a[0][-1] * 4 for a in args if a[0][0] == 450) > 8 << 20
+for s in range(3):
+    xs = values(s)
+    rt.clear_stats()
+    check(step([rt.from_torch(x) for x in xs]), xs)
+    assert rt.get_stat("StagingBlockReused") >= 1
+kept = [rt.from_torch(x) for x in xs]
+check(step(kept), xs)
+check(step(kept), xs)
+for i in (0, 4, 10, 12, 22):
+    xs[i] = values(9)[i]
+    kept[i] = rt.from_torch(xs[i])
+    check(step(kept), xs)
+""")
+    run(null_env, "ALONE = True" + TRACE + """
+for s in range(3):
+    check(step([rt.from_torch(x) for x in values(s)]), values(s))
+""")
+
+
+def test_a_traced_step_that_failed_leaves_no_stale_input(null_env):  # noqa: F811
+    """A launch of a step's uploads fails; the step before it, given again, must not find the new values where the failed one had brought them."""
+    run(null_env, "ALONE = False" + TRACE + """
+import ctypes
+null = ctypes.CDLL(os.environ["TTMLIR_AMD_HIP_LIB"])
+before = values(1)
+kept = [rt.from_torch(x) for x in before]
+check(step(kept), before)
+check(step(kept), before)
+for n in range(1, 40):
+    null.ttm_set_option(b"null_device_fail_in", n)
+    try:
+        step([rt.from_torch(x) for x in values(1 + n)])
+    except RuntimeError as e:
+        assert "was to fail" in str(e)
+    else:
+        break
+    check(step(kept), before)
+assert 5 < n < 39
+null.ttm_set_option(b"null_device_fail_in", 0)
+check(step(kept), before)
+""")

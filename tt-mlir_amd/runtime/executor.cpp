@@ -2255,6 +2255,7 @@ void updateTraceInputSlots(const fb::Table &op, ProgramContext &ctx, std::vector
     Tensor &in = ctx.get(ins[i], "trace input");
     if (in.handle->data.get() == slots[i].handle->data.get()) continue;
     if (in.handle->version == slots[i].handle->version) continue;
+    slots[i].handle->version = nextTensorVersion();   // no input's, should the step fail between here and the end
     if (batch.add(in, slots[i])) {
       batched.push_back({i, in.handle->version});
       continue;
