@@ -1964,8 +1964,8 @@ static bool mid_allowed() {
 // kernel per row tile (block-float weights; [4096, 14336] bfp8_b at 48 rows 27 us against 19, [4096, 6144] 23.6 / 13.5,
 // [1024, 1024] 10.8 / 5.9: never the better one) or ttm_linear_small_k (bf16 weights, one row tile: one workgroup per 32 columns,
 // four wavefronts over K).
-// `measured`: what it takes rather than what the models say, which judge plans of one kernel against each other and are 3 (fused),
-// 18 (images of block-float weights) and 23 % (of bf16 weights) too high on average.
+// `measured`: what it takes rather than what the models say, which judge plans of one kernel against each other and are 3 (fused; bfp4_b 8: its
+// conversion by table look-up), 18 (images of block-float weights) and 23 % (of bf16 weights) too high where the line lies.
 template <int WF>
 static double other_us(const LinearArgs &a, bool measured = false) {
   constexpr bool BFP = WF == WF_BFP8 || WF == WF_BFP4;
@@ -1985,13 +1985,13 @@ static double other_us(const LinearArgs &a, bool measured = false) {
   const double first = 3.0 + (double)a.Kt * a.Nt * (a.w_batch ? a.plan_batch : 1) * ((WF == WF_BFP8 ? 1088.0 : WF == WF_BFP4 ? 576.0 : 2048.0) + 2048.0) / 5.5e6;
   const double gain = WF == WF_BFP4 ? (slices == 1 ? 0.22 : 0.08) : (slices == 1 ? 0.28 : 0.18);
   const double two = first + (1.0 - gain) * us;
-  if (measured) return !BFP ? 0.77 * two : us <= two ? 0.97 * us : 0.82 * two;
+  if (measured) return !BFP ? 0.77 * two : us <= two ? (WF == WF_BFP4 ? 0.92 : 0.97) * us : 0.82 * two;
   return BFP ? std::min(us, two) : two;
 }
 // Whether the mid-size kernel's plan beats it.  4096 x 6144 bf16, image route / mid-size kernel: 520 rows 60.5 / 48.3 us, 661 rows 61.7 / 71.3;
-// 5120 x 2880 bfp8_b, 400 rows 38.6 / 28.1, 661 rows 52.3 / 49.6, 930 rows 56.0 / 54.1, 1600 rows 71.5 / 85.8.  Of 600 random shapes (33 .. 2048 rows,
-// weights of 512 .. 8192 x 512 .. 14336, all formats) it is taken at 473, on average in 0.60 of the other's time; it is the slower one at 3 of
-// them, by 4 .. 8 %, and is left out at 19 where it would be more than 5 % faster, at worst 29 % (787 rows x 7392 x 9202 bfp8_b).  The models scatter
+// 5120 x 2880 bfp8_b, 400 rows 38.6 / 28.1, 661 rows 52.3 / 49.6, 930 rows 56.0 / 54.1, 1600 rows 71.5 / 85.8.  Of 1012 random shapes (33 .. 2048 rows,
+// weights of 512 .. 8192 x 512 .. 14336, all formats) it is taken at 758, on average in 0.57 of the other's time; it is the slower one at 4 of
+// them, by 3 .. 11 %, and is left out at 9 where it would be more than 5 % faster, at worst 13 % (546 rows x 7712 x 5216 bf16).  The models scatter
 // by 5 .. 8 %: a line that is right at one of those shapes is wrong at others.
 template <int WF>
 static bool mid_beats_other(const LinearArgs &a, const MidPlan &plan) {
@@ -1999,7 +1999,7 @@ static bool mid_beats_other(const LinearArgs &a, const MidPlan &plan) {
   // one row tile of bf16 weights: the kernel without shares of K only where K is short ([18, 1120] x [1120, 1258] 6.1 us, mid-size 7.1; [27, 1472] x [1472,
   // 3552] 7.9 / 7.4, [13, 1856] x [1856, 3008] 9.7 / 8.5)
   if (!BFP && a.Mt == 1) return plan.us < (a.Kt > 40 ? 1.1 : 0.93) * other_us<WF>(a);
-  return (BFP ? 1.0 : 0.97) * plan.us < other_us<WF>(a, true);
+  return (BFP ? 1.0 : 0.94) * plan.us < other_us<WF>(a, true);
 }
 
 template <int WF>

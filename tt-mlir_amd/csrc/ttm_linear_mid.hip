@@ -288,17 +288,22 @@ MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu, int max_slice
   const int f = wf == WF_BFP8 ? 0 : wf == WF_BFP4 ? 1 : 2;
   // row tiles, shares of K; us of the sums of a round; how whole a last round counts (two or three of the smaller workgroups share a CU), and every
   // round behind the first; us per k-tile of a wavefront of bfp8_b / bfp4_b / bf16 weights (wavefronts of a SIMD share it, so they add up)
-  static const struct { int mt, wk; double sums, whole, further, chunk[3]; } kPlain[] = {{2, 4, 1.57, 0.75, 0.87, {0.440, 0.356, 0.466}},
-                                                                                         {1, 8, 0.64, 0.87, 1.00, {0.297, 0.242, 0.345}},
-                                                                                         {2, 8, 2.15, 0.89, 1.25, {0.355, 0.285, 0.391}},
-                                                                                         {4, 8, 4.74, 0.84, 1.17, {0.491, 0.414, 0.565}}};
+  static const struct { int mt, wk; double sums, whole, further, chunk[3], drift; } kPlain[] = {{2, 4, 1.57, 0.75, 0.87, {0.440, 0.356, 0.466}, 0.75e-4},
+                                                                                                {1, 8, 0.64, 0.87, 1.00, {0.297, 0.242, 0.345}, 0.0},
+                                                                                                {2, 8, 2.15, 0.89, 1.25, {0.355, 0.285, 0.391}, 2.30e-4},
+                                                                                                {4, 8, 4.74, 0.84, 1.17, {0.491, 0.414, 0.565}, 0.95e-4}};
   // the gated form: eight wavefronts, four shares of K of either matrix (36 shapes)
   static const struct { int mt, wk; double sums, chunk; } kGated[] = {{2, 4, 2.1, 0.44}, {4, 4, 4.0, 0.57}};
   static const double kAlone[3] = {1.08, 1.0, 0.80};   // of a k-tile where a SIMD has one wavefront
   // us per slice of K beside the reduction's launch and traffic: with bf16 weights alone (1085 shapes of 1 .. 2048 rows: the plan picked is 0.36 % slower
   // than the best one, without the term 0.69 %, [36, 2432] x [2432, 3424] 11.6 us in four slices, 9.8 in one)
   static const double kSlice[3] = {0.0, 0.0, 0.3};
-  const auto consider = [&](int mt, int wk, double sums, double whole, double further, double chunk) {
+  // Every column unit passes all activations by; beyond 1024 rows the workgroups of a unit drift apart along K and out of their XCD's L2 the further, the more
+  // there are: kPlain's last figure (of the workgroups of 64 rows on half a CU per round) per row tile beyond 32 and MB of activations, times this.
+  // Over 834 shapes of 1000 .. 2048 rows the modelled time of the plan picked is 5 % rms off (6 / 9 / 6 % without, bfp8_b / bfp4_b / bf16) and the plan
+  // 0.13 % slower than the best one (0.31 %): 1900 rows x 3000 x 3400 bfp4_b 84 us with 64 rows, modelled at 62 before; 1952 x 3872 x 3298 111, 77 before.
+  static const double kDrift[3] = {1.0, 2.0, 0.9};
+  const auto consider = [&](int mt, int wk, double sums, double whole, double further, double chunk, double drift) {
     const int blocks = (units + 7) / 8 * 8 * ((p.Mt + mt - 1) / mt) * p.plan_batch;   // a column unit's row blocks run on one XCD
     for (int slices = 1; slices <= (glu ? 1 : max_slices); slices *= 2) {
       if (force >= 1000) {
@@ -312,23 +317,15 @@ MidPlan ttm_linear_plan_mid(const LinearArgs &p, int wf, bool glu, int max_slice
       double us;
       if (glu) us = 3.3 + r * 2 * chunks * chunk + r * sums;
       else us = 3.0 + r * (wk / 4) * chunks * chunk * (wk == 4 && rounds == 1 ? kAlone[f] : 1.0) + (wk == 8 ? r : 0.5 + 0.5 * r) * sums;
+      us *= 1 + drift * (wk == 4 ? (double)blocks * slices / cus : 1.0) * std::max(0, p.Mt - 32) * p.Mt * p.Kt * 2048e-6;
       if (slices > 1) us += 2.65 + kSlice[f] * slices + (slices + 0.5) * (double)p.Mt * p.Nt * p.plan_batch * 4096.0 / 3.8e6;
       if (us < best.us) { best.us = us; best.mt = mt; best.wk = wk; best.slices = slices; }
     }
   };
   if (glu) {
-    for (const auto &k : kGated) consider(k.mt, k.wk, k.sums, 1.0, 1.0, k.chunk);
+    for (const auto &k : kGated) consider(k.mt, k.wk, k.sums, 1.0, 1.0, k.chunk, 0.0);
   } else {
-    for (const auto &k : kPlain) {
-      // every column unit passes all activations by; from three times an XCD's L2 on the workgroups of 64 rows wait for them (1952 rows x 3872 x 3298 bfp4_b,
-      // 15 MB: 111 us, 77 by the rounds, with 128 rows 90 and 82; 1656 x 7136 x 1344 73 / 62; but 1292 x 3424 x 1376 bfp8_b, 8.8 MB, 28 / 31)
-      if (k.wk == 4 && force < 1000 && (int64_t)p.Mt * p.Kt * 2048 > 12000000) continue;
-      consider(k.mt, k.wk, k.sums, k.whole, k.further, k.chunk[f]);
-    }
-    // and from two rounds on, whose workgroups are not at the same k, their bytes bound the launch: 2048 rows x 4096 x 4096 bfp4_b, 16.8 MB for 64
-    // units, 102 us (84 by the rounds; the fused kernel 88), 2000 x 5000 x 3000 89 (83); in one round 512 x 14336 x 4096 takes 63
-    const double activations = (double)p.Mt * p.Kt * 2048.0;
-    if (activations > 10e6 && best.mt && (int64_t)units * ((p.Mt + best.mt - 1) / best.mt) * best.slices * p.plan_batch >= 2 * cus) best.us = std::max(best.us, 3.0 + units * activations * p.plan_batch / 10.5e6);
+    for (const auto &k : kPlain) consider(k.mt, k.wk, k.sums, k.whole, k.further, k.chunk[f], kDrift[f] * k.drift);
   }
   return best;
 }
