@@ -345,19 +345,19 @@ def make_workloads(torch, hip, datagen, dev, names):
 # what the same counters read for the plain copy kernel of known size (factors 1.9998 and 0.9999); these are measured
 # constants of the committed kernels, not computed here (profiles/bench_kernels_hbm_traffic_pmc.md holds the table and
 # the commands).  linear2048 is a two-pass launch: 181.9 MB for the pass that writes the weights as bf16 fragment images
-# plus 447.5 MB for the matrix pass (every XCD's L2 fetches the activations and its share of the images again).  Each
+# plus 447.4 MB for the matrix pass (every XCD's L2 fetches the activations and its share of the images again).  Each
 # figure belongs to one version of a kernel source file: it is reported only while that file still has the content it
 # was measured on (first 12 hex digits of its SHA-1), else `traffic` is null and `traffic_source` says so.
 MEASURED_TRAFFIC_BYTES = {
-    "linear2048": (629.4e6, "ttm_linear.hip"), "linear32": (65.6e6, "ttm_linear.hip"), "pack_bfp8": (340.5e6, "ttm_bfp.hip"),
-    "unpack_bfp8": (340.1e6, "ttm_bfp.hip"), "pack_bfp4": (306.2e6, "ttm_bfp.hip"), "unpack_bfp4": (306.6e6, "ttm_bfp.hip"),
-    "tilize_f32": (537.0e6, "ttm_layout.hip"), "untilize_f32": (536.9e6, "ttm_layout.hip"), "copy": (536.9e6, "ttm_layout.hip"),
-    "sdpa_decode32": (269.1e6, "ttm_decode.hip"), "sdpa2048": (42.3e6, "ttm_sdpa.hip"), "rmsnorm2048": (34.0e6, "ttm_rowwise.hip"),
-    "softmax65536": (1073.8e6, "ttm_rowwise.hip"), "reduce65536": (545.2e6, "ttm_rowwise.hip"), "silu_mul512": (44.2e6, "ttm_eltwise.hip"),
+    "linear2048": (629.3e6, "ttm_linear.hip"), "linear32": (65.6e6, "ttm_linear.hip"), "pack_bfp8": (340.5e6, "ttm_bfp.hip"),
+    "unpack_bfp8": (340.1e6, "ttm_bfp.hip"), "pack_bfp4": (306.2e6, "ttm_bfp.hip"), "unpack_bfp4": (306.5e6, "ttm_bfp.hip"),
+    "tilize_f32": (537.0e6, "ttm_layout.hip"), "untilize_f32": (537.0e6, "ttm_layout.hip"), "copy": (536.9e6, "ttm_layout.hip"),
+    "sdpa_decode32": (269.2e6, "ttm_decode.hip"), "sdpa2048": (42.3e6, "ttm_sdpa.hip"), "rmsnorm2048": (33.9e6, "ttm_rowwise.hip"),
+    "softmax65536": (1073.9e6, "ttm_rowwise.hip"), "reduce65536": (545.2e6, "ttm_rowwise.hip"), "silu_mul512": (44.1e6, "ttm_eltwise.hip"),
 }
-MEASURED_ON = {"ttm_linear.hip": ("8bd42722c72a",), "ttm_bfp.hip": ("decc4fec81ad",), "ttm_layout.hip": ("bfc2725cebb3",),
-               "ttm_decode.hip": ("2c7f2e8df2c6",), "ttm_rowwise.hip": ("0819544c7ff3",), "ttm_eltwise.hip": ("62019175607e",),
-               "ttm_sdpa.hip": ("a16ad50409ff",)}
+MEASURED_ON = {"ttm_linear.hip": ("f96f656ba81a",), "ttm_bfp.hip": ("a934d3881685",), "ttm_layout.hip": ("6459989b6a63",),
+               "ttm_decode.hip": ("dcd57b741f02",), "ttm_rowwise.hip": ("825be5fa49de",), "ttm_eltwise.hip": ("e47be3adccd1",),
+               "ttm_sdpa.hip": ("9a570461fc71",)}
 TRAFFIC_HOW = ("rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE (two runs), KiB per dispatch scaled by what the same counters "
                "read for the 256 MiB copy kernel; profiles/bench_kernels_hbm_traffic_pmc.md")
 

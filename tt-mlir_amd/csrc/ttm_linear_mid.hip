@@ -12,8 +12,8 @@
 // the LDS-direct kernels' blocks cost 12 k-steps (20 us) before and after theirs - what bounded every product below some
 // 10 GFLOP.  Bounds inside the loop, per 32 k of a wavefront: about 670 cycles of vector issue for the conversion of bfp8_b (bfp4_b: 400, bf16
 // weights: 64), 128 MT of the matrix core, 32 + 32 MT of L1; MT = 2 balances them for short launches, MT = 4 halves the weight
-// traffic and conversions where the row count fills it.  Vector issue and products mostly add up (512 rows x 14336 x 4096 bfp4_b, when its
-// conversion took 820: 106k and 57k of 160k cycles per SIMD; interleaving one column's products with the next one's conversion gave nothing).
+// traffic and conversions where the row count fills it.  Vector issue and products mostly add up (512 rows x 14336 x 4096: 74k and 57k of 150k
+// cycles per SIMD with bfp4_b, 99k and 57k of 169k with bfp8_b; interleaving one column's products with the next one's conversion gave nothing).
 // bfp4_b by table look-up: 74.9 -> 63.4 us there, 113 rows x 5515 x 5253 28.8 -> 21.2, 259 x 576 x 8256 12.5 -> 10.7.
 // =============================================================================================
 template <int WF, int MT, int WK, bool TT, bool GLU, class ARGS>
@@ -272,8 +272,8 @@ __global__ __launch_bounds__((GLU ? 2 : 1) * WK * 64) void ttm_linear_mid_k(ARGS
 // ---- the mid-size kernel's launch plan
 static int mid_units(const LinearArgs &p, bool glu) { return glu ? (p.gNt[0] + 1) / 2 : column_units(p, 2); }
 
-// The model was fitted to 2700 random shapes (33 .. 2048 rows, weights of 512 .. 8192 x 512 .. 14336, all formats) under every plan: 6 % rms
-// over 15000 timings, and the plan it picks is 0.4 % slower than the best one on average, 3 % at the 95th percentile (one without figures of their
+// The model was fitted to 2700 random shapes (33 .. 2048 rows, weights of 512 .. 8192 x 512 .. 14336, all formats) under every plan, two terms of it to
+// 1000 more: 5 % rms (bf16 8 %) for the plan it picks, which is 0.3 % slower than the best one on average, 2 % at the 95th percentile (one without figures of their
 // own for the formats and wavefront counts 2 - 3 %, 15 %: 113 rows x 5515 x 5253 bfp4_b 21.2 / 18.4 us, 64 x 4096 x 14336
 // bfp8_b 19.8 / 17.8).  us = 3.0 for launch, first loads and the last wavefronts; per round of workgroups the k-tiles that
 // the wavefronts of a SIMD take and the sums through LDS; for a split K the reduction's launch and its traffic.
