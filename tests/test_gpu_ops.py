@@ -219,7 +219,7 @@ def test_softmax_and_reduce_lastdim(hip, dev, orc, dtype, shape, rowwise_variant
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
-@pytest.mark.parametrize("rows,cols", [(1000, 1024), (993, 1030), (1000, 2056), (512, 2100), (480, 4096), (512, 4100), (1025, 4100), (97, 8192), (481, 8192), (1030, 8100), (8200, 3100)])
+@pytest.mark.parametrize("rows,cols", [(1000, 1024), (993, 1030), (1000, 2056), (512, 2100), (480, 4096), (512, 4100), (1025, 4100), (97, 8192), (481, 8192), (1030, 8100), (8200, 3100), (13000, 2048)])
 def test_rowwise_lanes_by_width(hip, dev, dtype, rows, cols):
     """Every width at which a row-wise launch takes more lanes per workgroup, either side of the row counts at which it takes four rows
     per workgroup, and an input read past the caches; against float64.  fp32: a sum of n terms in any tree of 256 to 1024 lanes and up

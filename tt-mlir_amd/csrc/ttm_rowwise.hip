@@ -831,9 +831,18 @@ static int launch_rowwise(const RowArgs &p, int dtype, int64_t trows, hipStream_
       // can be there is read past it, and that of a reduction always, whose short workgroups the choice itself delays (sum over twelve tensors, us: plain /
       // past the caches, bf16 [8192, 2048] 7.6 / 7.1, [2048, 8192] 7.7 / 7.2, fp32 [4096, 2048] 7.4 / 6.9, [500, 8000] 4.9 / 5.5, [8192, 8192] 47.6 / 42.7)
       q.stream = (int64_t)p.ct * 1024 * elem * trows > 100000000;
+      // LDS that only limits how many bands are on the way in a CU: 32 KiB each, three for reductions (65536 fp32 rows of 2048 86 -> 82 us, of bf16 4096
+      // 82.3 -> 81.3; narrower ones are faster without: bf16 3000 60.7, 64.1), two for fp32 softmax past the caches (192 -> 188; 8192 rows 20.9, 21.7)
+      size_t lds = 0;
+      if (nk == 8 && MODE != RW_RMSNORM && MODE != RW_SOFTMAX) lds = 50 << 10;
+      if (nk == 8 && MODE == RW_SOFTMAX && elem == 4 && q.stream) {
+        lds = 72 << 10;
+        const hipError_t e = hipFuncSetAttribute((const void *)ttm_rowwise_band_k<MODE, 4, 4, 512>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return ttm_set_error(TTM_ERR_HIP, "hipFuncSetAttribute(LDS %zu): %s", lds, hipGetErrorString(e));
+      }
 #define TTM_BAND(N, T) \
-      do { if (dtype == TTM_BF16) hipLaunchKernelGGL((ttm_rowwise_band_k<MODE, 2, N, T>), grid, dim3(T), 0, s, q); \
-           else hipLaunchKernelGGL((ttm_rowwise_band_k<MODE, 4, N, T>), grid, dim3(T), 0, s, q); } while (0)
+      do { if (dtype == TTM_BF16) hipLaunchKernelGGL((ttm_rowwise_band_k<MODE, 2, N, T>), grid, dim3(T), lds, s, q); \
+           else hipLaunchKernelGGL((ttm_rowwise_band_k<MODE, 4, N, T>), grid, dim3(T), lds, s, q); } while (0)
       // lanes by width: measured per mode at 500 to 8192 rows.  RMSNorm of 3 and 4 chunks: [6738, 1920] bf16 10.4 us, 11.4 with 256 lanes
       // (softmax 11.5 / 11.1); 9 to 16 chunks: softmax [4000, 6000] bf16 26.8 with 512 lanes, 31.3 with 1024 (843 rows 9.5 / 8.4, RMSNorm
       // 26.5 / 23.1)
