@@ -355,7 +355,7 @@ MEASURED_TRAFFIC_BYTES = {
     "sdpa_decode32": (269.2e6, "ttm_decode.hip"), "sdpa2048": (42.3e6, "ttm_sdpa.hip"), "rmsnorm2048": (33.9e6, "ttm_rowwise.hip"),
     "softmax65536": (1073.9e6, "ttm_rowwise.hip"), "reduce65536": (545.2e6, "ttm_rowwise.hip"), "silu_mul512": (44.1e6, "ttm_eltwise.hip"),
 }
-MEASURED_ON = {"ttm_linear.hip": ("f96f656ba81a",), "ttm_bfp.hip": ("a934d3881685",), "ttm_layout.hip": ("6459989b6a63",),
+MEASURED_ON = {"ttm_linear.hip": ("1117f8e465f1",), "ttm_bfp.hip": ("a934d3881685",), "ttm_layout.hip": ("6459989b6a63",),
                "ttm_decode.hip": ("dcd57b741f02",), "ttm_rowwise.hip": ("d26d372225a3",), "ttm_eltwise.hip": ("e47be3adccd1",),
                "ttm_sdpa.hip": ("9a570461fc71",)}
 TRAFFIC_HOW = ("rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE (two runs), KiB per dispatch scaled by what the same counters "

@@ -893,7 +893,7 @@ __device__ __forceinline__ void linear_dma_block(const LinearArgs &p, int bid, i
   const int kbase = blockIdx.y * p.k_slice, kt_end = min(p.Kt, kbase + p.k_slice);
   const int ksteps = (kt_end - kbase + 1) / 2;
   u32x2 exps = {0, 0}, exps_next = {0, 0};
-  uint32_t keep = 0, keep_next = 0, live = 0xFFFFFFFFu;   // live (bfp4_b): the mask that belongs to exps
+  uint32_t keep = 0, keep_next = 0;
   u32x4 fw[2][NTW], fa[2][MB], out[4];
 
   // instructions [i0, i1) of the four that stage this wavefront's 32 activation rows of step kt0
@@ -930,8 +930,7 @@ __device__ __forceinline__ void linear_dma_block(const LinearArgs &p, int bid, i
       lds_dma16(row, dmaW, lds0 + LDS_RAW + stage_off + (uint32_t)(2 * wave) * 512u);
     }
   };
-  // exponents of step kt0: the raw load and, separately, the k-tail mask (of bfp8_b's exponents, of bfp4_b's nibbles: a bfp4_b exponent of zero leaves
-  // magnitudes of 5 and more a few subnormal steps).
+  // exponents of step kt0: the raw load and, separately, the k-tail mask (zero exponents dequantise to zero weights, bfp4_b's all but: clear_tail).
   // The mask is applied when the value is taken into use; masking right behind the load would wait for it, and with
   // it for every LDS-direct load issued before.
   auto load_exps = [&](int kt0, uint32_t &keep) {
@@ -940,14 +939,6 @@ __device__ __forceinline__ void linear_dma_block(const LinearArgs &p, int bid, i
     const int kt = min(kt0 + ukt, p.Kt - 1);
     keep = kt0 + ukt >= kt_end ? 0u : 0xFFFFFFFFu;
     return *(const u32x2 *)(We + (int64_t)kt * NtW * W_TILE + offWe);
-  };
-  auto take_exps = [&](const u32x2 &e, uint32_t k) {
-    if constexpr (WF == WF_BFP4) {
-      exps = e;
-      live = k;
-    } else {
-      exps = u32x2{e.x & k, e.y & k};
-    }
   };
   auto fetch = [&](int s2, uint32_t so, u32x4 (&w)[NTW], u32x4 (&a)[MB]) {
 #pragma unroll
@@ -977,7 +968,7 @@ __device__ __forceinline__ void linear_dma_block(const LinearArgs &p, int bid, i
       for (int j = 0; j < 4; ++j) out[j][c] = pack_hi(f[0][j], f[1][j]);
     } else {
       const uint8_t *raw = (const uint8_t *)lds + rawRd + c * 16 + raw_off;
-      const uint32_t pk = ((uint32_t) * (const uint16_t *)raw | (uint32_t) * (const uint16_t *)(raw + 8) << 16) & live, sub = bfp4_exponent_pair(exps, c);
+      const uint32_t pk = (uint32_t) * (const uint16_t *)raw | (uint32_t) * (const uint16_t *)(raw + 8) << 16, sub = bfp4_exponent_pair(exps, c);
 #pragma unroll
       for (int n = 0; n < 2; ++n) {
         uint32_t a, b;
@@ -994,6 +985,16 @@ __device__ __forceinline__ void linear_dma_block(const LinearArgs &p, int bid, i
     if (c == 3) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) *(u32x2 *)(lds + wrW[j] + 8 + w_off) = u32x2{out[j][2], out[j][3]};
+    }
+  };
+  // bfp4_b: under an exponent of zero the table look-up leaves magnitudes of 5 and more a few subnormal steps, so a k-tile past the end is overwritten
+  // once it is converted (a mask over the nibbles of every step took 1 .. 7 % of the launch: 2048 rows x 14336 x 4096 215 -> 229 us)
+  auto clear_tail = [&](int step, uint32_t w_off) {
+    if constexpr (WF == WF_BFP4 && !IMG) {
+      if (kbase + 2 * step + ukt >= kt_end && converts) {   // wavefront-uniform
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *(u32x4 *)(lds + wrW[j] + w_off) = u32x4{0, 0, 0, 0};
+      }
     }
   };
   auto mfma_chunk = [&](int buf) {
@@ -1020,12 +1021,13 @@ __device__ __forceinline__ void linear_dma_block(const LinearArgs &p, int bid, i
   issue_raw(2, RAW_STAGE);
   exps = load_exps(0, keep);
   landed_barrier();
-  take_exps(exps, keep);
+  exps = u32x2{exps.x & keep, exps.y & keep};
 #pragma unroll
   for (int c = 0; c < 4; ++c) quarter(c, 0, 0);
+  clear_tail(0, 0);
   exps = load_exps(2, keep);
   landed_barrier();            // weights of step 0 visible, raw stage 0 free
-  take_exps(exps, keep);
+  exps = u32x2{exps.x & keep, exps.y & keep};
   issue_a(2, STAGE);
   if constexpr (IMG) issue_img(1, STAGE);
   issue_raw(4, 0);
@@ -1057,8 +1059,9 @@ __device__ __forceinline__ void linear_dma_block(const LinearArgs &p, int bid, i
       mfma_chunk(q & 1);
       __builtin_amdgcn_sched_barrier(0);
     }
+    clear_tail(ks + 1, NXT);
     landed_barrier();
-    take_exps(exps_next, keep_next);
+    exps = u32x2{exps_next.x & keep_next, exps_next.y & keep_next};
     // stage CUR of the activations and stage RNXT of the mantissas are free now
     exps_next = load_exps((ks + 3) * 2, keep_next);
     issue_raw((ks + 3) * 2, RNXT);
